@@ -1,5 +1,6 @@
-// bf16 MFMA GEMM for gfx950:  C[M][N] = epilogue(A[M][K] . W[N][K]^T)
-// with an int8-weight (W8A16) variant dequantised on the way into LDS.
+// bf16 MFMA GEMM for gfx950:  C[M][N] = epilogue(A[M][K] . W[N][K]^T), with an int8-weight (W8A16) variant
+// dequantised on the way into LDS: the C entry points, the choice of a kernel by shape, and the kernels for few tokens
+// and for int8 weights.  Many tokens with 16-bit weights -- where the work is -- run the kernel of gemm8.h.
 //
 // Both operands are K-contiguous, which is exactly the MFMA operand layout (a
 // lane holds 8 consecutive k of one row), so nothing is transposed.  The MFMA
@@ -19,12 +20,7 @@
 // remapped so that each XCD (own L2) works on a compact group of tiles.
 #include <algorithm>
 
-#include "common.h"
-
-// No implicit fused multiply-adds in this file: the epilogues reproduce the stock op chain's roundings (product
-// rounded to the io dtype, THEN the sum), and for fp16 -- which has native arithmetic -- the compiler would otherwise
-// contract "round(g * y) + r" into one v_fma_f16 and drop the product's rounding.  Wanted fmas are written as fmaf.
-#pragma clang fp contract(off)
+#include "gemm_common.h"
 
 // Tuning knobs: non-temporal hint on the output stores (one bit per epilogue kind: 1 none, 2 bias, 4 bias + SiLU,
 // 8 gated residual; measured on the 20-block step, all four on is best: 2.307 ms per block against 2.319-2.324 with
@@ -100,125 +96,6 @@ __global__ __launch_bounds__(256) void dequant_w8_kernel(const int8_t* __restric
   uint16_t* o = out + n * ldo + 16 * p;
   *reinterpret_cast<u32x4_t*>(o) = lo;
   *reinterpret_cast<u32x4_t*>(o + 8) = hi;
-}
-
-// Epilogue operands.  SANA_EPI_GATE_RES: C = res + gate[row / rows_per_gate] * (acc + bias), i.e. the
-// gated residual update of the block (x + gate * module(x)), with the reference's three roundings
-// (linear output, gate product, residual sum) reproduced in registers.
-struct EpiArgs {
-  const uint16_t* bias;  // [N] or null
-  const uint16_t* gate;  // [*, N] rows gate_stride apart, one row per rows_per_gate rows of C
-  const uint16_t* res;   // [M, N] with row stride ldr
-  int64_t ldr, gate_stride;
-  int rows_per_gate;
-  // SANA_EPI_QKV_STATE only: per-token-tile partial states, [B * heads][tiles_per_batch][33 * 32] fp32
-  float* part;
-  int q_cols, q_pad, heads, tiles_per_batch;  // q_cols = C (columns of the q region), q_pad = C rounded up to the tile
-};
-#define SANA_EPI_GATE_RES 3
-// (not part of the C ABI's epilogue codes) qkv projection of the linear attention with the k / v column tiles
-// contracted over their tokens in the epilogue instead of stored: see state_tile16
-#define SANA_EPI_QKV_STATE 4
-
-// Virtual concatenation of the A operand along k: columns [t*kc, (t+1)*kc) of the GEMM's A are columns
-// [0, kc) of the matrix whose row m is row m + t*stride of the buffer (a convolution over rows as one GEMM,
-// without materialising its im2col matrix).  rows = rows of the buffer that exist, counted from A: reads
-// past them return zero (the convolution's zero padding on that side).
-struct Taps {
-  int kc;          // columns per tap, a multiple of the k-tile
-  int64_t stride;  // rows between taps
-  int64_t rows;
-  // split-k launches (SPLIT, never together with taps): grid row z works on k-tiles
-  // [z*split_tiles + min(z, split_rem), ...) -- split_tiles of them, one more for z < split_rem
-  int split_tiles, split_rem;
-  // taps only, may be null: one byte per block of `stride` output rows; non-zero = the LAST tap reads zeros for
-  // these rows (a chunk boundary behind the block: the convolution's zero padding inside the buffer)
-  const unsigned char* zero_last;
-};
-
-// 8 outputs of one row: accumulator (+bias) -> io dtype, per the epilogue kind (everything except
-// the gated residual, which needs the row's residual and gate and is applied at store time).
-template <int EPI, typename T = BF16>
-__device__ __forceinline__ u32x4_t epi_pack8(const float* a, const float* bv) {
-  float v[8];
-#pragma unroll
-  for (int r = 0; r < 8; ++r) v[r] = EPI != SANA_EPI_NONE ? a[r] + bv[r] : a[r];
-  u32x4_t o;
-  o.x = pk16<T>(v[0], v[1]);
-  o.y = pk16<T>(v[2], v[3]);
-  o.z = pk16<T>(v[4], v[5]);
-  o.w = pk16<T>(v[6], v[7]);
-  if (EPI == SANA_EPI_BIAS_SILU) {
-    // The reference rounds the linear output to bf16 before the activation.  x * rcp(1 + 2^(-x log2 e)),
-    // written stage by stage over the eight values (and pinned that way): one value at a time is a
-    // chain of dependent instructions with two slow transcendentals, which a lone wave per SIMD
-    // cannot hide.
-    float x[8], t[8];
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      x[2 * p] = lo16<T>(o[p]);
-      x[2 * p + 1] = hi16<T>(o[p]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int r = 0; r < 8; ++r) t[r] = -1.44269504088896341f * x[r];
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int r = 0; r < 8; ++r) t[r] = __builtin_amdgcn_exp2f(t[r]);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int r = 0; r < 8; ++r) t[r] = 1.0f + t[r];
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int r = 0; r < 8; ++r) t[r] = __builtin_amdgcn_rcpf(t[r]);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int r = 0; r < 8; ++r) x[r] *= t[r];
-    __builtin_amdgcn_sched_barrier(0);
-    o.x = pk16<T>(x[0], x[1]);
-    o.y = pk16<T>(x[2], x[3]);
-    o.z = pk16<T>(x[4], x[5]);
-    o.w = pk16<T>(x[6], x[7]);
-  }
-  return o;
-}
-template <typename T = BF16>
-__device__ __forceinline__ uint32_t gate_res2(uint32_t y, uint32_t g, uint32_t r) {
-  const float t0 = rnd16<T>(lo16<T>(g) * lo16<T>(y)), t1 = rnd16<T>(hi16<T>(g) * hi16<T>(y));
-  return pk16<T>(lo16<T>(r) + t0, hi16<T>(r) + t1);
-}
-// y: 8 linear outputs (already rounded to bf16), g / r: the gate and residual values of the same 8 columns
-template <typename T = BF16>
-__device__ __forceinline__ u32x4_t gate_res8v(u32x4_t y, u32x4_t g, u32x4_t r) {
-  u32x4_t o;
-  o.x = gate_res2<T>(y.x, g.x, r.x);
-  o.y = gate_res2<T>(y.y, g.y, r.y);
-  o.z = gate_res2<T>(y.z, g.z, r.z);
-  o.w = gate_res2<T>(y.w, g.w, r.w);
-  return o;
-}
-// the same with the gate values already unpacked (they are the same for every row a lane handles)
-template <typename T = BF16>
-__device__ __forceinline__ u32x4_t gate_res8f(u32x4_t y, const float* g, u32x4_t r) {
-  u32x4_t o;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const uint32_t t = pk16<T>(g[2 * e] * lo16<T>(y[e]), g[2 * e + 1] * hi16<T>(y[e]));  // one convert rounds both
-    o[e] = pk16<T>(lo16<T>(r[e]) + lo16<T>(t), hi16<T>(r[e]) + hi16<T>(t));
-  }
-  return o;
-}
-// y: 8 linear outputs (already rounded to bf16) of row m, columns n..n+7
-template <typename T = BF16>
-__device__ __forceinline__ u32x4_t gate_res8(u32x4_t y, const EpiArgs& e, int m, int n) {
-  const u32x4_t g = *reinterpret_cast<const u32x4_t*>(e.gate + (int64_t)(m / e.rows_per_gate) * e.gate_stride + n);
-  const u32x4_t r = *reinterpret_cast<const u32x4_t*>(e.res + (int64_t)m * e.ldr + n);
-  u32x4_t o;
-  o.x = gate_res2<T>(y.x, g.x, r.x);
-  o.y = gate_res2<T>(y.y, g.y, r.y);
-  o.z = gate_res2<T>(y.z, g.z, r.z);
-  o.w = gate_res2<T>(y.w, g.w, r.w);
-  return o;
 }
 
 // Compiler-scheduled kernel, any K % 8 == 0 (int8: K % 16 == 0).  Workgroup tile 64*TT tokens x 64*TC channels,
@@ -414,113 +291,6 @@ __global__ __launch_bounds__(256, (TT * TC <= 4 ? 2 : 1)) void gemm_kernel(const
 }
 
 
-// Epilogue of a k / v column tile of the fused qkv projection (SANA_EPI_QKV_STATE, 256-wide tiles only).  The tile's
-// 256 weight rows are, per wave column wc, [K of head 4T+2wc | V of it | K of head 4T+2wc+1 | V of it] (32 rows
-// each; the caller lays the weight out that way, see sana_hip_qkv_state_rows), so lane group g = lane / 16 of a wave
-// holds, for its tokens lane % 16 + 16 j, all 32 channels of one of those four blocks.  Instead of storing k and v,
-// the wave contracts them over its 128 tokens: S[dv][dk] += v[n][dv] * relu(k[n][dk]) and ksum[dk] += relu(k[n][dk])
-// with v and k rounded to bf16 first (what the unfused path stores and reads back), products in fp32 on the MFMA.
-// The contraction index of v_mfma_f32_16x16x32_bf16 is the token, and which token sits in which k slot is free as
-// long as both operands agree: the 8 tokens a lane holds for one channel (j = 0 .. 7) ARE one operand fragment, it
-// only sits in the wrong lane (the lane is the token group, the MFMA wants the channel there), so it takes one trip
-// through the wave's LDS: written at [channel][token group ^ channel % 16] (16 bytes each, conflict-free both ways),
-// read back as [channel = lane % 16][token group 4 m + lane / 16] for the m-th MFMA of a chain of four.  The two
-// token halves of the workgroup are added through LDS and the sum goes to this token tile's slot of the partial
-// states, which a second kernel adds up in tile order (deterministic, no atomics).
-__device__ __forceinline__ void state_tile16(f32x4_t (&acc)[8][8], const u32x4_t (&bpk)[4], unsigned char* smem,
-                                             const EpiArgs& ep, int m0, int n0) {
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int wc = wave & 1, wt = wave >> 1;
-  const int fr = lane & 15, fg = lane >> 4;
-  __syncthreads();  // every wave is done with the operand tiles
-  unsigned char* stg = smem + wave * 32768;
-  // relu for the k blocks (fg even) as a packed signed-integer max on the bf16 pairs; int16 minimum = no-op for v
-  const uint32_t floor2 = (fg & 1) ? 0x80008000u : 0u;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const uint32_t bw0 = bpk[i >> 1][2 * (i & 1)], bw1 = bpk[i >> 1][2 * (i & 1) + 1];
-    const float b4[4] = {bf16_lo(bw0), bf16_hi(bw0), bf16_lo(bw1), bf16_hi(bw1)};  // channels 4 i + r of the lane's 32
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      u32x4_t o;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t pk = pack_bf16(acc[i][2 * e][r] + b4[r], acc[i][2 * e + 1][r] + b4[r]);
-        o[e] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(s16x2_t, pk),
-                                                                    __builtin_bit_cast(s16x2_t, floor2)));
-      }
-      const int row = 32 * fg + 4 * i + r;
-      *reinterpret_cast<u32x4_t*>(stg + row * 256 + ((fr ^ (row & 15)) << 4)) = o;
-    }
-  }
-  // wave-private LDS is in order: the reads below see the writes above.  hh: the wave's two heads.  The products
-  // are formed transposed (rows = dk, columns = dv), so that a lane ends with four consecutive dk of one dv:
-  // 16-byte stores into the [dv][dk] state.
-  f32x4_t S[2][2][2], Ks[2][2];  // S[hh][a][b]: dk 16 a + 4 fg + r, dv 16 b + fr;  Ks[hh][a]: dk 16 a + 4 fg + r
-#pragma unroll
-  for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) Ks[hh][b][r] = 0.f, S[hh][0][b][r] = 0.f, S[hh][1][b][r] = 0.f;
-    }
-  const u32x4_t ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
-#pragma unroll
-  for (int hh = 0; hh < 2; ++hh) {
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const int slot = ((4 * m + fg) ^ fr) << 4;
-      u32x4_t kf[2], vf[2];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        kf[b] = *reinterpret_cast<const u32x4_t*>(stg + (64 * hh + 16 * b + fr) * 256 + slot);
-        vf[b] = *reinterpret_cast<const u32x4_t*>(stg + (64 * hh + 32 + 16 * b + fr) * 256 + slot);
-      }
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        // (the builtin, not the main loop's asm statement: the compiler then places the wait states itself)
-        S[hh][a][0] = mfma_16x16x32_bf16(kf[a], vf[0], S[hh][a][0]);
-        S[hh][a][1] = mfma_16x16x32_bf16(kf[a], vf[1], S[hh][a][1]);
-        Ks[hh][a] = mfma_16x16x32_bf16(kf[a], ones, Ks[hh][a]);
-      }
-    }
-  }
-  // add the two token halves: wave wt = 1 hands its 48 values per lane to wave wt = 0 of the same channel half
-  f32x4_t* xch = reinterpret_cast<f32x4_t*>(stg) + lane;
-  if (wt == 1) {
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        xch[((hh * 2 + a) * 3 + 0) * 64] = S[hh][a][0];
-        xch[((hh * 2 + a) * 3 + 1) * 64] = S[hh][a][1];
-        xch[((hh * 2 + a) * 3 + 2) * 64] = Ks[hh][a];
-      }
-  }
-  __syncthreads();
-  if (wt == 0) {
-    const f32x4_t* oth = reinterpret_cast<const f32x4_t*>(smem + (wave + 2) * 32768) + lane;
-    const int tile_kv = (n0 - ep.q_pad) >> 8;
-    const int tile_m = m0 >> 8;
-    const int bi = tile_m / ep.tiles_per_batch, split = tile_m - bi * ep.tiles_per_batch;
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const int head = 4 * tile_kv + 2 * wc + hh;
-      if (head < ep.heads) {
-        float* o = ep.part + (((int64_t)bi * ep.heads + head) * ep.tiles_per_batch + split) * (33 * 32);
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-          const int dk0 = 16 * a + 4 * fg;
-#pragma unroll
-          for (int b = 0; b < 2; ++b)
-            *reinterpret_cast<f32x4_t*>(o + (16 * b + fr) * 32 + dk0) = S[hh][a][b] + oth[((hh * 2 + a) * 3 + b) * 64];
-          if (fr == 0) *reinterpret_cast<f32x4_t*>(o + 32 * 32 + dk0) = Ks[hh][a] + oth[((hh * 2 + a) * 3 + 2) * 64];
-        }
-      }
-    }
-  }
-}
-
 // Epilogue of the pipelined kernels.  acc[i][j][r] (MFMA 16x16 tiles: i = channel tile of the wave, j = token tile):
 // token m0 + wt*128 + 16*j + lane%16, channel n0 + wc*32*NI + 8*NI*(lane/16) + 4*i + r.  bpk: the lane's 8*NI bias
 // values, packed (the caller requests them ahead of its last k-tile so that their latency hides behind its MFMAs).
@@ -530,14 +300,6 @@ __device__ __forceinline__ void finish_tile16(f32x4_t (&acc)[2 * NI][8], const u
                                               int m0, int n0) {
   constexpr int NWT = 2 * NI;
   constexpr bool HAS_BIAS = EPI != SANA_EPI_NONE;
-  if constexpr (EPI == SANA_EPI_QKV_STATE) {
-    static_assert(NI == 4 && !SPLIT && !is_f16<T>, "the fused qkv projection runs 256-wide bf16 tiles, unsplit");
-    if (n0 >= ep.q_pad) {  // uniform per workgroup: a k / v tile
-      state_tile16(acc, bpk, smem, ep, m0, n0);
-      return;
-    }
-    N = ep.q_cols;  // a q tile: stored like any biased output, columns past C dropped
-  }
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int wc = wave & 1, wt = wave >> 1;
   const int fr = lane & 15, fg = lane >> 4;
@@ -641,7 +403,7 @@ __device__ __forceinline__ void finish_tile16(f32x4_t (&acc)[2 * NI][8], const u
     float a8[8];
 #pragma unroll
     for (int r = 0; r < 4; ++r) a8[r] = acc[2 * c][j][r], a8[4 + r] = acc[2 * c + 1][j][r];
-    const u32x4_t o = epi_pack8<(EPI == SANA_EPI_GATE_RES || EPI == SANA_EPI_QKV_STATE) ? SANA_EPI_BIAS : EPI, T>(a8, bv[c]);
+    const u32x4_t o = epi_pack8<EPI == SANA_EPI_GATE_RES ? SANA_EPI_BIAS : EPI, T>(a8, bv[c]);
     const int chunk = NI * fg + c;
     *reinterpret_cast<u32x4_t*>(stg + tok * 256 + ((chunk ^ (tok & 15)) << 4)) = o;
   };
@@ -733,8 +495,7 @@ __device__ __forceinline__ void finish_tile16(f32x4_t (&acc)[2 * NI][8], const u
 // SPLIT (split-k, for shapes with too few tiles to fill the chip): grid row z multiplies its own range of
 // k-tiles and stores the raw fp32 accumulators to C taken as float [gridDim.y][M][N]; splitk_epilogue_kernel
 // adds the ranges up in order and applies the epilogue.
-// TAPS: 0 = plain A operand, 1 = tap-concatenated A operand, 2 = the same with per-row-block zero_last flags.
-template <bool W8, int EPI, int NI, int TAPS = 0, bool SPLIT = false, typename T = BF16>
+template <bool W8, int EPI, int NI, bool SPLIT = false, typename T = BF16>
 __global__ __launch_bounds__(256) void gemm4_kernel(const uint16_t* __restrict__ A_, const void* __restrict__ Wv_,
                                                     const float* __restrict__ scale, const EpiArgs ep,
                                                     uint16_t* __restrict__ C, int M, int N, int K_, int64_t lda,
@@ -824,39 +585,9 @@ __global__ __launch_bounds__(256) void gemm4_kernel(const uint16_t* __restrict__
   // address is scalar, so a load costs one vector add.  The resource ends with the last valid row's
   // K-th element: rows past M / N and anything past the end of the matrix read as zero instead of
   // faulting (k chunks past K inside the matrix read the next row: they are never multiplied).
-  // (TAPS: the resource ends with the buffer's last existing row instead, so a tap that reaches past it is zero)
-  const int64_t a_bytes = TAPS ? (tp.rows > m0 ? ((tp.rows - m0 - 1) * lda + tp.kc) * 2 : 0)
-                               : ((int64_t)a_last * lda + K) * 2;
+  const int64_t a_bytes = ((int64_t)a_last * lda + K) * 2;
   const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(A + (int64_t)m0 * lda), 0, (int)a_bytes, 0x00020000);
-  // byte offset of k-tile k0 inside a row of A (TAPS: tap k0 / kc starts tp.stride rows further down)
-  const int tap_b = TAPS ? (int)(tp.stride * lda * 2) : 0;
-  auto a_koff = [&](int k0) { return TAPS ? (k0 / tp.kc) * tap_b + (k0 % tp.kc) * 2 : k0 * 2; };
-  int a_kb = 0, a_kin = 0;  // offset of the k-tile being requested, and its column inside the tap
-  // rows of this thread (bit q: row g_row + 32*q) whose last tap is zero padding.  While the k-tile being
-  // requested belongs to the last tap, those rows' vector offsets carry 2^31 -- outside the resource, so the
-  // loads return zeros -- at no cost in the loop: the per-row offsets live in registers and change with the tap.
-  uint32_t zlast = 0;
-  int voffq[8];
-  int a_tap = 0;
-  const int last_tap = TAPS ? K / tp.kc - 1 : 0;
-  if (TAPS == 2 && tp.zero_last) {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int r = m0 + (tid >> 3) + 32 * q;
-      if (r < M && tp.zero_last[r / tp.stride]) zlast |= 1u << q;
-    }
-  }
-  const int voff_a0 = ((tid >> 3) * (int)lda + 8 * (tid & 7)) * 2;  // the thread's (row, k chunk) inside the tile
-  auto poison = [&](bool last) {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) voffq[q] = voff_a0;
-    if (TAPS == 2 && last) {
-#pragma unroll
-      for (int q = 0; q < 8; ++q) voffq[q] = voff_a0 + (((zlast >> q) & 1u) ? (int)0x80000000u : 0);
-    }
-  };
-  poison(false);
   const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<char*>(static_cast<const char*>(Wv) + (int64_t)n0 * ldw * (W8 ? 1 : 2)), 0,
       (int)(((int64_t)w_last * ldw + K) * (W8 ? 1 : 2)), 0x00020000);
@@ -865,7 +596,7 @@ __global__ __launch_bounds__(256) void gemm4_kernel(const uint16_t* __restrict__
   const int step_a = 32 * (int)ulda * 2, step_w1 = (int)uldw * 2;
   auto gload = [&](int q, int k0) {
     if (q < 8) {
-      const int off = (TAPS == 2 ? voffq[q] : voff_a) + (q * step_a + (TAPS ? a_kb : k0 * 2));
+      const int off = voff_a + (q * step_a + k0 * 2);
       const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, off, 0, 0);
       rs[q] = __builtin_bit_cast(u32x4_t, v);
     } else {
@@ -912,10 +643,6 @@ __global__ __launch_bounds__(256) void gemm4_kernel(const uint16_t* __restrict__
   // prologue: k-tile 0 -> stage 0, k-tile 1 in flight
 #pragma unroll
   for (int q = 0; q < NQ; ++q) gload(q, 0);
-  if (TAPS) {
-    a_kb = a_koff(BK);
-    if (TAPS == 2 && zlast) poison(BK / tp.kc == last_tap);
-  }
 #pragma unroll
   for (int q = 0; q < (W8 ? 8 : NQ); ++q) lstore(q, 0);
   if (W8) {
@@ -924,12 +651,6 @@ __global__ __launch_bounds__(256) void gemm4_kernel(const uint16_t* __restrict__
   }
 #pragma unroll
   for (int q = 0; q < NQ; ++q) gload(q, BK);
-  if (TAPS) {
-    a_kb = a_koff(2 * BK);
-    a_kin = (2 * BK) % tp.kc;
-    a_tap = (2 * BK) / tp.kc;
-    if (TAPS == 2 && zlast) poison(a_tap == last_tap);
-  }
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < NFR; ++q) fread(smem, 0, 0, q);
@@ -996,16 +717,6 @@ __global__ __launch_bounds__(256) void gemm4_kernel(const uint16_t* __restrict__
             gload(8 + (((slot - 3) / PSTR) >> 3), (kt + 2) * BK);
         }
         SANA_G4_PIN();
-      }
-    }
-    if (TAPS) {  // the next iteration requests k-tile kt + 3
-      a_kin += BK;
-      a_kb += BK * 2;
-      if (a_kin >= tp.kc) {
-        a_kin -= tp.kc;
-        a_kb += tap_b - tp.kc * 2;
-        ++a_tap;
-        if (TAPS == 2 && zlast) poison(a_tap == last_tap);
       }
     }
   }
@@ -1094,25 +805,6 @@ int pick_ni(int M, int N) {
   return cost192 < cost256 ? 3 : 4;
 }
 
-// Channels to cover with 256-wide tiles when the rest goes to 192-wide ones in a second launch, or 0 when one width
-// for all of N is at least as good.  Costs in rounds of 256 workgroups: a 192-wide round counts 0.78 (3/4 of the
-// math, 4 % more operand traffic per MFMA), the second launch 0.05; the mix must win by 2 %.
-int mixed_split(int M, int N) {
-  const int64_t cu = compute_units(), tiles_t = (M + BT - 1) / BT;
-  auto rounds = [&](int64_t col_tiles) { return (double)((tiles_t * col_tiles + cu - 1) / cu); };
-  const double pure = std::min(rounds((N + 255) / 256), 0.78 * rounds((N + 191) / 192));
-  double best = pure * 0.98;
-  int best_wide = 0;
-  for (int a = 1; a * 256 < N; ++a) {
-    const double cost = rounds(a) + 0.78 * rounds((N - a * 256 + 191) / 192) + 0.05;
-    if (cost < best) {
-      best = cost;
-      best_wide = a * 256;
-    }
-  }
-  return best_wide;
-}
-
 // Which kernel, and whether K is split.  A workgroup's K loop is a latency chain whatever the grid: about
 // 1.1 us per k-tile for the 256-wide pipelined kernel, 0.8 us for the 128 x 128 one (a quarter of the math, but
 // the same load / LDS / barrier round trip).  A grid that covers the chip keeps the 256-wide kernel (throughput
@@ -1164,17 +856,16 @@ size_t split_bytes(const GemmPlan& pl, int M, int N) { return pl.S > 1 ? (size_t
 
 template <bool W8, int NI, typename T = BF16>
 int launch4(const uint16_t* a, const void* W, const float* scale, const EpiArgs& ep, uint16_t* c, int M, int N, int K,
-            int64_t lda, int64_t ldw, int64_t ldc, int epilogue, hipStream_t s, const Taps* taps = nullptr,
-            float* ws = nullptr, size_t ws_bytes = 0) {
+            int64_t lda, int64_t ldw, int64_t ldc, int epilogue, hipStream_t s, float* ws = nullptr, size_t ws_bytes = 0) {
   const int tiles_t = (M + BT - 1) / BT, tiles_c = (N + 64 * NI - 1) / (64 * NI);
   dim3 grid((unsigned)(tiles_t * tiles_c)), block(256);
   const Taps none = {0, 0, 0, 0, 0, nullptr};
-  if constexpr (NI != 2) {  // the 128-wide tile exists unsplit and without taps only
-    if (!taps && ws) {  // split-k when it pays and the caller's workspace holds the partial planes
+  if constexpr (NI != 2) {  // the 128-wide tile exists unsplit only
+    if (ws) {  // split-k when it pays and the caller's workspace holds the partial planes
       const GemmPlan pl = plan_gemm(M, N, K, W8);
       if (pl.S > 1 && ws_bytes >= split_bytes(pl, M, N)) {
         const Taps split = {0, 0, 0, pl.tiles, pl.rem, nullptr};
-        hipLaunchKernelGGL((gemm4_kernel<W8, SANA_EPI_NONE, NI, 0, true, T>), dim3(grid.x, (unsigned)pl.S), block, 0, s,
+        hipLaunchKernelGGL((gemm4_kernel<W8, SANA_EPI_NONE, NI, true, T>), dim3(grid.x, (unsigned)pl.S), block, 0, s,
                            a, W, scale, ep, reinterpret_cast<uint16_t*>(ws), M, N, K, lda, ldw, ldc, tiles_t, tiles_c,
                            split);
         if (hipGetLastError() != hipSuccess) return SANA_ERR_LAUNCH;
@@ -1193,21 +884,11 @@ int launch4(const uint16_t* a, const void* W, const float* scale, const EpiArgs&
         return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
       }
     }
-    if (taps) {  // only the bf16 gated-residual instance exists with taps
-      if (W8 || is_f16<T> || epilogue != SANA_EPI_GATE_RES) return SANA_ERR_ARG;
-      if (taps->zero_last)
-        hipLaunchKernelGGL((gemm4_kernel<false, SANA_EPI_GATE_RES, NI, 2>), grid, block, 0, s, a, W, scale, ep, c, M, N, K,
-                           lda, ldw, ldc, tiles_t, tiles_c, *taps);
-      else
-        hipLaunchKernelGGL((gemm4_kernel<false, SANA_EPI_GATE_RES, NI, 1>), grid, block, 0, s, a, W, scale, ep, c, M, N, K,
-                           lda, ldw, ldc, tiles_t, tiles_c, *taps);
-      return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
-    }
-  } else {
-    if (taps) return SANA_ERR_ARG;
   }
+  if constexpr (!W8 && NI != 2) return SANA_ERR_WORKSPACE;  // (16-bit operands unsplit: the many-token kernel)
+  else {
 #define SANA_LAUNCH4(EPI)                                                                                         \
-  hipLaunchKernelGGL((gemm4_kernel<W8, EPI, NI, 0, false, T>), grid, block, 0, s, a, W, scale, ep, c, M, N, K, lda, ldw, ldc, \
+  hipLaunchKernelGGL((gemm4_kernel<W8, EPI, NI, false, T>), grid, block, 0, s, a, W, scale, ep, c, M, N, K, lda, ldw, ldc, \
                      tiles_t, tiles_c, none)
   switch (epilogue) {
     case SANA_EPI_NONE: SANA_LAUNCH4(SANA_EPI_NONE); break;
@@ -1218,6 +899,7 @@ int launch4(const uint16_t* a, const void* W, const float* scale, const EpiArgs&
   }
 #undef SANA_LAUNCH4
   return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
+  }
 }
 
 template <bool W8, typename T = BF16>
@@ -1239,63 +921,93 @@ int launch_small(const uint16_t* a, const void* W, const float* scale, const Epi
   return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
 }
 
+// Channel tile of the many-token kernel, in units of 64.  One persistent workgroup per compute unit, so the grid runs in
+// rounds of 256 tiles; a round of 192-wide tiles takes 0.83 of one of 256-wide tiles and a round of 128-wide ones 0.62
+// (16384 x 2240 x 5600: 2.25 -> 3 rounds of 256 wide 328 us, 3 of 192 wide 305 us; 4096 x 2240 x 2240: 46.5 us for one
+// round of 256 wide, 43.5 of 192 wide, 56.5 for two of 128 wide).
+constexpr double kRound8[5] = {0, 0, 0.62, 0.83, 1.0};
+double cost8(int64_t tiles_t, int64_t N, int nb) {
+  const int64_t cu = compute_units();
+  return (double)((tiles_t * ((N + 64 * nb - 1) / (64 * nb)) + cu - 1) / cu) * kRound8[nb];
+}
+int pick_nb(int M, int N) {
+  const int64_t tiles_t = (M + BT - 1) / BT;
+  int best = 4;
+  for (int nb = 3; nb >= 2; --nb)
+    if (cost8(tiles_t, N, nb) < cost8(tiles_t, N, best)) best = nb;
+  return best;
+}
+// Channels to cover with 256-wide tiles when the rest goes to 192-wide ones in a second launch, or 0 when one width
+// for all of N is at least as good: the second launch costs 0.1 of a round, the mix must win by 1 % (32760 x 6720
+// tokens x channels: 14 rounds of 256 wide, 12 + 2 x 0.83 mixed).
+int mixed_split(int M, int N) {
+  const int64_t tiles_t = (M + BT - 1) / BT;
+  double best = std::min(cost8(tiles_t, N, 4), cost8(tiles_t, N, 3)) * 0.99;
+  int best_wide = 0;
+  for (int a = 1; a * 256 < N; ++a) {
+    const double cost = cost8(tiles_t, a * 256, 4) + cost8(tiles_t, N - a * 256, 3) + 0.1;
+    if (cost < best) {
+      best = cost;
+      best_wide = a * 256;
+    }
+  }
+  return best_wide;
+}
+
 template <bool W8, typename T = BF16>
 int launch(const void* A, const void* W, const float* scale, const EpiArgs& ep, void* C, int M, int N, int K,
-           int64_t lda, int64_t ldw, int64_t ldc, int epilogue, hipStream_t s, const Taps* taps = nullptr,
-           void* workspace = nullptr, size_t workspace_bytes = 0) {
+           int64_t lda, int64_t ldw, int64_t ldc, int epilogue, hipStream_t s, void* workspace = nullptr,
+           size_t workspace_bytes = 0) {
   const int64_t tiles_t = (M + BT - 1) / BT;
   if (tiles_t * ((N + 127) / 128) > (1 << 30)) return SANA_ERR_SHAPE;
   const uint16_t* a = static_cast<const uint16_t*>(A);
   uint16_t* c = static_cast<uint16_t*>(C);
-  if (!taps && plan_gemm(M, N, K, W8).small)
-    return launch_small<W8, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s);
-  if (K % 32 == 0 && K >= 64) {  // the pipelined kernel; the generic one takes any K % 8 == 0 (int8: K % 16 == 0)
-    float* ws = aligned16(workspace) ? static_cast<float*>(workspace) : nullptr;
-    // Mixed channel tiling: the first n_wide channels in 256-wide tiles, the rest in 192-wide ones, as two launches
-    // over disjoint column ranges of C, when that needs fewer rounds of the chip than either width alone (qkv at
-    // 16384 tokens, N = 6720: 27 x 256 is 7 rounds of 256 tiles, 24 x 256 + 3 x 192 is 6 rounds + one of 192-wide
-    // tiles, 6.8 round-equivalents).  Same k order per output: bit-identical to the single launch.
-    if (!taps && plan_gemm(M, N, K, W8).S == 1) {
+  const GemmPlan pl = plan_gemm(M, N, K, W8);
+  if (pl.small) return launch_small<W8, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s);
+  const bool pipelined = K % 32 == 0 && K >= 64;
+  float* ws = aligned16(workspace) ? static_cast<float*>(workspace) : nullptr;
+  // Few tokens, wide N (qkv of one 1024 px image: 4 x 35 tiles of 192 channels on 256 CUs): 128-wide tiles put
+  // half as much math behind every k-tile of the chain and fill more of the chip (4 x 53 workgroups: 37 -> 31 us).
+  // Taken when the 192-wide grid leaves a fifth of the CUs idle and the 128-wide one still fits.
+  const int64_t t128 = tiles_t * ((N + 127) / 128), t192 = tiles_t * ((N + 191) / 192);
+  const bool narrow = pipelined && t128 <= compute_units() && t192 < compute_units() * 4 / 5 && pl.S == 1;
+  if (narrow) return launch4<W8, 2, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s);
+  if constexpr (!W8) {
+    const bool split = pl.S > 1 && ws && workspace_bytes >= split_bytes(pl, M, N);
+    if (!split) {
+      const uint16_t* w = static_cast<const uint16_t*>(W);
       const int n_wide = mixed_split(M, N);
-      if (n_wide > 0) {
-        const int rc = launch4<W8, 4, T>(a, W, scale, ep, c, M, n_wide, K, lda, ldw, ldc, epilogue, s, nullptr, nullptr, 0);
-        if (rc != SANA_OK) return rc;
-        EpiArgs ep2 = ep;
-        if (ep2.bias) ep2.bias += n_wide;
-        if (ep2.gate) ep2.gate += n_wide;
-        if (ep2.res) ep2.res += n_wide;
-        return launch4<W8, 3, T>(a, static_cast<const char*>(W) + (int64_t)n_wide * ldw * (W8 ? 1 : 2),
-                              scale ? scale + n_wide : nullptr, ep2, c + n_wide, M, N - n_wide, K, lda, ldw, ldc, epilogue,
-                              s, nullptr, nullptr, 0);
-      }
+      if (n_wide == 0) return gemm8_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, pick_nb(M, N), nullptr, s);
+      const int rc = gemm8_launch(a, w, ep, c, M, n_wide, K, lda, ldw, ldc, epilogue, is_f16<T>, 4, nullptr, s);
+      if (rc != SANA_OK) return rc;
+      EpiArgs ep2 = ep;
+      if (ep2.bias) ep2.bias += n_wide;
+      if (ep2.gate) ep2.gate += n_wide;
+      if (ep2.res) ep2.res += n_wide;
+      return gemm8_launch(a, w + (int64_t)n_wide * ldw, ep2, c + n_wide, M, N - n_wide, K, lda, ldw, ldc, epilogue, is_f16<T>,
+                          3, nullptr, s);
     }
-    // Few tokens, wide N (qkv of one 1024 px image: 4 x 35 tiles of 192 channels on 256 CUs): 128-wide tiles put
-    // half as much math behind every k-tile of the chain and fill more of the chip (4 x 53 workgroups: 37 -> 31 us).
-    // Taken when the 192-wide grid leaves a fifth of the CUs idle and the 128-wide one still fits.
-    {
-      const int64_t t128 = tiles_t * ((N + 127) / 128), t192 = tiles_t * ((N + 191) / 192);
-      if (!taps && t128 <= compute_units() && t192 < compute_units() * 4 / 5 && plan_gemm(M, N, K, W8).S == 1)
-        return launch4<W8, 2, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, nullptr, nullptr, 0);
-    }
-    return pick_ni(M, N) == 3
-               ? launch4<W8, 3, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, taps, ws, workspace_bytes)
-               : launch4<W8, 4, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, taps, ws, workspace_bytes);
   }
-  if (taps) return SANA_ERR_SHAPE;
-  const int tiles_c = (N + BC - 1) / BC;
-  dim3 grid((unsigned)(tiles_t * tiles_c)), block(256);
+  if (pipelined)  // int8 weights, or split over k
+    return pick_ni(M, N) == 3 ? launch4<W8, 3, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, ws, workspace_bytes)
+                              : launch4<W8, 4, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, ws, workspace_bytes);
+  if constexpr (W8) {  // any K % 16 == 0
+    const int tiles_c = (N + BC - 1) / BC;
+    dim3 grid((unsigned)(tiles_t * tiles_c)), block(256);
 #define SANA_LAUNCH(EPI)                                                                                        \
-  hipLaunchKernelGGL((gemm_kernel<W8, EPI, 4, 4, T>), grid, block, 0, s, a, W, scale, ep, c, M, N, K, lda, ldw, ldc, \
+  hipLaunchKernelGGL((gemm_kernel<true, EPI, 4, 4, T>), grid, block, 0, s, a, W, scale, ep, c, M, N, K, lda, ldw, ldc, \
                      (int)tiles_t, tiles_c)
-  switch (epilogue) {
-    case SANA_EPI_NONE: SANA_LAUNCH(SANA_EPI_NONE); break;
-    case SANA_EPI_BIAS: SANA_LAUNCH(SANA_EPI_BIAS); break;
-    case SANA_EPI_BIAS_SILU: SANA_LAUNCH(SANA_EPI_BIAS_SILU); break;
-    case SANA_EPI_GATE_RES: SANA_LAUNCH(SANA_EPI_GATE_RES); break;
-    default: return SANA_ERR_ARG;
-  }
+    switch (epilogue) {
+      case SANA_EPI_NONE: SANA_LAUNCH(SANA_EPI_NONE); break;
+      case SANA_EPI_BIAS: SANA_LAUNCH(SANA_EPI_BIAS); break;
+      case SANA_EPI_BIAS_SILU: SANA_LAUNCH(SANA_EPI_BIAS_SILU); break;
+      case SANA_EPI_GATE_RES: SANA_LAUNCH(SANA_EPI_GATE_RES); break;
+      default: return SANA_ERR_ARG;
+    }
 #undef SANA_LAUNCH
-  return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
+    return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
+  }
+  return SANA_ERR_SHAPE;
 }
 
 int check_common(const void* A, const void* W, const void* bias, const void* C, int M, int N, int K, int64_t lda,
@@ -1384,7 +1096,7 @@ SANA_API int sana_hip_gemm_bf16(const void* A, const void* W, const void* bias, 
   const int rc = check_common(A, W, bias, C, M, N, K, lda, ldw, ldc, epilogue, 8, 8);
   if (rc != SANA_OK) return rc;
   return launch<false>(A, W, nullptr, plain_epi(bias), C, M, N, K, lda, ldw, ldc, epilogue,
-                       static_cast<hipStream_t>(stream), nullptr, workspace, workspace_bytes);
+                       static_cast<hipStream_t>(stream), workspace, workspace_bytes);
 }
 
 SANA_API int sana_hip_gemm_f16(const void* A, const void* W, const void* bias, void* C, int M, int N, int K,
@@ -1394,7 +1106,7 @@ SANA_API int sana_hip_gemm_f16(const void* A, const void* W, const void* bias, v
   const int rc = check_common(A, W, bias, C, M, N, K, lda, ldw, ldc, epilogue, 8, 8);
   if (rc != SANA_OK) return rc;
   return launch<false, F16>(A, W, nullptr, plain_epi(bias), C, M, N, K, lda, ldw, ldc, epilogue,
-                            static_cast<hipStream_t>(stream), nullptr, workspace, workspace_bytes);
+                            static_cast<hipStream_t>(stream), workspace, workspace_bytes);
 }
 
 SANA_API int sana_hip_gemm_w8a16(const void* A, const int8_t* Wq, const float* scale, const void* bias, void* C,
@@ -1404,7 +1116,7 @@ SANA_API int sana_hip_gemm_w8a16(const void* A, const int8_t* Wq, const float* s
   const int rc = check_common(A, Wq, bias, C, M, N, K, lda, ldw, ldc, epilogue, 16, 16);
   if (rc != SANA_OK) return rc;
   return launch<true>(A, Wq, scale, plain_epi(bias), C, M, N, K, lda, ldw, ldc, epilogue,
-                      static_cast<hipStream_t>(stream), nullptr, workspace, workspace_bytes);
+                      static_cast<hipStream_t>(stream), workspace, workspace_bytes);
 }
 
 SANA_API int sana_hip_gemm_gate_residual(const void* A, const void* W, const float* w8_scale, const void* bias,
@@ -1420,9 +1132,9 @@ SANA_API int sana_hip_gemm_gate_residual(const void* A, const void* W, const flo
   const EpiArgs e = {static_cast<const uint16_t*>(bias), static_cast<const uint16_t*>(gate),
                      static_cast<const uint16_t*>(residual), ldr, gate_stride, rows_per_gate, nullptr, 0, 0, 0, 0};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return w8 ? launch<true>(A, W, w8_scale, e, C, M, N, K, lda, ldw, ldc, SANA_EPI_GATE_RES, s, nullptr, workspace,
+  return w8 ? launch<true>(A, W, w8_scale, e, C, M, N, K, lda, ldw, ldc, SANA_EPI_GATE_RES, s, workspace,
                            workspace_bytes)
-            : launch<false>(A, W, nullptr, e, C, M, N, K, lda, ldw, ldc, SANA_EPI_GATE_RES, s, nullptr, workspace,
+            : launch<false>(A, W, nullptr, e, C, M, N, K, lda, ldw, ldc, SANA_EPI_GATE_RES, s, workspace,
                             workspace_bytes);
 }
 
@@ -1438,7 +1150,7 @@ SANA_API int sana_hip_gemm_gate_residual_f16(const void* A, const void* W, const
   const EpiArgs e = {static_cast<const uint16_t*>(bias), static_cast<const uint16_t*>(gate),
                      static_cast<const uint16_t*>(residual), ldr, gate_stride, rows_per_gate, nullptr, 0, 0, 0, 0};
   return launch<false, F16>(A, W, nullptr, e, C, M, N, K, lda, ldw, ldc, SANA_EPI_GATE_RES,
-                            static_cast<hipStream_t>(stream), nullptr, workspace, workspace_bytes);
+                            static_cast<hipStream_t>(stream), workspace, workspace_bytes);
 }
 
 SANA_API int sana_hip_tconv_residual(const void* X, const void* W, void* out, int M, int C, int taps,
@@ -1454,8 +1166,8 @@ SANA_API int sana_hip_tconv_residual(const void* X, const void* W, void* out, in
   const uint16_t* x = static_cast<const uint16_t*>(X);
   const EpiArgs e = {nullptr, nullptr, x + (taps / 2) * tap_rows * ldx, ldx, 0, M, nullptr, 0, 0, 0, 0};
   const Taps tp = {C, tap_rows, x_rows, 0, 0, zero_last_tap};
-  return launch<false>(X, W, nullptr, e, out, M, C, taps * C, ldx, ldw, ldo, SANA_EPI_GATE_RES,
-                       static_cast<hipStream_t>(stream), &tp);
+  return gemm8_launch(x, static_cast<const uint16_t*>(W), e, static_cast<uint16_t*>(out), M, C, taps * C, ldx, ldw, ldo,
+                      SANA_EPI_GATE_RES, false, std::max(3, pick_nb(M, C)), &tp, static_cast<hipStream_t>(stream));
 }
 
 SANA_API int sana_hip_dequant_w8(const int8_t* Wq, const float* scale, void* W, int N, int K, int64_t ldw,
@@ -1513,11 +1225,9 @@ SANA_API int sana_hip_gemm_qkv_state(const void* A, const void* W_tiled, const v
   hipStream_t s = static_cast<hipStream_t>(stream);
   const EpiArgs e = {static_cast<const uint16_t*>(bias_tiled), nullptr, nullptr, 0, 0, 1, static_cast<float*>(workspace),
                      C, qkv_state_q_pad(C), heads, (N + 255) / 256};
-  const Taps none = {0, 0, 0, 0, 0, nullptr};
-  hipLaunchKernelGGL((gemm4_kernel<false, SANA_EPI_QKV_STATE, 4>), dim3((unsigned)(tiles_t * tiles_c)), dim3(256), 0, s,
-                     static_cast<const uint16_t*>(A), W_tiled, static_cast<const float*>(nullptr), e,
-                     static_cast<uint16_t*>(Q), M, rows_t, C, lda, ldw, ldq, (int)tiles_t, (int)tiles_c, none);
-  if (hipGetLastError() != hipSuccess) return SANA_ERR_LAUNCH;
+  const int rc = gemm8_launch(static_cast<const uint16_t*>(A), static_cast<const uint16_t*>(W_tiled), e, static_cast<uint16_t*>(Q),
+                              M, rows_t, C, lda, ldw, ldq, SANA_EPI_QKV_STATE, false, 4, nullptr, s);
+  if (rc != SANA_OK) return rc;
   const int total = B * heads * 33 * 32, nsplit = (N + 255) / 256;
   if (nsplit > 16)
     hipLaunchKernelGGL(qkv_state_reduce_kernel<4>, dim3((unsigned)((total + 63) / 64)), dim3(256), 0, s,
