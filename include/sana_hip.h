@@ -248,7 +248,8 @@ int sana_hip_dwconv3x3_silu_gate(const void* u, const void* w, const void* bias,
  * K: the proj and point-conv GEMMs of a single 1024 px image) runs faster as a split-k GEMM -- K cut into
  * up to 8 ranges whose fp32 partial results go through the workspace and are summed in a fixed order by a
  * second kernel that applies the epilogue.  sana_hip_gemm_workspace_bytes(M, N, K) is the size that
- * needs (0: this shape is never split).  With workspace NULL, misaligned or smaller than that, the GEMM
+ * needs (0: this shape is never split); given it, the GEMM splits where that is expected to be faster than its best
+ * unsplit tiling.  With workspace NULL, misaligned or smaller than that, the GEMM
  * runs unsplit -- same result up to the fp32 summation order.  The plan depends on (M, N, K) only, so the
  * int8-weight GEMM and the gated-residual GEMM split the same way and stay bit-identical to this one.
  */
@@ -358,6 +359,10 @@ int sana_hip_add_layernorm_modulate(const void* x, const void* y, const void* sc
  */
 int sana_hip_dequant_w8(const int8_t* Wq, const float* scale, void* W, int N, int K,
                         int64_t ldw, int64_t ldo, void* stream);
+
+/* 1 if an int8-weight GEMM of this shape is expected to be faster as sana_hip_dequant_w8 followed by the bf16 GEMM (the
+ * bits are the same), 0 if sana_hip_gemm_w8a16 is.  A host-side rule on the sizes; nothing depends on it being followed. */
+int sana_hip_gemm_w8_expand(int M, int N, int K);
 
 /* Softmax attention of many queries over a short key set, bf16: the core of the block's cross-attention to the
  * text tokens (diffusion/model/nets/sana_blocks.py:69-98: F.scaled_dot_product_attention(q, k, v, attn_mask) at

@@ -1,6 +1,6 @@
 // bf16 MFMA GEMM for gfx950:  C[M][N] = epilogue(A[M][K] . W[N][K]^T), with an int8-weight (W8A16) variant
-// dequantised on the way into LDS: the C entry points, the choice of a kernel by shape, and the kernels for few tokens
-// and for int8 weights.  Many tokens with 16-bit weights -- where the work is -- run the kernel of gemm8.h.
+// dequantised on the way into LDS: the C entry points, the choice of a kernel by shape, and the kernels for int8
+// weights and for k split into ranges.  Unsplit 16-bit GEMMs run the kernels of gemm8.h (many tokens) and gemm_ring.h (few).
 //
 // Both operands are K-contiguous, which is exactly the MFMA operand layout (a
 // lane holds 8 consecutive k of one row), so nothing is transposed.  The MFMA
@@ -37,7 +37,6 @@ namespace sana {
 namespace {
 
 constexpr int BT = 256;   // tokens (rows of A / C) per workgroup
-constexpr int BC = 256;   // output channels (rows of W) per workgroup
 constexpr int BK = 64;
 constexpr int ROW_BYTES = BK * 2;            // 128
 constexpr int TILE_BYTES = 256 * ROW_BYTES;  // 32 KB per operand per stage
@@ -98,7 +97,7 @@ __global__ __launch_bounds__(256) void dequant_w8_kernel(const int8_t* __restric
   *reinterpret_cast<u32x4_t*>(o + 8) = hi;
 }
 
-// Compiler-scheduled kernel, any K % 8 == 0 (int8: K % 16 == 0).  Workgroup tile 64*TT tokens x 64*TC channels,
+// Compiler-scheduled kernel for int8 weights, any K % 16 == 0.  Workgroup tile 64*TT tokens x 64*TC channels,
 // four waves in 2x2, each TT x TC MFMA tiles.  <4, 4>: the 256 x 256 tile of the pipelined kernel, for the K
 // values that one does not take.  <2, 2>: 128 x 128 with 64 accumulators and 64 KB of LDS, two workgroups per
 // CU -- a quarter of the work per k-tile, so a much shorter latency chain for shapes whose 256-wide grid would
@@ -106,12 +105,13 @@ __global__ __launch_bounds__(256) void dequant_w8_kernel(const int8_t* __restric
 // (three register sets in rotation), because with so little math per k-tile the chain is otherwise one global
 // load latency per k-tile.  Every output sums its k products in the same order in all of these kernels, so
 // they agree bit for bit.
-template <bool W8, int EPI, int TT = 4, int TC = 4, typename T = BF16>
-__global__ __launch_bounds__(256, (TT * TC <= 4 ? 2 : 1)) void gemm_kernel(const uint16_t* __restrict__ A, const void* __restrict__ Wv,
-                                                   const float* __restrict__ scale, const EpiArgs ep,
-                                                   uint16_t* __restrict__ C,
+template <int EPI, int TT, int TC>
+__global__ __launch_bounds__(256, (TT * TC <= 4 ? 2 : 1)) void gemm_w8_kernel(const uint16_t* __restrict__ A,
+                                                   const int8_t* __restrict__ Wq, const float* __restrict__ scale,
+                                                   const EpiArgs ep, uint16_t* __restrict__ C,
                                                    int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
                                                    int tiles_t, int tiles_c) {
+  typedef BF16 T;
   constexpr int BT = 64 * TT, BC = 64 * TC;              // shadow the file-scope 256 x 256
   constexpr int A_BYTES = BT * ROW_BYTES, STAGE_BYTES = (BT + BC) * ROW_BYTES;
   __shared__ __attribute__((aligned(16))) unsigned char smem[2 * STAGE_BYTES];  // [stage][A | W]
@@ -138,30 +138,28 @@ __global__ __launch_bounds__(256, (TT * TC <= 4 ? 2 : 1)) void gemm_kernel(const
   // ---- global -> register staging
   // A tile: BT rows x 8 chunks(16 B); thread -> chunk tid%8, rows tid/8 + 32*i
   const int a_chunk = tid & 7, a_row = tid >> 3;
-  constexpr int NA = 2 * TT, NW = W8 ? TC : 2 * TC;
+  constexpr int NA = 2 * TT, NW = TC;
   constexpr int DEPTH = TT * TC <= 4 ? 3 : 1;  // k-tiles in flight in registers
   u32x4_t ra[DEPTH][NA];
-  // W tile bf16: same shape.  W8: BC rows x 4 chunks of 16 int8; thread -> chunk tid%4, rows tid/4 + 64*i
+  // W tile: BC rows x 4 chunks of 16 int8; thread -> chunk tid%4, rows tid/4 + 64*i
   u32x4_t rw[DEPTH][NW];
-  const int w_chunk = W8 ? (tid & 3) : (tid & 7), w_row = W8 ? (tid >> 2) : (tid >> 3);
+  const int w_chunk = tid & 3, w_row = tid >> 2;
 
   // Operand tiles are read with buffer loads, one resource per operand over the tile's valid rows (ending with
   // the last valid row's K-th element): rows past M / N fall outside it and read as zero, and a k chunk past K
   // gets an offset outside it -- no branches around the loads, so that several k-tiles can stay in flight.
   // (The whole offset is the vector offset: only that one is range-checked.)
   const int a_last = min(BT, M - m0) - 1, w_last = min(BC, N - n0) - 1;
-  constexpr int WB = W8 ? 1 : 2;  // bytes per weight
   const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(A + (int64_t)m0 * lda), 0, (int)(((int64_t)a_last * lda + K) * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<char*>(static_cast<const char*>(Wv) + (int64_t)n0 * ldw * WB), 0,
-      (int)(((int64_t)w_last * ldw + K) * WB), 0x00020000);
+      const_cast<int8_t*>(Wq + (int64_t)n0 * ldw), 0, (int)((int64_t)w_last * ldw + K), 0x00020000);
   const int idle_off = (int)0x80000000u;
   const int voff_a = (a_row * (int)lda + a_chunk * 8) * 2, step_a = 32 * (int)lda * 2;
-  const int voff_w = (w_row * (int)ldw + w_chunk * (W8 ? 16 : 8)) * WB, step_w = (W8 ? 64 : 32) * (int)ldw * WB;
+  const int voff_w = w_row * (int)ldw + w_chunk * 16, step_w = 64 * (int)ldw;
   auto load_tile = [&](int set, int k0) {  // k chunks past K load zeros
     const int off_a = k0 + a_chunk * 8 < K ? voff_a + k0 * 2 : idle_off;
-    const int off_w = k0 + w_chunk * (W8 ? 16 : 8) < K ? voff_w + k0 * WB : idle_off;
+    const int off_w = k0 + w_chunk * 16 < K ? voff_w + k0 : idle_off;
 #pragma unroll
     for (int i = 0; i < NA; ++i)
       ra[set][i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, off_a + i * step_a, 0, 0));
@@ -170,44 +168,36 @@ __global__ __launch_bounds__(256, (TT * TC <= 4 ? 2 : 1)) void gemm_kernel(const
       rw[set][i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, off_w + i * step_w, 0, 0));
   };
   float wscale[TC], woff[TC];
-  if (W8) {
 #pragma unroll
-    for (int i = 0; i < TC; ++i) {
-      const int n = n0 + w_row + 64 * i;
-      wscale[i] = n < N ? scale[n] : 0.f;
-      woff[i] = -128.f * wscale[i];
-    }
+  for (int i = 0; i < TC; ++i) {
+    const int n = n0 + w_row + 64 * i;
+    wscale[i] = n < N ? scale[n] : 0.f;
+    woff[i] = -128.f * wscale[i];
   }
   auto store_tile = [&](int set, int stage) {
     unsigned char* sa = smem + stage * STAGE_BYTES;
     unsigned char* sw = sa + A_BYTES;
 #pragma unroll
     for (int i = 0; i < NA; ++i) *reinterpret_cast<u32x4_t*>(sa + swz(a_row + 32 * i, a_chunk)) = ra[set][i];
-    if (W8) {
 #pragma unroll
-      for (int i = 0; i < NW; ++i) {
-        const int lrow = wrow_to_lds(w_row + 64 * i);
-        u32x4_t q = rw[set][i];
-        q.x ^= 0x80808080u;
-        q.y ^= 0x80808080u;
-        q.z ^= 0x80808080u;
-        q.w ^= 0x80808080u;
-        u32x4_t lo, hi;
-        lo.x = dequant2(q.x, 0, wscale[i], woff[i]);
-        lo.y = dequant2(q.x, 1, wscale[i], woff[i]);
-        lo.z = dequant2(q.y, 0, wscale[i], woff[i]);
-        lo.w = dequant2(q.y, 1, wscale[i], woff[i]);
-        hi.x = dequant2(q.z, 0, wscale[i], woff[i]);
-        hi.y = dequant2(q.z, 1, wscale[i], woff[i]);
-        hi.z = dequant2(q.w, 0, wscale[i], woff[i]);
-        hi.w = dequant2(q.w, 1, wscale[i], woff[i]);
-        *reinterpret_cast<u32x4_t*>(sw + swz(lrow, 2 * w_chunk)) = lo;
-        *reinterpret_cast<u32x4_t*>(sw + swz(lrow, 2 * w_chunk + 1)) = hi;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < NW; ++i)
-        *reinterpret_cast<u32x4_t*>(sw + swz(wrow_to_lds(w_row + 32 * i), w_chunk)) = rw[set][i];
+    for (int i = 0; i < NW; ++i) {
+      const int lrow = wrow_to_lds(w_row + 64 * i);
+      u32x4_t q = rw[set][i];
+      q.x ^= 0x80808080u;
+      q.y ^= 0x80808080u;
+      q.z ^= 0x80808080u;
+      q.w ^= 0x80808080u;
+      u32x4_t lo, hi;
+      lo.x = dequant2(q.x, 0, wscale[i], woff[i]);
+      lo.y = dequant2(q.x, 1, wscale[i], woff[i]);
+      lo.z = dequant2(q.y, 0, wscale[i], woff[i]);
+      lo.w = dequant2(q.y, 1, wscale[i], woff[i]);
+      hi.x = dequant2(q.z, 0, wscale[i], woff[i]);
+      hi.y = dequant2(q.z, 1, wscale[i], woff[i]);
+      hi.z = dequant2(q.w, 0, wscale[i], woff[i]);
+      hi.w = dequant2(q.w, 1, wscale[i], woff[i]);
+      *reinterpret_cast<u32x4_t*>(sw + swz(lrow, 2 * w_chunk)) = lo;
+      *reinterpret_cast<u32x4_t*>(sw + swz(lrow, 2 * w_chunk + 1)) = hi;
     }
   };
 
@@ -854,104 +844,116 @@ GemmPlan plan_gemm(int M, int N, int K, bool w8) {
 }
 size_t split_bytes(const GemmPlan& pl, int M, int N) { return pl.S > 1 ? (size_t)pl.S * M * N * sizeof(float) : 0; }
 
+// Time of an unsplit 16-bit GEMM in a given tile, us: ceil(K / 64) k-tiles per round of workgroups, at a rate per k-tile that
+// grows from `lone` (an eighth of the chip or less at work) to `full` (all of it: a compute unit takes 107 bytes/ns from
+// its L2 and about 50 while most of the chip misses it), plus launch, first loads and epilogue.  Fitted to 128 shapes
+// (64 .. 5000 tokens, the eight projections of the two image widths, weights cold): 8 - 13 % off, choice 2.5 % from the best.
+struct Tile16 {
+  int bm, bn;    // tokens, channels; 256 tokens: gemm8_kernel, else gemm_ring_kernel
+  int resident;  // workgroups on the chip at a time
+  double fixed, lone, full;
+};
+constexpr Tile16 kTiles16[] = {
+    {256, 128, 256, 3.8, 0.73, 0.85}, {256, 192, 256, 5.7, 0.86, 1.17}, {256, 256, 256, 6.1, 1.12, 1.37},
+    {64, 64, 512, 2.1, 0.255, 0.466}, {64, 128, 256, 2.0, 0.42, 0.42},  {128, 128, 256, 2.4, 0.50, 0.59},
+    {128, 160, 256, 4.2, 0.58, 0.68},
+};
+double cost16(const Tile16& t, int64_t M, int64_t N, int K) {
+  const int64_t n = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn), rounds = n / t.resident, rest = n % t.resident;
+  const double kt = (K + BK - 1) / BK, eighth = t.resident / 8;
+  double us = t.fixed + rounds * (kt * t.full + 0.5 * t.fixed);
+  if (rest) us += kt * (t.lone + (t.full - t.lone) * std::min(1.0, std::max(0.0, (rest - eighth) / (t.resident - eighth))));
+  return us;
+}
+struct Plan16 {
+  const Tile16* tile;
+  int n_wide;  // > 0: the first n_wide channels in 256 x 256 tiles, the rest in 256 x 192 ones, two launches
+  double us;
+};
+Plan16 plan16(int M, int N, int K) {
+  Plan16 p = {&kTiles16[0], 0, 1e30};
+  for (const Tile16& t : kTiles16) {
+    const double us = cost16(t, M, N, K);
+    if (us < p.us) p.tile = &t, p.us = us;
+  }
+  // two widths, where their last rounds fill better (32760 x 6720 tokens x channels: 14 rounds of 256 wide, 12 + 2 mixed)
+  const double single = p.us;
+  for (int a = 256; a < N; a += 256) {
+    const double us = cost16(kTiles16[2], M, a, K) + cost16(kTiles16[1], M, N - a, K);
+    if (us < 0.98 * single && us < p.us) p.n_wide = a, p.us = us;
+  }
+  return p;
+}
+// Split over k, or not: the split GEMM against the best unsplit one (16-bit and int8 weights decide alike, so that they
+// keep giving the same bits).  Time of the split one: fitted to 49 shapes, 4 % off.
+bool split_pays(const GemmPlan& pl, int M, int N, int K) {
+  if (pl.S <= 1) return false;
+  const int kt = (K + BK - 1) / BK;
+  return 9.4 + 1.12 * ((kt + pl.S - 1) / pl.S) + 0.139e-6 * pl.S * M * N * 8 < 0.97 * plan16(M, N, K).us;
+}
+
+// The pipelined kernel: split over k into pl.S ranges (ws holds the partial planes), or, int8 weights, unsplit (ws null).
 template <bool W8, int NI, typename T = BF16>
 int launch4(const uint16_t* a, const void* W, const float* scale, const EpiArgs& ep, uint16_t* c, int M, int N, int K,
-            int64_t lda, int64_t ldw, int64_t ldc, int epilogue, hipStream_t s, float* ws = nullptr, size_t ws_bytes = 0) {
+            int64_t lda, int64_t ldw, int64_t ldc, int epilogue, hipStream_t s, const GemmPlan& pl, float* ws) {
   const int tiles_t = (M + BT - 1) / BT, tiles_c = (N + 64 * NI - 1) / (64 * NI);
   dim3 grid((unsigned)(tiles_t * tiles_c)), block(256);
-  const Taps none = {0, 0, 0, 0, 0, nullptr};
   if constexpr (NI != 2) {  // the 128-wide tile exists unsplit only
-    if (ws) {  // split-k when it pays and the caller's workspace holds the partial planes
-      const GemmPlan pl = plan_gemm(M, N, K, W8);
-      if (pl.S > 1 && ws_bytes >= split_bytes(pl, M, N)) {
-        const Taps split = {0, 0, 0, pl.tiles, pl.rem, nullptr};
-        hipLaunchKernelGGL((gemm4_kernel<W8, SANA_EPI_NONE, NI, true, T>), dim3(grid.x, (unsigned)pl.S), block, 0, s,
-                           a, W, scale, ep, reinterpret_cast<uint16_t*>(ws), M, N, K, lda, ldw, ldc, tiles_t, tiles_c,
-                           split);
-        if (hipGetLastError() != hipSuccess) return SANA_ERR_LAUNCH;
-        const int64_t threads = (int64_t)M * (N / 8);
-        dim3 egrid((unsigned)((threads + 255) / 256));
-#define SANA_SPLIT_EPI(EPI) \
-  hipLaunchKernelGGL((splitk_epilogue_kernel<EPI, T>), egrid, block, 0, s, ws, pl.S, ep, c, M, N, ldc)
-        switch (epilogue) {
-          case SANA_EPI_NONE: SANA_SPLIT_EPI(SANA_EPI_NONE); break;
-          case SANA_EPI_BIAS: SANA_SPLIT_EPI(SANA_EPI_BIAS); break;
-          case SANA_EPI_BIAS_SILU: SANA_SPLIT_EPI(SANA_EPI_BIAS_SILU); break;
-          case SANA_EPI_GATE_RES: SANA_SPLIT_EPI(SANA_EPI_GATE_RES); break;
-          default: return SANA_ERR_ARG;
-        }
-#undef SANA_SPLIT_EPI
-        return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
+    if (ws) {
+      const Taps split = {0, 0, 0, pl.tiles, pl.rem, nullptr};
+      hipLaunchKernelGGL((gemm4_kernel<W8, SANA_EPI_NONE, NI, true, T>), dim3(grid.x, (unsigned)pl.S), block, 0, s, a, W,
+                         scale, ep, reinterpret_cast<uint16_t*>(ws), M, N, K, lda, ldw, ldc, tiles_t, tiles_c, split);
+      if (hipGetLastError() != hipSuccess) return SANA_ERR_LAUNCH;
+      const int64_t threads = (int64_t)M * (N / 8);
+      dim3 egrid((unsigned)((threads + 255) / 256));
+#define SANA_SPLIT_EPI(EPI) hipLaunchKernelGGL((splitk_epilogue_kernel<EPI, T>), egrid, block, 0, s, ws, pl.S, ep, c, M, N, ldc)
+      switch (epilogue) {
+        case SANA_EPI_NONE: SANA_SPLIT_EPI(SANA_EPI_NONE); break;
+        case SANA_EPI_BIAS: SANA_SPLIT_EPI(SANA_EPI_BIAS); break;
+        case SANA_EPI_BIAS_SILU: SANA_SPLIT_EPI(SANA_EPI_BIAS_SILU); break;
+        case SANA_EPI_GATE_RES: SANA_SPLIT_EPI(SANA_EPI_GATE_RES); break;
+        default: return SANA_ERR_ARG;
       }
+#undef SANA_SPLIT_EPI
+      return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
     }
   }
-  if constexpr (!W8 && NI != 2) return SANA_ERR_WORKSPACE;  // (16-bit operands unsplit: the many-token kernel)
-  else {
-#define SANA_LAUNCH4(EPI)                                                                                         \
+  if constexpr (W8) {
+    const Taps none = {0, 0, 0, 0, 0, nullptr};
+#define SANA_LAUNCH4(EPI)                                                                                              \
   hipLaunchKernelGGL((gemm4_kernel<W8, EPI, NI, false, T>), grid, block, 0, s, a, W, scale, ep, c, M, N, K, lda, ldw, ldc, \
                      tiles_t, tiles_c, none)
-  switch (epilogue) {
-    case SANA_EPI_NONE: SANA_LAUNCH4(SANA_EPI_NONE); break;
-    case SANA_EPI_BIAS: SANA_LAUNCH4(SANA_EPI_BIAS); break;
-    case SANA_EPI_BIAS_SILU: SANA_LAUNCH4(SANA_EPI_BIAS_SILU); break;
-    case SANA_EPI_GATE_RES: SANA_LAUNCH4(SANA_EPI_GATE_RES); break;
-    default: return SANA_ERR_ARG;
-  }
-#undef SANA_LAUNCH4
-  return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
-  }
-}
-
-template <bool W8, typename T = BF16>
-int launch_small(const uint16_t* a, const void* W, const float* scale, const EpiArgs& ep, uint16_t* c, int M, int N,
-                 int K, int64_t lda, int64_t ldw, int64_t ldc, int epilogue, hipStream_t s) {
-  const int tiles_t = (M + 127) / 128, tiles_c = (N + 127) / 128;
-  dim3 grid((unsigned)(tiles_t * tiles_c)), block(256);
-#define SANA_LAUNCH_S(EPI)                                                                                          \
-  hipLaunchKernelGGL((gemm_kernel<W8, EPI, 2, 2, T>), grid, block, 0, s, a, W, scale, ep, c, M, N, K, lda, ldw, ldc, \
-                     tiles_t, tiles_c)
-  switch (epilogue) {
-    case SANA_EPI_NONE: SANA_LAUNCH_S(SANA_EPI_NONE); break;
-    case SANA_EPI_BIAS: SANA_LAUNCH_S(SANA_EPI_BIAS); break;
-    case SANA_EPI_BIAS_SILU: SANA_LAUNCH_S(SANA_EPI_BIAS_SILU); break;
-    case SANA_EPI_GATE_RES: SANA_LAUNCH_S(SANA_EPI_GATE_RES); break;
-    default: return SANA_ERR_ARG;
-  }
-#undef SANA_LAUNCH_S
-  return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
-}
-
-// Channel tile of the many-token kernel, in units of 64.  One persistent workgroup per compute unit, so the grid runs in
-// rounds of 256 tiles; a round of 192-wide tiles takes 0.83 of one of 256-wide tiles and a round of 128-wide ones 0.62
-// (16384 x 2240 x 5600: 2.25 -> 3 rounds of 256 wide 328 us, 3 of 192 wide 305 us; 4096 x 2240 x 2240: 46.5 us for one
-// round of 256 wide, 43.5 of 192 wide, 56.5 for two of 128 wide).
-constexpr double kRound8[5] = {0, 0, 0.62, 0.83, 1.0};
-double cost8(int64_t tiles_t, int64_t N, int nb) {
-  const int64_t cu = compute_units();
-  return (double)((tiles_t * ((N + 64 * nb - 1) / (64 * nb)) + cu - 1) / cu) * kRound8[nb];
-}
-int pick_nb(int M, int N) {
-  const int64_t tiles_t = (M + BT - 1) / BT;
-  int best = 4;
-  for (int nb = 3; nb >= 2; --nb)
-    if (cost8(tiles_t, N, nb) < cost8(tiles_t, N, best)) best = nb;
-  return best;
-}
-// Channels to cover with 256-wide tiles when the rest goes to 192-wide ones in a second launch, or 0 when one width
-// for all of N is at least as good: the second launch costs 0.1 of a round, the mix must win by 1 % (32760 x 6720
-// tokens x channels: 14 rounds of 256 wide, 12 + 2 x 0.83 mixed).
-int mixed_split(int M, int N) {
-  const int64_t tiles_t = (M + BT - 1) / BT;
-  double best = std::min(cost8(tiles_t, N, 4), cost8(tiles_t, N, 3)) * 0.99;
-  int best_wide = 0;
-  for (int a = 1; a * 256 < N; ++a) {
-    const double cost = cost8(tiles_t, a * 256, 4) + cost8(tiles_t, N - a * 256, 3) + 0.1;
-    if (cost < best) {
-      best = cost;
-      best_wide = a * 256;
+    switch (epilogue) {
+      case SANA_EPI_NONE: SANA_LAUNCH4(SANA_EPI_NONE); break;
+      case SANA_EPI_BIAS: SANA_LAUNCH4(SANA_EPI_BIAS); break;
+      case SANA_EPI_BIAS_SILU: SANA_LAUNCH4(SANA_EPI_BIAS_SILU); break;
+      case SANA_EPI_GATE_RES: SANA_LAUNCH4(SANA_EPI_GATE_RES); break;
+      default: return SANA_ERR_ARG;
     }
+#undef SANA_LAUNCH4
+    return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
   }
-  return best_wide;
+  return SANA_ERR_ARG;
+}
+
+// The compiler-scheduled kernel (int8 weights): 64*TT tokens x 64*TC channels.
+template <int TT, int TC>
+int launch_w8(const uint16_t* a, const void* W, const float* scale, const EpiArgs& ep, uint16_t* c, int M, int N, int K,
+              int64_t lda, int64_t ldw, int64_t ldc, int epilogue, hipStream_t s) {
+  const int tiles_t = (M + 64 * TT - 1) / (64 * TT), tiles_c = (N + 64 * TC - 1) / (64 * TC);
+  dim3 grid((unsigned)(tiles_t * tiles_c)), block(256);
+#define SANA_LAUNCH_W8(EPI)                                                                                      \
+  hipLaunchKernelGGL((gemm_w8_kernel<EPI, TT, TC>), grid, block, 0, s, a, static_cast<const int8_t*>(W), scale, ep, c, M, N, \
+                     K, lda, ldw, ldc, tiles_t, tiles_c)
+  switch (epilogue) {
+    case SANA_EPI_NONE: SANA_LAUNCH_W8(SANA_EPI_NONE); break;
+    case SANA_EPI_BIAS: SANA_LAUNCH_W8(SANA_EPI_BIAS); break;
+    case SANA_EPI_BIAS_SILU: SANA_LAUNCH_W8(SANA_EPI_BIAS_SILU); break;
+    case SANA_EPI_GATE_RES: SANA_LAUNCH_W8(SANA_EPI_GATE_RES); break;
+    default: return SANA_ERR_ARG;
+  }
+#undef SANA_LAUNCH_W8
+  return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
 }
 
 template <bool W8, typename T = BF16>
@@ -963,51 +965,42 @@ int launch(const void* A, const void* W, const float* scale, const EpiArgs& ep, 
   const uint16_t* a = static_cast<const uint16_t*>(A);
   uint16_t* c = static_cast<uint16_t*>(C);
   const GemmPlan pl = plan_gemm(M, N, K, W8);
-  if (pl.small) return launch_small<W8, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s);
-  const bool pipelined = K % 32 == 0 && K >= 64;
   float* ws = aligned16(workspace) ? static_cast<float*>(workspace) : nullptr;
-  // Few tokens, wide N (qkv of one 1024 px image: 4 x 35 tiles of 192 channels on 256 CUs): 128-wide tiles put
-  // half as much math behind every k-tile of the chain and fill more of the chip (4 x 53 workgroups: 37 -> 31 us).
-  // Taken when the 192-wide grid leaves a fifth of the CUs idle and the 128-wide one still fits.
-  const int64_t t128 = tiles_t * ((N + 127) / 128), t192 = tiles_t * ((N + 191) / 192);
-  const bool narrow = pipelined && t128 <= compute_units() && t192 < compute_units() * 4 / 5 && pl.S == 1;
-  if (narrow) return launch4<W8, 2, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s);
+  if (ws && workspace_bytes >= split_bytes(pl, M, N) && split_pays(pl, M, N, K))
+    return pick_ni(M, N) == 3 ? launch4<W8, 3, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, pl, ws)
+                              : launch4<W8, 4, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, pl, ws);
   if constexpr (!W8) {
-    const bool split = pl.S > 1 && ws && workspace_bytes >= split_bytes(pl, M, N);
-    if (!split) {
-      const uint16_t* w = static_cast<const uint16_t*>(W);
-      const int n_wide = mixed_split(M, N);
-      if (n_wide == 0) return gemm8_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, pick_nb(M, N), nullptr, s);
-      const int rc = gemm8_launch(a, w, ep, c, M, n_wide, K, lda, ldw, ldc, epilogue, is_f16<T>, 4, nullptr, s);
+    const uint16_t* w = static_cast<const uint16_t*>(W);
+    const Plan16 p = plan16(M, N, K);
+    if (p.n_wide) {
+      const int rc = gemm8_launch(a, w, ep, c, M, p.n_wide, K, lda, ldw, ldc, epilogue, is_f16<T>, 4, nullptr, s);
       if (rc != SANA_OK) return rc;
       EpiArgs ep2 = ep;
-      if (ep2.bias) ep2.bias += n_wide;
-      if (ep2.gate) ep2.gate += n_wide;
-      if (ep2.res) ep2.res += n_wide;
-      return gemm8_launch(a, w + (int64_t)n_wide * ldw, ep2, c + n_wide, M, N - n_wide, K, lda, ldw, ldc, epilogue, is_f16<T>,
-                          3, nullptr, s);
+      if (ep2.bias) ep2.bias += p.n_wide;
+      if (ep2.gate) ep2.gate += p.n_wide;
+      if (ep2.res) ep2.res += p.n_wide;
+      return gemm8_launch(a, w + (int64_t)p.n_wide * ldw, ep2, c + p.n_wide, M, N - p.n_wide, K, lda, ldw, ldc, epilogue,
+                          is_f16<T>, 3, nullptr, s);
     }
+    if (p.tile->bm == 256)
+      return gemm8_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, p.tile->bn / 64, nullptr, s);
+    return gemm_ring_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, p.tile->bm, p.tile->bn, s);
+  } else {
+    const bool pipelined = K % 32 == 0 && K >= 64;
+    const int KT = (K + BK - 1) / BK;
+    // the 128 x 128 tile where its grid fits one workgroup per compute unit and its chain is the shorter one (plan_gemm)
+    if (pl.small || (pl.S > 1 && (int64_t)((M + 127) / 128) * ((N + 127) / 128) <= compute_units() && KT >= 11))
+      return launch_w8<2, 2>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s);
+    if (!pipelined) return launch_w8<4, 4>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s);
+    // Few tokens, wide N (qkv of one 1024 px image: 4 x 35 tiles of 192 channels on 256 CUs): 128-wide tiles put
+    // half as much math behind every k-tile of the chain and fill more of the chip (4 x 53 workgroups).
+    // Taken when the 192-wide grid leaves a fifth of the CUs idle and the 128-wide one still fits.
+    const int64_t t128 = tiles_t * ((N + 127) / 128), t192 = tiles_t * ((N + 191) / 192);
+    if (t128 <= compute_units() && t192 < compute_units() * 4 / 5)
+      return launch4<true, 2>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, pl, nullptr);
+    return pick_ni(M, N) == 3 ? launch4<true, 3>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, pl, nullptr)
+                              : launch4<true, 4>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, pl, nullptr);
   }
-  if (pipelined)  // int8 weights, or split over k
-    return pick_ni(M, N) == 3 ? launch4<W8, 3, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, ws, workspace_bytes)
-                              : launch4<W8, 4, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, ws, workspace_bytes);
-  if constexpr (W8) {  // any K % 16 == 0
-    const int tiles_c = (N + BC - 1) / BC;
-    dim3 grid((unsigned)(tiles_t * tiles_c)), block(256);
-#define SANA_LAUNCH(EPI)                                                                                        \
-  hipLaunchKernelGGL((gemm_kernel<true, EPI, 4, 4, T>), grid, block, 0, s, a, W, scale, ep, c, M, N, K, lda, ldw, ldc, \
-                     (int)tiles_t, tiles_c)
-    switch (epilogue) {
-      case SANA_EPI_NONE: SANA_LAUNCH(SANA_EPI_NONE); break;
-      case SANA_EPI_BIAS: SANA_LAUNCH(SANA_EPI_BIAS); break;
-      case SANA_EPI_BIAS_SILU: SANA_LAUNCH(SANA_EPI_BIAS_SILU); break;
-      case SANA_EPI_GATE_RES: SANA_LAUNCH(SANA_EPI_GATE_RES); break;
-      default: return SANA_ERR_ARG;
-    }
-#undef SANA_LAUNCH
-    return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
-  }
-  return SANA_ERR_SHAPE;
 }
 
 int check_common(const void* A, const void* W, const void* bias, const void* C, int M, int N, int K, int64_t lda,
@@ -1089,6 +1082,15 @@ SANA_API size_t sana_hip_gemm_workspace_bytes(int M, int N, int K) {
   return split_bytes(plan_gemm(M, N, K, false), M, N);
 }
 
+// From 4096 rows on always (converting in the main loop costs it 14 % at every M, the expansion a fixed 10 - 20 us); below
+// that where N <= K and the GEMM is not split: there the bf16 GEMM has its small tiles and the int8 one a chain of long
+// k-tiles.  us, converting / expanding: 256 x 1152 x 2880 37 / 20, 2048 x 2240 x 2240 40 / 33, 2048 x 2240 x 5600 91 / 68;
+// but 2048 x 5760 x 1152 32 / 40, 1024 x 11200 x 2240 56 / 63, and split 512 x 2240 x 5600 33 / 42.
+SANA_API int sana_hip_gemm_w8_expand(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  return M >= 4096 || (N <= K && !split_pays(plan_gemm(M, N, K, true), M, N, K));
+}
+
 SANA_API int sana_hip_gemm_bf16(const void* A, const void* W, const void* bias, void* C, int M, int N, int K,
                                 int64_t lda, int64_t ldw, int64_t ldc, int epilogue, void* workspace,
                                 size_t workspace_bytes, void* stream) {
@@ -1167,7 +1169,8 @@ SANA_API int sana_hip_tconv_residual(const void* X, const void* W, void* out, in
   const EpiArgs e = {nullptr, nullptr, x + (taps / 2) * tap_rows * ldx, ldx, 0, M, nullptr, 0, 0, 0, 0};
   const Taps tp = {C, tap_rows, x_rows, 0, 0, zero_last_tap};
   return gemm8_launch(x, static_cast<const uint16_t*>(W), e, static_cast<uint16_t*>(out), M, C, taps * C, ldx, ldw, ldo,
-                      SANA_EPI_GATE_RES, false, std::max(3, pick_nb(M, C)), &tp, static_cast<hipStream_t>(stream));
+                      SANA_EPI_GATE_RES, false,
+                     cost16(kTiles16[1], M, C, taps * C) < cost16(kTiles16[2], M, C, taps * C) ? 3 : 4, &tp, static_cast<hipStream_t>(stream));
 }
 
 SANA_API int sana_hip_dequant_w8(const int8_t* Wq, const float* scale, void* W, int N, int K, int64_t ldw,

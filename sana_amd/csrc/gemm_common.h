@@ -49,6 +49,11 @@ struct Taps {
 int gemm8_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
                  int64_t ldw, int64_t ldc, int epilogue, bool f16, int nb, const Taps* taps, hipStream_t s);
 
+// The GEMM for few tokens (gemm_ring.hip): the same operands and epilogues up to SANA_EPI_GATE_RES (gate not null), in tiles
+// of bm tokens x bn channels: 64 x 64, 64 x 128, 128 x 128 or 128 x 160.
+int gemm_ring_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
+                     int64_t ldw, int64_t ldc, int epilogue, bool f16, int bm, int bn, hipStream_t s);
+
 namespace {
 
 // 8 outputs of one row: accumulator (+bias) -> io dtype, per the epilogue kind (everything except

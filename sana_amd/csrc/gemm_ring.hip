@@ -1,0 +1,52 @@
+#include "gemm_ring.h"
+
+#include <algorithm>
+
+namespace sana {
+namespace {
+
+template <int WM, int WN, int TM, int TN, int ST, typename T>
+int launch_ring(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
+                int64_t ldw, int64_t ldc, int epilogue, hipStream_t s) {
+  constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
+  const int tiles_t = (M + BM - 1) / BM, tiles_c = (N + BN - 1) / BN;
+  const dim3 grid((unsigned)(tiles_t * tiles_c)), block(64 * WM * WN);
+  // An XCD works on an eighth of the tiles, g token tiles x the rest: the shape that reads the fewest operand rows.
+  const int per = std::max(1, tiles_t * tiles_c / 8);
+  int group = 1;
+  int64_t best = INT64_MAX;
+  for (int g = 1; g <= std::min(tiles_t, 64); ++g) {
+    const int64_t cost = (int64_t)g * BM + (int64_t)((per + g - 1) / g) * BN;
+    if (cost < best) best = cost, group = g;
+  }
+#define SANA_LAUNCH_R(EPI)                                                                                              \
+  hipLaunchKernelGGL((gemm_ring_kernel<WM, WN, TM, TN, ST, EPI, T>), grid, block, 0, s, a, w, ep, c, M, N, K, lda, ldw, ldc, \
+                     tiles_t, tiles_c, group)
+  switch (epilogue) {
+    case SANA_EPI_NONE: SANA_LAUNCH_R(SANA_EPI_NONE); break;
+    case SANA_EPI_BIAS: SANA_LAUNCH_R(SANA_EPI_BIAS); break;
+    case SANA_EPI_BIAS_SILU: SANA_LAUNCH_R(SANA_EPI_BIAS_SILU); break;
+    case SANA_EPI_GATE_RES: SANA_LAUNCH_R(SANA_EPI_GATE_RES); break;
+    default: return SANA_ERR_ARG;
+  }
+#undef SANA_LAUNCH_R
+  return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
+}
+
+}  // namespace
+
+int gemm_ring_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
+                     int64_t ldw, int64_t ldc, int epilogue, bool f16, int bm, int bn, hipStream_t s) {
+#define SANA_RING(WM, WN, TM, TN, ST)                                                                          \
+  if (bm == 16 * TM * WM && bn == 16 * TN * WN)                                                                 \
+  return f16 ? launch_ring<WM, WN, TM, TN, ST, F16>(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, s)            \
+             : launch_ring<WM, WN, TM, TN, ST, BF16>(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, s)
+  SANA_RING(2, 2, 2, 2, 5);   // 64 x 64, 80 KB: two workgroups per compute unit
+  SANA_RING(2, 4, 2, 2, 6);   // 64 x 128
+  SANA_RING(4, 2, 2, 4, 4);   // 128 x 128 (five stages: the same time)
+  SANA_RING(4, 1, 2, 10, 4);  // 128 x 160
+#undef SANA_RING
+  return SANA_ERR_ARG;
+}
+
+}  // namespace sana

@@ -379,10 +379,16 @@ def gemm_bf16(a: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor
     return out
 
 
-# From this many rows on, an int8 weight is expanded to bf16 once per call (a streaming pass over N*K bytes) and
-# the bf16 GEMM runs; below it the GEMM converts inside its main loop.  Both give the same bits; the conversion
-# costs the main loop about 14 % at every M, the expansion a fixed 10-20 us.
+# From this many rows on, and below it where the library's rule says so (``sana_hip_gemm_w8_expand``), an int8 weight
+# is expanded to bf16 once per call (a streaming pass over N*K bytes) and the bf16 GEMM runs; otherwise the GEMM converts
+# inside its main loop.  Both give the same bits.
 W8_EXPAND_MIN_ROWS = 4096
+
+
+def _w8_expands(expand: Optional[bool], M: int, N: int, K: int) -> bool:
+    if expand is None:
+        return M >= W8_EXPAND_MIN_ROWS or bool(_lib.load().sana_hip_gemm_w8_expand(M, N, K))
+    return expand
 
 
 def dequant_w8(wq: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
@@ -471,11 +477,11 @@ def gemm_w8a16(a: torch.Tensor, wq: torch.Tensor, scale: torch.Tensor, bias: Opt
                epilogue: Optional[str] = None, out: Optional[torch.Tensor] = None,
                expand: Optional[bool] = None) -> torch.Tensor:
     """a: [M, K] bf16; wq: [N, K] int8; scale: [N] fp32.  Equals gemm_bf16 on (wq.float()*scale).bfloat16().
-    ``expand``: True = expand the weight to bf16 first, False = convert inside the GEMM, None = by M."""
+    ``expand``: True = expand the weight to bf16 first, False = convert inside the GEMM, None = by the sizes."""
     _need_cuda(a, wq, scale, bias)
     if a.dtype != torch.bfloat16 or wq.dtype != torch.int8 or scale.dtype != torch.float32:
         raise SanaHipError("gemm_w8a16 needs bf16 activations, int8 weights and fp32 scales")
-    if expand or (expand is None and a.shape[0] >= W8_EXPAND_MIN_ROWS):
+    if _w8_expands(expand, a.shape[0], wq.shape[0], a.shape[-1]):
         return gemm_bf16(a, dequant_w8(wq, scale), bias, epilogue, out)
     a, lda = _rows(a, "a")
     wq, ldw = _rows(wq, "wq")
@@ -524,7 +530,7 @@ def gemm_gate_residual(a: torch.Tensor, weight: torch.Tensor, bias: Optional[tor
     weight is bf16 [C, K], or int8 with ``weight_scale`` (W8A16; ``expand`` as in :func:`gemm_w8a16`)."""
     _need_cuda(a, weight, bias, gate, residual, weight_scale)
     B, Ntok, K = a.shape
-    if weight_scale is not None and (expand or (expand is None and B * Ntok >= W8_EXPAND_MIN_ROWS)):
+    if weight_scale is not None and _w8_expands(expand, B * Ntok, weight.shape[0], K):
         weight, weight_scale = dequant_w8(weight.reshape(weight.shape[0], -1), weight_scale), None
     C = weight.shape[0]
     dt = a.dtype

@@ -20,7 +20,13 @@ MANY = [(1030, 8200, 8), (1030, 8200, 64), (1030, 8200, 72), (1030, 8200, 184), 
         (4099, 2240, 136), (8200, 6720, 128), (4352, 4360, 192)]
 
 
-@pytest.mark.parametrize("M,N,K", MANY)
+# tiles of 64 x 64, 64 x 128, 128 x 128 and 128 x 160: one row and eight channels, ragged edges, fewer k-tiles than the
+# ring has stages and more, k tails of 8, 32 and 56
+FEW = [(1, 8, 8), (65, 72, 40), (200, 264, 184), (33, 16, 320), (206, 3456, 8), (700, 2240, 328), (1500, 1160, 1152),
+       (3679, 536, 8), (999, 2248, 392), (2049, 1160, 120), (3671, 1120, 200), (2000, 2232, 1032), (2040, 2240, 2240)]
+
+
+@pytest.mark.parametrize("M,N,K", MANY + FEW)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_many_token_tiles_are_exact_on_integers(cuda, M, N, K, dtype):
     a, w, bias = (_ints(M, K, seed=1, dtype=dtype).to(cuda), _ints(N, K, seed=2, dtype=dtype).to(cuda),
@@ -36,7 +42,8 @@ def test_many_token_tiles_are_exact_on_integers(cuda, M, N, K, dtype):
     assert ((y.double() - want).abs() <= ulp * want.abs() + 1e-7).all()
 
 
-@pytest.mark.parametrize("B,Ntok,C,K", [(3, 1365, 2240, 72), (41, 100, 2240, 64), (2, 4100, 2240, 136), (1, 4096, 4360, 64)])
+@pytest.mark.parametrize("B,Ntok,C,K", [(3, 1365, 2240, 72), (41, 100, 2240, 64), (2, 4100, 2240, 136), (1, 4096, 4360, 64),
+                                           (7, 9, 72, 40), (5, 140, 2240, 328), (9, 111, 2248, 392), (3, 667, 2232, 1032)])
 def test_many_token_gated_residual_across_batch_boundaries(cuda, B, Ntok, C, K):
     a, w, bias = _ints(B, Ntok, K, seed=1).to(cuda), _ints(C, K, seed=2).to(cuda), _ints(C, lo=-9, hi=9, seed=3).to(cuda)
     gate, res = _ints(B, 1, C, lo=-4, hi=4, seed=4).to(cuda), _ints(B, Ntok, C, lo=-99, hi=99, seed=5).to(cuda)
