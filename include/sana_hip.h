@@ -377,6 +377,10 @@ int sana_hip_gemm_w8_expand(int M, int N, int K);
 int sana_hip_cross_attention(const void* q, const void* kv, const float* key_bias, void* out, int B, int N,
                              int Nk, int H, int d, int64_t ldq, int64_t ldkv, int64_t ldo,
                              int64_t bias_stride, float scale, void* stream);
+/* the same with q, kv and out in f16 (probabilities rounded to f16) */
+int sana_hip_cross_attention_f16(const void* q, const void* kv, const float* key_bias, void* out, int B, int N,
+                                 int Nk, int H, int d, int64_t ldq, int64_t ldkv, int64_t ldo,
+                                 int64_t bias_stride, float scale, void* stream);
 
 /* Gated residual update as one elementwise pass:
  *   out[m][:] = residual[m][:] + gate[m / rows_per_gate][:] * y[m][:]

@@ -100,6 +100,13 @@ __device__ __forceinline__ f32x16_t mfma_32x32x16<F16>(u32x4_t a, u32x4_t b, f32
 __device__ __forceinline__ f32x4_t mfma_16x16x32_bf16(u32x4_t a, u32x4_t b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
+template <typename T>
+__device__ __forceinline__ f32x4_t mfma_16x16x32(u32x4_t a, u32x4_t b, f32x4_t c) {
+  if constexpr (is_f16<T>)
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  else
+    return mfma_16x16x32_bf16(a, b, c);
+}
 
 // acc + lo(x) + hi(x) for two packed 16-bit floats: one dot2 against (1, 1), fp32 accumulate
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));

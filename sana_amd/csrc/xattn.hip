@@ -1,5 +1,5 @@
 // Softmax attention of many queries over a SHORT key set (the block's cross-attention to the text tokens:
-// 16384 image tokens x 300 text tokens x 20 heads of 112 at the 4096 px latent), bf16 in and out.
+// 16384 image tokens x 300 text tokens x 20 heads of 112 at the 4096 px latent), bf16 or f16 in and out.
 //
 //   out[b, n, h*d + :] = softmax_m(q[b, n, h, :] . k[b, m, h, :] * scale + bias[b, m]) . v[b, m, h, :]
 //
@@ -13,6 +13,8 @@
 // feeds the probabilities straight back as the column operand of out^T = V^T . P^T -- the k index of that
 // product is permuted so that the 8 values a lane needs are the ones its own accumulators hold (keys
 // 32s + 4g + {0..3} and 32s + 16 + 4g + {0..3} for lane group g), and V^T is stored in that key order.
+// Few queries (one 512 px image: 32 workgroups of one item) are bound by the staging, a chain of load latencies: all of K
+// and V is requested before the first LDS write, and V is transposed four keys at a time (8-byte writes).
 // Workgroups are persistent over consecutive (batch, head, query block) items and restage K / V only when the
 // (batch, head) changes.  Every K / V fragment read from LDS feeds QT MFMAs.
 #include "common.h"
@@ -47,7 +49,7 @@ __device__ __forceinline__ int xa_vpos(int m) {
   return 32 * s + 8 * g + 4 * hi + e;
 }
 
-template <int DK, int DT, int QT, int NW, int NKT>
+template <typename T, int DK, int DT, int QT, int NW, int NKT>
 __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv,
                                                          const float* __restrict__ bias, uint16_t* __restrict__ out, int B,
                                                          int N, int Nk, int H, int d, int64_t ldq, int64_t ldkv, int64_t ldo,
@@ -71,47 +73,50 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
       __syncthreads();   // everyone is done with the previous head's K / V
       const uint16_t* kbase = kv + (int64_t)b * Nk * ldkv + (int64_t)h * d;
       const uint16_t* vbase = kbase + (int64_t)H * d;
-      // a thread's loads go out in batches of SB before the LDS writes of the batch (the rows come out of the L2: one
-      // load per round trip would make staging a chain of ~20 latencies)
-      constexpr int NT = 64 * NW, SB = 5;
-      for (int base = tid; base < XA_NKP * KCH; base += SB * NT) {
-        u32x4_t val[SB];
+      // all of a thread's loads go out before its first LDS write.  K: pieces of 8 channels; V: 8 channels of 4 keys
+      // (key tiles past NKT are not read)
+      constexpr int NT = 64 * NW, KEYS = 16 * NKT, VCH = 2 * DT;
+      constexpr int KN = (KEYS * KCH + NT - 1) / NT, VN = (KEYS / 4 * VCH + NT - 1) / NT;
+      u32x4_t kval[KN], vval[VN][4];
+      int ht = tid;  // hidden from the optimiser: the addresses are not worth registers across the items
+      asm volatile("" : "+v"(ht));
 #pragma unroll
-        for (int i = 0; i < SB; ++i) {
-          const int idx = base + i * NT, row = idx / KCH, c = idx - row * KCH;
-          val[i] = u32x4_t{0u, 0u, 0u, 0u};
-          if (row < Nk && 8 * c < d) val[i] = *reinterpret_cast<const u32x4_t*>(kbase + (int64_t)row * ldkv + 8 * c);
-        }
+      for (int i = 0; i < KN; ++i) {
+        const int idx = ht + i * NT, row = idx / KCH, c = idx - row * KCH;
+        kval[i] = u32x4_t{0u, 0u, 0u, 0u};
+        if (row < Nk && 8 * c < d) kval[i] = *reinterpret_cast<const u32x4_t*>(kbase + (int64_t)row * ldkv + 8 * c);
+      }
 #pragma unroll
-        for (int i = 0; i < SB; ++i) {
-          const int idx = base + i * NT, row = idx / KCH, c = idx - row * KCH;
-          if (row < XA_NKP) *reinterpret_cast<u32x4_t*>(sk + row * KPITCH + ((c ^ xa_kkey<DK>(row)) << 4)) = val[i];
+      for (int i = 0; i < VN; ++i) {
+        const int idx = ht + i * NT, quad = idx / VCH, c = idx - quad * VCH;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          vval[i][k] = u32x4_t{0u, 0u, 0u, 0u};
+          if (4 * quad + k < Nk && 8 * c < d)
+            vval[i][k] = *reinterpret_cast<const u32x4_t*>(vbase + (int64_t)(4 * quad + k) * ldkv + 8 * c);
         }
       }
-      // V^T: a thread takes 8 channels of one key and scatters them over 8 rows
-      for (int base = tid; base < XA_NKP * DT * 2; base += SB * NT) {
-        u32x4_t val[SB];
 #pragma unroll
-        for (int i = 0; i < SB; ++i) {
-          const int idx = base + i * NT, row = idx / (DT * 2), c = idx - row * (DT * 2);
-          val[i] = u32x4_t{0u, 0u, 0u, 0u};
-          if (row < Nk && 8 * c < d) val[i] = *reinterpret_cast<const u32x4_t*>(vbase + (int64_t)row * ldkv + 8 * c);
-        }
+      for (int i = 0; i < KN; ++i) {
+        const int idx = ht + i * NT, row = idx / KCH, c = idx - row * KCH;
+        if (row < KEYS) *reinterpret_cast<u32x4_t*>(sk + row * KPITCH + ((c ^ xa_kkey<DK>(row)) << 4)) = kval[i];
+      }
 #pragma unroll
-        for (int i = 0; i < SB; ++i) {
-          const int idx = base + i * NT, row = idx / (DT * 2), c = idx - row * (DT * 2);
-          if (row < XA_NKP) {
-            const int p = xa_vpos(row);
+      for (int i = 0; i < VN; ++i) {
+        const int idx = ht + i * NT, quad = idx / VCH, c = idx - quad * VCH;
+        if (quad < KEYS / 4) {
+          const int p = xa_vpos(4 * quad);  // four keys stand side by side
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              const int dr = 8 * c + e;
-              const uint16_t x = (uint16_t)(e & 1 ? val[i][e >> 1] >> 16 : val[i][e >> 1] & 0xffffu);
-              *reinterpret_cast<uint16_t*>(sv + dr * XA_VPITCH + (((p >> 3) ^ xa_vkey(dr)) << 4) + (p & 7) * 2) = x;
-            }
+          for (int e = 0; e < 8; ++e) {
+            const int dr = 8 * c + e;
+            const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;
+            const u32x2_t x = {__builtin_amdgcn_perm(vval[i][1][e >> 1], vval[i][0][e >> 1], sel),
+                               __builtin_amdgcn_perm(vval[i][3][e >> 1], vval[i][2][e >> 1], sel)};
+            *reinterpret_cast<u32x2_t*>(sv + dr * XA_VPITCH + (((p >> 3) ^ xa_vkey(dr)) << 4) + (p & 7) * 2) = x;
           }
         }
       }
-      for (int m = tid; m < XA_NKP; m += 64 * NW)
+      for (int m = tid; m < KEYS; m += NT)
         sb[m] = m < Nk ? (bias ? bias[(int64_t)b * bias_stride + m] * 1.44269504088896341f : 0.f) : -INFINITY;
       __syncthreads();
       staged = bh;
@@ -161,9 +166,9 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
         for (int j = 0; j < 2; ++j)
 #pragma unroll
           for (int t = 0; t < QT; ++t)
-            sc[t][2 * kp + j] = mfma_16x16x32_bf16(kf[kp & 1][j][ks], qf[t][ks], sc[t][2 * kp + j]);
+            sc[t][2 * kp + j] = mfma_16x16x32<T>(kf[kp & 1][j][ks], qf[t][ks], sc[t][2 * kp + j]);
     }
-    // ---- softmax over the keys of each query (log2 domain), probabilities back as packed bf16
+    // ---- softmax over the keys of each query (log2 domain), probabilities back as packed 16-bit values
     float rsum[QT];
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
@@ -184,7 +189,7 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
       for (int kt = 0; kt < NKT; ++kt) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float p = __builtin_amdgcn_exp2f(sc[t][kt][r] - mx);  // rounded to bf16 where it is packed below
+          const float p = __builtin_amdgcn_exp2f(sc[t][kt][r] - mx);  // rounded to 16 bits where it is packed below
           sc[t][kt][r] = p;
           sum += p;
         }
@@ -214,15 +219,15 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
       u32x4_t pf[QT];
 #pragma unroll
       for (int t = 0; t < QT; ++t) {
-        pf[t].x = pack_bf16(sc[t][2 * s][0], sc[t][2 * s][1]);
-        pf[t].y = pack_bf16(sc[t][2 * s][2], sc[t][2 * s][3]);
-        pf[t].z = pack_bf16(sc[t][2 * s + 1][0], sc[t][2 * s + 1][1]);
-        pf[t].w = pack_bf16(sc[t][2 * s + 1][2], sc[t][2 * s + 1][3]);
+        pf[t].x = pk16<T>(sc[t][2 * s][0], sc[t][2 * s][1]);
+        pf[t].y = pk16<T>(sc[t][2 * s][2], sc[t][2 * s][3]);
+        pf[t].z = pk16<T>(sc[t][2 * s + 1][0], sc[t][2 * s + 1][1]);
+        pf[t].w = pk16<T>(sc[t][2 * s + 1][2], sc[t][2 * s + 1][3]);
       }
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int t = 0; t < QT; ++t) oc[t][dt] = mfma_16x16x32_bf16(vf[s & 1][dt], pf[t], oc[t][dt]);
+        for (int t = 0; t < QT; ++t) oc[t][dt] = mfma_16x16x32<T>(vf[s & 1][dt], pf[t], oc[t][dt]);
     }
     // ---- normalise and store: a lane holds 4 consecutive channels of its query per channel tile
     uint16_t* obase = out + ((int64_t)b * N) * ldo + (int64_t)h * d;
@@ -234,8 +239,8 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
         const int c0 = 16 * dt + 4 * fg;
         if (qi < N && c0 < d) {
           u32x2_t o;
-          o.x = pack_bf16(oc[t][dt][0] * rsum[t], oc[t][dt][1] * rsum[t]);
-          o.y = pack_bf16(oc[t][dt][2] * rsum[t], oc[t][dt][3] * rsum[t]);
+          o.x = pk16<T>(oc[t][dt][0] * rsum[t], oc[t][dt][1] * rsum[t]);
+          o.y = pk16<T>(oc[t][dt][2] * rsum[t], oc[t][dt][3] * rsum[t]);
           *reinterpret_cast<u32x2_t*>(obase + (int64_t)qi * ldo + c0) = o;
         }
       }
@@ -243,7 +248,7 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
   }
 }
 
-template <int DK, int DT, int QT, int NW, int NKT>
+template <typename T, int DK, int DT, int QT, int NW, int NKT>
 int launch_xa(const uint16_t* q, const uint16_t* kv, const float* bias, uint16_t* out, int B, int N, int Nk, int H, int d,
               int64_t ldq, int64_t ldkv, int64_t ldo, int64_t bias_stride, float scale, hipStream_t s) {
   const int qblocks = (N + NW * 16 * QT - 1) / (NW * 16 * QT);
@@ -252,19 +257,14 @@ int launch_xa(const uint16_t* q, const uint16_t* kv, const float* bias, uint16_t
   const int items = (int)items64, cus = 256;
   const int ipw = (items + cus - 1) / cus;
   const int grid = (items + ipw - 1) / ipw;
-  hipLaunchKernelGGL((cross_attn_kernel<DK, DT, QT, NW, NKT>), dim3((unsigned)grid), dim3(64 * NW), 0, s, q, kv, bias, out, B, N, Nk, H, d,
+  hipLaunchKernelGGL((cross_attn_kernel<T, DK, DT, QT, NW, NKT>), dim3((unsigned)grid), dim3(64 * NW), 0, s, q, kv, bias, out, B, N, Nk, H, d,
                      ldq, ldkv, ldo, bias_stride, scale * 1.44269504088896341f, qblocks, items, ipw);
   return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
 }
 
-}  // namespace
-}  // namespace sana
-
-using namespace sana;
-
-extern "C" __attribute__((visibility("default"))) int sana_hip_cross_attention(
-    const void* q, const void* kv, const float* key_bias, void* out, int B, int N, int Nk, int H, int d, int64_t ldq,
-    int64_t ldkv, int64_t ldo, int64_t bias_stride, float scale, void* stream) {
+template <typename T>
+int cross_attention(const void* q, const void* kv, const float* key_bias, void* out, int B, int N, int Nk, int H, int d,
+                    int64_t ldq, int64_t ldkv, int64_t ldo, int64_t bias_stride, float scale, void* stream) {
   if (!q || !kv || !out || B <= 0 || N <= 0 || Nk <= 0 || H <= 0 || d <= 0) return SANA_ERR_ARG;
   if (Nk > XA_NKP || d % 8 || d > 112 || d <= 64) return SANA_ERR_SHAPE;  // LDS: K + V^T of one head at d <= 112
   if (ldq < (int64_t)H * d || ldkv < 2 * (int64_t)H * d || ldo < (int64_t)H * d || (key_bias && bias_stride < Nk))
@@ -276,9 +276,28 @@ extern "C" __attribute__((visibility("default"))) int sana_hip_cross_attention(
   uint16_t* op = static_cast<uint16_t*>(out);
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define SANA_XA_GO(DK, DT, NKT) \
-  launch_xa<DK, DT, SANA_XA_QT, SANA_XA_NW, NKT>(qp, kp, key_bias, op, B, N, Nk, H, d, ldq, ldkv, ldo, bias_stride, scale, s)
+  launch_xa<T, DK, DT, SANA_XA_QT, SANA_XA_NW, NKT>(qp, kp, key_bias, op, B, N, Nk, H, d, ldq, ldkv, ldo, bias_stride, scale, s)
   // key tiles of 16 that are multiplied: all 20, or 10 for up to 160 keys (tiles past Nk hold zeros and -inf)
   if (d > 96) return Nk > 160 ? SANA_XA_GO(4, 7, 20) : SANA_XA_GO(4, 7, 10);
   return Nk > 160 ? SANA_XA_GO(3, 6, 20) : SANA_XA_GO(3, 6, 10);
 #undef SANA_XA_GO
+}
+
+}  // namespace
+}  // namespace sana
+
+using namespace sana;
+
+#define SANA_API extern "C" __attribute__((visibility("default")))
+
+SANA_API int sana_hip_cross_attention(const void* q, const void* kv, const float* key_bias, void* out, int B, int N, int Nk,
+                                      int H, int d, int64_t ldq, int64_t ldkv, int64_t ldo, int64_t bias_stride,
+                                      float scale, void* stream) {
+  return cross_attention<BF16>(q, kv, key_bias, out, B, N, Nk, H, d, ldq, ldkv, ldo, bias_stride, scale, stream);
+}
+
+SANA_API int sana_hip_cross_attention_f16(const void* q, const void* kv, const float* key_bias, void* out, int B, int N,
+                                          int Nk, int H, int d, int64_t ldq, int64_t ldkv, int64_t ldo,
+                                          int64_t bias_stride, float scale, void* stream) {
+  return cross_attention<F16>(q, kv, key_bias, out, B, N, Nk, H, d, ldq, ldkv, ldo, bias_stride, scale, stream);
 }

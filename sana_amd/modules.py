@@ -325,7 +325,7 @@ class LiteLA(nn.Module):
         if rotary_emb is None and x.dtype == torch.bfloat16 and self._state_in_qkv_gemm(x):
             # k and v never reach memory: their column tiles are contracted over the tokens in the qkv GEMM's epilogue
             wt, bt = self._tiled_qkv()
-            if self.qkv.is_quantized:       # int8 weights: expanded to bf16 per call, as the plain GEMM does from 4096 rows
+            if self.qkv.is_quantized:       # int8 weights: expanded to bf16 per call, as the plain GEMM does at this size
                 wt = ops.dequant_w8(*wt)
             q, state = ops.gemm_qkv_state(x, wt, bt, self.heads)
             out = ops.linattn_apply(q, state, self.eps)
@@ -850,8 +850,8 @@ def t2i_modulate(x, shift, scale):
 
 class MultiHeadCrossAttention(nn.Module):
     """Cross-attention to the text tokens (reference: sana_blocks.py:48-98, the scaled_dot_product_attention
-    branch): bf16 inference runs the attention itself as the short-key softmax kernel; its linears are this library's
-    GEMM from 4096 rows and library GEMM calls below; everything else (other dtypes, training, more than 320 text tokens, 4-d masks) is stock ops."""
+    branch): bf16 / fp16 inference runs the attention itself as the short-key softmax kernel and its linears on this library's
+    GEMM; everything else (other dtypes, training, more than 320 text tokens, 4-d masks) is stock ops."""
 
     def __init__(self, d_model, num_heads, attn_drop=0.0, proj_drop=0.0, qk_norm=False, **block_kwargs):
         super().__init__()
@@ -892,49 +892,66 @@ class MultiHeadCrossAttention(nn.Module):
             self.__dict__["_pad_cache"] = cache
         return cache[1]
 
+    def _on_hip_path(self, x, cond, mask) -> bool:
+        B, N, C = x.shape
+        return (x.is_cuda and x.dtype in ops.IO16 and cond.dtype == x.dtype and not torch.is_grad_enabled()
+                and cond.dim() == 3 and cond.shape[0] == B and ops.cross_attention_supported(self.head_dim, cond.shape[1])
+                and (mask is None or (mask.ndim == 2 and tuple(mask.shape) == (B, cond.shape[1])))
+                and self.q_linear.weight.dtype == x.dtype)
+
+    @staticmethod
+    def _gemm_takes(linear, x) -> bool:
+        """Rows, alignment and dtypes of this library's GEMM (anything else is a stock linear, as it always was)."""
+        w, b = linear.weight, linear.bias
+        return (x.is_contiguous() and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0
+                and w.dtype == x.dtype and b is not None and b.dtype == x.dtype and b.is_contiguous()
+                and b.data_ptr() % 16 == 0 and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0)
+
+    @staticmethod
+    def _linear(linear, x):
+        if MultiHeadCrossAttention._gemm_takes(linear, x):
+            return ops.gemm_bf16(x.view(-1, x.shape[-1]), linear.weight, linear.bias, "bias").view(*x.shape[:-1], -1)
+        return F.linear(x, linear.weight, linear.bias)
+
     def _attend(self, x, cond, mask, kv=None):
         """The HIP path up to proj's input -- softmax(q k^T) v over the short text sequence as one kernel that reads
         q_linear's output and writes proj's input token-major (no head transposes, no padded head_dim) -- or None
         when the call is outside it.  ``kv``: kv_linear(cond) computed by the caller ([B, Nk, 2C] rows, see
         ``StepConditioning``)."""
         B, N, C = x.shape
-        H, d = self.num_heads, self.head_dim
-        if not (x.is_cuda and x.dtype == torch.bfloat16 and cond.dtype == torch.bfloat16 and not torch.is_grad_enabled()
-                and cond.dim() == 3 and cond.shape[0] == B and ops.cross_attention_supported(d, cond.shape[1])
-                and (mask is None or (mask.ndim == 2 and tuple(mask.shape) == (B, cond.shape[1])))
-                and self.q_linear.weight.dtype == torch.bfloat16):
+        H = self.num_heads
+        if not self._on_hip_path(x, cond, mask):
             return None
-        # (below 4096 rows q_linear and kv_linear are library GEMM calls: at a few hundred to a few thousand rows
-        # they are faster than this library's GEMM and cost less host time per call)
-        if B * N >= self.RESIDUAL_GEMM_MIN_ROWS and self.q_linear.bias is not None and x.is_contiguous():
-            q = ops.gemm_bf16(x.view(B * N, C), self.q_linear.weight, self.q_linear.bias, "bias").view(B, N, C)
-        else:
-            q = F.linear(x, self.q_linear.weight, self.q_linear.bias)
+        q = self._linear(self.q_linear, x)
         if kv is None:
-            kv = F.linear(cond, self.kv_linear.weight, self.kv_linear.bias)       # [B, Nk, 2C]
+            kv = self._linear(self.kv_linear, cond)       # [B, Nk, 2C]
         if not isinstance(self.q_norm, nn.Identity):
             q = self.q_norm(q)
         if not isinstance(self.k_norm, nn.Identity):
             kv = torch.cat([self.k_norm(kv[:, :, :C]), kv[:, :, C:]], dim=-1)
         bias = None if mask is None else (1.0 - mask.to(torch.float32)) * -10000.0   # sana_blocks.py:89-90
-        return ops.cross_attention(q, kv, H, bias)
+        return ops.cross_attention16(q, kv, H, bias)
 
     # rows from which proj + the block's residual add run as ONE GEMM of this library (its gated-residual epilogue
-    # with a gate of ones: x + (o W^T + b), the same two roundings as the stock linear and add) instead of a
-    # library GEMM and an elementwise pass; below it the library GEMM's shorter latency chain wins
-    RESIDUAL_GEMM_MIN_ROWS = 4096
+    # with a gate of ones: x + (o W^T + b), the same two roundings as the stock linear and add): all.  us, library GEMM
+    # and the add's share of the pass behind it against this: 256 x 1152 7.0 + 1 / 6.8, 2048 x 1152 12.5 + 3 / 11.9,
+    # 1024 x 2240 19.3 + 4 / 17.9, 3000 x 2240 37.6 + 7 / 34.2.
+    RESIDUAL_GEMM_MIN_ROWS = 1
+
+    def _residual_in_gemm(self, x, cond, mask) -> bool:
+        return (x.shape[0] * x.shape[1] >= self.RESIDUAL_GEMM_MIN_ROWS and isinstance(self.proj_drop, nn.Dropout)
+                and self.proj_drop.p == 0.0 and self._on_hip_path(x, cond, mask) and self._gemm_takes(self.proj, x))
 
     def forward_residual(self, x, cond, mask=None, kv=None):
         """x + self(x, cond, mask) -- what the blocks compute (sana_multi_scale.py:154) -- with the add inside the
         projection GEMM's epilogue when the call is on the HIP path and large enough."""
         B, N, C = x.shape
-        if B * N >= self.RESIDUAL_GEMM_MIN_ROWS and isinstance(self.proj_drop, nn.Dropout) and self.proj_drop.p == 0.0:
+        if self._residual_in_gemm(x, cond, mask):
             o = self._attend(x, cond, mask, kv)
-            if o is not None:
-                ones = self.__dict__.get("_ones_gate")
-                if ones is None or ones.device != x.device or ones.shape[-1] != C:
-                    ones = self.__dict__["_ones_gate"] = torch.ones(1, 1, C, dtype=torch.bfloat16, device=x.device)
-                return ops.gemm_gate_residual(o, self.proj.weight, self.proj.bias, ones.expand(B, 1, C), x)
+            ones = self.__dict__.get("_ones_gate")
+            if ones is None or ones.device != x.device or ones.dtype != x.dtype or ones.shape[-1] != C:
+                ones = self.__dict__["_ones_gate"] = torch.ones(1, 1, C, dtype=x.dtype, device=x.device)
+            return ops.gemm_gate_residual(o, self.proj.weight, self.proj.bias, ones.expand(B, 1, C), x)
         return x + self(x, cond, mask, kv)
 
     def forward(self, x, cond, mask=None, kv=None):
@@ -942,10 +959,10 @@ class MultiHeadCrossAttention(nn.Module):
         H, d = self.num_heads, self.head_dim
         o = self._attend(x, cond, mask, kv)
         if o is not None:
-            return self.proj_drop(F.linear(o, self.proj.weight, self.proj.bias))
+            return self.proj_drop(self._linear(self.proj, o))
         if x.is_cuda:
             stock_path("cross-attention",
-                       f"the HIP path is bf16 inference with head_dim 72 .. 112, at most {ops.CROSS_ATTN_MAX_KEYS} text tokens "
+                       f"the HIP path is bf16 / fp16 inference with head_dim 72 .. 112, at most {ops.CROSS_ATTN_MAX_KEYS} text tokens "
                        f"and no mask or a [B, Nk] one; got {x.dtype}, head_dim {d}, cond {tuple(cond.shape)}, "
                        f"mask {None if mask is None else tuple(mask.shape)}, grad {'on' if torch.is_grad_enabled() else 'off'}")
         fast = (96 < d < 128 and x.is_cuda and not torch.is_grad_enabled()
@@ -1024,7 +1041,7 @@ class SanaMSBlock(nn.Module):
                 x = ops.gate_residual(self.attn(h, HW=HW, rotary_emb=image_rotary_emb), gate_msa, x)
             else:
                 x = self.attn.forward_gated(h, gate_msa, x, rotary_emb=image_rotary_emb)
-            if B * N >= self.cross_attn.RESIDUAL_GEMM_MIN_ROWS:
+            if self.cross_attn._residual_in_gemm(x, y, mask):
                 # the cross-attention's residual add inside its projection GEMM, then norm2 + modulate
                 x = self.cross_attn.forward_residual(x, y, mask, text_kv)
                 h = ops.layernorm_modulate(x, scale_mlp, shift_mlp, self.norm2.eps)
@@ -1062,7 +1079,7 @@ class StepConditioning:
             x = blk(x, y, t, mask, HW, **c)
 
     The stacked weights are a derived copy (2 * C * C * 2 bytes per block), rebuilt when a block's parameters
-    change, and not part of any state_dict.  Outside bf16 inference on the GPU the call returns empty dicts and
+    change, and not part of any state_dict.  Outside bf16 / fp16 inference on the GPU the call returns empty dicts and
     the blocks compute their own."""
 
     def __init__(self, blocks):
@@ -1083,9 +1100,9 @@ class StepConditioning:
     def __call__(self, y, t):
         L = len(self.blocks)
         ca = self.blocks[0].cross_attn if L else None
-        if not (L and y.is_cuda and y.dtype == torch.bfloat16 and t.dtype == torch.bfloat16 and y.dim() == 3
-                and not torch.is_grad_enabled() and ca.kv_linear.weight.dtype == torch.bfloat16
-                and self.blocks[0].scale_shift_table.dtype == torch.bfloat16
+        if not (L and y.is_cuda and y.dtype in ops.IO16 and t.dtype == y.dtype and y.dim() == 3
+                and not torch.is_grad_enabled() and ca.kv_linear.weight.dtype == y.dtype
+                and self.blocks[0].scale_shift_table.dtype == y.dtype
                 and all(b.cross_attn.d_model == ca.d_model for b in self.blocks)):
             return [{} for _ in self.blocks]
         w, b, tab = self._stacked()

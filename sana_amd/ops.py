@@ -679,9 +679,17 @@ def cross_attention(q: torch.Tensor, kv: torch.Tensor, num_heads: int, key_bias:
     """softmax(q k^T * scale + key_bias) v per head, bf16.  q: [B, N, C] (q_linear's output), kv: [B, Nk, 2C]
     (kv_linear's output: keys then values), key_bias: fp32 [B, Nk] added to every head's and query's scores
     (0 / -10000 for a padding mask) or None.  Returns [B, N, C], token-major like q."""
-    _need_cuda(q, kv, key_bias)
-    if q.dim() != 3 or kv.dim() != 3 or q.dtype != torch.bfloat16 or kv.dtype != torch.bfloat16:
+    if q.dtype != torch.bfloat16:
         raise SanaHipError("cross_attention needs bf16 q [B, N, C] and kv [B, Nk, 2C]")
+    return cross_attention16(q, kv, num_heads, key_bias, scale, out)
+
+
+def cross_attention16(q: torch.Tensor, kv: torch.Tensor, num_heads: int, key_bias: Optional[torch.Tensor] = None,
+                      scale: Optional[float] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """:func:`cross_attention` for bf16 or fp16 operands of one dtype."""
+    _need_cuda(q, kv, key_bias)
+    if q.dim() != 3 or kv.dim() != 3 or q.dtype not in IO16 or kv.dtype != q.dtype:
+        raise SanaHipError("cross_attention needs bf16 or fp16 q [B, N, C] and kv [B, Nk, 2C] of one dtype")
     B, N, C = q.shape
     Nk = kv.shape[1]
     if kv.shape[0] != B or kv.shape[2] != 2 * C or C % num_heads:
@@ -695,12 +703,14 @@ def cross_attention(q: torch.Tensor, kv: torch.Tensor, num_heads: int, key_bias:
         if key_bias.dtype != torch.float32 or key_bias.shape != (B, Nk) or key_bias.stride(1) != 1:
             raise SanaHipError("key_bias must be fp32 [B, Nk] with unit inner stride")
     if out is None:
-        out = torch.empty(B, N, C, dtype=torch.bfloat16, device=q.device)
-    elif out.shape != (B, N, C) or out.dtype != torch.bfloat16 or not out.is_contiguous():
-        raise SanaHipError("out must be a contiguous bf16 [B, N, C] tensor")
+        out = torch.empty(B, N, C, dtype=q.dtype, device=q.device)
+    elif out.shape != (B, N, C) or out.dtype != q.dtype or not out.is_contiguous():
+        raise SanaHipError("out must be a contiguous [B, N, C] tensor of q's dtype")
     if B * N == 0:
         return out
-    code = _lib.load().sana_hip_cross_attention(
+    lib = _lib.load()
+    fn = lib.sana_hip_cross_attention if q.dtype == torch.bfloat16 else lib.sana_hip_cross_attention_f16
+    code = fn(
         q.data_ptr(), kv.data_ptr(), None if key_bias is None else key_bias.data_ptr(), out.data_ptr(), B, N, Nk,
         num_heads, d, q.stride(1), kv.stride(1), C, 0 if key_bias is None else key_bias.stride(0),
         float(d ** -0.5 if scale is None else scale), _stream())

@@ -134,3 +134,50 @@ def test_residual_add_inside_the_projection_gemm(cuda):
     assert (mx > 2e-2 + 2.0 ** -7 * ref.double().abs()).sum().item() == 0 and rel_l2(fused.cpu(), ref) <= 1e-2
     small = hm.forward_residual(x[:, :64].to(cuda), y.to(cuda))       # below the threshold: the composition itself
     assert torch.equal(small, x[:, :64].to(cuda) + hm(x[:, :64].to(cuda), y.to(cuda)))
+
+
+@pytest.mark.parametrize("B,N,Nk,H,d,masked", [(2, 1024, 300, 16, 72, True), (1, 37, 1, 2, 112, False),
+                                              (3, 130, 159, 4, 112, True), (1, 129, 161, 3, 96, False),
+                                              (2, 17, 320, 2, 104, True)])
+def test_cross_attention_fp16_matches_the_formula(cuda, B, N, Nk, H, d, masked):
+    """The same kernel on f16 operands, around the two key-tile counts (160 keys) and the padded head dims.  Probabilities
+    and outputs carry a relative 2^-11 each, the probabilities' errors average over the keys: 2e-3 in norm."""
+    g = torch.Generator().manual_seed(B * 1000 + N + Nk + d)
+    C = H * d
+    q = (torch.randn(B, N, C, generator=g) * 1.5).half()
+    kv = torch.randn(B, Nk, 2 * C, generator=g).half()
+    keep = torch.ones(B, Nk)
+    if masked:
+        for b in range(B):
+            keep[b, max(1, Nk - 7 * (b + 1)):] = 0
+    bias = (1 - keep) * -10000.0
+    out = ops.cross_attention16(q.to(cuda), kv.to(cuda), H, bias.to(cuda) if masked else None)
+    ref = formula(q, kv, H, bias if masked else None)
+    assert out.dtype == torch.float16
+    assert (out.cpu().double() - ref).abs().max().item() <= 5e-3 and rel_l2(out.cpu(), ref) <= 2e-3
+
+
+@pytest.mark.parametrize("C,H,B,N,Nk,dtype", [(1152, 16, 2, 100, 300, torch.float16), (2240, 20, 1, 7, 40, torch.bfloat16),
+                                             (1152, 16, 1, 1000, 77, torch.bfloat16)])
+def test_residual_projection_of_few_rows(cuda, C, H, B, N, Nk, dtype):
+    """x + cross_attn(x, y) on this library's GEMMs at row counts below a tile and above, against the oracle in fp32; an x
+    at an odd address takes the stock linears and gives the same up to the sums' order."""
+    g = torch.Generator().manual_seed(N)
+    om = O.MultiHeadCrossAttention(C, H)
+    with torch.no_grad():
+        for p in om.parameters():
+            p.copy_(torch.nn.init.trunc_normal_(torch.empty(p.shape), std=0.02, generator=g))
+    om = om.to(dtype)
+    hm = S.modules.MultiHeadCrossAttention(C, H).to(dtype)
+    hm.load_state_dict(om.state_dict())
+    hm = hm.to(cuda)
+    x, y = torch.randn(B, N, C, generator=g).to(dtype), torch.randn(B, Nk, C, generator=g).to(dtype)
+    with torch.no_grad():
+        out = hm.forward_residual(x.to(cuda), y.to(cuda))
+        odd = torch.empty(x.numel() + 1, dtype=dtype, device=cuda)[1:].view(x.shape).copy_(x)
+        assert odd.data_ptr() % 16
+        stock = hm._linear(hm.q_linear, odd)
+        ref = x.float() + om.float()(x.float(), y.float())
+    tol = 1e-2 if dtype == torch.bfloat16 else 2e-3
+    assert rel_l2(out.cpu(), ref) <= tol
+    assert rel_l2(stock.cpu(), torch.nn.functional.linear(x.float(), om.q_linear.weight, om.q_linear.bias)) <= tol
