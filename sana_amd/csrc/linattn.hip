@@ -25,6 +25,9 @@
 #include "linattn_common.h"
 
 // tuning knobs of the bf16 apply kernel: tokens per workgroup, 16-token steps in flight per wave
+#ifndef SANA_LA_APPLY_MINWG
+#define SANA_LA_APPLY_MINWG 256  // halve the tokens of a workgroup (to no less than 32) until the launch has this many
+#endif
 #ifndef SANA_LA_APPLY_TOKENS
 #define SANA_LA_APPLY_TOKENS 128
 #endif
@@ -218,6 +221,8 @@ __global__ __launch_bounds__(256) void linattn_state16_kernel(
 // ----------------------------------------------------------------------------
 // phase 1, fp32 io: MFMA 32x32x2 f32 straight from global memory.
 // grid: x = nsplit, y = n_chunks, z = B * ceil(h/4); block 256, wave = one head.
+// Bound by load latency: 64 tokens in flight without a branch around a load (it was 16 behind branches); the key sum is
+// adds, not a second MFMA chain.  Tokens x heads, us with the reduction: 1024 x 36 12.1 -> 7.6, 16384 x 70 136 -> 82.
 // ----------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void linattn_state32_kernel(
     const float* __restrict__ K, const float* __restrict__ V, float* __restrict__ dst,
@@ -234,33 +239,37 @@ __global__ __launch_bounds__(256) void linattn_state32_kernel(
   const int j = lane & 31, g = lane >> 5;
   const float* kp = K + (int64_t)b * stride_b + head * D + j;
   const float* vp = V + (int64_t)b * stride_b + head * D + j;
-  f32x16_t accS, accK;
+  f32x16_t accS;
+  float accK = 0.f;  // the "1" row of [V|1]: this lane's half of the tokens
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    accS[i] = 0.f;
-    accK[i] = 0.f;
-  }
-  constexpr int U = 8;  // 16 tokens in flight per wave
+  for (int i = 0; i < 16; ++i) accS[i] = 0.f;
+  constexpr int U = 32;  // 64 tokens in flight per wave: a small input is one round trip
   for (int t = t0; t < t1; t += 2 * U) {
     float kk[U], vv[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int tok = t + 2 * u + g;
-      const bool ok = tok < t1;
-      kk[u] = ok ? fmaxf(kp[(int64_t)tok * stride_n], 0.f) : 0.f;
-      vv[u] = ok ? vp[(int64_t)tok * stride_n] : 0.f;
+      const int64_t at = (int64_t)min(tok, t1 - 1) * stride_n;  // (no branch around a load)
+      kk[u] = kp[at], vv[u] = vp[at];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool ok = t + 2 * u + g < t1;
+      kk[u] = ok ? fmaxf(kk[u], 0.f) : 0.f;
+      vv[u] = ok ? vv[u] : 0.f;
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       accS = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[u], kk[u], accS, 0, 0, 0);
-      accK = __builtin_amdgcn_mfma_f32_32x32x2f32(1.0f, kk[u], accK, 0, 0, 0);
+      accK += kk[u];
     }
   }
   const int64_t slot = ((int64_t)(b * h + head) * n_chunks + c) * nsplit + split;
   float* o = dst + slot * STATE_ELEMS;
 #pragma unroll
   for (int r = 0; r < 16; ++r) o[(8 * (r >> 2) + 4 * g + (r & 3)) * D + j] = accS[r];
-  if (g == 0) o[D * D + j] = accK[0];
+  accK += __shfl_xor(accK, 32, 64);
+  if (g == 0) o[D * D + j] = accK;
 }
 
 // ----------------------------------------------------------------------------
@@ -295,7 +304,7 @@ __global__ __launch_bounds__(256) void linattn_reduce_scan_kernel(const float* _
 }
 
 // ----------------------------------------------------------------------------
-// phase 2, bf16 io.  grid: x = token ranges per chunk, y = n_chunks,
+// phase 2, bf16 and f16 io.  grid: x = token ranges per chunk, y = n_chunks,
 // z = B * ceil(pairs/4); block 256; wave = pair of heads.
 // ----------------------------------------------------------------------------
 struct SplitState {     // A operands of one head: 3 row blocks x 3 bf16 terms
@@ -321,8 +330,21 @@ __device__ __forceinline__ void split3(const float x[8], u32x4_t out[3]) {
   }
 }
 
-template <bool OUT_F32, int PRE>
-__global__ __launch_bounds__(256) void linattn_apply_bf16_kernel(
+// f16 queries go to the bf16 MFMA as the exact sum of two bf16 values (11 significant bits = 8 + 3): the state keeps its
+// range and its 24 bits, which f16 terms would not.
+__device__ __forceinline__ void f16_to_2bf16(u32x4_t q, u32x4_t& hi, u32x4_t& lo) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float a = lo16<F16>(q[e]), b = hi16<F16>(q[e]);
+    hi[e] = pack_bf16(a, b);
+    lo[e] = pack_bf16(a - bf16_lo(hi[e]), b - bf16_hi(hi[e]));
+  }
+}
+
+// T = F16 replaces MFMAs in fp32 (32x32x2) and 2-byte loads and stores: tokens x heads, us: 2048 x 36
+// 16.5 -> 7.1, 16384 x 70 125 -> 34.
+template <typename T, bool OUT_F32, int PRE>
+__global__ __launch_bounds__(256) void linattn_apply16_kernel(
     const uint16_t* __restrict__ Q, const float* __restrict__ state, void* __restrict__ out,
     const int32_t* __restrict__ chunk_starts, int N, int h, int n_chunks, int wg_tokens,
     int64_t q_stride_b, int64_t q_stride_n, int64_t o_stride_b, int64_t o_stride_n, float eps,
@@ -423,6 +445,7 @@ __global__ __launch_bounds__(256) void linattn_apply_bf16_kernel(
     unsigned char* ostage = stage + SANA_LA_APPLY_U * 2048;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
+      if (t + 16 * u >= t1) break;  // uniform
       const int tok = t + 16 * u + n;
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) {
@@ -431,14 +454,25 @@ __global__ __launch_bounds__(256) void linattn_apply_bf16_kernel(
         if (rope_first) qd = rope8(qd, cs[u][0], cs[u][1]);              // rotated first: both operands
         qd = relu_pk16(qd);                                              // denominator operand
         const u32x4_t qb = (has_rope && !rope_first) ? rope8(qd, cs[u][0], cs[u][1]) : qd;  // numerator operand
+        u32x4_t q_hi, q_lo;
+        if constexpr (is_f16<T>) f16_to_2bf16(qd, q_hi, q_lo);
         f32x4_t acc[3];
 #pragma unroll
         for (int rb = 0; rb < 3; ++rb) {
-          const u32x4_t bop = rb < 2 ? qb : qd;
+          [[maybe_unused]] const u32x4_t bop = rb < 2 ? qb : qd;
           f32x4_t a = {0.f, 0.f, 0.f, 0.f};
-          a = mfma_16x16x32_bf16(st[hh].a[rb][2], bop, a);  // smallest term first
-          a = mfma_16x16x32_bf16(st[hh].a[rb][1], bop, a);
-          a = mfma_16x16x32_bf16(st[hh].a[rb][0], bop, a);
+          if constexpr (is_f16<T>) {  // (no PRE: bop is qd)
+            a = mfma_16x16x32_bf16(st[hh].a[rb][2], q_lo, a);  // smallest terms first
+            a = mfma_16x16x32_bf16(st[hh].a[rb][2], q_hi, a);
+            a = mfma_16x16x32_bf16(st[hh].a[rb][1], q_lo, a);
+            a = mfma_16x16x32_bf16(st[hh].a[rb][1], q_hi, a);
+            a = mfma_16x16x32_bf16(st[hh].a[rb][0], q_lo, a);
+            a = mfma_16x16x32_bf16(st[hh].a[rb][0], q_hi, a);
+          } else {
+            a = mfma_16x16x32_bf16(st[hh].a[rb][2], bop, a);  // smallest term first
+            a = mfma_16x16x32_bf16(st[hh].a[rb][1], bop, a);
+            a = mfma_16x16x32_bf16(st[hh].a[rb][0], bop, a);
+          }
           acc[rb] = a;
         }
         const float den = acc[2][0] + eps;
@@ -458,10 +492,10 @@ __global__ __launch_bounds__(256) void linattn_apply_bf16_kernel(
         } else {
           const float inv = __builtin_amdgcn_rcpf(den);
           u32x4_t o;
-          o.x = pack_bf16(acc[0][0] * inv, acc[0][1] * inv);
-          o.y = pack_bf16(acc[0][2] * inv, acc[0][3] * inv);
-          o.z = pack_bf16(acc[1][0] * inv, acc[1][1] * inv);
-          o.w = pack_bf16(acc[1][2] * inv, acc[1][3] * inv);
+          o.x = pk16<T>(acc[0][0] * inv, acc[0][1] * inv);
+          o.y = pk16<T>(acc[0][2] * inv, acc[0][3] * inv);
+          o.z = pk16<T>(acc[1][0] * inv, acc[1][1] * inv);
+          o.w = pk16<T>(acc[1][2] * inv, acc[1][3] * inv);
           *reinterpret_cast<u32x4_t*>(ostage + slot_r[hh]) = o;
         }
       }
@@ -483,23 +517,14 @@ __global__ __launch_bounds__(256) void linattn_apply_bf16_kernel(
 }
 
 // ----------------------------------------------------------------------------
-// phase 2, fp32 / f16 io: MFMA 32x32x2 f32.  grid as above but wave = one head,
+// phase 2, fp32 io: MFMA 32x32x2 f32.  grid as above but wave = one head,
 // z = B * ceil(h/4).  A lane -> state row lane%32, contraction index 16*(lane/32)+s;
-// B lane -> token lane%32, same contraction index.  The denominator MFMA uses the
-// ksum row in every A row, so the divide is lane-local.
+// B lane -> token lane%32, same contraction index.  The denominator is 16 fused multiply-adds per lane and one exchange
+// with the lane that holds the token's other half.  Tokens x heads, us, against a second
+// MFMA chain for the denominator and scalar loads: 1024 x 36 9.2 -> 5.4, 16384 x 70 167 -> 88.
 // ----------------------------------------------------------------------------
-template <typename TIn, typename TOut>
-__device__ __forceinline__ TOut cvt_out(float x);
-template <>
-__device__ __forceinline__ float cvt_out<float, float>(float x) { return x; }
-template <>
-__device__ __forceinline__ float cvt_out<_Float16, float>(float x) { return x; }
-template <>
-__device__ __forceinline__ _Float16 cvt_out<_Float16, _Float16>(float x) { return (_Float16)x; }
-
-template <typename TIn, typename TOut>
 __global__ __launch_bounds__(256) void linattn_apply32_kernel(
-    const TIn* __restrict__ Q, const float* __restrict__ state, TOut* __restrict__ out,
+    const float* __restrict__ Q, const float* __restrict__ state, float* __restrict__ out,
     const int32_t* __restrict__ chunk_starts, int N, int h, int n_chunks, int wg_tokens,
     int64_t q_stride_b, int64_t q_stride_n, int64_t o_stride_b, int64_t o_stride_n, float eps) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -513,36 +538,41 @@ __global__ __launch_bounds__(256) void linattn_apply32_kernel(
   if (t0 >= t1) return;
   const int n = lane & 31, g = lane >> 5;
   const float* sp = state + ((int64_t)(b * h + head) * n_chunks + c) * STATE_ELEMS;
-  float a_num[16], a_den[16];
+  f32x4_t qn[4];  // (rows start at multiples of 16 bytes)
+  auto load_q = [&](int t) {
+    const float* qp = Q + (int64_t)b * q_stride_b + (int64_t)min(t + n, t1 - 1) * q_stride_n + head * D + 16 * g;
 #pragma unroll
-  for (int s = 0; s < 16; ++s) {
-    a_num[s] = sp[n * D + 16 * g + s];
-    a_den[s] = sp[D * D + 16 * g + s];
+    for (int i = 0; i < 4; ++i) qn[i] = *reinterpret_cast<const f32x4_t*>(qp + 4 * i);
+  };
+  load_q(t0);
+  f32x4_t a_num[4], a_den[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    a_num[i] = *reinterpret_cast<const f32x4_t*>(sp + n * D + 16 * g + 4 * i);
+    a_den[i] = *reinterpret_cast<const f32x4_t*>(sp + D * D + 16 * g + 4 * i);
   }
   for (int t = t0; t < t1; t += 32) {
     const int tok = t + n;
     const bool ok = tok < t1;
-    float qv[16];
-    const TIn* qp = Q + (int64_t)b * q_stride_b + (int64_t)tok * q_stride_n + head * D + 16 * g;
+    float qv[16], den = 0.f;
 #pragma unroll
-    for (int s = 0; s < 16; ++s) qv[s] = ok ? fmaxf((float)qp[s], 0.f) : 0.f;
-    f32x16_t num, den;
+    for (int s = 0; s < 16; ++s) qv[s] = ok ? fmaxf(qn[s >> 2][s & 3], 0.f) : 0.f;
+    if (t + 32 < t1) load_q(t + 32);
+    f32x16_t num;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      num[i] = 0.f;
-      den[i] = 0.f;
-    }
+    for (int i = 0; i < 16; ++i) num[i] = 0.f;
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      num = __builtin_amdgcn_mfma_f32_32x32x2f32(a_num[s], qv[s], num, 0, 0, 0);
-      den = __builtin_amdgcn_mfma_f32_32x32x2f32(a_den[s], qv[s], den, 0, 0, 0);
-    }
+    for (int s = 0; s < 16; ++s) num = __builtin_amdgcn_mfma_f32_32x32x2f32(a_num[s >> 2][s & 3], qv[s], num, 0, 0, 0);
+#pragma unroll
+    for (int s = 0; s < 16; ++s) den = fmaf(a_den[s >> 2][s & 3], qv[s], den);
+    den += __shfl_xor(den, 32, 64);
     if (ok) {
       // D layout: lane -> token (column) lane%32; register r -> channel 8*(r/4)+4*g+r%4
-      const float dd = den[0] + eps;
-      TOut* op = out + (int64_t)b * o_stride_b + (int64_t)tok * o_stride_n + head * D;
+      const float dd = den + eps;
+      float* op = out + (int64_t)b * o_stride_b + (int64_t)tok * o_stride_n + head * D;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) op[8 * (r >> 2) + 4 * g + (r & 3)] = cvt_out<TIn, TOut>(num[r] / dd);
+      for (int r = 0; r < 16; r += 4)
+        *reinterpret_cast<f32x4_t*>(op + 2 * r + 4 * g) = f32x4_t{num[r] / dd, num[r + 1] / dd, num[r + 2] / dd, num[r + 3] / dd};
     }
   }
 }
@@ -826,9 +856,14 @@ static int apply_impl(const void* q, const float* state, void* out, int B, int N
   if (d == 112)
     return launch_apply112(q, state, out, B, N, h, q_stride_b, q_stride_n, o_stride_b, o_stride_n, chunk_starts,
                            n_chunks, max_chunk_tokens, eps, io_dtype, out_dtype, pre, s);
-  const int wg_tokens = io_dtype == SANA_DT_BF16 ? SANA_LA_APPLY_TOKENS : 64;
+  // tokens per workgroup: enough to share the state's preparation, fewer where the grid would not fill the chip (bf16,
+  // tokens x heads, us: 256 x 36 7.1 -> 4.2, 1024 x 36 7.3 -> 4.5, 1024 x 70 7.6 -> 5.9; with 512 workgroups as the
+  // target 2916 x 70 would go from 9.4 to 12.4, with 256 it is 8.9)
+  const int64_t combos = (int64_t)n_chunks * B * (io_dtype == SANA_DT_F32 ? (h + 3) / 4 : ((h + 1) / 2 + 3) / 4);
+  int wg_tokens = io_dtype == SANA_DT_F32 ? 64 : SANA_LA_APPLY_TOKENS;
+  while (wg_tokens > 32 && combos * ((max_chunk_tokens + wg_tokens - 1) / wg_tokens) < SANA_LA_APPLY_MINWG) wg_tokens /= 2;
   const unsigned gx = (unsigned)((max_chunk_tokens + wg_tokens - 1) / wg_tokens);
-  if (io_dtype == SANA_DT_BF16) {
+  if (io_dtype != SANA_DT_F32) {
     const int pairs = (h + 1) / 2;
     dim3 grid(gx, n_chunks, B * ((pairs + 3) / 4));
     // many distinct states (chunk-causal video shapes): keep the readers of one state on one XCD
@@ -837,41 +872,35 @@ static int apply_impl(const void* q, const float* state, void* out, int B, int N
       grid = dim3((unsigned)((ngroups + 7) / 8 * 8) * gx, 1, 1);
     else
       ngroups = 0;
-#define SANA_APPLY(F32, PRE)                                                                                   \
-  hipLaunchKernelGGL((linattn_apply_bf16_kernel<F32, PRE>), grid, dim3(256), 0, s, static_cast<const uint16_t*>(q), \
+#define SANA_APPLY(T, F32, PRE)                                                                                \
+  hipLaunchKernelGGL((linattn_apply16_kernel<T, F32, PRE>), grid, dim3(256), 0, s, static_cast<const uint16_t*>(q), \
                      state, out, chunk_starts, N, h, n_chunks, wg_tokens, q_stride_b, q_stride_n, o_stride_b,     \
                      o_stride_n, eps, pre, (int)gx, ngroups)
     const int mode = (pre.rinv ? 1 : 0) | (pre.rope ? 2 : 0) | (pre.rope_first ? 4 : 0);
-    if (out_dtype == SANA_DT_F32) {
-      if (mode == 7) SANA_APPLY(true, 7);
-      else if (mode == 6) SANA_APPLY(true, 6);
-      else if (mode == 3) SANA_APPLY(true, 3);
-      else if (mode == 2) SANA_APPLY(true, 2);
-      else if (mode == 1) SANA_APPLY(true, 1);
-      else SANA_APPLY(true, 0);
+    if (io_dtype == SANA_DT_F16) {  // (check_pre: no norm or rotation on load)
+      if (out_dtype == SANA_DT_F32) SANA_APPLY(F16, true, 0);
+      else SANA_APPLY(F16, false, 0);
+    } else if (out_dtype == SANA_DT_F32) {
+      if (mode == 7) SANA_APPLY(BF16, true, 7);
+      else if (mode == 6) SANA_APPLY(BF16, true, 6);
+      else if (mode == 3) SANA_APPLY(BF16, true, 3);
+      else if (mode == 2) SANA_APPLY(BF16, true, 2);
+      else if (mode == 1) SANA_APPLY(BF16, true, 1);
+      else SANA_APPLY(BF16, true, 0);
     } else {
-      if (mode == 7) SANA_APPLY(false, 7);
-      else if (mode == 6) SANA_APPLY(false, 6);
-      else if (mode == 3) SANA_APPLY(false, 3);
-      else if (mode == 2) SANA_APPLY(false, 2);
-      else if (mode == 1) SANA_APPLY(false, 1);
-      else SANA_APPLY(false, 0);
+      if (mode == 7) SANA_APPLY(BF16, false, 7);
+      else if (mode == 6) SANA_APPLY(BF16, false, 6);
+      else if (mode == 3) SANA_APPLY(BF16, false, 3);
+      else if (mode == 2) SANA_APPLY(BF16, false, 2);
+      else if (mode == 1) SANA_APPLY(BF16, false, 1);
+      else SANA_APPLY(BF16, false, 0);
     }
 #undef SANA_APPLY
   } else {
     dim3 grid(gx, n_chunks, B * ((h + 3) / 4));
-    if (io_dtype == SANA_DT_F32)
-      hipLaunchKernelGGL((linattn_apply32_kernel<float, float>), grid, dim3(256), 0, s, static_cast<const float*>(q),
-                         state, static_cast<float*>(out), chunk_starts, N, h, n_chunks, wg_tokens, q_stride_b,
-                         q_stride_n, o_stride_b, o_stride_n, eps);
-    else if (out_dtype == SANA_DT_F32)
-      hipLaunchKernelGGL((linattn_apply32_kernel<_Float16, float>), grid, dim3(256), 0, s,
-                         static_cast<const _Float16*>(q), state, static_cast<float*>(out), chunk_starts, N, h,
-                         n_chunks, wg_tokens, q_stride_b, q_stride_n, o_stride_b, o_stride_n, eps);
-    else
-      hipLaunchKernelGGL((linattn_apply32_kernel<_Float16, _Float16>), grid, dim3(256), 0, s,
-                         static_cast<const _Float16*>(q), state, static_cast<_Float16*>(out), chunk_starts, N, h,
-                         n_chunks, wg_tokens, q_stride_b, q_stride_n, o_stride_b, o_stride_n, eps);
+    hipLaunchKernelGGL(linattn_apply32_kernel, grid, dim3(256), 0, s, static_cast<const float*>(q), state,
+                       static_cast<float*>(out), chunk_starts, N, h, n_chunks, wg_tokens, q_stride_b, q_stride_n, o_stride_b,
+                       o_stride_n, eps);
   }
   return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
 }

@@ -140,3 +140,24 @@ def test_chunk_scan_entry_point(cuda):
     ref = st.cumsum(2)
     ops.linattn_chunk_scan_(st)
     torch.testing.assert_close(st, ref, rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("N", [1, 31, 33, 64, 65, 129, 700])
+@pytest.mark.parametrize("dtype,heads", [(torch.float16, 3), (torch.float16, 9), (torch.float32, 5), (torch.bfloat16, 3)])
+def test_phases_at_the_edges_of_their_token_steps(cuda, dtype, heads, N):
+    """Ragged steps, the odd last head of a pair or group, one token; f16 with states beyond the f16 range (its queries are
+    split into two bf16 terms, not the state into f16 ones).  Against fp64: half an ulp of the output per element, 1e-6 in
+    fp32 (sums of up to 700 products)."""
+    g = torch.Generator().manual_seed(N + heads)
+    big = 200.0 if dtype == torch.float16 else 1.0
+    qkv = torch.randn(2, N, 3, 32 * heads, generator=g)
+    qkv[:, :, 1:] *= big
+    qkv = qkv.to(dtype)
+    q, k, v = (t.double().view(2, N, heads, 32).transpose(1, 2) for t in qkv.unbind(2))
+    q, k = q.relu(), k.relu()
+    ref = (q @ (k.transpose(-1, -2) @ v)) / (q @ k.sum(2)[..., None] + 1e-8)
+    ref = ref.transpose(1, 2).reshape(2, N, -1)
+    d = qkv.to(cuda)
+    out = ops.relu_linear_attention(d[:, :, 0], d[:, :, 1], d[:, :, 2], 1e-8).cpu().double()
+    tol = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 1e-6}[dtype]
+    assert ((out - ref).norm() / ref.norm()).item() <= tol
