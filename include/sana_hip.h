@@ -422,6 +422,26 @@ int sana_hip_tconv_residual(const void* X, const void* W, void* out, int M, int 
                             int64_t tap_rows, int64_t x_rows, const unsigned char* zero_last_tap,
                             int64_t ldx, int64_t ldw, int64_t ldo, void* stream);
 
+/* A whole image block (diffusion/model/nets/sana_multi_scale.py:141-157, attn_type "linear", ffn_type "glumbconv") in one
+ * call: the entry points above in the block's order, on one scratch buffer -- for few tokens, where issuing them one by one
+ * takes longer than they run.  16-bit weights of x's dtype (bf16 or f16), head_dim 32 without q/k norm or rotary embedding,
+ * text keys and values computed by the caller.  All rows are dense (row stride = width); every pointer 16-byte aligned.
+ *   x, out [B][N][C]; text_kv [B][text_len] rows of keys, then values, text_ld apart; key_bias [B] rows key_bias_ld apart
+ *   or NULL; the six modulation rows: one per batch entry, mod_stride apart; ones: C values of 1;
+ *   qkv_b, dw_b, point_b may be NULL; split_k: hand the GEMMs a split-k workspace. */
+typedef struct sana_block_args {
+  const void *x, *text_kv, *shift_msa, *scale_msa, *gate_msa, *shift_mlp, *scale_mlp, *gate_mlp;
+  const void *qkv_w, *qkv_b, *proj_w, *proj_b, *q_w, *q_b, *o_w, *o_b, *ones, *inv_w, *inv_b, *dw_w, *dw_b, *point_w, *point_b;
+  const float* key_bias;
+  void *out, *scratch;
+  size_t scratch_bytes;
+  int64_t text_ld, key_bias_ld, mod_stride;
+  int B, N, C, hidden, cross_heads, text_len, H, W, round_like_reference, split_k, io_dtype;
+  float eps_norm1, eps_norm2, eps_attn, cross_scale;
+} sana_block_args;
+size_t sana_hip_block_scratch_bytes(const sana_block_args* args); /* 0: sizes that cannot be */
+int sana_hip_block(const sana_block_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -15,6 +15,19 @@ LIB_PATH = os.path.join(_HERE, "libsana_hip.so")
 DT_F32, DT_BF16, DT_F16 = 0, 1, 2
 EPI_NONE, EPI_BIAS, EPI_BIAS_SILU = 0, 1, 2
 
+
+class BlockArgs(ctypes.Structure):
+    """``sana_block_args`` of include/sana_hip.h."""
+    _fields_ = [(n, c_void_p) for n in (
+        "x", "text_kv", "shift_msa", "scale_msa", "gate_msa", "shift_mlp", "scale_mlp", "gate_mlp",
+        "qkv_w", "qkv_b", "proj_w", "proj_b", "q_w", "q_b", "o_w", "o_b", "ones", "inv_w", "inv_b", "dw_w", "dw_b",
+        "point_w", "point_b", "key_bias", "out", "scratch")] + [("scratch_bytes", c_size_t)] + [
+        (n, c_int64) for n in ("text_ld", "key_bias_ld", "mod_stride")] + [
+        (n, c_int) for n in ("B", "N", "C", "hidden", "cross_heads", "text_len", "H", "W", "round_like_reference",
+                             "split_k", "io_dtype")] + [
+        (n, c_float) for n in ("eps_norm1", "eps_norm2", "eps_attn", "cross_scale")]
+
+
 # name -> (restype, argtypes); must list every symbol include/sana_hip.h declares
 SIGNATURES = {
     "sana_hip_abi_version": (c_int, []),
@@ -79,6 +92,8 @@ SIGNATURES = {
                                          c_int64, c_int64, c_int64, c_int64, c_float, c_void_p]),
     "sana_hip_cross_attention_f16": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                                              c_int64, c_int64, c_int64, c_int64, c_float, c_void_p]),
+    "sana_hip_block_scratch_bytes": (c_size_t, [c_void_p]),
+    "sana_hip_block": (c_int, [c_void_p, c_void_p]),
     "sana_hip_layernorm_modulate": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int,
                                             c_int64, c_int64, c_int, c_int64, c_float, c_int, c_void_p]),
 }

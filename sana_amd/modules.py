@@ -929,8 +929,18 @@ class MultiHeadCrossAttention(nn.Module):
             q = self.q_norm(q)
         if not isinstance(self.k_norm, nn.Identity):
             kv = torch.cat([self.k_norm(kv[:, :, :C]), kv[:, :, C:]], dim=-1)
-        bias = None if mask is None else (1.0 - mask.to(torch.float32)) * -10000.0   # sana_blocks.py:89-90
-        return ops.cross_attention16(q, kv, H, bias)
+        return ops.cross_attention16(q, kv, H, None if mask is None else self._key_bias(mask))
+
+    @staticmethod
+    def _key_bias(mask):
+        return (1.0 - mask.to(torch.float32)) * -10000.0   # sana_blocks.py:89-90
+
+    def _ones(self, x):
+        """[1, 1, C] ones like x: the gate of a plain residual add."""
+        ones = self.__dict__.get("_ones_gate")
+        if ones is None or ones.device != x.device or ones.dtype != x.dtype or ones.shape[-1] != x.shape[-1]:
+            ones = self.__dict__["_ones_gate"] = torch.ones(1, 1, x.shape[-1], dtype=x.dtype, device=x.device)
+        return ones
 
     # rows from which proj + the block's residual add run as ONE GEMM of this library (its gated-residual epilogue
     # with a gate of ones: x + (o W^T + b), the same two roundings as the stock linear and add): all.  us, library GEMM
@@ -948,10 +958,7 @@ class MultiHeadCrossAttention(nn.Module):
         B, N, C = x.shape
         if self._residual_in_gemm(x, cond, mask):
             o = self._attend(x, cond, mask, kv)
-            ones = self.__dict__.get("_ones_gate")
-            if ones is None or ones.device != x.device or ones.dtype != x.dtype or ones.shape[-1] != C:
-                ones = self.__dict__["_ones_gate"] = torch.ones(1, 1, C, dtype=x.dtype, device=x.device)
-            return ops.gemm_gate_residual(o, self.proj.weight, self.proj.bias, ones.expand(B, 1, C), x)
+            return ops.gemm_gate_residual(o, self.proj.weight, self.proj.bias, self._ones(x).expand(B, 1, C), x)
         return x + self(x, cond, mask, kv)
 
     def forward(self, x, cond, mask=None, kv=None):
@@ -1021,6 +1028,56 @@ class SanaMSBlock(nn.Module):
         self.drop_path = nn.Identity()
         self.scale_shift_table = nn.Parameter(torch.randn(6, hidden_size) / hidden_size ** 0.5)
 
+    # What a caller may put over a submodule: found in the instance, the block calls the submodules one by one.
+    _PATCHABLE = frozenset(("forward", "forward_gated", "forward_residual", "_attend", "_linear"))
+
+    def _one_call(self, x, y, modulation, mask, HW, text_kv):
+        """The block as one call into the library (``sana_hip_block``: the same launches in the same order), or None where
+        it does not apply: q/k norm, int8 weights, anything patched, hooked or replaced, unusual strides -- and many bf16
+        tokens, whose qkv projection takes the attention's first phase along and where the host is ahead anyway."""
+        B, N, C = x.shape
+        attn, ca, mlp = self._modules["attn"], self._modules["cross_attn"], self._modules["mlp"]
+        if B * N == 0 or HW is None or len(HW) != 2 or HW[0] * HW[1] != N or type(attn) is not LiteLA \
+                or (x.dtype == torch.bfloat16 and B * N >= attn.STATE_IN_QKV_GEMM_MIN_ROWS) or type(ca) is not MultiHeadCrossAttention \
+                or type(mlp) not in (GLUMBConv, GLUMBConvLinear) or attn.dim != HEAD_DIM or mlp.dilation != 1 \
+                or mlp.out_feature != C or torch.nn.modules.module._has_any_global_hook():
+            return None
+        linears = (attn._modules["qkv"], attn._modules["proj"], ca._modules["q_linear"], ca._modules["proj"])
+        for m, kind in zip(linears, (HipLinear, HipLinear, nn.Linear, nn.Linear)):
+            if type(m) is not kind or m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+                return None
+        for m in (attn, ca, mlp):
+            if not self._PATCHABLE.isdisjoint(m.__dict__):
+                return None
+        for m in (attn, ca):
+            if type(m._modules["q_norm"]) is not nn.Identity or type(m._modules["k_norm"]) is not nn.Identity:
+                return None
+        if not ca._residual_in_gemm(x, y, mask):
+            return None
+        ic, pc, dc = mlp._pointwise_params(mlp.inverted_conv), mlp._pointwise_params(mlp.point_conv), mlp.depth_conv.conv
+        hid, dt = mlp.hidden_features, x.dtype
+        ps = []
+        for m, shape in zip((*linears, ic, dc, pc), ((3 * C, C), (C, C), (C, C), (C, C), (2 * hid, C), (2 * hid, 1), (C, hid))):
+            w, b = m._parameters.get("weight"), m._parameters.get("bias")
+            if w is None or w.dtype != dt or w.shape[:2] != shape or not w.is_cuda or not w.is_contiguous() or w.data_ptr() % 16:
+                return None
+            if b is not None and (b.dtype != dt or b.numel() != shape[0] or not b.is_cuda or not b.is_contiguous()
+                                  or b.data_ptr() % 16):
+                return None
+            ps += (w.data_ptr(), None if b is None else b.data_ptr())
+        if None in (ps[3], ps[5], ps[7], ps[9]) or dc.weight.numel() != 18 * hid or hid % 8 or not x.is_contiguous() \
+                or x.data_ptr() % 16 or modulation.shape != (B, 6, C) or not modulation.is_contiguous() \
+                or not modulation.is_cuda or modulation.data_ptr() % 16:
+            return None
+        kv = ca._linear(ca.kv_linear, y) if text_kv is None else text_kv
+        Nk = y.shape[1]
+        if kv.dtype != dt or not kv.is_cuda or kv.shape != (B, Nk, 2 * C) or kv.stride(2) != 1 or kv.stride(1) % 8 \
+                or kv.stride(0) != Nk * kv.stride(1) or kv.data_ptr() % 16:
+            return None
+        bias = None if mask is None else ca._key_bias(mask)
+        return ops.block(x, kv, bias, modulation, ps, ca._ones(x), hid, ca.num_heads, HW, mlp.round_like_reference,
+                         self.norm1.eps, self.norm2.eps, attn.eps)
+
     def forward(self, x, y, t, mask=None, HW=None, image_rotary_emb=None, **kwargs):
         """The reference's signature (sana_multi_scale.py:141).  Two optional keywords ride in ``kwargs``:
         ``text_kv`` / ``modulation``, this block's share of a ``StepConditioning`` call (kv_linear(y) and
@@ -1034,6 +1091,9 @@ class SanaMSBlock(nn.Module):
         # fused kernels read the modulation rows as x's dtype, so that case takes the stock composition below)
         if x.is_cuda and x.dtype in ops.IO16 and shift_msa.dtype == x.dtype and C % 8 == 0 and C <= 8192 \
                 and not torch.is_grad_enabled():
+            out = self._one_call(x, y, modulation, mask, HW, text_kv) if image_rotary_emb is None else None
+            if out is not None:
+                return out
             # fused seams: LayerNorm + modulate in one kernel, gate * out + residual in the GEMM epilogue
             h = ops.layernorm_modulate(x, scale_msa, shift_msa, self.norm1.eps)
             if "forward" in self.attn.__dict__:

@@ -666,6 +666,31 @@ def add_layernorm_modulate(x: torch.Tensor, y: torch.Tensor, scale: torch.Tensor
     _lib.check(code, "sana_hip_add_layernorm_modulate")
     return total.view(B, Ntok, C), out.view(B, Ntok, C)
 
+
+def block(x, text_kv, key_bias, modulation, weights, ones, hidden, cross_heads, HW, round_like_reference, eps_norm1,
+          eps_norm2, eps_attn) -> torch.Tensor:
+    """A whole image block in one call (``sana_hip_block``).  The caller has checked devices, dtypes, shapes and alignment:
+    x [B, N, C] and modulation [B, 6, C] dense, text_kv [B, Nk, 2C] rows, key_bias fp32 [B, Nk] or None, ``weights`` the
+    weight and bias pointers of qkv, proj, q_linear, cross-attention proj, inverted, depthwise and point convolution."""
+    B, N, C = x.shape
+    lib = _lib.load()
+    out = torch.empty_like(x)
+    mod = modulation.data_ptr()
+    if key_bias is not None:
+        key_bias = key_bias.contiguous()
+    args = _lib.BlockArgs(
+        x.data_ptr(), text_kv.data_ptr(), mod, mod + 2 * C, mod + 4 * C, mod + 6 * C, mod + 8 * C, mod + 10 * C,
+        *weights[:8], ones.data_ptr(), *weights[8:], None if key_bias is None else key_bias.data_ptr(), out.data_ptr(), None, 0,
+        text_kv.stride(1), text_kv.shape[1], 6 * C if B > 1 else 0,
+        B, N, C, hidden, cross_heads, text_kv.shape[1], int(HW[0]), int(HW[1]), 1 if round_like_reference else 0, 1 if SPLIT_K else 0,
+        _dt(x), eps_norm1, eps_norm2, eps_attn, (C // cross_heads) ** -0.5)
+    ref = _lib.ctypes.byref(args)
+    scratch = torch.empty(lib.sana_hip_block_scratch_bytes(ref), dtype=torch.uint8, device=x.device)
+    args.scratch, args.scratch_bytes = scratch.data_ptr(), scratch.numel()
+    _lib.check(lib.sana_hip_block(ref, _stream()), "sana_hip_block")
+    return out
+
+
 CROSS_ATTN_MAX_KEYS = 320     # keys of one (batch, head) that fit LDS together with their values
 
 
