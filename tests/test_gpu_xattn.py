@@ -181,3 +181,38 @@ def test_residual_projection_of_few_rows(cuda, C, H, B, N, Nk, dtype):
     tol = 1e-2 if dtype == torch.bfloat16 else 2e-3
     assert rel_l2(out.cpu(), ref) <= tol
     assert rel_l2(stock.cpu(), torch.nn.functional.linear(x.float(), om.q_linear.weight, om.q_linear.bias)) <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_hooks_and_patches_on_the_cross_attention_of_a_block_run(cuda, dtype):
+    """A hook on, or another forward put over, a block's cross-attention is called at few rows too; a fp16 model's replaced
+    or hooked linears are called, not read past."""
+    C, H = 288, 4
+    torch.manual_seed(0)
+    b = S.SanaMSBlock(C, H, mlp_ratio=2.5).to(dtype).to(cuda).eval()
+    x, y = torch.randn(1, 64, C, dtype=dtype, device=cuda), torch.randn(1, 20, C, dtype=dtype, device=cuda)
+    t = torch.randn(1, 6 * C, dtype=dtype, device=cuda)
+    ca = b.cross_attn
+    with torch.no_grad():
+        ref, seen = b(x, y, t, None, (8, 8)), []
+        handle = ca.register_forward_hook(lambda m, i, o: seen.append(1))
+        b(x, y, t, None, (8, 8))
+        handle.remove()
+        assert seen == [1]
+        ca.forward = lambda x, *a, **k: torch.zeros_like(x)
+        patched = b(x, y, t, None, (8, 8))
+        del ca.forward
+        assert not torch.equal(patched, ref) and torch.equal(b(x, y, t, None, (8, 8)), ref)
+        if dtype == torch.float16:
+            class Doubled(torch.nn.Linear):
+                def forward(self, x):
+                    return 2 * super().forward(x)
+
+            for name in ("q_linear", "kv_linear", "proj"):
+                own = getattr(ca, name)
+                new = Doubled(own.in_features, own.out_features).to(dtype).to(cuda)
+                new.load_state_dict(own.state_dict())
+                setattr(ca, name, new)
+                assert not torch.equal(b(x, y, t, None, (8, 8), **S.StepConditioning([b])(y, t)[0]), ref), name
+                setattr(ca, name, own)
+            assert torch.equal(b(x, y, t, None, (8, 8)), ref)
