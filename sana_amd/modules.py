@@ -1068,23 +1068,24 @@ class SanaMSBlock(nn.Module):
         if not ca._residual_in_gemm(x, y, mask):
             return None
         ic, pc, dc = mlp._pointwise_params(mlp.inverted_conv), mlp._pointwise_params(mlp.point_conv), mlp.depth_conv.conv
-        hid, dt = mlp.hidden_features, x.dtype
+        hid, dt, dev = mlp.hidden_features, x.dtype, x.get_device()
         ps = []
         for m, shape in zip((*linears, ic, dc, pc), ((3 * C, C), (C, C), (C, C), (C, C), (2 * hid, C), (2 * hid, 1), (C, hid))):
             w, b = m._parameters.get("weight"), m._parameters.get("bias")
-            if w is None or w.dtype != dt or w.shape[:2] != shape or not w.is_cuda or not w.is_contiguous() or w.data_ptr() % 16:
+            if w is None or w.dtype != dt or w.shape[:2] != shape or w.get_device() != dev or not w.is_contiguous() or w.data_ptr() % 16:
                 return None
-            if b is not None and (b.dtype != dt or b.numel() != shape[0] or not b.is_cuda or not b.is_contiguous()
+            if b is not None and (b.dtype != dt or b.numel() != shape[0] or b.get_device() != dev or not b.is_contiguous()
                                   or b.data_ptr() % 16):
                 return None
             ps += (w.data_ptr(), None if b is None else b.data_ptr())
         if None in (ps[3], ps[5], ps[7], ps[9]) or dc.weight.numel() != 18 * hid or hid % 8 or not x.is_contiguous() \
                 or x.data_ptr() % 16 or modulation.shape != (B, 6, C) or not modulation.is_contiguous() \
-                or not modulation.is_cuda or modulation.data_ptr() % 16:
+                or modulation.get_device() != dev or modulation.data_ptr() % 16 \
+                or (mask is not None and mask.get_device() != dev):
             return None
         kv = ca._linear(ca.kv_linear, y) if text_kv is None else text_kv
         Nk = y.shape[1]
-        if kv.dtype != dt or not kv.is_cuda or kv.shape != (B, Nk, 2 * C) or kv.stride(2) != 1 or kv.stride(1) % 8 \
+        if kv.dtype != dt or kv.get_device() != dev or kv.shape != (B, Nk, 2 * C) or kv.stride(2) != 1 or kv.stride(1) % 8 \
                 or kv.stride(0) != Nk * kv.stride(1) or kv.data_ptr() % 16:
             return None
         bias = None if mask is None else ca._key_bias(mask)

@@ -86,3 +86,7 @@ def test_what_keeps_the_composition(cuda, monkeypatch):
     big = x.repeat(1, 64, 1)
     run(b, big, (64, 64))
     assert calls == [1, 1]
+    with pytest.raises((ops.SanaHipError, RuntimeError)):       # a mask left on the host: refused, as the composition refuses it
+        with torch.no_grad():
+            b(x, y, t, torch.ones(1, 20), HW)
+    assert calls == [1, 1]
