@@ -189,7 +189,7 @@ def test_hooks_and_patches_on_the_cross_attention_of_a_block_run(cuda, dtype):
     or hooked linears are called, not read past."""
     C, H = 288, 4
     torch.manual_seed(0)
-    b = S.SanaMSBlock(C, H, mlp_ratio=2.5).to(dtype).to(cuda).eval()
+    b = S.SanaMSBlock(C, H, mlp_ratio=2.5, attn_type="linear", ffn_type="glumbconv").to(dtype).to(cuda).eval()
     x, y = torch.randn(1, 64, C, dtype=dtype, device=cuda), torch.randn(1, 20, C, dtype=dtype, device=cuda)
     t = torch.randn(1, 6 * C, dtype=dtype, device=cuda)
     ca = b.cross_attn
