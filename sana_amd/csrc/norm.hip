@@ -11,6 +11,10 @@
 // pass normalises, modulates and stores.  The four roundings of the stock op
 // chain (layer_norm -> 1+scale -> product -> +shift, each a bf16 tensor) are
 // reproduced in registers.
+// Few rows are one latency chain: row, two wave sums, modulation rows, store.  The modulation rows are therefore requested
+// with the row, and the wave sums stay in the vector unit (through LDS a step of the butterfly takes over 100 cycles, twelve of
+// them a row); the row is unpacked once.  us, rows x channels, before and now: 256 x 1152 3.8 -> 3.2, 1024 x 1152 4.3 -> 3.8,
+// 2048 x 1152 5.6 -> 5.0, 1024 x 2240 5.9 -> 5.2, 2048 x 2240 7.6 -> 6.9; 16384 x 2240 (memory) 33.5 -> 32.5.  Same bits.
 #include "common.h"
 
 // No implicit fused multiply-adds in this file: the epilogues reproduce the stock op chain's roundings (product
@@ -28,10 +32,22 @@
 namespace sana {
 namespace {
 
+// The butterfly over lane ^ 32, 16, 8, 4, 2, 1 in the vector unit: v_permlane*_swap of a value with itself puts the two
+// halves (rows) beside each other, and once the lanes i and i ^ 8 agree, a rotation by 4 of a row of 16 is lane ^ 4.
+template <int CTRL>
+__device__ __forceinline__ float lane_move(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+  uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto h = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  u = __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, (uint32_t)h[0]) + __builtin_bit_cast(float, (uint32_t)h[1]));
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+  v += lane_move<0x128>(v);  // row_ror:8
+  v += lane_move<0x124>(v);  // row_ror:4
+  v += lane_move<0x4e>(v);   // quad_perm:[2,3,0,1]
+  return v + lane_move<0xb1>(v);  // quad_perm:[1,0,3,2]
 }
 
 // NCH: 16-byte chunks per lane (C <= 512 * NCH).  ADD: the row is x + y (rounded to bf16, as the stock add
@@ -50,62 +66,72 @@ __global__ __launch_bounds__(256) void ln_modulate_kernel(const uint16_t* __rest
   if (row >= M) return;  // no barriers in this kernel
   const int nchunks = C >> 3;
   const uint16_t* xr = x + row * ldx;
-  u32x4_t raw[NCH];
-  const u32x4_t zero4 = {0u, 0u, 0u, 0u};
+  const int64_t mod = (row / rows_per_mod) * mod_stride;
+  // A lane's chunks, past the row's end its last one once more: no branch around a load, all of them in flight at once.
+  auto chunk = [&](const uint16_t* p, int i) {
+    return reinterpret_cast<const u32x4_t*>(p + 8 * min(lane + 64 * i, nchunks - 1));
+  };
+  constexpr bool AHEAD = NCH <= 5;  // the modulation rows with the row itself, while registers allow
+  u32x4_t raw[NCH], b[ADD ? NCH : 1], sc[AHEAD ? NCH : 1], sh[AHEAD ? NCH : 1];
 #pragma unroll
-  for (int i = 0; i < NCH; ++i) {
-    const int ch = lane + 64 * i;
-    raw[i] = ch < nchunks ? load_stream<SANA_LN_NT_LOAD != 0>(reinterpret_cast<const u32x4_t*>(xr + 8 * ch)) : zero4;
+  for (int i = 0; i < NCH; ++i) raw[i] = load_stream<SANA_LN_NT_LOAD != 0>(chunk(xr, i));
+  if constexpr (ADD) {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) b[i] = load_stream<SANA_LN_NT_LOAD != 0>(chunk(y + row * ldy, i));
   }
-  if (ADD) {
-    const uint16_t* yr = y + row * ldy;
+  if constexpr (AHEAD) {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) sc[i] = *chunk(scale + mod, i), sh[i] = *chunk(shift + mod, i);
+  }
+  if constexpr (ADD) {
     uint16_t* sr = sum + row * lds;
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
-      const int ch = lane + 64 * i;
-      if (ch < nchunks) {
-        const u32x4_t b = load_stream<SANA_LN_NT_LOAD != 0>(reinterpret_cast<const u32x4_t*>(yr + 8 * ch));
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          raw[i][e] = pk16<T>(lo16<T>(raw[i][e]) + lo16<T>(b[e]), hi16<T>(raw[i][e]) + hi16<T>(b[e]));
-        store_stream<SANA_LN_NT_STORE != 0>(raw[i], reinterpret_cast<u32x4_t*>(sr + 8 * ch));
-      }
+      for (int e = 0; e < 4; ++e)
+        raw[i][e] = pk16<T>(lo16<T>(raw[i][e]) + lo16<T>(b[i][e]), hi16<T>(raw[i][e]) + hi16<T>(b[i][e]));
+      if (lane + 64 * i < nchunks)
+        store_stream<SANA_LN_NT_STORE != 0>(raw[i], reinterpret_cast<u32x4_t*>(sr + 8 * (lane + 64 * i)));
     }
   }
-  float s = 0.f;
+  float f[NCH][8], s = 0.f;  // the row, then centred: unpacked once
 #pragma unroll
-  for (int i = 0; i < NCH; ++i)
+  for (int i = 0; i < NCH; ++i) {
+    const bool in = lane + 64 * i < nchunks;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) s += lo16<T>(raw[i][e]) + hi16<T>(raw[i][e]);
+    for (int e = 0; e < 4; ++e) {
+      f[i][2 * e] = lo16<T>(raw[i][e]);
+      f[i][2 * e + 1] = hi16<T>(raw[i][e]);
+      const float pair = f[i][2 * e] + f[i][2 * e + 1];
+      s += in ? pair : 0.f;
+    }
+  }
   const float mean = wave_sum(s) / (float)C;
   float v = 0.f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[i][e] -= mean;
     if (lane + 64 * i < nchunks) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float a = lo16<T>(raw[i][e]) - mean, b = hi16<T>(raw[i][e]) - mean;
-        v = fmaf(a, a, v);
-        v = fmaf(b, b, v);
-      }
+      for (int e = 0; e < 8; ++e) v = fmaf(f[i][e], f[i][e], v);
     }
   }
   const float rstd = rsqrtf(wave_sum(v) / (float)C + eps);
-  const int64_t mod = (row / rows_per_mod) * mod_stride;
   uint16_t* orow = out + row * ldo;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     const int ch = lane + 64 * i;
     if (ch < nchunks) {
-      const u32x4_t sc = *reinterpret_cast<const u32x4_t*>(scale + mod + 8 * ch);
-      const u32x4_t sh = *reinterpret_cast<const u32x4_t*>(shift + mod + 8 * ch);
-      u32x4_t o;
+      u32x4_t c, h, o;
+      if constexpr (AHEAD) c = sc[i], h = sh[i];
+      else c = *chunk(scale + mod, i), h = *chunk(shift + mod, i);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const uint32_t ln = pk16<T>((lo16<T>(raw[i][e]) - mean) * rstd, (hi16<T>(raw[i][e]) - mean) * rstd);
-        const uint32_t s1 = pk16<T>(1.0f + lo16<T>(sc[e]), 1.0f + hi16<T>(sc[e]));
+        const uint32_t ln = pk16<T>(f[i][2 * e] * rstd, f[i][2 * e + 1] * rstd);
+        const uint32_t s1 = pk16<T>(1.0f + lo16<T>(c[e]), 1.0f + hi16<T>(c[e]));
         const uint32_t t = pk16<T>(lo16<T>(ln) * lo16<T>(s1), hi16<T>(ln) * hi16<T>(s1));
-        o[e] = pk16<T>(lo16<T>(t) + lo16<T>(sh[e]), hi16<T>(t) + hi16<T>(sh[e]));
+        o[e] = pk16<T>(lo16<T>(t) + lo16<T>(h[e]), hi16<T>(t) + hi16<T>(h[e]));
       }
       store_stream<SANA_LN_NT_STORE != 0>(o, reinterpret_cast<u32x4_t*>(orow + 8 * ch));
     }

@@ -336,6 +336,26 @@ def test_add_layernorm_modulate_equals_add_then_norm(cuda, B, Ntok, C):
     assert torch.equal(out, ops.layernorm_modulate(x + y, scale, shift, 1e-6))
 
 
+@pytest.mark.parametrize("C", [8, 512, 1032, 1536, 2560, 2568, 4104, 8192])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_layernorm_modulate_at_the_edges_of_a_lanes_chunks(cuda, C, dtype):
+    """One 8-channel chunk, whole and nearly empty rounds of 64 chunks, the first width whose modulation rows are loaded behind
+    the statistics, the widest row; strided rows whose neighbours hold NaN (a chunk read past a row must not count)."""
+    g = torch.Generator().manual_seed(C)
+    wide = torch.full((3, C + 8), float("nan"), dtype=dtype, device=cuda)
+    x = wide[:, :C].view(1, 3, C)
+    x.copy_((torch.randn(3, C, generator=g) * 2 + 0.3).view(1, 3, C))
+    y = torch.randn(1, 3, C, generator=g).to(dtype).to(cuda)
+    mod = (torch.randn(1, 2, C, generator=g) * 0.3).to(dtype).to(cuda)
+    shift, scale = mod[:, 0:1], mod[:, 1:2]
+    tol = 4e-3 if dtype == torch.bfloat16 else 5e-4     # u: four roundings of at most u = 2^-8 (2^-11), u / 3 each in the 2-norm
+    total, out = ops.add_layernorm_modulate(x, y, scale, shift, 1e-6)
+    assert torch.equal(total, x + y) and torch.equal(out, ops.layernorm_modulate(total, scale, shift, 1e-6))
+    for v, o in ((x, ops.layernorm_modulate(x, scale, shift, 1e-6)), (total, out)):
+        ref = F.layer_norm(v.double(), (C,), eps=1e-6) * (1 + scale.double()) + shift.double()
+        assert rel_l2(o, ref) <= tol
+
+
 @pytest.mark.parametrize("C,T,P,B", [(64, 4, 30, 1), (128, 6, 35, 2), (2240, 3, 300, 1)])
 def test_temporal_conv_residual_matches_conv2d(cuda, C, T, P, B):
     """x + t_conv(x) over frames (zero frame in front, zeros behind) against F.conv2d in fp64, with the
