@@ -47,7 +47,7 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "kernels_cfg3_hbm_traffic.txt")
-DOMINANT_KERNEL_ROW = "gemm4_kernel<false, 2, 4>"   # the inverted-conv GEMM (bias + SiLU epilogue, 256-wide channel tile)
+DOMINANT_KERNEL_ROW = "gemm8_kernel<2, 4>"   # the inverted-conv GEMM (bias + SiLU epilogue, 256-wide channel tile)
 
 
 def dominant_kernel_traffic_bytes():
@@ -702,7 +702,7 @@ def main():
     dom = next((r for r in kernels if r["kernel"] == "gemm_inverted"), None)
     roofline = None
     if dom:
-        roofline = {"kernel": "gemm4_kernel<bf16, bias+silu> (inverted 1x1 conv, M=16384 N=11200 K=2240)",
+        roofline = {"kernel": "gemm8_kernel<bf16, bias+silu> (inverted 1x1 conv, M=16384 N=11200 K=2240)",
                     "bound": "mfma", "achieved": dom["achieved"], "peak": dom["peak"], "unit": "TFLOP/s",
                     "frac": dom["frac"], "traffic": dominant_kernel_traffic_bytes()}
     line = {

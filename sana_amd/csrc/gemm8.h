@@ -141,7 +141,7 @@ __device__ __forceinline__ void g8_state_tile(f32x4_t (&acc)[4][8], const float 
 // that settles at 1.68 - 1.8 GHz on random operands; a tile's epilogue costs ~6000 cycles, ~13000 with SiLU (two quarter-rate
 // transcendentals per output), and nothing else is exposed.  Against the one-wave-per-SIMD kernel with register-staged
 // operands that it replaced (2657 cycles per k-tile, 8600 / 15700 of epilogue, 3200 of prologue), us on one card: 16384
-// tokens, inverted conv + SiLU 646 -> 589, bias only 612 -> 562, qkv 378 -> 350, proj 147 -> 139, point conv 343 -> 305.
+// tokens, inverted conv + SiLU 646 -> 589, bias only 612 -> 562, qkv 378 -> 350, proj 147 -> 139, point conv 343 -> 333.
 //
 // Waves (wm, wn) = (wave / 4, wave % 4): 128 tokens x 16*NB channels each = 8 x NB tiles of v_mfma_f32_16x16x32 (the
 // weight tile is the row operand: a lane owns one token and, by the order in which weight rows are placed in LDS, 8

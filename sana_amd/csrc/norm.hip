@@ -14,7 +14,8 @@
 // Few rows are one latency chain: row, two wave sums, modulation rows, store.  The modulation rows are therefore requested
 // with the row, and the wave sums stay in the vector unit (through LDS a step of the butterfly takes over 100 cycles, twelve of
 // them a row); the row is unpacked once.  us, rows x channels, before and now: 256 x 1152 3.8 -> 3.2, 1024 x 1152 4.3 -> 3.8,
-// 2048 x 1152 5.6 -> 5.0, 1024 x 2240 5.9 -> 5.2, 2048 x 2240 7.6 -> 6.9; 16384 x 2240 (memory) 33.5 -> 32.5.  Same bits.
+// 2048 x 1152 5.6 -> 5.0, 1024 x 2240 5.9 -> 5.2, 2048 x 2240 7.6 -> 6.9; 16384 x 2240 33.5 -> 32.5 (vector unit 0.99 busy, at the copy rate).
+// Same bits.
 #include "common.h"
 
 // No implicit fused multiply-adds in this file: the epilogues reproduce the stock op chain's roundings (product
