@@ -1003,6 +1003,9 @@ int launch(const void* A, const void* W, const float* scale, const EpiArgs& ep, 
   }
 }
 
+// Row strides from which the 32-bit offsets inside a tile's 256 rows could overflow.
+constexpr int64_t kMaxTileStride = 1 << 22;
+
 int check_common(const void* A, const void* W, const void* bias, const void* C, int M, int N, int K, int64_t lda,
                  int64_t ldw, int64_t ldc, int epilogue, int kmult, int ldw_mult) {
   if (!A || !W || !C || M <= 0 || N <= 0 || K <= 0) return SANA_ERR_ARG;
@@ -1010,7 +1013,7 @@ int check_common(const void* A, const void* W, const void* bias, const void* C, 
   if (epilogue < SANA_EPI_NONE || epilogue > SANA_EPI_GATE_RES) return SANA_ERR_ARG;
   if (K % kmult || N % 8) return SANA_ERR_SHAPE;
   if (lda < K || ldw < K || ldc < N) return SANA_ERR_ARG;
-  if (lda >= (1 << 22) || ldw >= (1 << 22) || ldc >= (1 << 22)) return SANA_ERR_SHAPE;  // 32-bit offsets inside a tile's rows
+  if (lda >= kMaxTileStride || ldw >= kMaxTileStride || ldc >= kMaxTileStride) return SANA_ERR_SHAPE;
   if (lda % 8 || ldw % ldw_mult || ldc % 8 || !aligned16(A) || !aligned16(W) || !aligned16(C)) return SANA_ERR_ALIGN;
   return SANA_OK;
 }
@@ -1021,6 +1024,24 @@ int check_gate_res(const void* gate, const void* residual, int M, int N, int64_t
   if (ldr < N || gate_stride < 0) return SANA_ERR_ARG;
   if (ldr % 8 || gate_stride % 8 || !aligned16(gate) || !aligned16(residual)) return SANA_ERR_ALIGN;
   return SANA_OK;
+}
+
+// C = residual + gate * (A . W^T + bias).  Rows of the residual further apart than a tile's offsets reach (one token of each
+// of many long sequences, say) are added by the elementwise kernel, whose addresses have 64 bits, on the linear output in C:
+// the same three roundings.
+template <bool W8, typename T = BF16>
+int launch_gate_res(const void* A, const void* W, const float* scale, EpiArgs e, void* C, int M, int N, int K, int64_t lda,
+                    int64_t ldw, int64_t ldc, void* stream, void* workspace, size_t workspace_bytes) {
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (M == 1) e.ldr = N;  // a single row has no stride (and may be C itself)
+  if (e.ldr < kMaxTileStride)
+    return launch<W8, T>(A, W, scale, e, C, M, N, K, lda, ldw, ldc, SANA_EPI_GATE_RES, s, workspace, workspace_bytes);
+  EpiArgs lin = e;
+  lin.gate = lin.res = nullptr, lin.ldr = lin.gate_stride = 0;
+  const int rc = launch<W8, T>(A, W, scale, lin, C, M, N, K, lda, ldw, ldc, SANA_EPI_BIAS, s, workspace, workspace_bytes);
+  return rc != SANA_OK ? rc
+                       : sana_hip_gate_residual(C, e.gate, e.res, C, M, N, ldc, e.ldr, ldc, e.rows_per_gate, e.gate_stride,
+                                                is_f16<T> ? SANA_DT_F16 : SANA_DT_BF16, stream);
 }
 
 // Sum of the per-token-tile partial states of the fused qkv projection: part[bh][nsplit][33 * 32] -> state[bh][33 * 32].
@@ -1133,11 +1154,8 @@ SANA_API int sana_hip_gemm_gate_residual(const void* A, const void* W, const flo
   if (rc != SANA_OK) return rc;
   const EpiArgs e = {static_cast<const uint16_t*>(bias), static_cast<const uint16_t*>(gate),
                      static_cast<const uint16_t*>(residual), ldr, gate_stride, rows_per_gate, nullptr, 0, 0, 0, 0};
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  return w8 ? launch<true>(A, W, w8_scale, e, C, M, N, K, lda, ldw, ldc, SANA_EPI_GATE_RES, s, workspace,
-                           workspace_bytes)
-            : launch<false>(A, W, nullptr, e, C, M, N, K, lda, ldw, ldc, SANA_EPI_GATE_RES, s, workspace,
-                            workspace_bytes);
+  return w8 ? launch_gate_res<true>(A, W, w8_scale, e, C, M, N, K, lda, ldw, ldc, stream, workspace, workspace_bytes)
+            : launch_gate_res<false>(A, W, nullptr, e, C, M, N, K, lda, ldw, ldc, stream, workspace, workspace_bytes);
 }
 
 SANA_API int sana_hip_gemm_gate_residual_f16(const void* A, const void* W, const void* bias, const void* gate,
@@ -1151,8 +1169,7 @@ SANA_API int sana_hip_gemm_gate_residual_f16(const void* A, const void* W, const
   if (rc != SANA_OK) return rc;
   const EpiArgs e = {static_cast<const uint16_t*>(bias), static_cast<const uint16_t*>(gate),
                      static_cast<const uint16_t*>(residual), ldr, gate_stride, rows_per_gate, nullptr, 0, 0, 0, 0};
-  return launch<false, F16>(A, W, nullptr, e, C, M, N, K, lda, ldw, ldc, SANA_EPI_GATE_RES,
-                            static_cast<hipStream_t>(stream), workspace, workspace_bytes);
+  return launch_gate_res<false, F16>(A, W, nullptr, e, C, M, N, K, lda, ldw, ldc, stream, workspace, workspace_bytes);
 }
 
 SANA_API int sana_hip_tconv_residual(const void* X, const void* W, void* out, int M, int C, int taps,

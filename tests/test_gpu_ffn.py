@@ -304,6 +304,23 @@ def test_gemm_gate_residual_matches_stock_op_chain(cuda, B, Ntok, C, K, w8):
     assert rel_l2(out, ref) <= 4e-3
 
 
+@pytest.mark.parametrize("ldr", [2240 * 16384, (1 << 23) + 8, (1 << 22) + 8])
+@pytest.mark.parametrize("M,dtype,w8", [(64, torch.bfloat16, False), (64, torch.bfloat16, True), (130, torch.float16, False)])
+def test_gemm_gate_residual_rows_far_apart(cuda, M, dtype, w8, ldr):
+    """One token of each of many long sequences as the residual: the rows of one tile span more than 32-bit offsets reach
+    (64 rows of 16384 x 2240 values: 4.7 GB).  The same bits as with the residual's rows side by side."""
+    C, K = 264, 128
+    g = torch.Generator().manual_seed(M)
+    a = torch.randn(M, 1, K, generator=g).to(dtype).to(cuda)
+    w, bias = (torch.randn(C, K, generator=g) * 0.05).to(dtype), torch.randn(C, generator=g).to(dtype).to(cuda)
+    gate, res = (torch.randn(M, 1, C, generator=g).to(dtype).to(cuda) for _ in range(2))
+    far = torch.empty((M - 1) * ldr + C, dtype=dtype, device=cuda).as_strided((M, 1, C), (ldr, C, 1)).copy_(res)
+    wq, s = O.quantize_w8(w) if w8 else (w, None)
+    args = (a, wq.to(cuda), bias, gate)
+    kw = dict(weight_scale=s.to(cuda), expand=False) if w8 else {}
+    assert torch.equal(ops.gemm_gate_residual(*args, far, **kw), ops.gemm_gate_residual(*args, res, **kw))
+
+
 @pytest.mark.parametrize("B,Ntok,C", [(1, 16384, 2240), (4, 1024, 1152), (2, 77, 96), (1, 5, 4096)])
 def test_layernorm_modulate_matches_stock_op_chain(cuda, B, Ntok, C):
     g = torch.Generator().manual_seed(C)
