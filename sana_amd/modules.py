@@ -922,7 +922,8 @@ class MultiHeadCrossAttention(nn.Module):
     @staticmethod
     def _linear(linear, x):
         if MultiHeadCrossAttention._gemm_takes(linear, x):
-            return ops.gemm_bf16(x.view(-1, x.shape[-1]), linear.weight, linear.bias, "bias").view(*x.shape[:-1], -1)
+            w = linear.weight     # (no -1 in the view: x may be empty)
+            return ops.gemm_bf16(x.view(-1, x.shape[-1]), w, linear.bias, "bias").view(*x.shape[:-1], w.shape[0])
         return F.linear(x, linear.weight, linear.bias)
 
     def _attend(self, x, cond, mask, kv=None):

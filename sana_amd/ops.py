@@ -722,7 +722,9 @@ def cross_attention16(q: torch.Tensor, kv: torch.Tensor, num_heads: int, key_bia
     d = C // num_heads
     if not cross_attention_supported(d, Nk):
         raise SanaHipError(f"cross_attention holds one head's keys in LDS: head_dim {d} (72 .. 112), {Nk} keys (<= 320)")
-    if q.stride(2) != 1 or kv.stride(2) != 1 or q.stride(0) != N * q.stride(1) or kv.stride(0) != Nk * kv.stride(1):
+    # (the strides of an empty tensor mean nothing)
+    if B * N and (q.stride(2) != 1 or kv.stride(2) != 1 or q.stride(0) != N * q.stride(1)
+                  or kv.stride(0) != Nk * kv.stride(1)):
         raise SanaHipError("cross_attention needs q and kv rows with unit inner stride, batch entries back to back")
     if key_bias is not None:
         if key_bias.dtype != torch.float32 or key_bias.shape != (B, Nk) or key_bias.stride(1) != 1:

@@ -300,6 +300,22 @@ def test_empty_inputs(cuda):
         assert ob.attn(x0.cpu(), HW=(4, 4)).shape == (0, 16, C) and ob.mlp(x0.cpu(), HW=(4, 4)).shape == (0, 16, C)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_empty_inputs_of_the_cross_attention(cuda, dtype):
+    """No batch entries / no tokens, at a head_dim the short-key kernel takes: empty tensors, as the stock ops return."""
+    C, H = 288, 4
+    hb = S.SanaMSBlock(C, H, mlp_ratio=2.5, attn_type="linear", ffn_type="glumbconv").to(dtype).to(cuda).eval()
+    y, t = torch.randn(2, 20, C, dtype=dtype, device=cuda), torch.randn(2, 6 * C, dtype=dtype, device=cuda)
+    mask = torch.ones(2, 20, dtype=torch.int16, device=cuda)
+    with torch.no_grad():
+        x0, xn = (torch.zeros(*s, C, dtype=dtype, device=cuda) for s in ((0, 16), (2, 0)))
+        assert hb.cross_attn(x0, y[:0]).shape == (0, 16, C) and hb.cross_attn.forward_residual(x0, y[:0]).shape == (0, 16, C)
+        assert hb.cross_attn(xn, y, mask).shape == (2, 0, C) and hb.cross_attn.forward_residual(xn, y).shape == (2, 0, C)
+        for m in (None, mask):
+            assert hb(xn, y, t, m, (0, 0)).shape == (2, 0, C)
+            assert hb(xn, y, t, m, (0, 0), **S.StepConditioning([hb])(y, t)[0]).shape == (2, 0, C)
+
+
 def test_block_replays_from_a_hip_graph(cuda):
     """The whole block (hand-written kernels, stock cross-attention, the cached workspace) captured once into a HIP
     graph: every replay, with eager launches and synchronisations between them, reproduces the eager result bit
