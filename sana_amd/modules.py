@@ -948,13 +948,6 @@ class MultiHeadCrossAttention(nn.Module):
     def _key_bias(mask):
         return (1.0 - mask.to(torch.float32)) * -10000.0   # sana_blocks.py:89-90
 
-    def _ones(self, x):
-        """[1, 1, C] ones like x: the gate of a plain residual add."""
-        ones = self.__dict__.get("_ones_gate")
-        if ones is None or ones.device != x.device or ones.dtype != x.dtype or ones.shape[-1] != x.shape[-1]:
-            ones = self.__dict__["_ones_gate"] = torch.ones(1, 1, x.shape[-1], dtype=x.dtype, device=x.device)
-        return ones
-
     # rows from which proj + the block's residual add run as ONE GEMM of this library (its gated-residual epilogue
     # with a gate of ones: x + (o W^T + b), the same two roundings as the stock linear and add): all.  us, library GEMM
     # and the add's share of the pass behind it against this: 256 x 1152 7.0 + 1 / 6.8, 2048 x 1152 12.5 + 3 / 11.9,
@@ -972,7 +965,7 @@ class MultiHeadCrossAttention(nn.Module):
         B, N, C = x.shape
         if self._residual_in_gemm(x, cond, mask):
             o = self._attend(x, cond, mask, kv)
-            return ops.gemm_gate_residual(o, self.proj.weight, self.proj.bias, self._ones(x).expand(B, 1, C), x)
+            return ops.gemm_gate_residual(o, self.proj.weight, self.proj.bias, ops.ones_row(C, x.dtype, x.device).expand(B, 1, C), x)
         return x + self(x, cond, mask, kv)
 
     def forward(self, x, cond, mask=None, kv=None):
@@ -1090,7 +1083,7 @@ class SanaMSBlock(nn.Module):
                 or kv.stride(0) != Nk * kv.stride(1) or kv.data_ptr() % 16:
             return None
         bias = None if mask is None else ca._key_bias(mask)
-        return ops.block(x, kv, bias, modulation, ps, ca._ones(x), hid, ca.num_heads, HW, mlp.round_like_reference,
+        return ops.block(x, kv, bias, modulation, ps, ops.ones_row(C, x.dtype, x.device), hid, ca.num_heads, HW, mlp.round_like_reference,
                          self.norm1.eps, self.norm2.eps, attn.eps)
 
     def forward(self, x, y, t, mask=None, HW=None, image_rotary_emb=None, **kwargs):

@@ -570,6 +570,21 @@ def gemm_gate_residual(a: torch.Tensor, weight: torch.Tensor, bias: Optional[tor
     return out.view(B, Ntok, C)
 
 
+_ones_rows = {}      # (device index, dtype, C) -> [C] tensor of ones
+
+
+def ones_row(C: int, dtype: torch.dtype, device: torch.device) -> torch.Tensor:
+    """[C] ones, the gate of a plain residual add.  Kept for the process (a captured graph may hold the address) and copied
+    from the host, so that it is there for every stream when it is returned; made while a graph is captured it belongs to
+    that graph, whose replays fill it, and is not kept."""
+    t = _ones_rows.get((device.index, dtype, C))
+    if t is None:
+        if torch.cuda.is_current_stream_capturing():
+            return torch.ones(C, dtype=dtype, device=device)
+        t = _remember(_ones_rows, (device.index, dtype, C), lambda: torch.ones(C, dtype=dtype).to(device))
+    return t
+
+
 _frame_flags = {}    # (device index, n_frames, tuple of flagged frames) -> uint8 tensor
 
 

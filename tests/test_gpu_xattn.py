@@ -216,3 +216,26 @@ def test_hooks_and_patches_on_the_cross_attention_of_a_block_run(cuda, dtype):
                 assert not torch.equal(b(x, y, t, None, (8, 8), **S.StepConditioning([b])(y, t)[0]), ref), name
                 setattr(ca, name, own)
             assert torch.equal(b(x, y, t, None, (8, 8)), ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_residual_projection_first_called_inside_a_capture(cuda, dtype):
+    """A caller's own graph captures the call before anything ran eagerly, and is not replayed yet: eager calls must not
+    meet memory that only a replay fills, and replays (eager work between them) give the eager bits."""
+    C, H = (352 if dtype == torch.bfloat16 else 416), 4      # widths of no other test: nothing is kept for them yet
+    torch.manual_seed(1)
+    ca = S.modules.MultiHeadCrossAttention(C, H).to(dtype).to(cuda)
+    x, y = torch.randn(2, 24, C, dtype=dtype, device=cuda), torch.randn(2, 12, C, dtype=dtype, device=cuda)
+    with torch.no_grad():
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            captured = ca.forward_residual(x, y)
+        eager = ca.forward_residual(x, y)
+        plain = x + ca(x, y)
+        # the same products and roundings; the two GEMM calls may sum in another order
+        assert (eager.float() - plain.float()).abs().max().item() <= 2 ** -7 * plain.float().abs().max().item()
+        for _ in range(3):
+            captured.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(captured, eager) and torch.equal(ca.forward_residual(x, y), eager)
