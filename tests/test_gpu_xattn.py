@@ -239,3 +239,29 @@ def test_residual_projection_first_called_inside_a_capture(cuda, dtype):
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(captured, eager) and torch.equal(ca.forward_residual(x, y), eager)
+
+
+def test_fp16_cross_attention_stays_visible_to_who_watches_its_ops(cuda):
+    """vmap, torch.jit.trace and autocast to another dtype see stock ops (a call into the library is invisible to them: vmap
+    raised, a trace recorded an unfilled buffer, autocast lost its dtype), and a kv in other rows than the kernel reads or a
+    mask in other strides is taken as before."""
+    C, H = 288, 4
+    torch.manual_seed(2)
+    ca = S.modules.MultiHeadCrossAttention(C, H).half().to(cuda)
+    xs, y = torch.randn(3, 2, 16, C, dtype=torch.half, device=cuda), torch.randn(2, 12, C, dtype=torch.half, device=cuda)
+    with torch.no_grad():
+        refs = torch.stack([ca(x, y) for x in xs])
+        assert rel_l2(torch.vmap(lambda x: ca(x, y))(xs), refs) <= 2e-3
+        traced = torch.jit.trace(ca, (xs[0], y), check_trace=False)
+        assert rel_l2(traced(xs[1], y), refs[1]) <= 2e-3
+        with torch.autocast("cuda", torch.bfloat16):
+            assert ca(xs[0], y).dtype == torch.bfloat16
+        with torch.autocast("cuda", torch.float16):
+            assert torch.equal(ca(xs[0], y), refs[0])
+        kv = torch.nn.functional.linear(y, ca.kv_linear.weight, ca.kv_linear.bias)
+        wide = torch.cat([kv, kv], 1)[:, :12]         # batch entries not back to back
+        assert rel_l2(ca(xs[0], y, None, wide), refs[0]) <= 2e-3
+        mask = torch.ones(12, 2, device=cuda).t()
+        mask[1, 7:] = 0
+        assert mask.stride() == (1, 2)
+        assert torch.equal(ca(xs[0], y, mask), ca(xs[0], y, mask.contiguous()))
