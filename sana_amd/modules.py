@@ -931,10 +931,12 @@ class MultiHeadCrossAttention(nn.Module):
 
     @staticmethod
     def _gemm_takes(linear, x) -> bool:
-        """Rows, alignment and dtypes of this library's GEMM (anything else is a stock linear, as it always was)."""
+        """Rows, alignment, dtypes and devices of this library's GEMM, and weights that are what they seem (anything else,
+        a quantised tensor subclass say, is a stock linear, as it always was)."""
         w, b = linear.weight, linear.bias
-        return (x.is_contiguous() and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0
-                and w.dtype == x.dtype and b is not None and b.dtype == x.dtype and b.is_contiguous()
+        return (type(w) in _PLAIN and type(b) in _PLAIN and w.get_device() == x.get_device() == b.get_device()
+                and x.is_contiguous() and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0
+                and w.dtype == x.dtype and b.dtype == x.dtype and b.is_contiguous()
                 and b.data_ptr() % 16 == 0 and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0)
 
     @staticmethod
@@ -1084,9 +1086,9 @@ class SanaMSBlock(nn.Module):
         ps = []
         for m, shape in zip((*linears, ic, dc, pc), ((3 * C, C), (C, C), (C, C), (C, C), (2 * hid, C), (2 * hid, 1), (C, hid))):
             w, b = m._parameters.get("weight"), m._parameters.get("bias")
-            if w is None or w.dtype != dt or w.shape[:2] != shape or w.get_device() != dev or not w.is_contiguous() or w.data_ptr() % 16:
+            if type(w) not in _PLAIN or w.dtype != dt or w.shape[:2] != shape or w.get_device() != dev or not w.is_contiguous() or w.data_ptr() % 16:
                 return None
-            if b is not None and (b.dtype != dt or b.numel() != shape[0] or b.get_device() != dev or not b.is_contiguous()
+            if b is not None and (type(b) not in _PLAIN or b.dtype != dt or b.numel() != shape[0] or b.get_device() != dev or not b.is_contiguous()
                                   or b.data_ptr() % 16):
                 return None
             ps += (w.data_ptr(), None if b is None else b.data_ptr())

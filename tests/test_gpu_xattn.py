@@ -265,3 +265,39 @@ def test_fp16_cross_attention_stays_visible_to_who_watches_its_ops(cuda):
         mask[1, 7:] = 0
         assert mask.stride() == (1, 2)
         assert torch.equal(ca(xs[0], y, mask), ca(xs[0], y, mask.contiguous()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_tensor_subclass_weights_of_the_cross_attention_are_dispatched(cuda, dtype):
+    """A weight that is a tensor subclass (as quantisation libraries put in) sees its linear, alone and in a block."""
+    C, H = 288, 4
+    torch.manual_seed(3)
+    b = S.SanaMSBlock(C, H, mlp_ratio=2.5, attn_type="linear", ffn_type="glumbconv").to(dtype).to(cuda).eval()
+    x, y = torch.randn(1, 64, C, dtype=dtype, device=cuda), torch.randn(1, 20, C, dtype=dtype, device=cuda)
+    t = torch.randn(1, 6 * C, dtype=dtype, device=cuda)
+    seen = []
+
+    class Doubled(torch.Tensor):
+        """Stands for twice its memory."""
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            if func is torch.nn.functional.linear:
+                seen.append(1)
+                with torch._C.DisableTorchFunctionSubclass():
+                    return torch.nn.functional.linear(args[0], 2 * args[1].as_subclass(torch.Tensor), args[2])
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    with torch.no_grad():
+        ref = b(x, y, t, None, (8, 8))
+        for name in ("q_linear", "kv_linear", "proj"):
+            lin = getattr(b.cross_attn, name)
+            own = lin.weight
+            half = (own.detach() / 2).as_subclass(Doubled)
+            lin.weight = torch.nn.Parameter(half, requires_grad=False)
+            for f in (lambda: b(x, y, t, None, (8, 8)), lambda: x + b.cross_attn(x, y)):
+                seen.clear()
+                out = f()
+                assert seen, name
+            lin.weight = own
+            assert rel_l2(out, x + b.cross_attn(x, y)) <= (1e-2 if dtype == torch.bfloat16 else 2e-3), name
+        assert torch.equal(b(x, y, t, None, (8, 8)), ref)
