@@ -341,8 +341,25 @@ __device__ __forceinline__ void f16_to_2bf16(u32x4_t q, u32x4_t& hi, u32x4_t& lo
   }
 }
 
+// num / den for many numerators, rounded as the division is: the reciprocal with one Newton step, the product corrected by its
+// residual (an exact fma), and the division's own handling of zeros, infinities and NaN.  f16 outputs need it: where the
+// quotient lies halfway between two f16 values the error of num * rcp(den) decides the rounding.  Denominators beyond 2^126,
+// whose reciprocal is not a normal number, do not occur (the operands are f16).  16384 x 70, us: num * rcp(den) 36, the
+// compiler's division 48, this 39.
+struct Quotient {
+  float den, inv;
+  __device__ __forceinline__ explicit Quotient(float d) : den(d) {
+    inv = __builtin_amdgcn_rcpf(d);
+    inv = fmaf(fmaf(-d, inv, 1.0f), inv, inv);
+  }
+  __device__ __forceinline__ float operator()(float num) const {
+    const float q = num * inv;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-den, q, num), inv, q), den, num);
+  }
+};
+
 // T = F16 replaces MFMAs in fp32 (32x32x2) and 2-byte loads and stores: tokens x heads, us: 2048 x 36
-// 16.5 -> 7.1, 16384 x 70 125 -> 34.
+// 16.5 -> 7.2, 16384 x 70 125 -> 36.
 template <typename T, bool OUT_F32, int PRE>
 __global__ __launch_bounds__(256) void linattn_apply16_kernel(
     const uint16_t* __restrict__ Q, const float* __restrict__ state, void* __restrict__ out,
@@ -490,12 +507,16 @@ __global__ __launch_bounds__(256) void linattn_apply16_kernel(
             store_stream<SANA_LA_NT_STORE != 0>(o1, reinterpret_cast<f32x4_t*>(op + 4));
           }
         } else {
-          const float inv = __builtin_amdgcn_rcpf(den);
           u32x4_t o;
-          o.x = pk16<T>(acc[0][0] * inv, acc[0][1] * inv);
-          o.y = pk16<T>(acc[0][2] * inv, acc[0][3] * inv);
-          o.z = pk16<T>(acc[1][0] * inv, acc[1][1] * inv);
-          o.w = pk16<T>(acc[1][2] * inv, acc[1][3] * inv);
+          if constexpr (is_f16<T>) {
+            const Quotient by(den);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = pk16<T>(by(acc[e >> 1][2 * (e & 1)]), by(acc[e >> 1][2 * (e & 1) + 1]));
+          } else {
+            const float inv = __builtin_amdgcn_rcpf(den);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = pk16<T>(acc[e >> 1][2 * (e & 1)] * inv, acc[e >> 1][2 * (e & 1) + 1] * inv);
+          }
           *reinterpret_cast<u32x4_t*>(ostage + slot_r[hh]) = o;
         }
       }

@@ -161,3 +161,18 @@ def test_phases_at_the_edges_of_their_token_steps(cuda, dtype, heads, N):
     out = ops.relu_linear_attention(d[:, :, 0], d[:, :, 1], d[:, :, 2], 1e-8).cpu().double()
     tol = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 1e-6}[dtype]
     assert ((out - ref).norm() / ref.norm()).item() <= tol
+
+
+def test_f16_quotients_halfway_between_two_f16_values_round_to_even(cuda):
+    """Integers m D over D with m odd and of 12 bits: numerator, denominator and quotient are exact in fp32 and the quotient lies
+    halfway between two f16 values, so whatever a reciprocal is off by shows as a wrong rounding."""
+    heads, tokens = 3, 70
+    dk = torch.arange(32)
+    D = (2 * dk + 3).float()                                             # 3, 5, .. 65
+    m = 2049 + 2 * ((torch.arange(heads * 32).view(heads, 32, 1) * 37 + dk * 11) % 1023)      # [head][dv][dk]
+    state = torch.cat([m.float() * D, D.expand(heads, 1, 32)], 1).view(1, heads, 1, 33, 32).contiguous()
+    q = torch.zeros(1, tokens, heads, 32)
+    at = torch.arange(tokens) % 32
+    q[0, torch.arange(tokens), :, at] = 1                                # picks one dk per token
+    out = ops.linattn_apply(q.view(1, tokens, -1).half().to(cuda), state.to(cuda), 0.0)
+    assert torch.equal(out.cpu().view(tokens, heads, 32), m[:, :, at].permute(2, 0, 1).half())
