@@ -1100,7 +1100,8 @@ using namespace sana;
 
 SANA_API size_t sana_hip_gemm_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || N % 8) return 0;
-  return split_bytes(plan_gemm(M, N, K, false), M, N);
+  const GemmPlan pl = plan_gemm(M, N, K, false);
+  return split_pays(pl, M, N, K) ? split_bytes(pl, M, N) : 0;
 }
 
 // From 4096 rows on always (converting in the main loop costs it 14 % at every M, the expansion a fixed 10 - 20 us); below

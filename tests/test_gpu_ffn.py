@@ -227,14 +227,15 @@ def test_gemm_w8a16_equals_bf16_gemm_on_dequantised_weight(cuda, M, N, K, epilog
     assert rel_l2(y8.cpu(), ref) <= 4e-3
 
 
-@pytest.mark.parametrize("M,N,K", [(1024, 2240, 5600),    # point conv of one 1024 px image: 4 k ranges
-                                   (256, 2240, 2240),     # 4 ranges of 9, 9, 9 and 8 k-tiles
-                                   (1000, 1152, 2880),    # ragged rows, 600M widths
-                                   (300, 72, 1184),       # two tiles, k ranges of 10 and 9 k-tiles, a k tail of one k-step of 32
-                                   (2048, 2240, 5600)])   # 2 ranges
+@pytest.mark.parametrize("M,N,K", [(1024, 2240, 5600),    # point conv of one 1024 px image: k ranges of 18, 18, 18, 17 and 17 k-tiles
+                                   (700, 2240, 5600),     # ragged rows, 7 ranges
+                                   (1400, 1152, 5600),    # the narrower width, 7 ranges
+                                   (300, 264, 5664),      # few tiles, ranges of 12 and 11 k-tiles, a k tail of one k-step of 32
+                                   (1001, 1160, 5728),    # ragged rows and channels, a k tail
+                                   (1, 72, 5600)])        # one row
 def test_gemm_split_k(cuda, monkeypatch, M, N, K):
-    """Shapes with too few output tiles run as split-k through the workspace: against the fp64 oracle to the same
-    bounds as the fused path, against the unsplit kernel to fp32 summation-order noise, bit-identical between the
+    """Shapes with too few output tiles run as split-k through the workspace (the query answers 0 where they do not):
+    against the fp64 oracle to the same bounds as the fused path, against the unsplit kernel to fp32 summation-order noise, bit-identical between the
     bf16, int8 and gated-residual entry points (they share the plan), and exact on integer inputs."""
     from sana_amd import _lib
     assert _lib.load().sana_hip_gemm_workspace_bytes(M, N, K) > 0
@@ -272,6 +273,23 @@ def test_gemm_split_k(cuda, monkeypatch, M, N, K):
     ai = torch.randint(-2, 3, (M, K), generator=g).bfloat16()
     wi = torch.randint(-1, 2, (N, K), generator=g).bfloat16()
     assert torch.equal(ops.gemm_bf16(ai.to(cuda), wi.to(cuda)).cpu(), (ai.float() @ wi.float().T).bfloat16())
+
+
+@pytest.mark.parametrize("B,Ntok,C,K", [(2, 500, 2240, 5600), (3, 233, 1160, 5728), (9, 31, 264, 5664)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_split_k_gated_residual_across_batch_boundaries(cuda, monkeypatch, dtype, B, Ntok, C, K):
+    """Gate rows that change inside a tile of a split GEMM, both dtypes, on integers: every product and sum is exact in fp32
+    (|sum| <= 9 K < 2^24), so split and unsplit agree with the stock op chain bit for bit."""
+    from sana_amd import _lib
+    assert _lib.load().sana_hip_gemm_workspace_bytes(B * Ntok, C, K) > 0
+    g = torch.Generator().manual_seed(C)
+    ints = lambda *s, hi=3: torch.randint(-hi, hi + 1, s, generator=g).to(dtype).to(cuda)
+    a, w, bias, gate, res = ints(B, Ntok, K), ints(C, K), ints(C, hi=9), ints(B, 1, C, hi=4), ints(B, Ntok, C, hi=99)
+    y = (a.float() @ w.float().T + bias.float()).to(dtype)
+    assert torch.equal(ops.gemm_gate_residual(a, w, bias, gate, res), res + gate * y)
+    assert torch.equal(ops.gemm_bf16(a.view(-1, K), w, bias, "bias").view(y.shape), y)
+    monkeypatch.setattr(ops, "SPLIT_K", False)
+    assert torch.equal(ops.gemm_gate_residual(a, w, bias, gate, res), res + gate * y)
 
 
 # ---------------------------------------------------------------- fused seams of the block
