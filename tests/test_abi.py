@@ -97,6 +97,18 @@ def test_gemm_split_k_workspace_query():
         assert lib.sana_hip_gemm_workspace_bytes(M, N, K) == 0, (M, N, K)
 
 
+@pytest.mark.parametrize("B,N,C,hidden", [(16, 4096, 1152, 2880), (2, 16384, 2240, 5600), (1, 256, 288, 720)])
+def test_block_scratch_is_no_more_than_the_calls_one_by_one_hold(B, N, C, hidden):
+    """fp16 takes the block call at every size: its scratch stays within what the composition holds at its peak beside
+    input and output (normalised rows, the second residual sum, hidden pairs, gated hidden values)."""
+    lib = _lib.load()
+    args = _lib.BlockArgs(B=B, N=N, C=C, hidden=hidden, cross_heads=C // 72, text_len=300, split_k=1, io_dtype=_lib.DT_F16)
+    state = lib.sana_hip_linattn_workspace_bytes(B, C // 32, 32, 1, N, _lib.DT_F16) + B * (C // 32) * 33 * 32 * 4
+    most = 2 * B * N * (2 * C + 3 * hidden) + state + 4096
+    need = lib.sana_hip_block_scratch_bytes(ctypes.byref(args))
+    assert 2 * B * N * (C + 3 * C + 2 * hidden) <= need <= most
+
+
 def test_ops_refuse_cpu_tensors():
     import torch
     from sana_amd import ops
