@@ -28,6 +28,7 @@ from typing import List, Optional, Sequence, Tuple
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import ops
 from ._lib import SanaHipError
@@ -919,7 +920,7 @@ class MultiHeadCrossAttention(nn.Module):
         """Nothing hooked on, patched over or overriding forward: forward_residual may stand for the call."""
         return not (self._forward_hooks or self._forward_pre_hooks or "forward" in self.__dict__
                     or type(self).forward is not MultiHeadCrossAttention.forward
-                    or torch.nn.modules.module._has_any_global_hook())
+                    or _has_any_global_hook())
 
     def _on_hip_path(self, x, cond, mask, kv=None) -> bool:
         B, N, C = x.shape
@@ -930,10 +931,9 @@ class MultiHeadCrossAttention(nn.Module):
                 and self.q_linear.weight.dtype == x.dtype)
 
     @staticmethod
-    def _gemm_takes(linear, x) -> bool:
+    def _gemm_takes(w, b, x) -> bool:
         """Rows, alignment, dtypes and devices of this library's GEMM, and weights that are what they seem (anything else,
         a quantised tensor subclass say, is a stock linear, as it always was)."""
-        w, b = linear.weight, linear.bias
         return (type(w) in _PLAIN and type(b) in _PLAIN and w.get_device() == x.get_device() == b.get_device()
                 and x.is_contiguous() and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0
                 and w.dtype == x.dtype and b.dtype == x.dtype and b.is_contiguous()
@@ -941,20 +941,21 @@ class MultiHeadCrossAttention(nn.Module):
 
     @staticmethod
     def _linear(linear, x):
-        if MultiHeadCrossAttention._gemm_takes(linear, x):
-            w = linear.weight     # (no -1 in the view: x may be empty)
-            return ops.gemm_bf16(x.view(-1, x.shape[-1]), w, linear.bias, "bias").view(*x.shape[:-1], w.shape[0])
-        return F.linear(x, linear.weight, linear.bias)
+        w, b = linear.weight, linear.bias
+        if MultiHeadCrossAttention._gemm_takes(w, b, x):      # (no -1 in the last view: x may be empty)
+            return ops.gemm_bf16(x.view(-1, x.shape[-1]), w, b, "bias").view(*x.shape[:-1], w.shape[0])
+        return F.linear(x, w, b)
 
     def _attend(self, x, cond, mask, kv=None):
         """The HIP path up to proj's input -- softmax(q k^T) v over the short text sequence as one kernel that reads
         q_linear's output and writes proj's input token-major (no head transposes, no padded head_dim) -- or None
         when the call is outside it.  ``kv``: kv_linear(cond) computed by the caller ([B, Nk, 2C] rows, see
         ``StepConditioning``)."""
-        B, N, C = x.shape
-        H = self.num_heads
-        if not self._on_hip_path(x, cond, mask, kv):
-            return None
+        return self._attend_hip(x, cond, mask, kv) if self._on_hip_path(x, cond, mask, kv) else None
+
+    def _attend_hip(self, x, cond, mask, kv):
+        """:meth:`_attend` of a call that :meth:`_on_hip_path` has accepted."""
+        C = x.shape[-1]
         q = self._linear(self.q_linear, x)
         if kv is None:
             kv = self._linear(self.kv_linear, cond)       # [B, Nk, 2C]
@@ -962,7 +963,7 @@ class MultiHeadCrossAttention(nn.Module):
             q = self.q_norm(q)
         if not isinstance(self.k_norm, nn.Identity):
             kv = torch.cat([self.k_norm(kv[:, :, :C]), kv[:, :, C:]], dim=-1)
-        return ops.cross_attention16(q, kv, H, None if mask is None else self._key_bias(mask))
+        return ops.cross_attention16(q, kv, self.num_heads, None if mask is None else self._key_bias(mask))
 
     @staticmethod
     def _key_bias(mask):
@@ -975,18 +976,24 @@ class MultiHeadCrossAttention(nn.Module):
     RESIDUAL_GEMM_MIN_ROWS = 1
 
     def _residual_in_gemm(self, x, cond, mask, kv=None) -> bool:
-        return (x.shape[0] * x.shape[1] >= self.RESIDUAL_GEMM_MIN_ROWS and isinstance(self.proj_drop, nn.Dropout)
-                and self.proj_drop.p == 0.0 and self._called_as_is() and self._on_hip_path(x, cond, mask, kv)
-                and self._gemm_takes(self.proj, x))
+        drop, proj = self.proj_drop, self.proj
+        return (x.shape[0] * x.shape[1] >= self.RESIDUAL_GEMM_MIN_ROWS and isinstance(drop, nn.Dropout) and drop.p == 0.0
+                and self._called_as_is() and self._on_hip_path(x, cond, mask, kv)
+                and self._gemm_takes(proj.weight, proj.bias, x))
 
     def forward_residual(self, x, cond, mask=None, kv=None):
         """x + self(x, cond, mask) -- what the blocks compute (sana_multi_scale.py:154) -- with the add inside the
         projection GEMM's epilogue when the call is on the HIP path and large enough."""
-        B, N, C = x.shape
         if self._residual_in_gemm(x, cond, mask, kv):
-            o = self._attend(x, cond, mask, kv)
-            return ops.gemm_gate_residual(o, self.proj.weight, self.proj.bias, ops.ones_row(C, x.dtype, x.device).expand(B, 1, C), x)
+            return self._residual_hip(x, cond, mask, kv)
         return x + self(x, cond, mask, kv)
+
+    def _residual_hip(self, x, cond, mask, kv):
+        """:meth:`forward_residual` of a call that :meth:`_residual_in_gemm` has accepted."""
+        B, N, C = x.shape
+        o = self._attend(x, cond, mask, kv) if "_attend" in self.__dict__ else self._attend_hip(x, cond, mask, kv)
+        proj = self.proj
+        return ops.gemm_gate_residual(o, proj.weight, proj.bias, ops.ones_row(C, x.dtype, x.device).expand(B, 1, C), x)
 
     def forward(self, x, cond, mask=None, kv=None):
         B, N, C = x.shape
@@ -1060,14 +1067,12 @@ class SanaMSBlock(nn.Module):
 
     def _one_call(self, x, y, modulation, mask, HW, text_kv):
         """The block as one call into the library (``sana_hip_block``: the same launches in the same order), or None where
-        it does not apply: q/k norm, int8 weights, anything patched, hooked or replaced, unusual strides -- and many bf16
-        tokens, whose qkv projection takes the attention's first phase along and where the host is ahead anyway."""
+        it does not apply: q/k norm, int8 weights, anything patched, hooked or replaced, unusual strides."""
         B, N, C = x.shape
         attn, ca, mlp = self._modules["attn"], self._modules["cross_attn"], self._modules["mlp"]
-        if B * N == 0 or HW is None or len(HW) != 2 or HW[0] * HW[1] != N or type(attn) is not LiteLA \
-                or (x.dtype == torch.bfloat16 and B * N >= attn.STATE_IN_QKV_GEMM_MIN_ROWS) or type(ca) is not MultiHeadCrossAttention \
+        if B * N == 0 or HW is None or len(HW) != 2 or HW[0] * HW[1] != N or type(ca) is not MultiHeadCrossAttention \
                 or type(mlp) not in (GLUMBConv, GLUMBConvLinear) or attn.dim != HEAD_DIM or mlp.dilation != 1 \
-                or mlp.out_feature != C or torch.nn.modules.module._has_any_global_hook():
+                or mlp.out_feature != C or _has_any_global_hook():
             return None
         linears = (attn._modules["qkv"], attn._modules["proj"], ca._modules["q_linear"], ca._modules["proj"])
         for m, kind in zip(linears, (HipLinear, HipLinear, nn.Linear, nn.Linear)):
@@ -1079,8 +1084,6 @@ class SanaMSBlock(nn.Module):
         for m in (attn, ca):
             if type(m._modules["q_norm"]) is not nn.Identity or type(m._modules["k_norm"]) is not nn.Identity:
                 return None
-        if not ca._residual_in_gemm(x, y, mask, text_kv):
-            return None
         ic, pc, dc = mlp._pointwise_params(mlp.inverted_conv), mlp._pointwise_params(mlp.point_conv), mlp.depth_conv.conv
         hid, dt, dev = mlp.hidden_features, x.dtype, x.get_device()
         ps = []
@@ -1095,7 +1098,7 @@ class SanaMSBlock(nn.Module):
         if None in (ps[3], ps[5], ps[7], ps[9]) or dc.weight.numel() != 18 * hid or hid % 8 or not x.is_contiguous() \
                 or x.data_ptr() % 16 or modulation.shape != (B, 6, C) or not modulation.is_contiguous() \
                 or modulation.get_device() != dev or modulation.data_ptr() % 16 \
-                or (mask is not None and mask.get_device() != dev):
+                or (mask is not None and mask.get_device() != dev) or not ca._residual_in_gemm(x, y, mask, text_kv):
             return None
         kv = ca._linear(ca.kv_linear, y) if text_kv is None else text_kv
         Nk = y.shape[1]
@@ -1119,23 +1122,31 @@ class SanaMSBlock(nn.Module):
         # fused kernels read the modulation rows as x's dtype, so that case takes the stock composition below)
         if x.is_cuda and x.dtype in ops.IO16 and shift_msa.dtype == x.dtype and C % 8 == 0 and C <= 8192 \
                 and not torch.is_grad_enabled():
-            out = self._one_call(x, y, modulation, mask, HW, text_kv) if image_rotary_emb is None else None
-            if out is not None:
-                return out
+            attn = self.attn
+            # the block as one call; with many bf16 tokens the qkv projection takes the attention's first phase along, and
+            # the host is ahead anyway
+            if image_rotary_emb is None and type(attn) is LiteLA \
+                    and (x.dtype == torch.float16 or B * N < attn.STATE_IN_QKV_GEMM_MIN_ROWS):
+                out = self._one_call(x, y, modulation, mask, HW, text_kv)
+                if out is not None:
+                    return out
             # fused seams: LayerNorm + modulate in one kernel, gate * out + residual in the GEMM epilogue
             h = ops.layernorm_modulate(x, scale_msa, shift_msa, self.norm1.eps)
-            if "forward" in self.attn.__dict__:
+            if "forward" in attn.__dict__:
                 # a guidance processor was patched over attn.forward (dpm_solver.py:486-524): call it
-                x = ops.gate_residual(self.attn(h, HW=HW, rotary_emb=image_rotary_emb), gate_msa, x)
+                x = ops.gate_residual(attn(h, HW=HW, rotary_emb=image_rotary_emb), gate_msa, x)
             else:
-                x = self.attn.forward_gated(h, gate_msa, x, rotary_emb=image_rotary_emb)
-            if self.cross_attn._residual_in_gemm(x, y, mask, text_kv):
-                # the cross-attention's residual add inside its projection GEMM, then norm2 + modulate
-                x = self.cross_attn.forward_residual(x, y, mask, text_kv)
+                x = attn.forward_gated(h, gate_msa, x, rotary_emb=image_rotary_emb)
+            ca = self.cross_attn
+            if ca._residual_in_gemm(x, y, mask, text_kv):
+                # the cross-attention's residual add inside its projection GEMM, then norm2 + modulate (decided once: the
+                # walk over modules, hooks and pointers is as long as a launch)
+                own = type(ca) is MultiHeadCrossAttention and "forward_residual" not in ca.__dict__
+                x = (ca._residual_hip if own else ca.forward_residual)(x, y, mask, text_kv)
                 h = ops.layernorm_modulate(x, scale_mlp, shift_mlp, self.norm2.eps)
             else:
                 # the cross-attention's residual add and norm2 + modulate in one pass
-                x, h = ops.add_layernorm_modulate(x, self.cross_attn(x, y, mask, text_kv), scale_mlp, shift_mlp,
+                x, h = ops.add_layernorm_modulate(x, ca(x, y, mask, text_kv), scale_mlp, shift_mlp,
                                                    self.norm2.eps)
             return self.mlp.forward_gated(h, HW, gate_mlp, x)
         stock_path("SanaMSBlock LayerNorm / modulate / gate / residual seams",
