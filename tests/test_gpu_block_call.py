@@ -90,3 +90,18 @@ def test_what_keeps_the_composition(cuda, monkeypatch):
         with torch.no_grad():
             b(x, y, t, torch.ones(1, 20), HW)
     assert calls == [1, 1]
+
+
+@pytest.mark.parametrize("kw,int8", [({}, True), ({"qk_norm": True}, False)])
+def test_a_composed_block_decides_the_route_of_its_cross_attention_once(cuda, monkeypatch, kw, int8):
+    """The decision walks modules, hooks, strides and pointers on the host, which a small image waits for."""
+    b = _block(288, 4, torch.bfloat16, cuda, 1, **kw)
+    if int8:
+        b.quantize_w8_()
+    x, y, t, _ = _inputs(1, 64, 288, 20, torch.bfloat16, cuda, False)
+    asked, real = [], S.modules.MultiHeadCrossAttention._on_hip_path
+    monkeypatch.setattr(S.modules.MultiHeadCrossAttention, "_on_hip_path", lambda *a: (asked.append(1), real(*a))[1])
+    calls = _count(monkeypatch)
+    with torch.no_grad():
+        b(x, y, t, None, (8, 8))
+    assert asked == [1] and not calls
