@@ -417,6 +417,7 @@ int sana_hip_gate_residual(const void* y, const void* gate, const void* residual
  *         these rows reads zeros instead of the rows behind them.  That is the zero padding ChunkGLUMBConvTemp
  *         puts behind every chunk (:302-349: a chunk sees the previous chunk's last frame in front and zeros
  *         behind), so all chunks of a sequence run as one launch.  taps >= 3 when given.
+ * x_rows * ldx < 2^30 and ldo < 2^23 (32-bit byte offsets).
  */
 int sana_hip_tconv_residual(const void* X, const void* W, void* out, int M, int C, int taps,
                             int64_t tap_rows, int64_t x_rows, const unsigned char* zero_last_tap,

@@ -1183,6 +1183,8 @@ SANA_API int sana_hip_tconv_residual(const void* X, const void* W, void* out, in
   if (ldx < C || ldw < (int64_t)taps * C || ldo < C) return SANA_ERR_ARG;
   if (ldx % 8 || ldw % 8 || ldo % 8 || !aligned16(X) || !aligned16(W) || !aligned16(out)) return SANA_ERR_ALIGN;
   if (x_rows * ldx * 2 >= ((int64_t)1 << 31)) return SANA_ERR_SHAPE;  // 32-bit byte offsets inside the buffer
+  if (M == 1) ldo = C;  // a single row has no stride
+  if (ldo >= 2 * kMaxTileStride) return SANA_ERR_SHAPE;  // .. and inside the 128 rows of out that a wave stores
   const uint16_t* x = static_cast<const uint16_t*>(X);
   const EpiArgs e = {nullptr, nullptr, x + (taps / 2) * tap_rows * ldx, ldx, 0, M, nullptr, 0, 0, 0, 0};
   const Taps tp = {C, tap_rows, x_rows, 0, 0, zero_last_tap};

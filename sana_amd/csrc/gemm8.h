@@ -482,8 +482,10 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
     fresh = false;
     constexpr bool GATED = EPI == SANA_EPI_GATE_RES;
     const int rows = min(BM, M - m0t);
+    // (C per wave: its 128 rows reach twice as far in 32 bits as the tile's 256)
+    const int wrows = min(128, rows - 128 * wm);
     const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc(
-        C + (int64_t)m0t * ldc, 0, (int)((((int64_t)rows - 1) * ldc + n_end) * 2), 0x00020000);
+        C + (int64_t)(m0t + 128 * wm) * ldc, 0, wrows > 0 ? (int)((((int64_t)wrows - 1) * ldc + n_end) * 2) : 0, 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_r = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(GATED ? ep.res + (int64_t)m0t * ep.ldr : nullptr), 0,
         GATED ? (int)((((int64_t)rows - 1) * ep.ldr + n_end) * 2) : 0, 0x00020000);
@@ -509,7 +511,7 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
       rd[s] = out0 + out_at(row, pc);
       row_s[s] = 128 * wm + row;
       n_s[s] = n0t + wn * 16 * NB + 8 * pc;
-      coff[s] = n_s[s] < n_end ? (row_s[s] * (int)ldc + n_s[s]) * 2 : (int)kOut;
+      coff[s] = n_s[s] < n_end ? (row * (int)ldc + n_s[s]) * 2 : (int)kOut;
       roff[s] = n_s[s] < n_end ? (row_s[s] * (int)ep.ldr + n_s[s]) * 2 : (int)kOut;
     }
     u32x4_t res[GATED ? 4 : 1][NB], gate[NB];

@@ -629,6 +629,8 @@ def tconv_residual(xp: torch.Tensor, weight: torch.Tensor, n_rows: int, tap_rows
         raise SanaHipError("out has the wrong shape or dtype")
     if n_rows == 0:
         return out
+    if n_rows > 1 and ldo >= 1 << 23:      # rows further apart than the kernel's 32-bit offsets reach
+        return out.copy_(tconv_residual(xp, weight, n_rows, tap_rows, None, zero_last_tap))
     if zero_last_tap is not None and (zero_last_tap.dtype != torch.uint8 or not zero_last_tap.is_contiguous()
                                       or zero_last_tap.numel() < (n_rows + tap_rows - 1) // tap_rows):
         raise SanaHipError("zero_last_tap must be a contiguous uint8 tensor with one entry per frame")

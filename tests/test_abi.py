@@ -63,6 +63,7 @@ def test_argument_validation_needs_no_gpu():
     assert lib.sana_hip_tconv_residual(16, 16, 32, 64, 64, 3, 16, 64, None, 64, 192, 64, None) == -1
     assert lib.sana_hip_tconv_residual(16, 16, 32, 64, 64, 3, 16, 80, None, 64, 128, 64, None) == -1   # ldw < taps * C
     assert lib.sana_hip_tconv_residual(16, 16, 32, 64, 64, 1, 16, 80, 16, 64, 64, 64, None) == -1   # chunk flags need >= 3 taps
+    assert lib.sana_hip_tconv_residual(16, 16, 32, 64, 64, 3, 16, 80, None, 64, 192, 1 << 23, None) == -2   # 32-bit offsets
 
 
 def test_workspace_query():

@@ -437,6 +437,23 @@ def test_temporal_conv_chunk_flags_equal_per_chunk_launches(cuda, C, T, P, ends)
     assert ops.frame_flags(T, [], cuda) is None
 
 
+@pytest.mark.parametrize("ldo", [(1 << 22) + 8, (1 << 23) - 8, (1 << 23) + 8])
+def test_tconv_residual_into_rows_far_apart(cuda, ldo):
+    """Output rows that span more than 32-bit offsets reach (one token of each of many long sequences): the same bits as
+    with the rows side by side, and what lies between the rows is left alone.  320 channels: the last channel tile is
+    ragged, its lanes past the row's end must not store."""
+    P, C, rows = 5, 320, 200
+    g = torch.Generator().manual_seed(5)
+    buf = torch.randn(rows + P, C, generator=g).bfloat16().to(cuda)
+    w2 = (torch.randn(C, 3 * C, generator=g) * 0.05).bfloat16().to(cuda)
+    store = torch.zeros((rows - 1) * ldo + C, dtype=torch.bfloat16, device=cuda)
+    far = store.as_strided((rows, C), (ldo, 1))
+    near = ops.tconv_residual(buf, w2, rows, P)
+    assert torch.equal(ops.tconv_residual(buf, w2, rows, P, out=far), near)
+    far.zero_()
+    assert not store.any()
+
+
 def test_temporal_conv_zero_weight_is_identity(cuda):
     """t_conv is zero-initialised in the reference: x + 0 must come back bit for bit."""
     C, T, P = 128, 3, 50
