@@ -255,6 +255,11 @@ int sana_hip_dwconv3x3_silu_gate(const void* u, const void* w, const void* bias,
  */
 size_t sana_hip_gemm_workspace_bytes(int M, int N, int K);
 
+/* What a 16-bit GEMM of this shape runs as, given that workspace: plan[0], plan[1] = tokens and channels of a workgroup's
+ * tile; plan[2] > 0: its first plan[2] channels run in tiles of 256 x 256, the rest in tiles of 256 x 192 (two launches);
+ * plan[3] > 1: split into that many ranges of K.  A host-side query for tests and measurements. */
+int sana_hip_gemm_plan(int M, int N, int K, int plan[4]);
+
 int sana_hip_gemm_bf16(const void* A, const void* W, const void* bias, void* C,
                        int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
                        int epilogue, void* workspace, size_t workspace_bytes, void* stream);

@@ -1104,6 +1104,17 @@ SANA_API size_t sana_hip_gemm_workspace_bytes(int M, int N, int K) {
   return split_pays(pl, M, N, K) ? split_bytes(pl, M, N) : 0;
 }
 
+SANA_API int sana_hip_gemm_plan(int M, int N, int K, int plan[4]) {
+  if (!plan || M <= 0 || N <= 0 || K <= 0) return SANA_ERR_ARG;
+  if (N % 8 || K % 8) return SANA_ERR_SHAPE;
+  const GemmPlan split = plan_gemm(M, N, K, false);
+  const Plan16 p = plan16(M, N, K);
+  const bool cut = split_pays(split, M, N, K);
+  plan[0] = cut ? BT : p.tile->bm, plan[1] = cut ? 64 * pick_ni(M, N) : p.n_wide ? 256 : p.tile->bn;
+  plan[2] = cut ? 0 : p.n_wide, plan[3] = cut ? split.S : 1;
+  return SANA_OK;
+}
+
 // From 4096 rows on always (converting in the main loop costs it 14 % at every M, the expansion a fixed 10 - 20 us); below
 // that where N <= K and the GEMM is not split: there the bf16 GEMM has its small tiles and the int8 one a chain of long
 // k-tiles.  us, converting / expanding: 256 x 1152 x 2880 37 / 20, 2048 x 2240 x 2240 40 / 33, 2048 x 2240 x 5600 91 / 68;

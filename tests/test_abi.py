@@ -98,6 +98,22 @@ def test_gemm_split_k_workspace_query():
         assert lib.sana_hip_gemm_workspace_bytes(M, N, K) == 0, (M, N, K)
 
 
+def test_gemm_plan_query():
+    lib = _lib.load()
+    plan = (ctypes.c_int * 4)()
+    def of(*shape):
+        assert lib.sana_hip_gemm_plan(*shape, plan) == 0
+        return tuple(plan)
+    assert of(256, 1152, 1152) == (64, 64, 0, 1)
+    assert of(16384, 11200, 2240) == (256, 256, 0, 1)
+    assert of(4096, 6720, 2240) == (256, 256, 3840, 1)              # two widths, two launches
+    assert of(1024, 2240, 5600) == (256, 192, 0, 5)                 # five ranges of k
+    for M, N, K in ((1024, 2240, 5600), (256, 2240, 5600), (1024, 2240, 2240), (4096, 2240, 5600), (300, 264, 5664)):
+        assert (of(M, N, K)[3] > 1) == (lib.sana_hip_gemm_workspace_bytes(M, N, K) > 0)
+    assert lib.sana_hip_gemm_plan(256, 1152, 1152, None) == -1 and lib.sana_hip_gemm_plan(0, 8, 8, plan) == -1
+    assert lib.sana_hip_gemm_plan(8, 12, 8, plan) == -2 and lib.sana_hip_gemm_plan(8, 8, 12, plan) == -2
+
+
 @pytest.mark.parametrize("B,N,C,hidden", [(16, 4096, 1152, 2880), (2, 16384, 2240, 5600), (1, 256, 288, 720)])
 def test_block_scratch_is_no_more_than_the_calls_one_by_one_hold(B, N, C, hidden):
     """fp16 takes the block call at every size: its scratch stays within what the composition holds at its peak beside

@@ -140,11 +140,16 @@ def test_gemm_strided_views(cuda):
 
 @pytest.mark.parametrize("w8", [False, True])
 def test_gemm_mixed_channel_tiling_is_bit_identical(cuda, w8):
-    """qkv at 16384 tokens (N = 6720) runs as two launches: 24 tiles of 256 channels and 3 of 192.  Every output sums
-    its k products in the same order whatever the tiling, so the first 256 rows -- which alone are one launch of one
-    width -- must come out bit for bit the same; bias, SiLU, the gated residual and int8 weights ride along."""
+    """qkv at 4096 tokens (N = 6720) runs as two launches: 15 tiles of 256 channels and 15 of 192.  Every output sums
+    its k products in the same order whatever the tiling, so 256 of its rows -- which alone are one launch of one
+    tile -- must come out bit for bit the same; bias, SiLU, the gated residual and int8 weights ride along."""
+    from sana_amd import _lib
     from sana_amd.modules import quantize_w8
-    M, N, K = 16384, 6720, 192
+    M, N, K = 4096, 6720, 2240
+    plans = (_lib.ctypes.c_int * 4)(), (_lib.ctypes.c_int * 4)()
+    for m, p in zip((M, 256), plans):
+        _lib.check(_lib.load().sana_hip_gemm_plan(m, N, K, p), "sana_hip_gemm_plan")
+    assert plans[0][2] > 0 and plans[1][2] == 0 and plans[0][3] == plans[1][3] == 1
     g = torch.Generator().manual_seed(9)
     a = torch.randn(M, K, generator=g).bfloat16().to(cuda)
     w = (torch.randn(N, K, generator=g) * 0.05).bfloat16().to(cuda)
@@ -158,7 +163,7 @@ def test_gemm_mixed_channel_tiling_is_bit_identical(cuda, w8):
         whole, head = run(a, epi), run(a[:256], epi)
         assert torch.equal(whole[:256], head)
         # a tile row in the middle and the last one, against the same rows alone
-        assert torch.equal(whole[8192:8448], run(a[8192:8448], epi))
+        assert torch.equal(whole[2048:2304], run(a[2048:2304], epi))
         assert torch.equal(whole[-256:], run(a[-256:], epi))
     if not w8:
         ref = a[:512].double() @ w.double().T + bias.double()
@@ -172,7 +177,7 @@ def test_gemm_mixed_channel_tiling_is_bit_identical(cuda, w8):
 
 def test_gemm_128_wide_tiles_are_bit_identical_to_the_wider_ones(cuda):
     """1024 tokens x 6720 channels (qkv of one image) runs 128-wide tiles: 4 x 53 workgroups instead of 4 x 35 of 192
-    channels.  The same rows inside a 16384-token call run the 256- / 192-wide tiles: same k order per output, so
+    channels.  The same rows inside a 16384-token call run 256-wide tiles: same k order per output, so
     bit for bit the same; the int8-weight instances (also 128-wide here) as well; every epilogue kind."""
     from sana_amd.modules import quantize_w8
     M, N, K = 1024, 6720, 2240

@@ -1,10 +1,12 @@
 """The tile kernels of the 16-bit GEMM at the edges of their tiles: integer operands (every product, sum and bias is exact
 in fp32, so the result is bit for bit the rounded integer matrix product), ragged rows and channels, k tails, one and
 several tiles per workgroup, gate rows that change inside a tile."""
+import ctypes
+
 import pytest
 import torch
 
-from sana_amd import ops
+from sana_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -14,21 +16,47 @@ def _ints(*shape, lo=-3, hi=3, seed=0, dtype=torch.bfloat16):
     return torch.randint(lo, hi + 1, shape, generator=g).to(dtype)
 
 
-# (rows, channels, k): 256-token tiles of 256 / 192 / 128 channels, and the two-launch mix of 256 and 192; k of less
-# than one k-tile, of whole ones, and with tails of 8, 32 and 56
-MANY = [(1030, 8200, 8), (1030, 8200, 64), (1030, 8200, 72), (1030, 8200, 184), (1025, 8208, 160), (2563, 2240, 72),
-        (4099, 2240, 136), (8200, 6720, 128), (4352, 4360, 192)]
+# Tile (tokens, channels; "mix": the first channels in tiles of 256 x 256, the rest in 256 x 192, two launches) -> shapes
+# (rows, channels, k) that run in it, asserted through the library's own plan: k of less than one k-tile (8, 40), of one (64),
+# of an odd and an even number, with tails of 8, 32 and 56; ragged rows and channels; one row; more tiles than workgroups
+# that are resident (persistent workgroups then take several).  128 x 160 is not chosen for short k or for many tiles.
+TILES = {
+    (64, 64): [(1, 8, 8), (65, 72, 40), (200, 264, 184), (33, 16, 320), (12300, 264, 72)],
+    (64, 128): [(206, 3456, 8), (700, 2240, 328), (1500, 1160, 1152), (65, 6728, 40), (515, 6728, 64), (515, 6728, 136)],
+    (128, 128): [(1030, 8200, 8), (1030, 8200, 64), (3679, 536, 8), (999, 2248, 392), (2049, 1160, 120), (1030, 6728, 40),
+                 (1030, 6728, 184), (4100, 2240, 64)],
+    (128, 160): [(3671, 1120, 200), (2000, 2232, 1032), (2040, 2240, 2240), (5121, 776, 136), (5121, 776, 192)],
+    (256, 128): [(2563, 2240, 72), (4352, 4360, 192), (2563, 1544, 8), (9999, 1160, 40), (9999, 1160, 64), (16390, 776, 136),
+                 (8200, 2240, 136)],
+    (256, 192): [(1030, 8200, 72), (1030, 8200, 184), (1025, 8208, 160), (4099, 2240, 136), (6150, 5128, 40), (6150, 5128, 64),
+                 (12300, 1288, 192)],
+    (256, 256): [(8200, 6720, 128), (4613, 5128, 40), (4613, 5128, 64), (4613, 5128, 184), (1290, 8200, 136), (9999, 1160, 72)],
+    "mix": [(8200, 4432, 712), (2563, 8920, 1736)],
+}
+# the same for the gated residual, (batch entries, tokens of each, channels, k): boundaries between them inside a tile
+GATED = {
+    (64, 64): [(7, 9, 72, 40), (3, 67, 264, 184)],
+    (64, 128): [(5, 140, 2240, 328), (3, 172, 6728, 8)],
+    (128, 128): [(9, 111, 2248, 392), (41, 100, 2240, 64), (5, 206, 6728, 40)],
+    (128, 160): [(3, 667, 2232, 1032), (3, 1707, 776, 136)],
+    (256, 128): [(2, 4100, 2240, 136), (1, 4096, 4360, 64), (3, 855, 1544, 8)],
+    (256, 192): [(3, 1365, 2240, 72), (3, 2050, 5128, 40), (7, 147, 8200, 184)],
+    (256, 256): [(3, 1538, 5128, 40), (6, 215, 8200, 136)],
+    "mix": [(2, 4100, 4432, 712), (3, 855, 8920, 1736)],
+}
 
 
-# tiles of 64 x 64, 64 x 128, 128 x 128 and 128 x 160: one row and eight channels, ragged edges, fewer k-tiles than the
-# ring has stages and more, k tails of 8, 32 and 56
-FEW = [(1, 8, 8), (65, 72, 40), (200, 264, 184), (33, 16, 320), (206, 3456, 8), (700, 2240, 328), (1500, 1160, 1152),
-       (3679, 536, 8), (999, 2248, 392), (2049, 1160, 120), (3671, 1120, 200), (2000, 2232, 1032), (2040, 2240, 2240)]
+def _runs_in(tile, M, N, K):
+    plan = (ctypes.c_int * 4)()
+    _lib.check(_lib.load().sana_hip_gemm_plan(M, N, K, plan), "sana_hip_gemm_plan")
+    assert plan[3] == 1, "split over k: not these kernels"
+    assert plan[2] > 0 if tile == "mix" else (tuple(plan[:2]) == tile and plan[2] == 0), (tuple(plan), tile)
 
 
-@pytest.mark.parametrize("M,N,K", MANY + FEW)
+@pytest.mark.parametrize("tile,M,N,K", [(t, *s) for t, shapes in TILES.items() for s in shapes])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_many_token_tiles_are_exact_on_integers(cuda, M, N, K, dtype):
+def test_many_token_tiles_are_exact_on_integers(cuda, tile, M, N, K, dtype):
+    _runs_in(tile, M, N, K)
     a, w, bias = (_ints(M, K, seed=1, dtype=dtype).to(cuda), _ints(N, K, seed=2, dtype=dtype).to(cuda),
                   _ints(N, lo=-9, hi=9, seed=3, dtype=dtype).to(cuda))
     ref = a.float() @ w.float().T        # |sum| <= 9 k < 2^24: exact in any order
@@ -42,10 +70,12 @@ def test_many_token_tiles_are_exact_on_integers(cuda, M, N, K, dtype):
     assert ((y.double() - want).abs() <= ulp * want.abs() + 1e-7).all()
 
 
-@pytest.mark.parametrize("B,Ntok,C,K", [(3, 1365, 2240, 72), (41, 100, 2240, 64), (2, 4100, 2240, 136), (1, 4096, 4360, 64),
-                                           (7, 9, 72, 40), (5, 140, 2240, 328), (9, 111, 2248, 392), (3, 667, 2232, 1032)])
-def test_many_token_gated_residual_across_batch_boundaries(cuda, B, Ntok, C, K):
-    a, w, bias = _ints(B, Ntok, K, seed=1).to(cuda), _ints(C, K, seed=2).to(cuda), _ints(C, lo=-9, hi=9, seed=3).to(cuda)
-    gate, res = _ints(B, 1, C, lo=-4, hi=4, seed=4).to(cuda), _ints(B, Ntok, C, lo=-99, hi=99, seed=5).to(cuda)
-    y = (a.float() @ w.float().T + bias.float()).bfloat16()
+@pytest.mark.parametrize("tile,B,Ntok,C,K", [(t, *s) for t, shapes in GATED.items() for s in shapes])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_many_token_gated_residual_across_batch_boundaries(cuda, tile, B, Ntok, C, K, dtype):
+    _runs_in(tile, B * Ntok, C, K)
+    ints = lambda *s, hi=3, seed: _ints(*s, lo=-hi, hi=hi, seed=seed, dtype=dtype).to(cuda)
+    a, w, bias = ints(B, Ntok, K, seed=1), ints(C, K, seed=2), ints(C, hi=9, seed=3)
+    gate, res = ints(B, 1, C, hi=4, seed=4), ints(B, Ntok, C, hi=99, seed=5)
+    y = (a.float() @ w.float().T + bias.float()).to(dtype)
     assert torch.equal(ops.gemm_gate_residual(a, w, bias, gate, res), res + gate * y)   # the stock pair's roundings
