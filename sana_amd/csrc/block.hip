@@ -8,7 +8,7 @@
 namespace {
 
 struct Layout {  // byte offsets into the scratch buffer
-  size_t h, o, x1, y, x2, wide, state, ws, total, ws_bytes;  // y: on h, o and x1
+  size_t h, wide, o, x1, x2, y, state, ws, total, ws_bytes;  // o and x1: inside wide
 };
 
 bool plan(const sana_block_args& a, Layout& l) {
@@ -22,15 +22,17 @@ bool plan(const sana_block_args& a, Layout& l) {
     at += (bytes + 255) & ~(size_t)255;
     return p;
   };
-  // The hidden pairs and the gated hidden values are the largest, and when the latter are written the normalised input, the
-  // attention's output and the sum behind it are dead: they share their place.  9 C values per token at 2.5 C hidden channels,
-  // less than the calls one by one hold (h, x2, the pairs, the gated values: 9.5).
+  // The attention's output and the sum behind it lie behind q, k and v and are dead when the hidden pairs are written: 9.5 C
+  // values per token at 2.5 C hidden channels, what the calls one by one hold (h, x2, the pairs, the gated values).  A step of
+  // 8 blocks at 256 x 1152 bf16 / 2048 x 1152 f16, us: this 835 / 1462, all buffers side by side (11.5 C) 833 / 1462, the gated
+  // values on h, o and x1 (9 C) 845 / 1498.
   const size_t row = (M * a.C * 2 + 255) & ~(size_t)255;
-  l.h = l.y = take(std::max(3 * row, M * a.hidden * 2));               // h: normalised input; cross-attention's queries
-  l.o = l.h + row;                                                     // attention outputs
+  l.h = take(row);                                                     // normalised input; cross-attention's queries
+  l.wide = take(std::max(5 * row, M * 4 * (size_t)a.hidden));          // q, k, v; the Mix-FFN's hidden pairs
+  l.o = l.wide + 3 * row;                                              // attention outputs
   l.x1 = l.o + row;                                                    // behind the attention
-  l.x2 = take(M * a.C * 2);                                            // behind the cross-attention
-  l.wide = take(M * 2 * std::max<size_t>(3 * (size_t)a.C, 2 * (size_t)a.hidden));  // q, k, v; the Mix-FFN's hidden pairs
+  l.x2 = take(row);                                                    // behind the cross-attention
+  l.y = take(M * a.hidden * 2);                                        // gated hidden values
   l.state = take((size_t)a.B * heads * 33 * 32 * 4);
   l.ws_bytes = sana_hip_linattn_workspace_bytes(a.B, heads, 32, 1, a.N, a.io_dtype);
   if (a.split_k)
