@@ -1,6 +1,7 @@
 // bf16 MFMA GEMM for gfx950:  C[M][N] = epilogue(A[M][K] . W[N][K]^T), with an int8-weight (W8A16) variant
 // dequantised on the way into LDS: the C entry points, the choice of a kernel by shape, and the kernels for int8
-// weights and for k split into ranges.  Unsplit 16-bit GEMMs run the kernels of gemm8.h (many tokens) and gemm_ring.h (few).
+// weights and for k split into ranges, which the rest of this comment describes.  Unsplit 16-bit GEMMs run the kernels of
+// gemm8.h (many tokens) and gemm_ring.h (few).
 //
 // Both operands are K-contiguous, which is exactly the MFMA operand layout (a
 // lane holds 8 consecutive k of one row), so nothing is transposed.  The MFMA
@@ -21,17 +22,6 @@
 #include <algorithm>
 
 #include "gemm_common.h"
-
-// Tuning knobs: non-temporal hint on the output stores (one bit per epilogue kind: 1 none, 2 bias, 4 bias + SiLU,
-// 8 gated residual; measured on the 20-block step, all four on is best: 2.307 ms per block against 2.319-2.324 with
-// the gated-residual or the plain outputs cacheable and 2.332 with none) / on the residual loads of the pipelined
-// kernel's epilogue.
-#ifndef SANA_GEMM_NT_STORE
-#define SANA_GEMM_NT_STORE 15
-#endif
-#ifndef SANA_GEMM_NT_RES
-#define SANA_GEMM_NT_RES 0
-#endif
 
 namespace sana {
 namespace {
@@ -370,7 +360,7 @@ __device__ __forceinline__ void finish_tile16(f32x4_t (&acc)[2 * NI][8], const u
 #pragma unroll
       for (int it = 0; it < 8; ++it)
         res[j][it] = __builtin_bit_cast(
-            u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc_r, r_off0 + (8 * j + it) * r_step, 0, SANA_GEMM_NT_RES ? kBufferNt : 0));
+            u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc_r, r_off0 + (8 * j + it) * r_step, 0, 0));
   }
   float bv[NI][8];
   if (HAS_BIAS) {
@@ -437,7 +427,7 @@ __device__ __forceinline__ void finish_tile16(f32x4_t (&acc)[2 * NI][8], const u
       __builtin_amdgcn_sched_barrier(0);
       if (js >= 0) {
         if (EPI == SANA_EPI_GATE_RES) o = gate_res8f<T>(o, gf, res[js][st]);
-        __builtin_amdgcn_raw_buffer_store_b128(o, rsrc_c, c_off0 + (8 * js + st) * c_step, 0, ((SANA_GEMM_NT_STORE >> EPI) & 1) ? kBufferNt : 0);
+        __builtin_amdgcn_raw_buffer_store_b128(o, rsrc_c, c_off0 + (8 * js + st) * c_step, 0, kBufferNt);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -785,7 +775,7 @@ __global__ __launch_bounds__(256) void splitk_epilogue_kernel(const float* __res
 // every host, with or without a GPU.
 constexpr int compute_units() { return 256; }
 
-// Channel tile of the pipelined kernel (NI = 4: 256 channels, 3: 192).  One workgroup per compute unit at a
+// Channel tile of the pipelined kernel (int8 weights, and K split: NI = 4: 256 channels, 3: 192).  One workgroup per compute unit at a
 // time, so the grid runs in rounds: the tile whose rounds x tile size is smaller wins; the narrower tile
 // re-reads a little more per MFMA, hence its 4 % handicap.
 int pick_ni(int M, int N) {
@@ -795,17 +785,18 @@ int pick_ni(int M, int N) {
   return cost192 < cost256 ? 3 : 4;
 }
 
-// Which kernel, and whether K is split.  A workgroup's K loop is a latency chain whatever the grid: about
-// 1.1 us per k-tile for the 256-wide pipelined kernel, 0.8 us for the 128 x 128 one (a quarter of the math, but
-// the same load / LDS / barrier round trip).  A grid that covers the chip keeps the 256-wide kernel (throughput
-// is what counts, and that kernel has twice the math per byte).  A grid of fewer tiles than half the compute
-// units (M = 1024 tokens x N = 2240: 48 workgroups on 256 CUs) leaves most of the chip idle for the whole
-// chain; two remedies, by estimate:
+// The split of K that could pay, and the tile of an unsplit GEMM with int8 weights (16-bit weights unsplit: plan16).  A
+// workgroup's K loop is a latency chain whatever the grid: about 1.1 us per k-tile for the 256-wide pipelined kernel, 0.8 us
+// for the 128 x 128 one (a quarter of the math, but the same load / LDS / barrier round trip).  A grid that covers the chip
+// keeps the 256-wide kernel (throughput is what counts, and that kernel has twice the math per byte).  A grid of fewer tiles
+// than half the compute units (M = 1024 tokens x N = 2240: 48 workgroups on 256 CUs) leaves most of the chip idle for the
+// whole chain; two remedies, by estimate:
 //  * split-k: S ranges of >= 8 k-tiles (S <= 8, S x tiles <= CUs) shorten the chain to ceil(KT / S) k-tiles and
 //    cost the fp32 partial planes (S x M x N x 4 bytes written and read once, about 6 bytes/ns at these sizes)
-//    plus a second launch (about 5 us); taken when that beats the unsplit chain by 15 %.  Long-K narrow-N
-//    shapes (the point conv of a few thousand tokens or less) split, wide-N or short-K ones do not.
-//  * the 128 x 128 kernel, when its grid still fits one workgroup per CU and its chain beats the above.
+//    plus a second launch (about 5 us); a candidate where that beats the unsplit chain by 15 %.  Whether it is taken
+//    is split_pays' to say, against the best unsplit 16-bit tile.
+//  * the 128 x 128 kernel, when its grid still fits one workgroup per CU and its chain beats the above.  (It rules the
+//    split out for 16-bit weights too, which have better small tiles still: both kinds of weight split alike.)
 struct GemmPlan {
   bool small;         // the 128 x 128 kernel
   int S, tiles, rem;  // k ranges; k-tiles per range; ranges that take one more
@@ -876,7 +867,8 @@ Plan16 plan16(int M, int N, int K) {
     const double us = cost16(t, M, N, K);
     if (us < p.us) p.tile = &t, p.us = us;
   }
-  // two widths, where their last rounds fill better (32760 x 6720 tokens x channels: 14 rounds of 256 wide, 12 + 2 mixed)
+  // two widths, where their last rounds fill better (4096 x 6720 tokens x channels, K = 2240:
+  // 432 tiles of 256 are 1.7 rounds, 15 x 16 and 15 x 16 tiles of the mix two that are 94 % full)
   const double single = p.us;
   for (int a = 256; a < N; a += 256) {
     const double us = cost16(kTiles16[2], M, a, K) + cost16(kTiles16[1], M, N - a, K);
@@ -1117,8 +1109,10 @@ SANA_API int sana_hip_gemm_plan(int M, int N, int K, int plan[4]) {
 
 // From 4096 rows on always (converting in the main loop costs it 14 % at every M, the expansion a fixed 10 - 20 us); below
 // that where N <= K and the GEMM is not split: there the bf16 GEMM has its small tiles and the int8 one a chain of long
-// k-tiles.  us, converting / expanding: 256 x 1152 x 2880 37 / 20, 2048 x 2240 x 2240 40 / 33, 2048 x 2240 x 5600 91 / 68;
-// but 2048 x 5760 x 1152 32 / 40, 1024 x 11200 x 2240 56 / 63, and split 512 x 2240 x 5600 33 / 42.
+// k-tiles.  us, converting / expanding (the weights of 12 calls in turn): 256 x 1152 x 2880 37 / 20, 2048 x 2240 x 2240 36 / 32,
+// 2048 x 2240 x 5600 90 / 76; but 2048 x 5760 x 1152 32 / 41, 1024 x 11200 x 2240 56 / 65, and split 512 x 2240 x 5600 33 / 42.
+// Wide weights of 2240 at 2000 - 3000 rows are the tie between: 2048 x 11200 x 2240 107 - 112 / 109 - 110, 2048 x 6720 x 2240
+// 63 / 60, 2916 x 11200 x 2240 155 / 152, 2916 x 6720 x 2240 98 / 97.
 SANA_API int sana_hip_gemm_w8_expand(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   return M >= 4096 || (N <= K && !split_pays(plan_gemm(M, N, K, true), M, N, K));

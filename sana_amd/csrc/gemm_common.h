@@ -24,7 +24,7 @@ struct EpiArgs {
 };
 #define SANA_EPI_GATE_RES 3
 // (not part of the C ABI's epilogue codes) qkv projection of the linear attention with the k / v column tiles
-// contracted over their tokens in the epilogue instead of stored: see state_tile16
+// contracted over their tokens in the epilogue instead of stored: see g8_state_tile
 #define SANA_EPI_QKV_STATE 4
 
 // Virtual concatenation of the A operand along k: columns [t*kc, (t+1)*kc) of the GEMM's A are columns

@@ -283,6 +283,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
         }
         o[s] = gate_res8v<T>(o[s], g8, res[j][s]);
       }
+      // (cacheable: with the non-temporal hint of the many-token kernel a 512 px step takes 866 us instead of 845, 1024 - 2048
+      // tokens 0.5 % less)
       __builtin_amdgcn_raw_buffer_store_b128(o[s], rsrc_c, coff[s] + 32 * j * (int)ldc, 0, 0);
     }
   }

@@ -983,7 +983,7 @@ class MultiHeadCrossAttention(nn.Module):
 
     def forward_residual(self, x, cond, mask=None, kv=None):
         """x + self(x, cond, mask) -- what the blocks compute (sana_multi_scale.py:154) -- with the add inside the
-        projection GEMM's epilogue when the call is on the HIP path and large enough."""
+        projection GEMM's epilogue when the call is on the HIP path."""
         if self._residual_in_gemm(x, cond, mask, kv):
             return self._residual_hip(x, cond, mask, kv)
         return x + self(x, cond, mask, kv)
