@@ -840,7 +840,7 @@ size_t split_bytes(const GemmPlan& pl, int M, int N) { return pl.S > 1 ? (size_t
 // its L2 and about 50 while most of the chip misses it), plus launch, first loads and epilogue.  Fitted to 128 shapes
 // (64 .. 5000 tokens, the eight projections of the two image widths, weights cold): 8 - 13 % off, choice 2.5 % from the best.
 struct Tile16 {
-  int bm, bn;    // tokens, channels; 256 tokens: gemm8_kernel, else gemm_ring_kernel
+  int bm, bn;    // tokens, channels; 256 tokens: gemm8_kernel, 288 channels: gemm288_kernel; else gemm_ring_kernel
   int resident;  // workgroups on the chip at a time
   double fixed, lone, full;
 };
@@ -855,6 +855,27 @@ double cost16(const Tile16& t, int64_t M, int64_t N, int K) {
   double us = t.fixed + rounds * (kt * t.full + 0.5 * t.fixed);
   if (rest) us += kt * (t.lone + (t.full - t.lone) * std::min(1.0, std::max(0.0, (rest - eighth) / (t.resident - eighth))));
   return us;
+}
+// The 288-wide tile.  Its k-tile costs 1.18 times the 256-wide one's for 1.125 times the work, so it pays where it saves
+// rounds (2240 and 1152 channels are 8 and 4 tiles).  Fitted to 120 shapes (700 .. 32760 tokens, the same projections, weights
+// cold), and the tiles it is compared with to the same shapes, which reach further up than the ones above: 7 % off each.  Taken
+// at 0.99 of the others' estimate or less: of 140 shapes 29, at 0.90 of the time on the mean, none slower.  us, best other / this:
+// 8192 x 2240 x 5600 220 / 157, 16384 x 2240 x 5600 348 / 314, 32760 x 2240 x 5600 747 / 646, 16384 x 1152 x 2880 106 / 88,
+// 9720 x 5760 x 1152 123 / 119; not taken: 4096 x 2240 x 2240 43 / 56, 16384 x 11200 x 2240 591 / 626, 12288 x 2240 x 2240 111 / 123.
+constexpr Tile16 kTile288 = {256, 288, 256, 11.3, 1.17, 1.61};
+constexpr Tile16 kBeside288[] = {
+    {256, 128, 256, 4.8, 0.75, 0.89}, {256, 192, 256, 7.4, 0.85, 1.18}, {256, 256, 256, 7.0, 1.20, 1.40},
+    {128, 128, 256, 2.3, 0.51, 0.61}, {128, 160, 256, 4.1, 0.62, 0.68},
+};
+constexpr int64_t kMaxStride288 = 1 << 21;  // rows of W from which the 32-bit offsets inside a tile could overflow
+bool takes_288(int M, int N, int K, double others_us) {  // others_us: by the constants above, which are lower
+  const double us = cost16(kTile288, M, N, K) / 0.99;
+  if (us > 1.1 * others_us) return false;
+  for (const Tile16& t : kBeside288)
+    if (us > cost16(t, M, N, K)) return false;
+  for (int a = 256; a < N; a += 256)
+    if (us > cost16(kBeside288[2], M, a, K) + cost16(kBeside288[1], M, N - a, K)) return false;
+  return true;
 }
 struct Plan16 {
   const Tile16* tile;
@@ -874,6 +895,7 @@ Plan16 plan16(int M, int N, int K) {
     const double us = cost16(kTiles16[2], M, a, K) + cost16(kTiles16[1], M, N - a, K);
     if (us < 0.98 * single && us < p.us) p.n_wide = a, p.us = us;
   }
+  if (takes_288(M, N, K, p.us)) p = {&kTile288, 0, cost16(kTile288, M, N, K)};
   return p;
 }
 // Split over k, or not: the split GEMM against the best unsplit one (16-bit and int8 weights decide alike, so that they
@@ -974,6 +996,9 @@ int launch(const void* A, const void* W, const float* scale, const EpiArgs& ep, 
       return gemm8_launch(a, w + (int64_t)p.n_wide * ldw, ep2, c + p.n_wide, M, N - p.n_wide, K, lda, ldw, ldc, epilogue,
                           is_f16<T>, 3, nullptr, s);
     }
+    if (p.tile->bn == 288 && ldw < kMaxStride288)
+      return gemm288_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, nullptr, s);
+    if (p.tile->bn == 288) return gemm8_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, 4, nullptr, s);
     if (p.tile->bm == 256)
       return gemm8_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, p.tile->bn / 64, nullptr, s);
     return gemm_ring_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, p.tile->bm, p.tile->bn, s);
@@ -1193,9 +1218,13 @@ SANA_API int sana_hip_tconv_residual(const void* X, const void* W, void* out, in
   const uint16_t* x = static_cast<const uint16_t*>(X);
   const EpiArgs e = {nullptr, nullptr, x + (taps / 2) * tap_rows * ldx, ldx, 0, M, nullptr, 0, 0, 0, 0};
   const Taps tp = {C, tap_rows, x_rows, 0, 0, zero_last_tap};
-  return gemm8_launch(x, static_cast<const uint16_t*>(W), e, static_cast<uint16_t*>(out), M, C, taps * C, ldx, ldw, ldo,
-                      SANA_EPI_GATE_RES, false,
-                     cost16(kTiles16[1], M, C, taps * C) < cost16(kTiles16[2], M, C, taps * C) ? 3 : 4, &tp, static_cast<hipStream_t>(stream));
+  const uint16_t* w = static_cast<const uint16_t*>(W);
+  uint16_t* o = static_cast<uint16_t*>(out);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const double us192 = cost16(kTiles16[1], M, C, taps * C), us256 = cost16(kTiles16[2], M, C, taps * C);
+  if (takes_288(M, C, taps * C, std::min(us192, us256)) && ldw < kMaxStride288)
+    return gemm288_launch(x, w, e, o, M, C, taps * C, ldx, ldw, ldo, SANA_EPI_GATE_RES, false, &tp, s);
+  return gemm8_launch(x, w, e, o, M, C, taps * C, ldx, ldw, ldo, SANA_EPI_GATE_RES, false, us192 < us256 ? 3 : 4, &tp, s);
 }
 
 SANA_API int sana_hip_dequant_w8(const int8_t* Wq, const float* scale, void* W, int N, int K, int64_t ldw,

@@ -49,6 +49,10 @@ struct Taps {
 int gemm8_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
                  int64_t ldw, int64_t ldc, int epilogue, bool f16, int nb, const Taps* taps, hipStream_t s);
 
+// The same in tiles of 256 tokens x 288 channels (gemm288.hip); no SANA_EPI_QKV_STATE; rows of W less than 2^21 values apart.
+int gemm288_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
+                   int64_t ldw, int64_t ldc, int epilogue, bool f16, const Taps* taps, hipStream_t s);
+
 // The GEMM for few tokens (gemm_ring.hip): the same operands and epilogues up to SANA_EPI_GATE_RES (gate not null), in tiles
 // of bm tokens x bn channels: 64 x 64, 64 x 128, 128 x 128 or 128 x 160.
 int gemm_ring_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,

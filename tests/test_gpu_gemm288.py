@@ -1,0 +1,72 @@
+"""The 256 x 288 tile kernel of the 16-bit GEMM at the edges of its tiles: integer operands (every product, sum and bias is
+exact in fp32, so the result is bit for bit the rounded integer matrix product), ragged rows and channels, k tails, one and
+several tiles per workgroup, gate rows that change inside a tile, and the temporal convolution against narrower tiles."""
+import ctypes
+
+import pytest
+import torch
+
+from sana_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _ints(*shape, lo=-3, hi=3, seed=0, dtype=torch.bfloat16):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randint(lo, hi + 1, shape, generator=g).to(dtype)
+
+
+def _runs_in_288(M, N, K):
+    plan = (ctypes.c_int * 4)()
+    _lib.check(_lib.load().sana_hip_gemm_plan(M, N, K, plan), "sana_hip_gemm_plan")
+    assert tuple(plan) == (256, 288, 0, 1), tuple(plan)
+
+
+# k tails of 8, 56 and 0 in an odd and an even number of k-tiles; ragged rows; ragged channels in the first and the second
+# wave column and one whole tile; the last two have more tiles than workgroups
+@pytest.mark.parametrize("M,N,K", [(1413, 11016, 200), (3287, 5016, 248), (5257, 3400, 256), (4325, 4208, 320),
+                                   (2907, 5528, 488), (8471, 4256, 200), (14040, 2592, 248)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_288_wide_tile_is_exact_on_integers(cuda, M, N, K, dtype):
+    _runs_in_288(M, N, K)
+    a, w, bias = (_ints(M, K, seed=1, dtype=dtype).to(cuda), _ints(N, K, seed=2, dtype=dtype).to(cuda),
+                  _ints(N, lo=-9, hi=9, seed=3, dtype=dtype).to(cuda))
+    ref = a.float() @ w.float().T        # |sum| <= 9 k < 2^24: exact in any order
+    assert torch.equal(ops.gemm_bf16(a, w), ref.to(dtype))
+    ref = (ref + bias.float()).to(dtype)
+    assert torch.equal(ops.gemm_bf16(a, w, bias, "bias"), ref)
+    y = ops.gemm_bf16(a, w, bias, "bias_silu")
+    want = torch.nn.functional.silu(ref.double())
+    # the fp32 sigmoid is good to a few 2^-24, the rounding to the io dtype is half an ulp: at most one ulp apart
+    ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+    assert ((y.double() - want).abs() <= ulp * want.abs() + 1e-7).all()
+
+
+@pytest.mark.parametrize("B,Ntok,C,K", [(3, 1096, 5016, 248), (7, 202, 11016, 200), (5, 1052, 3400, 256), (1, 8471, 4256, 200)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_288_wide_gated_residual_across_batch_boundaries(cuda, B, Ntok, C, K, dtype):
+    _runs_in_288(B * Ntok, C, K)
+    ints = lambda *s, hi=3, seed: _ints(*s, lo=-hi, hi=hi, seed=seed, dtype=dtype).to(cuda)
+    a, w, bias = ints(B, Ntok, K, seed=1), ints(C, K, seed=2), ints(C, hi=9, seed=3)
+    gate, res = ints(B, 1, C, hi=4, seed=4), ints(B, Ntok, C, hi=99, seed=5)
+    y = (a.float() @ w.float().T + bias.float()).to(dtype)
+    assert torch.equal(ops.gemm_gate_residual(a, w, bias, gate, res), res + gate * y)   # the stock pair's roundings
+    y = (a.float() @ w.float().T).to(dtype)
+    assert torch.equal(ops.gemm_gate_residual(a, w, None, gate, res), res + gate * y)
+
+
+@pytest.mark.parametrize("T,P,C,ends", [(5, 1560, 2240, [1, 3]), (6, 2700, 1152, [])])
+def test_288_wide_temporal_convolution_equals_one_launch_per_chunk(cuda, T, P, C, ends):
+    """The whole clip in 288-wide tiles, its chunks (or its frames' first rows) in narrower ones: the same products in the
+    same order, so the same bits."""
+    _runs_in_288(T * P, C, 3 * C)
+    g = torch.Generator().manual_seed(C + T)
+    y = torch.randn((T + 1) * P, C, generator=g).bfloat16().to(cuda)          # a real frame in front (a cache's last one)
+    w2 = (torch.randn(C, 3 * C, generator=g) * (1.0 / (3 * C)) ** 0.5).bfloat16().to(cuda)
+    one = ops.tconv_residual(y, w2, T * P, P, zero_last_tap=ops.frame_flags(T, ends, cuda))
+    bounds = [0, *(e + 1 for e in ends), T]
+    if ends:
+        parts = [ops.tconv_residual(y[f0 * P:(f1 + 1) * P], w2, (f1 - f0) * P, P) for f0, f1 in zip(bounds[:-1], bounds[1:])]
+        assert torch.equal(one, torch.cat(parts))
+    else:
+        assert torch.equal(one[:4000], ops.tconv_residual(y, w2, 4000, P))
