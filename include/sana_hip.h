@@ -123,6 +123,23 @@ int sana_hip_linattn_apply(const void* q, const float* state, void* out,
                            float eps, int io_dtype, int out_dtype, void* stream);
 
 /* ---------------------------------------------------------------------------
+ * Both phases in one call: one chunk, d = 32, out in the io dtype, no state returned.  Short sequences are one kernel
+ * that keeps the state on the compute unit (the same values as the two calls, up to the order of the state's fp32 sums),
+ * others the launches of the two.  k and v share strides, as in sana_hip_linattn_state; q and out as in
+ * sana_hip_linattn_apply; out must not overlap the inputs.
+ *   scratch  at least sana_hip_linattn_scratch_bytes(...) bytes, 16-byte aligned (may be NULL when that is 0)
+ */
+size_t sana_hip_linattn_scratch_bytes(int B, int N, int h, int d, int io_dtype);
+
+int sana_hip_linattn(const void* q, const void* k, const void* v, void* out,
+                     void* scratch, size_t scratch_bytes,
+                     int B, int N, int h, int d,
+                     int64_t q_stride_b, int64_t q_stride_n,
+                     int64_t stride_b, int64_t stride_n,
+                     int64_t o_stride_b, int64_t o_stride_n,
+                     float eps, int io_dtype, void* stream);
+
+/* ---------------------------------------------------------------------------
  * q/k RMSNorm and rotary embedding inside the attention kernels (bf16 io)
  *
  * LiteLAReLURope / ChunkCausalAttention / CachedCausalAttention

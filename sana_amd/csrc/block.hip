@@ -8,7 +8,7 @@
 namespace {
 
 struct Layout {  // byte offsets into the scratch buffer
-  size_t h, wide, o, x1, x2, y, state, ws, total, ws_bytes;  // o and x1: inside wide
+  size_t h, wide, o, x1, x2, y, ws, total, ws_bytes;  // o and x1: inside wide
 };
 
 bool plan(const sana_block_args& a, Layout& l) {
@@ -33,8 +33,7 @@ bool plan(const sana_block_args& a, Layout& l) {
   l.x1 = l.o + row;                                                    // behind the attention
   l.x2 = take(row);                                                    // behind the cross-attention
   l.y = take(M * a.hidden * 2);                                        // gated hidden values
-  l.state = take((size_t)a.B * heads * 33 * 32 * 4);
-  l.ws_bytes = sana_hip_linattn_workspace_bytes(a.B, heads, 32, 1, a.N, a.io_dtype);
+  l.ws_bytes = sana_hip_linattn_scratch_bytes(a.B, a.N, heads, 32, a.io_dtype);
   if (a.split_k)
     for (size_t b : {sana_hip_gemm_workspace_bytes(rows, 3 * a.C, a.C), sana_hip_gemm_workspace_bytes(rows, a.C, a.C),
                      sana_hip_gemm_workspace_bytes(rows, 2 * a.hidden, a.C), sana_hip_gemm_workspace_bytes(rows, a.C, a.hidden)})
@@ -80,7 +79,6 @@ SANA_API int sana_hip_block(const sana_block_args* args, void* stream) {
   const bool f16 = dt == SANA_DT_F16;
   char* s = static_cast<char*>(a.scratch);
   void *h = s + l.h, *wide = s + l.wide, *o = s + l.o, *x1 = s + l.x1, *x2 = s + l.x2, *y = s + l.y;
-  float* state = reinterpret_cast<float*>(s + l.state);
   void* ws = l.ws_bytes ? s + l.ws : nullptr;
   void* gws = a.split_k ? ws : nullptr;
   auto gemm = [&](const void* A, const void* W, const void* bias, void* out, int N, int K, int epi) {
@@ -102,9 +100,8 @@ SANA_API int sana_hip_block(const sana_block_args* args, void* stream) {
   SANA_DO(gemm(h, a.qkv_w, a.qkv_b, wide, 3 * C, C, a.qkv_b ? SANA_EPI_BIAS : SANA_EPI_NONE));
   const char* qkv = static_cast<const char*>(wide);
   const int64_t sb = a.B > 1 ? (int64_t)a.N * 3 * C : 0, ob = a.B > 1 ? (int64_t)a.N * C : 0;
-  SANA_DO(sana_hip_linattn_state(qkv + 2 * (size_t)C, qkv + 4 * (size_t)C, state, ws, l.ws_bytes, a.B, a.N, heads, 32, sb, 3 * C,
-                                 nullptr, 1, a.N, 0, dt, stream));
-  SANA_DO(sana_hip_linattn_apply(qkv, state, o, a.B, a.N, heads, 32, sb, 3 * C, ob, C, nullptr, 1, a.N, a.eps_attn, dt, dt, stream));
+  SANA_DO(sana_hip_linattn(qkv, qkv + 2 * (size_t)C, qkv + 4 * (size_t)C, o, ws, l.ws_bytes, a.B, a.N, heads, 32, sb, 3 * C, sb,
+                           3 * C, ob, C, a.eps_attn, dt, stream));
   SANA_DO(gated(o, a.proj_w, a.proj_b, a.gate_msa, a.mod_stride, a.x, x1, C));
   // x2 = x1 + cross_attention(x1)
   SANA_DO(gemm(x1, a.q_w, a.q_b, h, C, C, SANA_EPI_BIAS));

@@ -599,6 +599,263 @@ __global__ __launch_bounds__(256) void linattn_apply32_kernel(
 }
 
 // ----------------------------------------------------------------------------
+// Both phases in one launch, for short sequences: one workgroup = one head of one batch entry, the state never leaves LDS.
+// Three launches (phase 1, reduction, phase 2) are 3 - 6 us of work each with a gap in front; here everything a head needs
+// for 1024 tokens is requested at once and the rest is one memory round trip, the transposes and the matrix products of one
+// compute unit.  That is also the bound: a head's tokens are one compute unit's work.  us, two calls / this, replayed from a
+// graph: bf16, 36 heads x 256 tokens 10.1 / 5.4, 36 x 1024 12.5 / 8.5, 140 x 1024 19.1 / 15.2; fp16 36 x 256 10.8 / 6.0; fp32
+// 36 x 256 10.8 / 8.5, 140 x 512 21.4 / 17.1.
+// ----------------------------------------------------------------------------
+constexpr int WHOLE_TOKENS = 1024;  // the most that one round of loads covers
+template <int OFF>
+__device__ __forceinline__ u32x2_t lds_read_tr16(uint32_t addr) {  // 4 tokens x 16 channels -> this lane's channel, 4 tokens
+  u32x2_t v;
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+  return v;
+}
+
+// 16-bit io.  grid: B * h; block 512.  Phase 1: wave w takes the 32-token tiles w, w + 8, .. through its own LDS (rows of 96
+// bytes: conflict-free transposing reads) as operands of MFMA 16x16x32, the key sum with an operand of ones; the waves'
+// sums are added in wave order.  Phase 2 as linattn_apply16_kernel, on the 16-token steps w, w + 8, ..
+template <typename T>
+__global__ __launch_bounds__(512) void linattn_whole16_kernel(
+    const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V, uint16_t* __restrict__ out,
+    int N, int h, int64_t q_stride_b, int64_t q_stride_n, int64_t stride_b, int64_t stride_n, int64_t o_stride_b,
+    int64_t o_stride_n, float eps) {
+  constexpr int WAVES = 8, ROW = 96, U1 = WHOLE_TOKENS / (WAVES * TILE), U2 = WHOLE_TOKENS / (WAVES * 16);
+  constexpr int STATE_AT = WAVES * U2 * 1024;
+  static_assert(STATE_AT >= WAVES * 2 * TILE * ROW && STATE_AT >= WAVES * STATE_ELEMS * 4, "the state lies behind the stages");
+  __shared__ __attribute__((aligned(16))) unsigned char smem[STATE_AT + STATE_ELEMS * 4];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int b = blockIdx.x / h, head = blockIdx.x - b * h;
+  const int ld_tok = lane >> 2, ld_chunk = lane & 3;  // a load instruction: 16 tokens x 64 bytes
+  const int n = lane & 15, g = lane >> 4;             // MFMA layout
+  const u32x4_t zero4 = {0u, 0u, 0u, 0u};
+  const uint16_t* kbase = K + (int64_t)b * stride_b + head * D + 8 * ld_chunk;
+  const uint16_t* vbase = V + (int64_t)b * stride_b + head * D + 8 * ld_chunk;
+  const uint16_t* qbase = Q + (int64_t)b * q_stride_b + head * D + 8 * ld_chunk;
+
+  // ---- phase 1
+  u32x4_t kreg[U1][2], vreg[U1][2], raw[U2];
+#pragma unroll
+  for (int u = 0; u < U1; ++u)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int tok = (wave + u * WAVES) * TILE + 16 * i + ld_tok;
+      kreg[u][i] = tok < N ? *reinterpret_cast<const u32x4_t*>(kbase + (int64_t)tok * stride_n) : zero4;
+      vreg[u][i] = tok < N ? *reinterpret_cast<const u32x4_t*>(vbase + (int64_t)tok * stride_n) : zero4;
+    }
+#pragma unroll
+  for (int u = 0; u < U2; ++u) {
+    const int tok = (wave + u * WAVES) * 16 + ld_tok;
+    raw[u] = tok < N ? *reinterpret_cast<const u32x4_t*>(qbase + (int64_t)tok * q_stride_n) : zero4;
+  }
+  unsigned char* stage = smem + wave * (2 * TILE * ROW);
+  const uint32_t stage_addr = (uint32_t)(size_t)(__attribute__((address_space(3))) const unsigned char*)stage;
+  const uint32_t k_at = stage_addr + (4 * g + (n >> 2)) * ROW + (n & 3) * 8, v_at = k_at + TILE * ROW;
+  const uint32_t one2 = is_f16<T> ? 0x3c003c00u : 0x3f803f80u;
+  const u32x4_t ones = {one2, one2, one2, one2};
+  f32x4_t S[2][2], ks[2];  // S[i][j]: dv 16 i + 4 g + r, dk 16 j + n;  ks[j]: dk 16 j + n, every row
+#pragma unroll
+  for (int j = 0; j < 2; ++j) S[0][j] = S[1][j] = ks[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < U1; ++u) {
+    if ((wave + u * WAVES) * TILE >= N) break;  // uniform
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      *reinterpret_cast<u32x4_t*>(stage + (16 * i + ld_tok) * ROW + 16 * ld_chunk) = relu_pk16(kreg[u][i]);
+      *reinterpret_cast<u32x4_t*>(stage + TILE * ROW + (16 * i + ld_tok) * ROW + 16 * ld_chunk) = vreg[u][i];
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // wave-private LDS: in-order, no barrier needed
+    u32x2_t kf[2][2], vf[2][2];  // [channels 16 j ..][tokens 16 i ..]
+    kf[0][0] = lds_read_tr16<0>(k_at), kf[0][1] = lds_read_tr16<16 * ROW>(k_at);
+    kf[1][0] = lds_read_tr16<32>(k_at), kf[1][1] = lds_read_tr16<32 + 16 * ROW>(k_at);
+    vf[0][0] = lds_read_tr16<0>(v_at), vf[0][1] = lds_read_tr16<16 * ROW>(v_at);
+    vf[1][0] = lds_read_tr16<32>(v_at), vf[1][1] = lds_read_tr16<32 + 16 * ROW>(v_at);
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+v"(kf[0][0]), "+v"(kf[0][1]), "+v"(kf[1][0]), "+v"(kf[1][1]), "+v"(vf[0][0]), "+v"(vf[0][1]),
+                   "+v"(vf[1][0]), "+v"(vf[1][1])::"memory");
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const u32x4_t kk = {kf[j][0].x, kf[j][0].y, kf[j][1].x, kf[j][1].y};
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        S[i][j] = mfma_16x16x32<T>(u32x4_t{vf[i][0].x, vf[i][0].y, vf[i][1].x, vf[i][1].y}, kk, S[i][j]);
+      ks[j] = mfma_16x16x32<T>(ones, kk, ks[j]);
+    }
+  }
+  __syncthreads();
+  float* red = reinterpret_cast<float*>(smem) + wave * STATE_ELEMS;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[(16 * i + 4 * g + r) * D + 16 * j + n] = S[i][j][r];
+    if (g == 0) red[D * D + 16 * j + n] = ks[j][0];
+  }
+  __syncthreads();
+  float* state = reinterpret_cast<float*>(smem + STATE_AT);
+  for (int e = tid; e < STATE_ELEMS; e += 64 * WAVES) {
+    const float* p = reinterpret_cast<const float*>(smem) + e;
+    float s = p[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) s += p[w * STATE_ELEMS];
+    state[e] = s;
+  }
+  __syncthreads();
+
+  // ---- phase 2 (operand layout: linattn_apply16_kernel)
+  u32x4_t st[3][3];
+#pragma unroll
+  for (int rb = 0; rb < 3; ++rb) {
+    const float* sp = state + (rb < 2 ? 8 * (n >> 2) + 4 * rb + (n & 3) : D) * D + 8 * g;
+    const f32x4_t x0 = *reinterpret_cast<const f32x4_t*>(sp), x1 = *reinterpret_cast<const f32x4_t*>(sp + 4);
+    const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+    split3(x, st[rb]);
+  }
+  unsigned char* qstage = smem + wave * (U2 * 1024);
+  const int slot_w = 16 * (4 * ld_tok + (ld_chunk ^ ((ld_tok >> 1) & 3)));
+  const int slot_r = 16 * (4 * n + (g ^ ((n >> 1) & 3)));
+  uint16_t* obase = out + (int64_t)b * o_stride_b + head * D + 8 * ld_chunk;
+#pragma unroll
+  for (int u = 0; u < U2; ++u) *reinterpret_cast<u32x4_t*>(qstage + u * 1024 + slot_w) = relu_pk16(raw[u]);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int u = 0; u < U2; ++u) {
+    if ((wave + u * WAVES) * 16 >= N) break;  // uniform
+    unsigned char* slot = qstage + u * 1024 + slot_r;
+    const u32x4_t qd = *reinterpret_cast<const u32x4_t*>(slot);
+    u32x4_t q_hi, q_lo;
+    if constexpr (is_f16<T>) f16_to_2bf16(qd, q_hi, q_lo);
+    f32x4_t acc[3];
+#pragma unroll
+    for (int rb = 0; rb < 3; ++rb) {
+      f32x4_t a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int term = 2; term >= 0; --term) {  // smallest terms first
+        if constexpr (is_f16<T>) {
+          a = mfma_16x16x32_bf16(st[rb][term], q_lo, a);
+          a = mfma_16x16x32_bf16(st[rb][term], q_hi, a);
+        } else {
+          a = mfma_16x16x32_bf16(st[rb][term], qd, a);
+        }
+      }
+      acc[rb] = a;
+    }
+    const float den = acc[2][0] + eps;
+    u32x4_t o;
+    if constexpr (is_f16<T>) {
+      const Quotient by(den);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = pk16<T>(by(acc[e >> 1][2 * (e & 1)]), by(acc[e >> 1][2 * (e & 1) + 1]));
+    } else {
+      const float inv = __builtin_amdgcn_rcpf(den);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = pk16<T>(acc[e >> 1][2 * (e & 1)] * inv, acc[e >> 1][2 * (e & 1) + 1] * inv);
+    }
+    *reinterpret_cast<u32x4_t*>(slot) = o;  // in the place of this lane's queries
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int u = 0; u < U2; ++u) {
+    const int tok = (wave + u * WAVES) * 16 + ld_tok;
+    const u32x4_t o = *reinterpret_cast<const u32x4_t*>(qstage + u * 1024 + slot_w);
+    if (tok < N) *reinterpret_cast<u32x4_t*>(obase + (int64_t)tok * o_stride_n) = o;
+  }
+}
+
+// fp32 io.  grid: B * h; block 1024.  Phase 1 as linattn_state32_kernel with the waves as its splits of 64 tokens (same sums
+// up to 1024 tokens), phase 2 as linattn_apply32_kernel on the 32-token tiles w, w + 16, ..
+__global__ __launch_bounds__(1024) void linattn_whole32_kernel(
+    const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V, float* __restrict__ out, int N, int h,
+    int64_t q_stride_b, int64_t q_stride_n, int64_t stride_b, int64_t stride_n, int64_t o_stride_b, int64_t o_stride_n,
+    float eps) {
+  constexpr int WAVES = WHOLE_TOKENS / 64, U = 16;
+  __shared__ __attribute__((aligned(16))) float smem[(WAVES + 1) * STATE_ELEMS];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int b = blockIdx.x / h, head = blockIdx.x - b * h;
+  const int j = lane & 31, g = lane >> 5;
+  const float* kp = K + (int64_t)b * stride_b + head * D + j;
+  const float* vp = V + (int64_t)b * stride_b + head * D + j;
+  f32x16_t accS;
+  float accK = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) accS[i] = 0.f;
+#pragma unroll 1
+  for (int t = wave * 64; t < min(wave * 64 + 64, N); t += 2 * U) {  // (both halves at once need more registers than there are)
+    float kk[U], vv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t at = (int64_t)min(t + 2 * u + g, N - 1) * stride_n;  // (no branch around a load)
+      kk[u] = kp[at], vv[u] = vp[at];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool ok = t + 2 * u + g < N;
+      kk[u] = ok ? fmaxf(kk[u], 0.f) : 0.f;
+      vv[u] = ok ? vv[u] : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      accS = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[u], kk[u], accS, 0, 0, 0);
+      accK += kk[u];
+    }
+  }
+  f32x4_t qn[4];
+  auto load_q = [&](int t) {
+    const float* qp = Q + (int64_t)b * q_stride_b + (int64_t)min(t + j, N - 1) * q_stride_n + head * D + 16 * g;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) qn[i] = *reinterpret_cast<const f32x4_t*>(qp + 4 * i);
+  };
+  load_q(wave * 32);  // (a wave without a tile: the last token)
+  float* red = smem + wave * STATE_ELEMS;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) red[(8 * (r >> 2) + 4 * g + (r & 3)) * D + j] = accS[r];
+  accK += __shfl_xor(accK, 32, 64);
+  if (g == 0) red[D * D + j] = accK;
+  __syncthreads();
+  float* state = smem + WAVES * STATE_ELEMS;
+  for (int e = threadIdx.x; e < STATE_ELEMS; e += 64 * WAVES) {
+    float s = smem[e];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) s += smem[w * STATE_ELEMS + e];
+    state[e] = s;
+  }
+  __syncthreads();
+  f32x4_t a_num[4], a_den[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    a_num[i] = *reinterpret_cast<const f32x4_t*>(state + j * D + 16 * g + 4 * i);
+    a_den[i] = *reinterpret_cast<const f32x4_t*>(state + D * D + 16 * g + 4 * i);
+  }
+  for (int t = wave * 32; t < N; t += WAVES * 32) {
+    const int tok = t + j;
+    const bool ok = tok < N;
+    float qv[16], den = 0.f;
+#pragma unroll
+    for (int s = 0; s < 16; ++s) qv[s] = ok ? fmaxf(qn[s >> 2][s & 3], 0.f) : 0.f;
+    if (t + WAVES * 32 < N) load_q(t + WAVES * 32);
+    f32x16_t num;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) num[i] = 0.f;
+#pragma unroll
+    for (int s = 0; s < 16; ++s) num = __builtin_amdgcn_mfma_f32_32x32x2f32(a_num[s >> 2][s & 3], qv[s], num, 0, 0, 0);
+#pragma unroll
+    for (int s = 0; s < 16; ++s) den = fmaf(a_den[s >> 2][s & 3], qv[s], den);
+    den += __shfl_xor(den, 32, 64);
+    if (ok) {
+      const float dd = den + eps;
+      float* op = out + (int64_t)b * o_stride_b + (int64_t)tok * o_stride_n + head * D;
+#pragma unroll
+      for (int r = 0; r < 16; r += 4)
+        *reinterpret_cast<f32x4_t*>(op + 2 * r + 4 * g) = f32x4_t{num[r] / dd, num[r + 1] / dd, num[r + 2] / dd, num[r + 3] / dd};
+    }
+  }
+}
+
+// ----------------------------------------------------------------------------
 // Per-token 1/rms of q and of k over all C channels (the statistic of the reference's
 // RMSNorm before the head split): rinv = rsqrt(mean(x^2) + eps).  One wave per (token, tensor).
 // grid: x = ceil(B*N/4), y = 2 (q, k); block 256.
@@ -952,4 +1209,57 @@ extern "C" __attribute__((visibility("default"))) int sana_hip_litela_apply(
   const QkPre pre = {q_rinv, static_cast<const uint16_t*>(q_weight), rope, rope ? 1 : 0};
   return apply_impl(q, state, out, B, N, h, d, q_stride_b, q_stride_n, o_stride_b, o_stride_n, nullptr, 1, N, eps,
                     io_dtype, out_dtype, pre, stream);
+}
+
+// One launch while a head is a short piece of work and every head has a compute unit.  us, two calls / one launch: bf16
+// 36 x 1024 12.5 / 8.5, 210 x 1024 21.3 / 19.0, but 36 x 1536 12.8 / 13.1 and 280 x 1024 26.4 / 30.2 (a second round); f16 210 x
+// 1024 23.7 / 21.2.  fp32 moves twice the bytes and has the slower matrix instruction, so that few heads leave too much of the
+// chip idle beyond 256 tokens: 36 x 256 10.8 / 8.5, 36 x 512 11.3 / 12.2, 70 x 512 13.5 / 12.9, 70 x 768 16.0 / 19.3, 108 x 768
+// 21.5 / 20.4, 140 x 1024 27.7 / 24.9.
+static bool one_launch(int B, int N, int h, int io_dtype) {
+  const int64_t heads = (int64_t)B * h;
+  if (N > WHOLE_TOKENS || heads > 256) return false;
+  return io_dtype != SANA_DT_F32 || N <= 256 || N <= 7 * heads;
+}
+static size_t state_bytes(int B, int h) { return ((size_t)B * h * STATE_ELEMS * sizeof(float) + 255) & ~(size_t)255; }
+
+extern "C" __attribute__((visibility("default"))) size_t sana_hip_linattn_scratch_bytes(int B, int N, int h, int d, int io_dtype) {
+  if (B <= 0 || N <= 0 || h <= 0 || d != D || one_launch(B, N, h, io_dtype)) return 0;
+  return state_bytes(B, h) + sana_hip_linattn_workspace_bytes(B, h, d, 1, N, io_dtype);
+}
+
+extern "C" __attribute__((visibility("default"))) int sana_hip_linattn(
+    const void* q, const void* k, const void* v, void* out, void* scratch, size_t scratch_bytes, int B, int N, int h, int d,
+    int64_t q_stride_b, int64_t q_stride_n, int64_t stride_b, int64_t stride_n, int64_t o_stride_b, int64_t o_stride_n, float eps,
+    int io_dtype, void* stream) {
+  if (!q || !k || !v || !out || B <= 0 || N <= 0 || h <= 0) return SANA_ERR_ARG;
+  if (d != D) return SANA_ERR_SHAPE;
+  if (io_dtype != SANA_DT_F32 && io_dtype != SANA_DT_BF16 && io_dtype != SANA_DT_F16) return SANA_ERR_DTYPE;
+  const int64_t C = (int64_t)h * d, vec = io_dtype == SANA_DT_F32 ? 4 : 8;  // values in 16 bytes
+  if (q_stride_n < C || stride_n < C || o_stride_n < C || q_stride_b < 0 || stride_b < 0 || o_stride_b < 0) return SANA_ERR_ARG;
+  if ((int64_t)B * h > (1 << 22)) return SANA_ERR_SHAPE;
+  if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out)) return SANA_ERR_ALIGN;
+  for (int64_t x : {q_stride_b, q_stride_n, stride_b, stride_n, o_stride_b, o_stride_n})
+    if (x % vec) return SANA_ERR_ALIGN;
+  if (!one_launch(B, N, h, io_dtype)) {
+    const size_t at = state_bytes(B, h);
+    if (!scratch || scratch_bytes < sana_hip_linattn_scratch_bytes(B, N, h, d, io_dtype)) return SANA_ERR_WORKSPACE;
+    float* state = static_cast<float*>(scratch);
+    const int rc = sana_hip_linattn_state(k, v, state, static_cast<char*>(scratch) + at, scratch_bytes - at, B, N, h, d, stride_b,
+                                          stride_n, nullptr, 1, N, 0, io_dtype, stream);
+    return rc != SANA_OK ? rc
+                         : sana_hip_linattn_apply(q, state, out, B, N, h, d, q_stride_b, q_stride_n, o_stride_b, o_stride_n,
+                                                  nullptr, 1, N, eps, io_dtype, io_dtype, stream);
+  }
+  const dim3 grid((unsigned)(B * h));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+#define SANA_WHOLE(kernel, threads, E)                                                                                 \
+  hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, static_cast<const E*>(q), static_cast<const E*>(k),           \
+                     static_cast<const E*>(v), static_cast<E*>(out), N, h, q_stride_b, q_stride_n, stride_b, stride_n, \
+                     o_stride_b, o_stride_n, eps)
+  if (io_dtype == SANA_DT_F32) SANA_WHOLE(linattn_whole32_kernel, WHOLE_TOKENS, float);
+  else if (io_dtype == SANA_DT_F16) SANA_WHOLE(linattn_whole16_kernel<F16>, 512, uint16_t);
+  else SANA_WHOLE(linattn_whole16_kernel<BF16>, 512, uint16_t);
+#undef SANA_WHOLE
+  return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
 }

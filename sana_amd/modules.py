@@ -423,6 +423,8 @@ class LiteLA(nn.Module):
     def _attend(self, qkv, rotary_emb, chunk_tokens=None):
         pre_q, pre_k = self._pre(qkv, rotary_emb)
         causal = chunk_tokens is not None and len(chunk_tokens) > 1
+        if pre_q is None and pre_k is None:
+            return ops.relu_linear_attention(qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], self.eps, chunk_tokens, head_dim=self.dim)
         state = ops.linattn_state(qkv[:, :, 1], qkv[:, :, 2], chunk_tokens, causal=causal, pre=pre_k,
                                   head_dim=self.dim)
         return ops.linattn_apply(qkv[:, :, 0], state, self.eps, chunk_tokens, pre=pre_q)

@@ -291,10 +291,32 @@ def linattn_apply(q: torch.Tensor, state: torch.Tensor, eps: float, chunk_tokens
     return out
 
 
+def _one_call(q, k, v, d: int) -> bool:
+    """Whether ``sana_hip_linattn`` takes these.  What it does not (mixed dtypes or shapes, k and v of different
+    strides, other head dims) goes to the two calls, which serve or refuse it."""
+    if d != HEAD_DIM or q.dim() != 3 or not q.is_cuda or q.shape != k.shape or k.shape != v.shape:
+        return False
+    if q.dtype != k.dtype or k.dtype != v.dtype or q.dtype not in _DT or q.shape[2] % d or q.numel() == 0:
+        return False
+    return q.device == k.device == v.device and all(a == b or n == 1 for a, b, n in zip(k.stride(), v.stride(), k.shape))
+
+
 def relu_linear_attention(q, k, v, eps: float, chunk_tokens=None, out_dtype=None,
                           head_dim: int = HEAD_DIM) -> torch.Tensor:
     """Both phases on token-major [B, N, C] views; chunk-causal when ``chunk_tokens`` has > 1 entry."""
     causal = chunk_tokens is not None and len(chunk_tokens) > 1
+    if not causal and out_dtype in (None, q.dtype) and _one_call(q, k, v, head_dim):
+        B, N, C = q.shape
+        h, dt, lib = C // head_dim, _dt(q), _lib.load()
+        qs, ks = _token_major_view(q, "q"), _token_major_view(k, "k")
+        out = torch.empty(B, N, C, dtype=q.dtype, device=q.device)
+        nbytes = lib.sana_hip_linattn_scratch_bytes(B, N, h, head_dim, dt)
+        ws = _workspace(q.device, nbytes)
+        code = lib.sana_hip_linattn(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                                    ws.data_ptr() if ws is not None else None, nbytes, B, N, h, head_dim, *qs, *ks,
+                                    N * C if B > 1 else 0, C, float(eps), dt, _stream())
+        _lib.check(code, "sana_hip_linattn")
+        return out
     state = linattn_state(k, v, chunk_tokens, causal=causal, head_dim=head_dim)
     return linattn_apply(q, state, eps, chunk_tokens, out_dtype)
 

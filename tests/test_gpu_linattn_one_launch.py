@@ -1,0 +1,67 @@
+"""Both phases of the linear attention in one kernel (short sequences): against the fp64 oracle, at the edges of its tiles
+(16-token steps, 32-token tiles, 64-token ranges, 256 heads, 1024 tokens) and just beyond them, and no further from it
+than the two calls."""
+import pytest
+import torch
+
+from oracle import sana_oracle as O
+from sana_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(a, b):
+    return ((a.double() - b).norm() / b.norm()).item()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,N,C", [(1, 1, 64), (2, 15, 32), (1, 17, 96), (3, 33, 160), (1, 255, 1152), (1, 256, 1152),
+                                   (2, 513, 64), (1, 972, 2240), (2, 1024, 1152), (3, 1023, 2240),
+                                   (1, 1025, 96), (8, 100, 1056)])
+def test_matches_the_oracle_and_the_two_calls(cuda, B, N, C, dtype):
+    eps = 1e-8
+    gen = torch.Generator().manual_seed(N + C)
+    wide = torch.randn(B, N, 3 * C + 32, generator=gen).to(dtype)      # rows with something between them
+    q, k, v = (wide[:, :, i * C:(i + 1) * C] for i in range(3))
+    heads = [t.double().reshape(B, N, C // 32, 32).permute(0, 2, 3, 1) for t in (q, k, v)]
+    ref = O.relu_linear_attention(heads[0], heads[1].transpose(-1, -2), heads[2], eps).permute(0, 3, 1, 2).reshape(B, N, C)
+    d = wide.to(cuda)
+    q, k, v = (d[:, :, i * C:(i + 1) * C] for i in range(3))
+    got = ops.relu_linear_attention(q, k, v, eps).cpu()
+    two = ops.linattn_apply(q, ops.linattn_state(k, v), eps).cpu()
+    assert bool(torch.isfinite(got).all())
+    # fp32: a sum of N products, rounded at 6e-8 each in random directions; 16 bits: one rounding of the result (2^-9, 2^-12)
+    bound = {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dtype]
+    assert _rel(got, ref) <= bound
+    assert _rel(got, ref) <= 1.05 * _rel(two, ref) + 1e-8
+    one = _lib.load().sana_hip_linattn_scratch_bytes(B, N, C // 32, 32, ops._dt(q)) == 0
+    assert one == (N <= 1024 and B * C // 32 <= 256 and (dtype != torch.float32 or N <= max(256, 7 * B * C // 32)))
+    if not one:
+        assert torch.equal(got, two)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_zeros_and_infinities_as_the_two_calls(cuda, dtype):
+    """Tokens without a positive key or query (0 / eps), a head of zeros, and an infinity in one head: the same classes."""
+    gen = torch.Generator().manual_seed(3)
+    qkv = torch.randn(2, 70, 3, 128, generator=gen)
+    qkv[0, :, 1, :32] = -1.0
+    qkv[0, 5, 0] = -2.0
+    qkv[1, 9, 1, 40], qkv[1, 11, 2, 70] = float("inf"), float("-inf")
+    q, k, v = (qkv.to(dtype).to(cuda)[:, :, i] for i in range(3))
+    got, two = ops.relu_linear_attention(q, k, v, 1e-8), ops.linattn_apply(q, ops.linattn_state(k, v), 1e-8)
+    assert torch.equal(torch.isnan(got), torch.isnan(two)) and torch.equal(torch.isinf(got), torch.isinf(two))
+    ok = torch.isfinite(two)
+    assert torch.allclose(got[ok].float(), two[ok].float(), rtol=2.0 ** -7, atol=1e-6)
+
+
+def test_what_it_does_not_take_goes_to_the_two_calls(cuda):
+    x = torch.randn(1, 64, 3, 64, device=cuda)
+    q, k, v = x[:, :, 0], x[:, :, 1], x[:, :, 2]
+    assert ops._one_call(q, k, v, 32)
+    assert not ops._one_call(q, k.contiguous(), v, 32)                       # k and v of different strides: refused
+    assert not ops._one_call(q, k.bfloat16(), v.bfloat16(), 32)
+    with pytest.raises(_lib.SanaHipError):
+        ops.relu_linear_attention(q, k.contiguous(), v, 1e-8)
+    out32 = ops.relu_linear_attention(q.bfloat16(), k.bfloat16(), v.bfloat16(), 1e-8, out_dtype=torch.float32)
+    assert out32.dtype == torch.float32
