@@ -140,6 +140,18 @@ int sana_hip_linattn(const void* q, const void* k, const void* v, void* out,
                      float eps, int io_dtype, void* stream);
 
 /* ---------------------------------------------------------------------------
+ * The cache of a stream's earlier chunks (CachedCausalAttention, CachedGLUMBConvTemp)
+ *
+ * sana_hip_state_cache: save_vk [B][h][d][d] and save_ks [B][h][1][d] receive the state's product rows and its last row
+ * (both or neither NULL), then state [B][h][1][d+1][d] += past_vk, past_ks (both or neither NULL); fp32, contiguous.
+ * sana_hip_transpose16: dst[b][p][c] = src[b][c][p] for 16-bit values, unit stride along the last axis of each.
+ */
+int sana_hip_state_cache(float* state, const float* past_vk, const float* past_ks, float* save_vk, float* save_ks,
+                         int B, int h, int d, void* stream);
+int sana_hip_transpose16(const void* src, void* dst, int B, int P, int C, int64_t src_b, int64_t src_c,
+                         int64_t dst_b, int64_t dst_p, void* stream);
+
+/* ---------------------------------------------------------------------------
  * q/k RMSNorm and rotary embedding inside the attention kernels (bf16 io)
  *
  * LiteLAReLURope / ChunkCausalAttention / CachedCausalAttention

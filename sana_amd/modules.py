@@ -504,13 +504,10 @@ class CachedCausalAttention(LiteLAReLURope):
         d = self.dim
         state = ops.linattn_state(qkv[:, :, 1], qkv[:, :, 2], pre=pre_k, head_dim=d)  # [B, h, 1, d+1, d]: this chunk only
         if kv_cache is not None:
-            past_vk, past_ks = kv_cache[0], kv_cache[1]
+            past = tuple(kv_cache[:2])
+            saved = ops.state_cache_(state, past if all(t is not None for t in past) else None, save_kv_cache)
             if save_kv_cache:
-                kv_cache[0] = state[:, :, 0, :d].clone()
-                kv_cache[1] = state[:, :, 0, d:].clone()
-            if past_vk is not None and past_ks is not None:
-                state[:, :, 0, :d] += past_vk.to(state)
-                state[:, :, 0, d:] += past_ks.to(state)
+                kv_cache[0], kv_cache[1] = saved
         out = self._proj_gated(ops.linattn_apply(qkv[:, :, 0], state, self.eps, pre=pre_q), gate, residual)
         if kv_cache is not None:
             return out, kv_cache
@@ -726,7 +723,7 @@ class GLUMBConvTemp(GLUMBConv):
         if left is None:
             buf[:, :P].zero_()
         else:
-            buf[:, :P].copy_(left)
+            ops.copy_tokens_(buf[:, :P], left)
         out = buf.new_empty(B, T * P, C)
         w2 = self._tconv_weight()
         # one launch per batch entry for all chunks: the frame behind a chunk's last frame reads as zeros

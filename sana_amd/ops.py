@@ -291,6 +291,41 @@ def linattn_apply(q: torch.Tensor, state: torch.Tensor, eps: float, chunk_tokens
     return out
 
 
+def state_cache_(state: torch.Tensor, past: Optional[Tuple[torch.Tensor, torch.Tensor]], save: bool):
+    """What a streamed chunk does with its state [B, h, 1, d+1, d]: with ``save`` returns copies of the products
+    [B, h, d, d] and of the key sums [B, h, 1, d] (else None), then adds ``past`` (the same pair of the chunks before)."""
+    B, h, _, _, d = state.shape
+    rows, last = (B, h, d, d), (B, h, 1, d)
+    fits = state.is_cuda and state.dtype == torch.float32 and state.is_contiguous() and state.data_ptr() % 16 == 0 and state.numel()
+    if past is not None:
+        fits = fits and all(t.dtype == torch.float32 and t.device == state.device and t.is_contiguous()
+                            and t.data_ptr() % 16 == 0 and tuple(t.shape) == s for t, s in zip(past, (rows, last)))
+    if not fits:   # a cache that was moved or cast
+        saved = (state[:, :, 0, :d].clone(), state[:, :, 0, d:].clone()) if save else None
+        if past is not None:
+            state[:, :, 0, :d] += past[0].to(state)
+            state[:, :, 0, d:] += past[1].to(state)
+        return saved
+    saved = (state.new_empty(rows), state.new_empty(last)) if save else None
+    ptrs = [t.data_ptr() for t in past] if past is not None else [None, None]
+    ptrs += [t.data_ptr() for t in saved] if save else [None, None]
+    _lib.check(_lib.load().sana_hip_state_cache(state.data_ptr(), *ptrs, B, h, d, _stream()), "sana_hip_state_cache")
+    return saved
+
+
+def copy_tokens_(dst: torch.Tensor, src: torch.Tensor) -> torch.Tensor:
+    """``dst.copy_(src)`` for token-major [B, P, C] dst; a channel-major src of its 16-bit dtype goes through LDS tiles."""
+    if dst.is_cuda and src.device == dst.device and src.dtype == dst.dtype and dst.dtype in IO16 and src.shape == dst.shape \
+            and dst.dim() == 3 and dst.numel() and src.stride(1) == 1 and src.stride(2) != 1 and dst.stride(2) == 1 \
+            and dst.shape[2] % 8 == 0 and dst.stride(1) % 8 == 0 and dst.stride(0) % 8 == 0 and dst.stride(1) >= dst.shape[2] \
+            and dst.data_ptr() % 16 == 0 and dst.shape[0] <= 65535 and dst.shape[2] < 1 << 22:
+        B, P, C = dst.shape
+        _lib.check(_lib.load().sana_hip_transpose16(src.data_ptr(), dst.data_ptr(), B, P, C, src.stride(0), src.stride(2),
+                                                    dst.stride(0), dst.stride(1), _stream()), "sana_hip_transpose16")
+        return dst
+    return dst.copy_(src)
+
+
 def _one_call(q, k, v, d: int) -> bool:
     """Whether ``sana_hip_linattn`` takes these.  What it does not (mixed dtypes or shapes, k and v of different
     strides, other head dims) goes to the two calls, which serve or refuse it."""
