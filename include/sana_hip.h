@@ -416,6 +416,13 @@ int sana_hip_cross_attention_f16(const void* q, const void* kv, const float* key
                                  int Nk, int H, int d, int64_t ldq, int64_t ldkv, int64_t ldo,
                                  int64_t bias_stride, float scale, void* stream);
 
+/* bias[i] = (1 - mask[i]) * -10000 in fp32 (sana_blocks.py:89-90): key_bias of the two calls above from n mask values of
+ * one of these types (bool counts as U8). */
+enum { SANA_MASK_U8 = 0, SANA_MASK_I16 = 1, SANA_MASK_I32 = 2, SANA_MASK_I64 = 3, SANA_MASK_F32 = 4, SANA_MASK_F16 = 5,
+       SANA_MASK_BF16 = 6 };
+int sana_hip_key_bias(const void* mask, float* bias, int64_t n, int mask_type, void* stream);
+
+
 /* Gated residual update as one elementwise pass:
  *   out[m][:] = residual[m][:] + gate[m / rows_per_gate][:] * y[m][:]
  * with the product and the sum each rounded to bf16, as the reference's two ops do.  Replaces

@@ -45,6 +45,7 @@ SIGNATURES = {
                                  c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_float, c_int, c_void_p]),
     "sana_hip_state_cache": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     "sana_hip_transpose16": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p]),
+    "sana_hip_key_bias": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p]),
     "sana_hip_qk_rms": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int64, c_int64,
                                 c_float, c_int, c_void_p]),
     "sana_hip_linattn_state_pre": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_size_t,

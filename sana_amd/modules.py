@@ -968,7 +968,7 @@ class MultiHeadCrossAttention(nn.Module):
 
     @staticmethod
     def _key_bias(mask):
-        return ((1.0 - mask.to(torch.float32)) * -10000.0).contiguous()   # sana_blocks.py:89-90
+        return ops.key_bias(mask)
 
     # rows from which proj + the block's residual add run as ONE GEMM of this library (its gated-residual epilogue
     # with a gate of ones: x + (o W^T + b), the same two roundings as the stock linear and add): all.  us, library GEMM

@@ -819,6 +819,21 @@ def cross_attention16(q: torch.Tensor, kv: torch.Tensor, num_heads: int, key_bia
     return out
 
 
+# SANA_MASK_* of include/sana_hip.h
+_MASK_TYPE = {torch.bool: 0, torch.uint8: 0, torch.int16: 1, torch.int32: 2, torch.int64: 3, torch.float32: 4, torch.float16: 5,
+              torch.bfloat16: 6}
+
+
+def key_bias(mask: torch.Tensor) -> torch.Tensor:
+    """``(1 - mask.float()) * -10000``, contiguous: the additive key bias of a 0 / 1 prompt mask (sana_blocks.py:89-90)."""
+    kind = _MASK_TYPE.get(mask.dtype)
+    if kind is None or type(mask) is not torch.Tensor or not mask.is_cuda or not mask.is_contiguous() or mask.numel() == 0:
+        return ((1.0 - mask.to(torch.float32)) * -10000.0).contiguous()
+    out = torch.empty(mask.shape, dtype=torch.float32, device=mask.device)
+    _lib.check(_lib.load().sana_hip_key_bias(mask.data_ptr(), out.data_ptr(), mask.numel(), kind, _stream()), "sana_hip_key_bias")
+    return out
+
+
 def gate_residual(y: torch.Tensor, gate: torch.Tensor, residual: torch.Tensor) -> torch.Tensor:
     """residual + gate * y in one pass with the stock op pair's two roundings; y, residual: [B, N, C] bf16;
     gate: [B, 1, C], or one row per group of consecutive tokens, [B, G, 1, C]."""
