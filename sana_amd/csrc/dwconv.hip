@@ -461,11 +461,13 @@ int launch(const void* u, const void* w, const void* bias, void* y, int BT, int 
     if ((int64_t)H * W * 2 * Ch * 2 < ((int64_t)1 << 31) && Ch % 8 == 0) {
       // Bands of rows so that the launch has at least SANA_DW_LDS_MINWG workgroups (four fit a compute unit).
       // Two halo rows are re-read per band: no band shorter than 8 rows, or than 4 where even that leaves
-      // the chip short of work (single small images).
+      // the chip short of work (single small images), or than 2 while those are at most one workgroup per compute unit:
+      // both groups of such a band's rows are requested at once, so it is one memory round trip instead of two.  us, bands of
+      // 4 / of 2: 16 x 16 x 2880 7.8 / 6.4 (184 workgroups of 2), 12 x 12 x 2880 7.7 / 6.3; 12 x 12 x 5600 7.8 / 8.5 (264).
       constexpr int NW = 4;
       const int xg = (W + 4 * NW - 1) / (4 * NW);
       const int64_t base = (int64_t)slabs * xg * BT;
-      const int min_rows = base * ((H + 7) / 8) >= 512 ? 8 : 4;
+      const int min_rows = base * ((H + 7) / 8) >= 512 ? 8 : base * ((H + 1) / 2) <= 256 ? 2 : 4;
       int nb = (int)((SANA_DW_LDS_MINWG + base - 1) / base);
       nb = std::max(1, std::min(nb, (H + min_rows - 1) / min_rows));
       const int R = (H + nb - 1) / nb, bands = (H + R - 1) / R;
