@@ -1,5 +1,5 @@
 // One image block (SanaMSBlock, 16-bit weights) as one call: the launches of the entry points below, in order, on one
-// scratch buffer.  No kernels of its own.  At a few hundred tokens a block is twelve to fourteen launches of 4 - 14 us, and issuing
+// scratch buffer.  No kernels of its own.  At a few hundred tokens a block is eleven to thirteen launches of 4 - 14 us, and issuing
 // them one by one from Python took 220 us per block where the device needs about 100.
 #include <algorithm>
 
