@@ -996,7 +996,7 @@ int launch(const void* A, const void* W, const float* scale, const EpiArgs& ep, 
       return gemm8_launch(a, w + (int64_t)p.n_wide * ldw, ep2, c + p.n_wide, M, N - p.n_wide, K, lda, ldw, ldc, epilogue,
                           is_f16<T>, 3, nullptr, s);
     }
-    if (p.tile->bn == 288 && ldw < kMaxStride288)
+    if (p.tile->bn == 288 && ldw < kMaxStride288 && aligned16(ep.bias))  // (its bias row is loaded straight to LDS, 16 bytes a lane)
       return gemm288_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, nullptr, s);
     if (p.tile->bn == 288) return gemm8_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, 4, nullptr, s);
     if (p.tile->bm == 256)

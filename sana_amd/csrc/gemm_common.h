@@ -49,7 +49,8 @@ struct Taps {
 int gemm8_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
                  int64_t ldw, int64_t ldc, int epilogue, bool f16, int nb, const Taps* taps, hipStream_t s);
 
-// The same in tiles of 256 tokens x 288 channels (gemm288.hip); no SANA_EPI_QKV_STATE; rows of W less than 2^21 values apart.
+// The same in tiles of 256 tokens x 288 channels (gemm288.hip); no SANA_EPI_QKV_STATE; rows of W less than 2^21 values apart,
+// bias 16-byte aligned (or null).
 int gemm288_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
                    int64_t ldw, int64_t ldc, int epilogue, bool f16, const Taps* taps, hipStream_t s);
 

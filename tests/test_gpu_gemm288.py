@@ -55,6 +55,32 @@ def test_288_wide_gated_residual_across_batch_boundaries(cuda, B, Ntok, C, K, dt
     assert torch.equal(ops.gemm_gate_residual(a, w, None, gate, res), res + gate * y)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("off", [1, 2, 4, 7])
+def test_bias_at_any_alignment(cuda, off, dtype):
+    """A bias that is a slice at an odd place gives what its aligned copy does (other tiles, the same sums)."""
+    M, N, K = 8471, 4256, 200
+    _runs_in_288(M, N, K)
+    a, w, stored = (_ints(M, K, seed=1, dtype=dtype).to(cuda), _ints(N, K, seed=2, dtype=dtype).to(cuda),
+                    _ints(N + 8, lo=-9, hi=9, seed=3, dtype=dtype).to(cuda))
+    bias = stored[off:off + N]
+    y = (a.float() @ w.float().T + bias.float()).to(dtype)
+    assert torch.equal(ops.gemm_bf16(a, w, bias, "bias"), y)
+    gate, res = _ints(1, 1, N, seed=4, dtype=dtype).to(cuda), _ints(1, M, N, hi=99, lo=-99, seed=5, dtype=dtype).to(cuda)
+    assert torch.equal(ops.gemm_gate_residual(a[None], w, bias, gate, res), res + gate * y)
+
+
+@pytest.mark.parametrize("ldw", [(1 << 21) - 8, 1 << 21])
+def test_weight_rows_around_the_limit_of_its_offsets(cuda, ldw):
+    M, N, K = 14040, 2592, 248
+    _runs_in_288(M, N, K)
+    w = torch.empty((N - 1) * ldw + K, dtype=torch.bfloat16, device=cuda).as_strided((N, K), (ldw, 1))
+    dense = _ints(N, K, seed=2).to(cuda)
+    w.copy_(dense)
+    a = _ints(M, K, seed=1).to(cuda)
+    assert torch.equal(ops.gemm_bf16(a, w), (a.float() @ dense.float().T).bfloat16())
+
+
 @pytest.mark.parametrize("T,P,C,ends", [(5, 1560, 2240, [1, 3]), (6, 2700, 1152, [])])
 def test_288_wide_temporal_convolution_equals_one_launch_per_chunk(cuda, T, P, C, ends):
     """The whole clip in 288-wide tiles, its chunks (or its frames' first rows) in narrower ones: the same products in the
