@@ -16,7 +16,7 @@
 //            into three bf16 terms (hi + mid + lo = all 24 mantissa bits) and
 //            applied with MFMA 16x16x32; rows 32..47 of the A operand all carry
 //            ksum so every lane gets its token's denominator in-lane.
-// fp32 io (and f16 phase 2) uses MFMA 32x32x2 f32 directly from global memory.
+// fp32 io uses MFMA 32x32x2 f32 directly from global memory.
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -603,8 +603,9 @@ __global__ __launch_bounds__(256) void linattn_apply32_kernel(
 // Three launches (phase 1, reduction, phase 2) are 3 - 6 us of work each with a gap in front; here everything a head needs
 // for 1024 tokens is requested at once and the rest is one memory round trip, the transposes and the matrix products of one
 // compute unit.  That is also the bound: a head's tokens are one compute unit's work.  us, two calls / this, replayed from a
-// graph: bf16, 36 heads x 256 tokens 10.1 / 5.4, 36 x 1024 12.5 / 8.5, 140 x 1024 19.1 / 15.2; fp16 36 x 256 10.8 / 6.0; fp32
-// 36 x 256 10.8 / 8.5, 140 x 512 21.4 / 17.1.
+// graph on one set of inputs (on 32 in turn): bf16, 36 heads x 256 tokens 10.5 / 5.6 (10.9 / 6.1), 36 x 1024 12.9 / 9.3 (13.7 /
+// 12.0), 140 x 1024 19.4 / 15.5 (21.6 / 16.6); fp16 36 x 256 11.2 / 6.2 (11.6 / 6.7); fp32 210 x 1024 34.2 / 26.6 (40.5 / 34.8).
+// (Adding the state up in the two calls' order costs 0.4 us at 1024 tokens: sixteen partial states in LDS, not eight.)
 // ----------------------------------------------------------------------------
 constexpr int WHOLE_TOKENS = 1024;  // the most that one round of loads covers
 template <int OFF>
@@ -614,99 +615,119 @@ __device__ __forceinline__ u32x2_t lds_read_tr16(uint32_t addr) {  // 4 tokens x
   return v;
 }
 
-// 16-bit io.  grid: B * h; block 512.  Phase 1: wave w takes the 32-token tiles w, w + 8, .. through its own LDS (rows of 96
-// bytes: conflict-free transposing reads) as operands of MFMA 16x16x32, the key sum with an operand of ones; the waves'
-// sums are added in wave order.  Phase 2 as linattn_apply16_kernel, on the 16-token steps w, w + 8, ..
+// 16-bit io.  grid: B * h; block 512.  The state is formed by the sums of linattn_state16_kernel and its reduction, in their
+// order (at most 256 heads: always splits of 256 tokens), so that the result is that of the two calls bit for bit: "chain" c is
+// what wave c % 4 of split c / 4 adds up there, the 32-token tiles 256 (c / 4) + 32 (c % 4) + {0, 128}.  Wave w takes chains w and
+// w + 8 through its own LDS (rows of 96 bytes: conflict-free transposing reads).  Phase 2 as linattn_apply16_kernel, on the
+// 16-token steps w, w + 8, ..
 template <typename T>
 __global__ __launch_bounds__(512) void linattn_whole16_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V, uint16_t* __restrict__ out,
     int N, int h, int64_t q_stride_b, int64_t q_stride_n, int64_t stride_b, int64_t stride_n, int64_t o_stride_b,
     int64_t o_stride_n, float eps) {
-  constexpr int WAVES = 8, ROW = 96, U1 = WHOLE_TOKENS / (WAVES * TILE), U2 = WHOLE_TOKENS / (WAVES * 16);
-  constexpr int STATE_AT = WAVES * U2 * 1024;
-  static_assert(STATE_AT >= WAVES * 2 * TILE * ROW && STATE_AT >= WAVES * STATE_ELEMS * 4, "the state lies behind the stages");
+  constexpr int WAVES = 8, ROW = 96, SPLIT = 256, CHAINS = 4 * WHOLE_TOKENS / SPLIT, U1 = CHAINS / WAVES,
+                U2 = WHOLE_TOKENS / (WAVES * 16);
+  constexpr int STATE_AT = CHAINS * STATE_ELEMS * 4;
+  static_assert(STATE_AT >= WAVES * 2 * TILE * ROW && STATE_AT >= WAVES * U2 * 1024, "the state lies behind the stages");
   __shared__ __attribute__((aligned(16))) unsigned char smem[STATE_AT + STATE_ELEMS * 4];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int b = blockIdx.x / h, head = blockIdx.x - b * h;
   const int ld_tok = lane >> 2, ld_chunk = lane & 3;  // a load instruction: 16 tokens x 64 bytes
-  const int n = lane & 15, g = lane >> 4;             // MFMA layout
   const u32x4_t zero4 = {0u, 0u, 0u, 0u};
   const uint16_t* kbase = K + (int64_t)b * stride_b + head * D + 8 * ld_chunk;
   const uint16_t* vbase = V + (int64_t)b * stride_b + head * D + 8 * ld_chunk;
   const uint16_t* qbase = Q + (int64_t)b * q_stride_b + head * D + 8 * ld_chunk;
 
   // ---- phase 1
-  u32x4_t kreg[U1][2], vreg[U1][2], raw[U2];
+  auto tile_of = [&](int u, int t) {
+    const int c = wave + WAVES * u;
+    return SPLIT * (c >> 2) + TILE * (c & 3) + 128 * t;
+  };
+  u32x4_t kreg[U1][2][2], vreg[U1][2][2], raw[U2];
 #pragma unroll
   for (int u = 0; u < U1; ++u)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int tok = (wave + u * WAVES) * TILE + 16 * i + ld_tok;
-      kreg[u][i] = tok < N ? *reinterpret_cast<const u32x4_t*>(kbase + (int64_t)tok * stride_n) : zero4;
-      vreg[u][i] = tok < N ? *reinterpret_cast<const u32x4_t*>(vbase + (int64_t)tok * stride_n) : zero4;
-    }
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int tok = tile_of(u, t) + 16 * i + ld_tok;
+        kreg[u][t][i] = tok < N ? *reinterpret_cast<const u32x4_t*>(kbase + (int64_t)tok * stride_n) : zero4;
+        vreg[u][t][i] = tok < N ? *reinterpret_cast<const u32x4_t*>(vbase + (int64_t)tok * stride_n) : zero4;
+      }
 #pragma unroll
   for (int u = 0; u < U2; ++u) {
     const int tok = (wave + u * WAVES) * 16 + ld_tok;
     raw[u] = tok < N ? *reinterpret_cast<const u32x4_t*>(qbase + (int64_t)tok * q_stride_n) : zero4;
   }
+  // MFMA 32x32x16: lane -> channel lane % 32, element r of k-step s is token 16 s + 2 r + lane / 32 of the tile.  A transposing
+  // read hands the 16 lanes of a group four rows, row i addressed by lanes 4 i .. 4 i + 3: two tokens apart here.
   unsigned char* stage = smem + wave * (2 * TILE * ROW);
   const uint32_t stage_addr = (uint32_t)(size_t)(__attribute__((address_space(3))) const unsigned char*)stage;
-  const uint32_t k_at = stage_addr + (4 * g + (n >> 2)) * ROW + (n & 3) * 8, v_at = k_at + TILE * ROW;
-  const uint32_t one2 = is_f16<T> ? 0x3c003c00u : 0x3f803f80u;
-  const u32x4_t ones = {one2, one2, one2, one2};
-  f32x4_t S[2][2], ks[2];  // S[i][j]: dv 16 i + 4 g + r, dk 16 j + n;  ks[j]: dk 16 j + n, every row
-#pragma unroll
-  for (int j = 0; j < 2; ++j) S[0][j] = S[1][j] = ks[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const uint32_t k_at = stage_addr + (2 * ((lane >> 2) & 3) + (lane >> 5)) * ROW + ((lane >> 4) & 1) * 32 + (lane & 3) * 8,
+                 v_at = k_at + TILE * ROW;
+  f32x16_t S[U1];
+  float ks[U1];
 #pragma unroll
   for (int u = 0; u < U1; ++u) {
-    if ((wave + u * WAVES) * TILE >= N) break;  // uniform
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      *reinterpret_cast<u32x4_t*>(stage + (16 * i + ld_tok) * ROW + 16 * ld_chunk) = relu_pk16(kreg[u][i]);
-      *reinterpret_cast<u32x4_t*>(stage + TILE * ROW + (16 * i + ld_tok) * ROW + 16 * ld_chunk) = vreg[u][i];
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // wave-private LDS: in-order, no barrier needed
-    u32x2_t kf[2][2], vf[2][2];  // [channels 16 j ..][tokens 16 i ..]
-    kf[0][0] = lds_read_tr16<0>(k_at), kf[0][1] = lds_read_tr16<16 * ROW>(k_at);
-    kf[1][0] = lds_read_tr16<32>(k_at), kf[1][1] = lds_read_tr16<32 + 16 * ROW>(k_at);
-    vf[0][0] = lds_read_tr16<0>(v_at), vf[0][1] = lds_read_tr16<16 * ROW>(v_at);
-    vf[1][0] = lds_read_tr16<32>(v_at), vf[1][1] = lds_read_tr16<32 + 16 * ROW>(v_at);
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(kf[0][0]), "+v"(kf[0][1]), "+v"(kf[1][0]), "+v"(kf[1][1]), "+v"(vf[0][0]), "+v"(vf[0][1]),
-                   "+v"(vf[1][0]), "+v"(vf[1][1])::"memory");
+    for (int i = 0; i < 16; ++i) S[u][i] = 0.f;
+    ks[u] = 0.f;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const u32x4_t kk = {kf[j][0].x, kf[j][0].y, kf[j][1].x, kf[j][1].y};
+    for (int t = 0; t < 2; ++t) {
+      if (tile_of(u, t) >= N) break;  // uniform
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
-        S[i][j] = mfma_16x16x32<T>(u32x4_t{vf[i][0].x, vf[i][0].y, vf[i][1].x, vf[i][1].y}, kk, S[i][j]);
-      ks[j] = mfma_16x16x32<T>(ones, kk, ks[j]);
+      for (int i = 0; i < 2; ++i) {
+        *reinterpret_cast<u32x4_t*>(stage + (16 * i + ld_tok) * ROW + 16 * ld_chunk) = relu_pk16(kreg[u][t][i]);
+        *reinterpret_cast<u32x4_t*>(stage + TILE * ROW + (16 * i + ld_tok) * ROW + 16 * ld_chunk) = vreg[u][t][i];
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // wave-private LDS: in-order, no barrier needed
+      u32x2_t kf[2][2], vf[2][2];  // [k-step][elements 4 i ..]
+      kf[0][0] = lds_read_tr16<0>(k_at), kf[0][1] = lds_read_tr16<8 * ROW>(k_at);
+      kf[1][0] = lds_read_tr16<16 * ROW>(k_at), kf[1][1] = lds_read_tr16<24 * ROW>(k_at);
+      vf[0][0] = lds_read_tr16<0>(v_at), vf[0][1] = lds_read_tr16<8 * ROW>(v_at);
+      vf[1][0] = lds_read_tr16<16 * ROW>(v_at), vf[1][1] = lds_read_tr16<24 * ROW>(v_at);
+      asm volatile("s_waitcnt lgkmcnt(0)"
+                   : "+v"(kf[0][0]), "+v"(kf[0][1]), "+v"(kf[1][0]), "+v"(kf[1][1]), "+v"(vf[0][0]), "+v"(vf[0][1]),
+                     "+v"(vf[1][0]), "+v"(vf[1][1])::"memory");
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const u32x4_t kk = {kf[s][0].x, kf[s][0].y, kf[s][1].x, kf[s][1].y};
+        S[u] = mfma_32x32x16<T>(u32x4_t{vf[s][0].x, vf[s][0].y, vf[s][1].x, vf[s][1].y}, kk, S[u]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ks[u] = add_pk16<T>(kk[e], ks[u]);
+      }
     }
   }
   __syncthreads();
-  float* red = reinterpret_cast<float*>(smem) + wave * STATE_ELEMS;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int u = 0; u < U1; ++u) {
+    const int c = wave + WAVES * u;
+    if (SPLIT * (c >> 2) >= N) break;  // uniform: no such split
+    float* red = reinterpret_cast<float*>(smem) + c * STATE_ELEMS;
+    const int j = lane & 31, g2 = lane >> 5;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) red[(16 * i + 4 * g + r) * D + 16 * j + n] = S[i][j][r];
-    if (g == 0) red[D * D + 16 * j + n] = ks[j][0];
+    for (int r = 0; r < 16; ++r) red[(8 * (r >> 2) + 4 * g2 + (r & 3)) * D + j] = S[u][r];
+    const float both = ks[u] + __shfl_xor(ks[u], 32, 64);
+    if (g2 == 0) red[D * D + j] = both;
   }
   __syncthreads();
   float* state = reinterpret_cast<float*>(smem + STATE_AT);
-  for (int e = tid; e < STATE_ELEMS; e += 64 * WAVES) {
-    const float* p = reinterpret_cast<const float*>(smem) + e;
-    float s = p[0];
+  if (tid < STATE_ELEMS / 4) {  // the waves of a split, then the splits
+    const f32x4_t* p = reinterpret_cast<const f32x4_t*>(smem) + tid;
+    constexpr int STEP = STATE_ELEMS / 4;
+    f32x4_t s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 1; w < WAVES; ++w) s += p[w * STATE_ELEMS];
-    state[e] = s;
+    for (int sp = 0; sp < CHAINS / 4; ++sp) {
+      if (SPLIT * sp >= N) break;  // uniform
+      s += ((p[(4 * sp) * STEP] + p[(4 * sp + 1) * STEP]) + p[(4 * sp + 2) * STEP]) + p[(4 * sp + 3) * STEP];
+    }
+    reinterpret_cast<f32x4_t*>(state)[tid] = s;
   }
   __syncthreads();
 
   // ---- phase 2 (operand layout: linattn_apply16_kernel)
+  const int n = lane & 15, g = lane >> 4;
   u32x4_t st[3][3];
 #pragma unroll
   for (int rb = 0; rb < 3; ++rb) {
@@ -766,12 +787,13 @@ __global__ __launch_bounds__(512) void linattn_whole16_kernel(
   }
 }
 
-// fp32 io.  grid: B * h; block 1024.  Phase 1 as linattn_state32_kernel with the waves as its splits of 64 tokens (same sums
-// up to 1024 tokens), phase 2 as linattn_apply32_kernel on the 32-token tiles w, w + 16, ..
+// fp32 io.  grid: B * h; block 1024.  Phase 1 as linattn_state32_kernel with the waves as its splits (split_tokens as planned for
+// it, at most 16 splits) and their sums added in its order: the two calls' result bit for bit.  Phase 2 as
+// linattn_apply32_kernel on the 32-token tiles w, w + 16, ..
 __global__ __launch_bounds__(1024) void linattn_whole32_kernel(
     const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V, float* __restrict__ out, int N, int h,
-    int64_t q_stride_b, int64_t q_stride_n, int64_t stride_b, int64_t stride_n, int64_t o_stride_b, int64_t o_stride_n,
-    float eps) {
+    int split_tokens, int64_t q_stride_b, int64_t q_stride_n, int64_t stride_b, int64_t stride_n, int64_t o_stride_b,
+    int64_t o_stride_n, float eps) {
   constexpr int WAVES = WHOLE_TOKENS / 64, U = 16;
   __shared__ __attribute__((aligned(16))) float smem[(WAVES + 1) * STATE_ELEMS];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -783,17 +805,18 @@ __global__ __launch_bounds__(1024) void linattn_whole32_kernel(
   float accK = 0.f;
 #pragma unroll
   for (int i = 0; i < 16; ++i) accS[i] = 0.f;
+  const int t1 = min((wave + 1) * split_tokens, N);
 #pragma unroll 1
-  for (int t = wave * 64; t < min(wave * 64 + 64, N); t += 2 * U) {  // (both halves at once need more registers than there are)
+  for (int t = wave * split_tokens; t < t1; t += 2 * U) {  // (64 tokens at once need more registers than there are)
     float kk[U], vv[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t at = (int64_t)min(t + 2 * u + g, N - 1) * stride_n;  // (no branch around a load)
+      const int64_t at = (int64_t)min(t + 2 * u + g, t1 - 1) * stride_n;  // (no branch around a load)
       kk[u] = kp[at], vv[u] = vp[at];
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const bool ok = t + 2 * u + g < N;
+      const bool ok = t + 2 * u + g < t1;
       kk[u] = ok ? fmaxf(kk[u], 0.f) : 0.f;
       vv[u] = ok ? vv[u] : 0.f;
     }
@@ -1253,13 +1276,14 @@ extern "C" __attribute__((visibility("default"))) int sana_hip_linattn(
   }
   const dim3 grid((unsigned)(B * h));
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define SANA_WHOLE(kernel, threads, E)                                                                                 \
+#define SANA_WHOLE(kernel, threads, E, ...)                                                                            \
   hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, static_cast<const E*>(q), static_cast<const E*>(k),           \
-                     static_cast<const E*>(v), static_cast<E*>(out), N, h, q_stride_b, q_stride_n, stride_b, stride_n, \
+                     static_cast<const E*>(v), static_cast<E*>(out), N, h, __VA_ARGS__, q_stride_n, stride_b, stride_n, \
                      o_stride_b, o_stride_n, eps)
-  if (io_dtype == SANA_DT_F32) SANA_WHOLE(linattn_whole32_kernel, WHOLE_TOKENS, float);
-  else if (io_dtype == SANA_DT_F16) SANA_WHOLE(linattn_whole16_kernel<F16>, 512, uint16_t);
-  else SANA_WHOLE(linattn_whole16_kernel<BF16>, 512, uint16_t);
+  if (io_dtype == SANA_DT_F32)
+    SANA_WHOLE(linattn_whole32_kernel, WHOLE_TOKENS, float, plan_state(B, h, 1, N, io_dtype).split_tokens, q_stride_b);
+  else if (io_dtype == SANA_DT_F16) SANA_WHOLE(linattn_whole16_kernel<F16>, 512, uint16_t, q_stride_b);
+  else SANA_WHOLE(linattn_whole16_kernel<BF16>, 512, uint16_t, q_stride_b);
 #undef SANA_WHOLE
   return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
 }

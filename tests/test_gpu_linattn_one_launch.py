@@ -1,6 +1,6 @@
 """Both phases of the linear attention in one kernel (short sequences): against the fp64 oracle, at the edges of its tiles
-(16-token steps, 32-token tiles, 64-token ranges, 256 heads, 1024 tokens) and just beyond them, and no further from it
-than the two calls."""
+(16-token steps, 32-token tiles, the two calls' splits of 48 to 256 tokens, 256 heads, 1024 tokens) and just beyond them, and
+bit for bit what the two calls give."""
 import pytest
 import torch
 
@@ -17,7 +17,8 @@ def _rel(a, b):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,N,C", [(1, 1, 64), (2, 15, 32), (1, 17, 96), (3, 33, 160), (1, 255, 1152), (1, 256, 1152),
                                    (2, 513, 64), (1, 972, 2240), (2, 1024, 1152), (3, 1023, 2240),
-                                   (1, 1025, 96), (8, 100, 1056)])
+                                   (1, 1025, 96), (8, 100, 1056), (1, 65, 1152), (1, 128, 64), (2, 129, 1152), (1, 144, 2240),
+                                   (1, 385, 2240), (1, 769, 1152), (256, 1024, 32), (85, 700, 96)])
 def test_matches_the_oracle_and_the_two_calls(cuda, B, N, C, dtype):
     eps = 1e-8
     gen = torch.Generator().manual_seed(N + C)
@@ -33,16 +34,14 @@ def test_matches_the_oracle_and_the_two_calls(cuda, B, N, C, dtype):
     # fp32: a sum of N products, rounded at 6e-8 each in random directions; 16 bits: one rounding of the result (2^-9, 2^-12)
     bound = {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dtype]
     assert _rel(got, ref) <= bound
-    assert _rel(got, ref) <= 1.05 * _rel(two, ref) + 1e-8
+    assert torch.equal(got, two)
     one = _lib.load().sana_hip_linattn_scratch_bytes(B, N, C // 32, 32, ops._dt(q)) == 0
     assert one == (N <= 1024 and B * C // 32 <= 256 and (dtype != torch.float32 or N <= max(256, 7 * B * C // 32)))
-    if not one:
-        assert torch.equal(got, two)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_zeros_and_infinities_as_the_two_calls(cuda, dtype):
-    """Tokens without a positive key or query (0 / eps), a head of zeros, and an infinity in one head: the same classes."""
+    """Tokens without a positive key or query (0 / eps), a head of zeros, and an infinity in one head."""
     gen = torch.Generator().manual_seed(3)
     qkv = torch.randn(2, 70, 3, 128, generator=gen)
     qkv[0, :, 1, :32] = -1.0
@@ -50,9 +49,7 @@ def test_zeros_and_infinities_as_the_two_calls(cuda, dtype):
     qkv[1, 9, 1, 40], qkv[1, 11, 2, 70] = float("inf"), float("-inf")
     q, k, v = (qkv.to(dtype).to(cuda)[:, :, i] for i in range(3))
     got, two = ops.relu_linear_attention(q, k, v, 1e-8), ops.linattn_apply(q, ops.linattn_state(k, v), 1e-8)
-    assert torch.equal(torch.isnan(got), torch.isnan(two)) and torch.equal(torch.isinf(got), torch.isinf(two))
-    ok = torch.isfinite(two)
-    assert torch.allclose(got[ok].float(), two[ok].float(), rtol=2.0 ** -7, atol=1e-6)
+    assert torch.isnan(two).any() and torch.allclose(got, two, rtol=0, atol=0, equal_nan=True)
 
 
 def test_what_it_does_not_take_goes_to_the_two_calls(cuda):
