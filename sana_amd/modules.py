@@ -345,11 +345,7 @@ class LiteLA(nn.Module):
             out = ops.linattn_apply(q, state, self.eps)
         elif rotary_emb is None and x.dtype == torch.bfloat16:   # qk-norm (if any) on load inside the kernels
             B, N, C = x.shape
-            qkv = self.qkv(x).view(B, N, 3, C)
-            if isinstance(self.q_norm, nn.Identity):
-                out = ops.relu_linear_attention(qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], self.eps, head_dim=self.dim)
-            else:
-                out = self._attend(qkv, None)
+            out = self._attend(self.qkv(x).view(B, N, 3, C), None)
         elif x.dtype == torch.bfloat16 and x.is_cuda and self.dim == 32 and \
                 (table := _rope_real_table_cached(rotary_emb, x.shape[1], x.device, self.dim)) is not None:
             # LiteLA.forward's own order (sana_blocks.py:274-286): norm, rotation BEFORE the ReLU, everything rotated --
@@ -426,6 +422,8 @@ class LiteLA(nn.Module):
 
     def _attend(self, qkv, rotary_emb, chunk_tokens=None):
         pre_q, pre_k = self._pre(qkv, rotary_emb)
+        if pre_k is None:
+            return ops.relu_linear_attention(qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], self.eps, chunk_tokens, head_dim=self.dim)
         causal = chunk_tokens is not None and len(chunk_tokens) > 1
         state = ops.linattn_state(qkv[:, :, 1], qkv[:, :, 2], chunk_tokens, causal=causal, pre=pre_k,
                                   head_dim=self.dim)

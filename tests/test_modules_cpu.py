@@ -228,3 +228,26 @@ def test_graphed_call_needs_a_warm_up():
         GraphedCall(lambda x: x, [torch.zeros(1)], warmup=1)      # CPU tensors
     src = inspect.getsource(GraphedCall.__init__)
     assert "warmup < 1" in src
+
+
+def test_an_attention_put_over_the_module_s_own_is_called():
+    """``_attend`` set on the instance or overridden in a subclass stands for the attention of the plain path too."""
+    seen = []
+
+    def values_only(qkv, rotary_emb, chunk_tokens=None):
+        seen.append(tuple(qkv.shape))
+        return qkv[:, :, 2]
+
+    class Sub(S.LiteLA):
+        def _attend(self, qkv, rotary_emb, chunk_tokens=None):
+            return values_only(qkv, rotary_emb, chunk_tokens)
+
+    x = torch.randn(2, 5, 64).bfloat16()
+    for attn in (S.LiteLA(64, 64, heads=2), Sub(64, 64, heads=2)):
+        attn.qkv, attn.proj = torch.nn.Linear(64, 192), torch.nn.Linear(64, 64)   # (the library's linears need a GPU)
+        attn.bfloat16()
+        if type(attn) is S.LiteLA:
+            attn._attend = values_only
+        with torch.no_grad():
+            assert torch.equal(attn(x), attn.proj(attn.qkv(x)[..., 128:]))
+    assert seen == [(2, 5, 3, 64)] * 2
