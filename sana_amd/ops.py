@@ -326,6 +326,9 @@ def copy_tokens_(dst: torch.Tensor, src: torch.Tensor) -> torch.Tensor:
     return dst.copy_(src)
 
 
+STATE_SCRATCH_KEPT = 64 << 20   # bytes of attention state and partial states that may stay in the stream's scratch buffer
+
+
 def _one_call(q, k, v, d: int) -> bool:
     """Whether ``sana_hip_linattn`` takes these.  What it does not (mixed dtypes or shapes, k and v of different
     strides, other head dims) goes to the two calls, which serve or refuse it."""
@@ -342,14 +345,20 @@ def relu_linear_attention(q, k, v, eps: float, chunk_tokens=None, out_dtype=None
     causal = chunk_tokens is not None and len(chunk_tokens) > 1
     if not causal and out_dtype in (None, q.dtype) and _one_call(q, k, v, head_dim):
         B, N, C = q.shape
-        h, dt, lib = C // head_dim, _dt(q), _lib.load()
+        h, dt, lib, stream = C // head_dim, _dt(q), _lib.load(), _stream()
         qs, ks = _token_major_view(q, "q"), _token_major_view(k, "k")
         out = torch.empty(B, N, C, dtype=q.dtype, device=q.device)
         nbytes = lib.sana_hip_linattn_scratch_bytes(B, N, h, head_dim, dt)
-        ws = _workspace(q.device, nbytes)
+        # The state is in there as well: of this call's own under capture (graphs that a caller captures on one stream and
+        # replays side by side must not share it) and where it is too large to be kept.  us, fp32 1024 tokens x 36 heads, own
+        # always / the stream's where it may be: 17.8 / 17.2.
+        if nbytes and (nbytes > STATE_SCRATCH_KEPT or torch._C._cuda_isCurrentStreamCapturing()):
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+        else:
+            ws = _workspace(q.device, nbytes, stream)
         code = lib.sana_hip_linattn(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                                     ws.data_ptr() if ws is not None else None, nbytes, B, N, h, head_dim, *qs, *ks,
-                                    N * C if B > 1 else 0, C, float(eps), dt, _stream())
+                                    N * C if B > 1 else 0, C, float(eps), dt, stream)
         _lib.check(code, "sana_hip_linattn")
         return out
     state = linattn_state(k, v, chunk_tokens, causal=causal, head_dim=head_dim)

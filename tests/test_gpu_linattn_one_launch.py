@@ -62,3 +62,49 @@ def test_what_it_does_not_take_goes_to_the_two_calls(cuda):
         ops.relu_linear_attention(q, k.contiguous(), v, 1e-8)
     out32 = ops.relu_linear_attention(q.bfloat16(), k.bfloat16(), v.bfloat16(), 1e-8, out_dtype=torch.float32)
     assert out32.dtype == torch.float32
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_graphs_captured_on_one_stream_keep_a_state_each(cuda, monkeypatch, dtype):
+    """Beyond one launch the state is in memory: nothing of it in the stream's scratch buffer, which graphs of one capture
+    stream would share, and two such graphs replayed on two streams give the eager results."""
+    stream, graphs, wants = torch.cuda.Stream(), [], []
+    monkeypatch.setattr(ops, "_workspaces", {})      # (stream handles come from a pool: not those of other tests)
+    for seed in (1, 2):
+        gen = torch.Generator().manual_seed(seed)
+        q, k, v = (t.to(cuda) for t in torch.randn(3, 2, 1500, 1152, generator=gen).to(dtype))
+        wants.append(ops.relu_linear_attention(q, k, v, 1e-8))
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            out = ops.relu_linear_attention(q, k, v, 1e-8)
+        graphs.append((graph, out, (q, k, v)))
+    assert (q.device.index, stream.cuda_stream) not in ops._workspaces
+    sides = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for _ in range(5):
+        for _, out, _ in graphs:
+            out.zero_()
+        torch.cuda.synchronize()
+        for side, (graph, _, _) in zip(sides, graphs):
+            with torch.cuda.stream(side):
+                graph.replay()
+        torch.cuda.synchronize()
+        for (_, out, _), want in zip(graphs, wants):
+            assert torch.equal(out, want)
+
+
+def test_a_large_state_is_not_kept(cuda, monkeypatch):
+    gen = torch.Generator().manual_seed(1)
+    q, k, v = (t.to(cuda) for t in torch.randn(3, 1, 1100, 64, generator=gen))
+    want = ops.linattn_apply(q, ops.linattn_state(k, v), 1e-8)
+    need = _lib.load().sana_hip_linattn_scratch_bytes(1, 1100, 2, 32, ops._dt(q))
+    torch.cuda.synchronize()
+    for kept in (need - 1, need):
+        monkeypatch.setattr(ops, "STATE_SCRATCH_KEPT", kept)
+        stream = torch.cuda.Stream()
+        monkeypatch.setattr(ops, "_workspaces", {})
+        with torch.cuda.stream(stream):
+            got = ops.relu_linear_attention(q, k, v, 1e-8)
+        stream.synchronize()
+        assert torch.equal(got, want)
+        assert ((q.device.index, stream.cuda_stream) in ops._workspaces) == (kept == need)
