@@ -16,10 +16,14 @@ def _ints(*shape, lo=-3, hi=3, seed=0, dtype=torch.bfloat16):
     return torch.randint(lo, hi + 1, shape, generator=g).to(dtype)
 
 
-def _runs_in_288(M, N, K):
+def _plan(M, N, K):
     plan = (ctypes.c_int * 4)()
     _lib.check(_lib.load().sana_hip_gemm_plan(M, N, K, plan), "sana_hip_gemm_plan")
-    assert tuple(plan) == (256, 288, 0, 1), tuple(plan)
+    return tuple(plan)
+
+
+def _runs_in_288(M, N, K):
+    assert _plan(M, N, K) == (256, 288, 0, 1)
 
 
 # k tails of 8, 56 and 0 in an odd and an even number of k-tiles; ragged rows; ragged channels in the first and the second
@@ -42,7 +46,9 @@ def test_288_wide_tile_is_exact_on_integers(cuda, M, N, K, dtype):
     assert ((y.double() - want).abs() <= ulp * want.abs() + 1e-7).all()
 
 
-@pytest.mark.parametrize("B,Ntok,C,K", [(3, 1096, 5016, 248), (7, 202, 11016, 200), (5, 1052, 3400, 256), (1, 8471, 4256, 200)])
+# the last two have more tiles than workgroups, with one batch entry and with boundaries inside tiles
+@pytest.mark.parametrize("B,Ntok,C,K", [(3, 1096, 5016, 248), (7, 202, 11016, 200), (5, 1052, 3400, 256), (1, 8471, 4256, 200),
+                                        (3, 2824, 4256, 200)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_288_wide_gated_residual_across_batch_boundaries(cuda, B, Ntok, C, K, dtype):
     _runs_in_288(B * Ntok, C, K)
@@ -81,18 +87,18 @@ def test_weight_rows_around_the_limit_of_its_offsets(cuda, ldw):
     assert torch.equal(ops.gemm_bf16(a, w), (a.float() @ dense.float().T).bfloat16())
 
 
-@pytest.mark.parametrize("T,P,C,ends", [(5, 1560, 2240, [1, 3]), (6, 2700, 1152, [])])
-def test_288_wide_temporal_convolution_equals_one_launch_per_chunk(cuda, T, P, C, ends):
-    """The whole clip in 288-wide tiles, its chunks (or its frames' first rows) in narrower ones: the same products in the
-    same order, so the same bits."""
+# 248 and 256 tiles, one a workgroup; 1024, 1024 and 512: workgroups with several, frames (and flagged ones) inside a tile
+@pytest.mark.parametrize("T,P,C,ends", [(5, 1560, 2240, [1, 3]), (6, 2700, 1152, []), (21, 1560, 2240, [4, 9, 17]),
+                                        (21, 1560, 2240, []), (21, 1560, 1152, [0, 6])])
+def test_288_wide_temporal_convolution_equals_one_launch_per_frame(cuda, T, P, C, ends):
+    """The whole clip in 288-wide tiles, each frame by itself in narrower ones: the same products in the same order, so the
+    same bits."""
     _runs_in_288(T * P, C, 3 * C)
+    assert _plan(P, C, 3 * C)[:2] != (256, 288)
     g = torch.Generator().manual_seed(C + T)
     y = torch.randn((T + 1) * P, C, generator=g).bfloat16().to(cuda)          # a real frame in front (a cache's last one)
     w2 = (torch.randn(C, 3 * C, generator=g) * (1.0 / (3 * C)) ** 0.5).bfloat16().to(cuda)
     one = ops.tconv_residual(y, w2, T * P, P, zero_last_tap=ops.frame_flags(T, ends, cuda))
-    bounds = [0, *(e + 1 for e in ends), T]
-    if ends:
-        parts = [ops.tconv_residual(y[f0 * P:(f1 + 1) * P], w2, (f1 - f0) * P, P) for f0, f1 in zip(bounds[:-1], bounds[1:])]
-        assert torch.equal(one, torch.cat(parts))
-    else:
-        assert torch.equal(one[:4000], ops.tconv_residual(y, w2, 4000, P))
+    for f in range(T):      # rows behind the last frame, or behind a flagged one, read as zeros
+        frame = ops.tconv_residual(y[f * P:(f + (2 if f in ends else 3)) * P], w2, P, P)
+        assert torch.equal(one[f * P:(f + 1) * P], frame), f
