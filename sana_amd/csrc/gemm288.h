@@ -8,37 +8,10 @@
 namespace sana {
 namespace {
 
-// A wave-uniform value into scalar registers, whatever the compiler thinks of it.
-__device__ __forceinline__ int g288_uniform(int x) {
-  int r;
-  asm volatile("s_mov_b32 %0, %1" : "=s"(r) : "s"(x));
-  return r;
-}
-__device__ __forceinline__ const uint16_t* g288_uniform(const uint16_t* x) {
-  const uint16_t* r;
-  asm volatile("s_mov_b64 %0, %1" : "=s"(r) : "s"(x));
-  return r;
-}
-template <int OFF>
-__device__ __forceinline__ u32x4_t g288_read(uint32_t addr) {
-  u32x4_t v;
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
-  return v;
-}
 __device__ __forceinline__ u32x2_t g288_read2(uint32_t addr) {
   u32x2_t v;
   asm volatile("ds_read_b64 %0, %1" : "=v"(v) : "v"(addr));
   return v;
-}
-template <int OFF, typename V>
-__device__ __forceinline__ void g288_write(uint32_t addr, V v) {
-  if constexpr (sizeof(V) == 16) asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(addr), "v"(v), "n"(OFF) : "memory");
-  else asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(addr), "v"(v), "n"(OFF) : "memory");
-}
-template <typename T>
-__device__ __forceinline__ void g288_mfma(f32x4_t& c, u32x4_t a, u32x4_t b) {
-  if constexpr (is_f16<T>) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
-  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
 }
 
 // What bounds it: the matrix pipes' power where the rounds are full (16384 x 2240 x 5600: 314 us = 1.31 PFLOP/s with the gated
@@ -150,26 +123,15 @@ __global__ __launch_bounds__(512) void gemm288_kernel(const uint16_t* __restrict
     }
   };
 
-  // workgroup -> tile: XCD x (ids x, x + 8, ..) takes the x-th contiguous eighth of the grouped tile order
   const int total = tiles_t * tiles_c;
   auto start_tile = [&](int id) {  // resources and offsets of a tile, and the loads in front of its first phase
-    int pid;
-    {
-      const int xcd = id & 7, local = id >> 3;
-      const int base = total >> 3, rem = total & 7;
-      pid = xcd * base + min(xcd, rem) + local;
-    }
-    const int GROUP = K >= 4096 ? 8 : 4;
-    const int group_sz = GROUP * tiles_c;
-    const int gid = pid / group_sz;
-    const int first_t = gid * GROUP;
-    const int gt = min(tiles_t - first_t, GROUP);
-    m0 = g288_uniform(__builtin_amdgcn_readfirstlane(first_t + (pid % group_sz) % gt) * BM);
-    n0 = g288_uniform(__builtin_amdgcn_readfirstlane((pid % group_sz) / gt) * BN);
+    gemm_tile_of(id, tiles_t, tiles_c, K >= 4096 ? 8 : 4, BM, BN, m0, n0);
+    m0 = gemm_uniform(__builtin_amdgcn_readfirstlane(m0));
+    n0 = gemm_uniform(__builtin_amdgcn_readfirstlane(n0));
     const int a_last = min(BM, M - m0) - 1, w_last = min(BN, N - n0) - 1;
     const int64_t a_bytes = TAPS ? (tp.rows > m0 ? ((tp.rows - m0 - 1) * lda + tp.kc) * 2 : 0) : ((int64_t)a_last * lda + K) * 2;
-    base_a = g288_uniform(A + (int64_t)m0 * lda), bytes_a = g288_uniform((int)a_bytes);
-    base_w = g288_uniform(W + (int64_t)n0 * ldw), bytes_w = g288_uniform((int)(((int64_t)w_last * ldw + K) * 2));
+    base_a = gemm_uniform(A + (int64_t)m0 * lda), bytes_a = gemm_uniform((int)a_bytes);
+    base_w = gemm_uniform(W + (int64_t)n0 * ldw), bytes_w = gemm_uniform((int)(((int64_t)w_last * ldw + K) * 2));
     const int lane = lane_id(), lr = lane >> 3;
     // bias and gate row of the tile's first token: older than every load that is waited for by number
     row_sel ^= 1024;
@@ -236,11 +198,11 @@ __global__ __launch_bounds__(512) void gemm288_kernel(const uint16_t* __restrict
     constexpr int O = decltype(off_c)::value, n = decltype(n_c)::value;
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      f[ks][0] = g288_read<O>(r[ks]);
-      f[ks][1] = g288_read<O + 2048>(r[ks]);
-      f[ks][2] = g288_read<O + 4096>(r[ks]);
-      f[ks][3] = g288_read<O + 6144>(r[ks]);
-      if constexpr (n > 4) f[ks][4] = g288_read<O + 8192>(r[ks]);
+      f[ks][0] = gemm_lds_read<O>(r[ks]);
+      f[ks][1] = gemm_lds_read<O + 2048>(r[ks]);
+      f[ks][2] = gemm_lds_read<O + 4096>(r[ks]);
+      f[ks][3] = gemm_lds_read<O + 6144>(r[ks]);
+      if constexpr (n > 4) f[ks][4] = gemm_lds_read<O + 8192>(r[ks]);
     }
   };
   auto wait_n = [&](auto& f, int n) {
@@ -258,7 +220,7 @@ __global__ __launch_bounds__(512) void gemm288_kernel(const uint16_t* __restrict
 #pragma unroll
         for (int jj = 0; jj < TM; ++jj) {
           const int j = ((ks * n + i) & 1) ? TM - 1 - jj : jj;  // every MFMA shares an operand with the one before
-          g288_mfma<T>(acc[i0 + i][j], fb[ks][i], fa[ks][j]);
+          gemm_mfma<T>(acc[i0 + i][j], fb[ks][i], fa[ks][j]);
           ++m;
           if (m % EVERY == 0 && m / EVERY <= D) {
             G288_PIN();
@@ -414,8 +376,8 @@ __global__ __launch_bounds__(512) void gemm288_kernel(const uint16_t* __restrict
           bv[4 * e + 2] = HAS_BIAS ? lo16<T>(bpk[i].y) : 0.f, bv[4 * e + 3] = HAS_BIAS ? hi16<T>(bpk[i].y) : 0.f;
         }
         const u32x4_t o = epi_pack8<CEPI, T>(a8, bv);
-        if constexpr (n == 2) g288_write<64 * p>(wr, o);
-        else g288_write<64 * p>(wr - 8 * fg, u32x2_t{o.x, o.y});
+        if constexpr (n == 2) gemm_lds_write<64 * p>(wr, o);
+        else gemm_lds_write<64 * p>(wr - 8 * fg, u32x2_t{o.x, o.y});
       };
       convert(C0{});
       convert(C1{});
@@ -429,7 +391,7 @@ __global__ __launch_bounds__(512) void gemm288_kernel(const uint16_t* __restrict
         int row, ch;
         const bool in = piece_of(s, row, ch);
         off[s] = in ? ((row + 16 * j) * (int)ldc + nw + ch) * 2 : (int)kOut;
-        o[s] = g288_read<0>(out0 + (in ? row * PITCH + 2 * ch : 0));
+        o[s] = gemm_lds_read<0>(out0 + (in ? row * PITCH + 2 * ch : 0));
       }
 #pragma unroll
       for (int s = 0; s < NS; ++s) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(o[s])::"memory");
@@ -442,7 +404,7 @@ __global__ __launch_bounds__(512) void gemm288_kernel(const uint16_t* __restrict
             int row, ch;
             const bool in = piece_of(s, row, ch);
             if (one_gate) {
-              g8 = g288_read<2048>(lds0 + rows_at + 2 * (wn * 16 * NT + ch));
+              g8 = gemm_lds_read<2048>(lds0 + rows_at + 2 * (wn * 16 * NT + ch));
               asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(g8)::"memory");
             } else if (in) {
               const int m = min((int)row0 + row + 16 * j, M - 1);

@@ -8,36 +8,6 @@
 namespace sana {
 namespace {
 
-// A wave-uniform value into scalar registers, whatever the compiler thinks of it.
-__device__ __forceinline__ int g8_uniform(int x) {
-  int r;
-  asm volatile("s_mov_b32 %0, %1" : "=s"(r) : "s"(x));
-  return r;
-}
-__device__ __forceinline__ const uint16_t* g8_uniform(const uint16_t* x) {
-  const uint16_t* r;
-  asm volatile("s_mov_b64 %0, %1" : "=s"(r) : "s"(x));
-  return r;
-}
-template <int OFF>
-__device__ __forceinline__ u32x4_t g8_read(uint32_t addr) {
-  u32x4_t v;
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
-  return v;
-}
-template <int OFF>
-__device__ __forceinline__ void g8_write(uint32_t addr, u32x4_t v) {
-  asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(addr), "v"(v), "n"(OFF) : "memory");
-}
-template <int OFF>
-__device__ __forceinline__ void g8_write(uint32_t addr, u32x2_t v) {
-  asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(addr), "v"(v), "n"(OFF) : "memory");
-}
-template <typename T>
-__device__ __forceinline__ void g8_mfma(f32x4_t& c, u32x4_t a, u32x4_t b) {
-  if constexpr (is_f16<T>) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
-  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
-}
 // 4 outputs of one row -> packed, per the epilogue kind (the gated residual is applied at store time)
 template <int EPI, typename T>
 __device__ __forceinline__ u32x2_t g8_pack4(f32x4_t a, const float* bv) {
@@ -252,26 +222,15 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
           rsrc_w, (__attribute__((address_space(3))) void*)(smem + W_BASE + st * W_STAGE + w_dst(q)), 16, (int)vw[q], kl * 128, 0, 0);
   };
 
-  // workgroup -> tile: XCD x (ids x, x + 8, ..) takes the x-th contiguous eighth of the grouped tile order
   const int total = tiles_t * tiles_c;
   auto start_tile = [&](int id) {  // resources and offsets of a tile, and the loads in front of its first phase
-    int pid;
-    {
-      const int xcd = id & 7, local = id >> 3;
-      const int base = total >> 3, rem = total & 7;
-      pid = xcd * base + min(xcd, rem) + local;
-    }
-    const int GROUP = K >= 4096 ? 8 : 4;
-    const int group_sz = GROUP * tiles_c;
-    const int gid = pid / group_sz;
-    const int first_t = gid * GROUP;
-    const int gt = min(tiles_t - first_t, GROUP);
-    m0 = g8_uniform(__builtin_amdgcn_readfirstlane(first_t + (pid % group_sz) % gt) * BM);
-    n0 = g8_uniform(__builtin_amdgcn_readfirstlane((pid % group_sz) / gt) * BN);
+    gemm_tile_of(id, tiles_t, tiles_c, K >= 4096 ? 8 : 4, BM, BN, m0, n0);
+    m0 = gemm_uniform(__builtin_amdgcn_readfirstlane(m0));
+    n0 = gemm_uniform(__builtin_amdgcn_readfirstlane(n0));
     const int a_last = min(BM, M - m0) - 1, w_last = min(BN, N - n0) - 1;
     const int64_t a_bytes = TAPS ? (tp.rows > m0 ? ((tp.rows - m0 - 1) * lda + tp.kc) * 2 : 0) : ((int64_t)a_last * lda + K) * 2;
-    base_a = g8_uniform(A + (int64_t)m0 * lda), bytes_a = g8_uniform((int)a_bytes);
-    base_w = g8_uniform(W + (int64_t)n0 * ldw), bytes_w = g8_uniform((int)(((int64_t)w_last * ldw + K) * 2));
+    base_a = gemm_uniform(A + (int64_t)m0 * lda), bytes_a = gemm_uniform((int)a_bytes);
+    base_w = gemm_uniform(W + (int64_t)n0 * ldw), bytes_w = gemm_uniform((int)(((int64_t)w_last * ldw + K) * 2));
     const int lane = lane_id(), lr = lane >> 3;
     const int piece = (lane & 7) ^ (4 * (wave & 1) + (lr >> 1));  // the global k piece of this lane's place in LDS
     const uint32_t la0 = ((uint32_t)(8 * wave + lr) * (uint32_t)lda + 8 * piece) * 2;
@@ -326,22 +285,22 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
     constexpr int O = decltype(st_c)::value * W_STAGE;
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      fb[ks][0] = g8_read<O>(rw[ks]);
-      fb[ks][1] = g8_read<O + 2048>(rw[ks]);
-      if constexpr (NB > 2) fb[ks][2] = g8_read<O + 4096>(rw[ks]);
-      if constexpr (NB > 3) fb[ks][3] = g8_read<O + 6144>(rw[ks]);
+      fb[ks][0] = gemm_lds_read<O>(rw[ks]);
+      fb[ks][1] = gemm_lds_read<O + 2048>(rw[ks]);
+      if constexpr (NB > 2) fb[ks][2] = gemm_lds_read<O + 4096>(rw[ks]);
+      if constexpr (NB > 3) fb[ks][3] = gemm_lds_read<O + 6144>(rw[ks]);
     }
   };
   auto read_a = [&](auto st_c, auto h_c) {
     constexpr int O = decltype(st_c)::value * A_STAGE + decltype(h_c)::value * 8192;
-    fa[0][0] = g8_read<O>(ra[0]);
-    fa[0][1] = g8_read<O + 2048>(ra[0]);
-    fa[0][2] = g8_read<O + 4096>(ra[0]);
-    fa[0][3] = g8_read<O + 6144>(ra[0]);
-    fa[1][0] = g8_read<O>(ra[1]);
-    fa[1][1] = g8_read<O + 2048>(ra[1]);
-    fa[1][2] = g8_read<O + 4096>(ra[1]);
-    fa[1][3] = g8_read<O + 6144>(ra[1]);
+    fa[0][0] = gemm_lds_read<O>(ra[0]);
+    fa[0][1] = gemm_lds_read<O + 2048>(ra[0]);
+    fa[0][2] = gemm_lds_read<O + 4096>(ra[0]);
+    fa[0][3] = gemm_lds_read<O + 6144>(ra[0]);
+    fa[1][0] = gemm_lds_read<O>(ra[1]);
+    fa[1][1] = gemm_lds_read<O + 2048>(ra[1]);
+    fa[1][2] = gemm_lds_read<O + 4096>(ra[1]);
+    fa[1][3] = gemm_lds_read<O + 6144>(ra[1]);
   };
   auto wait_a = [&]() {
     asm volatile("s_waitcnt lgkmcnt(0)"
@@ -360,7 +319,7 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
           const int j = ((ks * NB + i) & 1) ? 3 - jj : jj;  // every MFMA shares an operand with the one before
-          g8_mfma<T>(acc[i][4 * h + j], fb[ks][i], fa[ks][j]);
+          gemm_mfma<T>(acc[i][4 * h + j], fb[ks][i], fa[ks][j]);
         }
   };
   auto half_end = [&]() {
@@ -547,12 +506,12 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
 #pragma unroll
         for (int c = 0; c < NP; ++c) {
           if ((NB & 1) && c == NP - 1) {
-            g8_write<O>(wr[c], g8_pack4<CEPI, T>(acc[2 * c][j], bv + 8 * c));
+            gemm_lds_write<O>(wr[c], g8_pack4<CEPI, T>(acc[2 * c][j], bv + 8 * c));
           } else {
             float a8[8];
 #pragma unroll
             for (int r = 0; r < 4; ++r) a8[r] = acc[2 * c][j][r], a8[4 + r] = acc[2 * c + 1 < NB ? 2 * c + 1 : 2 * c][j][r];
-            g8_write<O>(wr[c], epi_pack8<CEPI, T>(a8, bv + 8 * c));
+            gemm_lds_write<O>(wr[c], epi_pack8<CEPI, T>(a8, bv + 8 * c));
           }
         }
       };
@@ -562,7 +521,7 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
     auto store = [&](int g) {
       u32x4_t o[NB];
 #pragma unroll
-      for (int s = 0; s < NB; ++s) o[s] = g8_read<0>(rd[s]);  // (a wave's LDS accesses are in order)
+      for (int s = 0; s < NB; ++s) o[s] = gemm_lds_read<0>(rd[s]);  // (a wave's LDS accesses are in order)
 #pragma unroll
       for (int s = 0; s < NB; ++s) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(o[s])::"memory");
 #pragma unroll

@@ -61,6 +61,47 @@ int gemm_ring_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, ui
 
 namespace {
 
+// A wave-uniform value into scalar registers, whatever the compiler thinks of it.
+__device__ __forceinline__ int gemm_uniform(int x) {
+  int r;
+  asm volatile("s_mov_b32 %0, %1" : "=s"(r) : "s"(x));
+  return r;
+}
+__device__ __forceinline__ const uint16_t* gemm_uniform(const uint16_t* x) {
+  const uint16_t* r;
+  asm volatile("s_mov_b64 %0, %1" : "=s"(r) : "s"(x));
+  return r;
+}
+// LDS accesses and MFMAs of the tile kernels as asm statements: to the compiler an ordinary LDS access may alias the direct
+// loads in flight.  The caller waits.
+template <int OFF>
+__device__ __forceinline__ u32x4_t gemm_lds_read(uint32_t addr) {
+  u32x4_t v;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+  return v;
+}
+template <int OFF>
+__device__ __forceinline__ void gemm_lds_write(uint32_t addr, u32x4_t v) {
+  asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(addr), "v"(v), "n"(OFF) : "memory");
+}
+template <int OFF>
+__device__ __forceinline__ void gemm_lds_write(uint32_t addr, u32x2_t v) {
+  asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(addr), "v"(v), "n"(OFF) : "memory");
+}
+template <typename T>
+__device__ __forceinline__ void gemm_mfma(f32x4_t& c, u32x4_t a, u32x4_t b) {
+  if constexpr (is_f16<T>) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+// Workgroup id -> first token and first channel of its tile of bm x bn: XCD x (ids x, x + 8, ..) takes the x-th contiguous
+// eighth of the order in groups of `group` token tiles.
+__device__ __forceinline__ void gemm_tile_of(int id, int tiles_t, int tiles_c, int group, int bm, int bn, int& m0, int& n0) {
+  const int total = tiles_t * tiles_c, xcd = id & 7, local = id >> 3, base = total >> 3, rem = total & 7;
+  const int pid = xcd * base + min(xcd, rem) + local;
+  const int group_sz = group * tiles_c, gid = pid / group_sz, first_t = gid * group, gt = min(tiles_t - first_t, group);
+  m0 = (first_t + (pid % group_sz) % gt) * bm, n0 = ((pid % group_sz) / gt) * bn;
+}
+
 // 8 outputs of one row: accumulator (+bias) -> io dtype, per the epilogue kind (everything except
 // the gated residual, which needs the row's residual and gate and is applied at store time).
 template <int EPI, typename T = BF16>

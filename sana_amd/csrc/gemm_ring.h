@@ -8,19 +8,10 @@
 namespace sana {
 namespace {
 
-template <int OFF>
-__device__ __forceinline__ u32x4_t gr_read(uint32_t addr) {
-  u32x4_t v;
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
-  return v;
-}
-__device__ __forceinline__ void gr_write(uint32_t addr, u32x4_t v) {
-  asm volatile("ds_write_b128 %0, %1" ::"v"(addr), "v"(v) : "memory");
-}
 // N fragments, 2048 bytes (16 rows) apart
 template <size_t N, size_t... I>
 __device__ __forceinline__ void gr_read_n(u32x4_t (&f)[N], uint32_t addr, std::index_sequence<I...>) {
-  ((f[I] = gr_read<2048 * (int)I>(addr)), ...);
+  ((f[I] = gemm_lds_read<2048 * (int)I>(addr)), ...);
 }
 // wait for the reads issued so far, tied to the registers they fill
 template <size_t N>
@@ -29,12 +20,6 @@ __device__ __forceinline__ void gr_landed(u32x4_t (&f)[N]) {
 #pragma unroll
   for (size_t i = 1; i < N; ++i) asm volatile("" : "+v"(f[i])::"memory");
 }
-template <typename T>
-__device__ __forceinline__ void gr_mfma(f32x4_t& c, u32x4_t a, u32x4_t b) {
-  if constexpr (is_f16<T>) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
-  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
-}
-
 // Workgroup tile BM = 16 TM WM tokens x BN = 16 TN WN channels, WM x WN waves of TM x TN MFMA tiles of 16x16x32.
 //
 // LDS: ST stages of a k-tile of 64 ([A rows | W rows], 128 bytes a row, the 16-byte piece index XORed with (row / 2) % 8),
@@ -66,16 +51,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
   const int wm = wave / WN, wn = wave % WN;
   const int fr = lane & 15, fg = lane >> 4, lr = lane >> 3;
 
-  // workgroup -> tile: XCD x (ids x, x + 8, ..) takes the x-th contiguous eighth of the order in groups of `group` token tiles
-  const int total = tiles_t * tiles_c;
-  int pid;
-  {
-    const int id = blockIdx.x, xcd = id & 7, local = id >> 3;
-    const int base = total >> 3, rem = total & 7;
-    pid = xcd * base + min(xcd, rem) + local;
-  }
-  const int group_sz = group * tiles_c, gid = pid / group_sz, first_t = gid * group, gt = min(tiles_t - first_t, group);
-  const int m0 = (first_t + (pid % group_sz) % gt) * BM, n0 = ((pid % group_sz) / gt) * BN;
+  int m0, n0;
+  gemm_tile_of(blockIdx.x, tiles_t, tiles_c, group, BM, BN, m0, n0);
 
   // ---- direct loads: rows past M / N, k pieces past K and k-tiles past the last one lie outside the resource: zeros
   constexpr uint32_t kOut = 0x80000000u;
@@ -156,7 +133,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
       const int i = m / TM, j = (i & 1) ? TM - 1 - m % TM : m % TM;  // every MFMA shares an operand with the one before
-      gr_mfma<T>(acc[i][j], fb[KS][i], fa[KS][j]);
+      gemm_mfma<T>(acc[i][j], fb[KS][i], fa[KS][j]);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int r = RPM * m; r < RPM * (m + 1) && r < NR; ++r) {
@@ -266,11 +243,11 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
       float a8[8];
 #pragma unroll
       for (int r = 0; r < 4; ++r) a8[r] = acc[2 * c][j][r], a8[4 + r] = acc[2 * c + 1][j][r];
-      gr_write(wr + 64 * c, epi_pack8<GATED ? SANA_EPI_BIAS : EPI, T>(a8, bv[c]));
+      gemm_lds_write<0>(wr + 64 * c, epi_pack8<GATED ? SANA_EPI_BIAS : EPI, T>(a8, bv[c]));
     }
     u32x4_t o[NS];
 #pragma unroll
-    for (int s = 0; s < NS; ++s) o[s] = gr_read<0>(rd[s]);  // (a wave's LDS accesses are in order)
+    for (int s = 0; s < NS; ++s) o[s] = gemm_lds_read<0>(rd[s]);  // (a wave's LDS accesses are in order)
 #pragma unroll
     for (int s = 0; s < NS; ++s) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(o[s])::"memory");
 #pragma unroll
