@@ -603,8 +603,8 @@ __global__ __launch_bounds__(256) void linattn_apply32_kernel(
 // Three launches (phase 1, reduction, phase 2) are 3 - 6 us of work each with a gap in front; here everything a head needs
 // for 1024 tokens is requested at once and the rest is one memory round trip, the transposes and the matrix products of one
 // compute unit.  That is also the bound: a head's tokens are one compute unit's work.  us, two calls / this, replayed from a
-// graph on one set of inputs (on 32 in turn): bf16, 36 heads x 256 tokens 10.5 / 5.6 (10.9 / 6.1), 36 x 1024 12.9 / 9.3 (13.7 /
-// 12.0), 140 x 1024 19.4 / 15.5 (21.6 / 16.6); fp16 36 x 256 11.2 / 6.2 (11.6 / 6.7); fp32 210 x 1024 34.2 / 26.6 (40.5 / 34.8).
+// graph on one set of inputs (on 16 in turn): bf16, 36 heads x 256 tokens 9.8 / 5.2 (10.5 / 6.0), 36 x 1024 12.1 / 8.8 (13.3 /
+// 11.5), 140 x 1024 18.9 / 15.4 (22.2 / 17.0); fp16 36 x 256 10.5 / 5.8 (11.2 / 6.6); fp32 256 x 1024 35.9 / 26.7 (45.6 / 38.4).
 // (Adding the state up in the two calls' order costs 0.4 us at 1024 tokens: sixteen partial states in LDS, not eight.)
 // ----------------------------------------------------------------------------
 constexpr int WHOLE_TOKENS = 1024;  // the most that one round of loads covers
@@ -1234,15 +1234,17 @@ extern "C" __attribute__((visibility("default"))) int sana_hip_litela_apply(
                     io_dtype, out_dtype, pre, stream);
 }
 
-// One launch while a head is a short piece of work and every head has a compute unit.  us, two calls / one launch: bf16
-// 36 x 1024 12.5 / 8.5, 210 x 1024 21.3 / 19.0, but 36 x 1536 12.8 / 13.1 and 280 x 1024 26.4 / 30.2 (a second round); f16 210 x
-// 1024 23.7 / 21.2.  fp32 moves twice the bytes and has the slower matrix instruction, so that few heads leave too much of the
-// chip idle beyond 256 tokens: 36 x 256 10.8 / 8.5, 36 x 512 11.3 / 12.2, 70 x 512 13.5 / 12.9, 70 x 768 16.0 / 19.3, 108 x 768
-// 21.5 / 20.4, 140 x 1024 27.7 / 24.9.
+// One launch while a head is a short piece of work and every head has a compute unit.  us, the launches of the two calls / one,
+// from a graph on 16 sets of inputs in turn (what another kernel has just written is not in the reading XCD's L2 either):
+// bf16 36 x 1024 13.3 / 11.5, 256 x 1024 27.6 / 25.1, but 280 x 1024 32.2 / 38.4 (a second round); f16 36 x 1024 14.0 / 14.0, 256 x
+// 1024 29.5 / 27.2.  fp32 moves twice the bytes and has the slower matrix instruction, so that beyond 256 tokens a head is too much
+// for one compute unit while others idle: 70 x 512 18.6 / 22.9, 108 x 768 25.0 / 27.6, 140 x 768 26.3 / 28.2, and 180 x 512 25.5 /
+// 25.5, 180 x 768 33.0 / 29.2, 256 x 1024 45.6 / 38.4.  Up to 256 the spared launches decide, issued eagerly 15.7 / 14.3 for 36 x
+// 256 (from the graph 13.3 / 14.5), 16.4 / 13.5 for 70 x 128 (13.3 / 13.5).
 static bool one_launch(int B, int N, int h, int io_dtype) {
   const int64_t heads = (int64_t)B * h;
   if (N > WHOLE_TOKENS || heads > 256) return false;
-  return io_dtype != SANA_DT_F32 || N <= 256 || N <= 7 * heads;
+  return io_dtype != SANA_DT_F32 || N <= 256 || heads >= 160;
 }
 static size_t state_bytes(int B, int h) { return ((size_t)B * h * STATE_ELEMS * sizeof(float) + 255) & ~(size_t)255; }
 
