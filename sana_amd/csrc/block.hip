@@ -1,6 +1,7 @@
 // One image block (SanaMSBlock, 16-bit weights) as one call: the launches of the entry points below, in order, on one
-// scratch buffer.  No kernels of its own.  At a few hundred tokens a block is eleven to thirteen launches of 4 - 14 us, and issuing
-// them one by one from Python took 220 us per block where the device needs about 100.
+// scratch buffer.  No kernels of its own.  A block is eleven launches (4 - 14 us each at a few hundred tokens), plus up to two where
+// the attention is not one launch and one for each GEMM in two widths or split over k, and issuing them one by one from Python
+// took 220 us per block where the device needs about 100.
 #include <algorithm>
 
 #include "common.h"

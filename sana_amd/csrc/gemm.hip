@@ -858,10 +858,14 @@ double cost16(const Tile16& t, int64_t M, int64_t N, int K) {
 }
 // The 288-wide tile.  Its k-tile costs 1.18 times the 256-wide one's for 1.125 times the work, so it pays where it saves
 // rounds (2240 and 1152 channels are 8 and 4 tiles).  Fitted to 120 shapes (700 .. 32760 tokens, the same projections, weights
-// cold), and the tiles it is compared with to the same shapes, which reach further up than the ones above: 7 % off each.  Taken
-// at 0.99 of the others' estimate or less: of 140 shapes 29, at 0.90 of the time on the mean, none slower.  us, best other / this:
-// 8192 x 2240 x 5600 220 / 157, 16384 x 2240 x 5600 348 / 314, 32760 x 2240 x 5600 747 / 646, 16384 x 1152 x 2880 106 / 88,
-// 9720 x 5760 x 1152 123 / 119; not taken: 4096 x 2240 x 2240 43 / 56, 16384 x 11200 x 2240 591 / 626, 12288 x 2240 x 2240 111 / 123.
+// cold), and the tiles it is compared with to the same shapes, which reach further up than the ones above (two fits: the constants
+// of one tile differ by up to 30 % between them, and a plan's estimate is by one or the other): 7 % off each.  Taken
+// at 0.99 of the others' estimate or less: of 128 shapes 21, at 0.90 of the time on the mean, none slower, and two of the other
+// 107 would have been faster in it (3 and 6 %; profiles/gemm288_against_other_tiles.txt).  Of 330 random shapes that take it
+// (K 256 .. 5600, odd sizes) it is at 0.90 on the mean; three are 6 - 12 % slower, at K 600 - 830 with several rounds and no
+// epilogue, where the constants make too much of the 256- and 128-wide tiles.  us, best other / this:
+// 8192 x 2240 x 5600 225 / 152, 16384 x 2240 x 5600 352 / 308, 32760 x 2240 x 5600 751 / 642, 16384 x 1152 x 2880 103 / 84,
+// 9720 x 5760 x 1152 122 / 120; not taken: 4096 x 2240 x 2240 42 / 55, 16384 x 11200 x 2240 577 / 621, 12288 x 2240 x 2240 109 / 121.
 constexpr Tile16 kTile288 = {256, 288, 256, 11.3, 1.17, 1.61};
 constexpr Tile16 kBeside288[] = {
     {256, 128, 256, 4.8, 0.75, 0.89}, {256, 192, 256, 7.4, 0.85, 1.18}, {256, 256, 256, 7.0, 1.20, 1.40},
@@ -1221,6 +1225,7 @@ SANA_API int sana_hip_tconv_residual(const void* X, const void* W, void* out, in
   const uint16_t* w = static_cast<const uint16_t*>(W);
   uint16_t* o = static_cast<uint16_t*>(out);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // (takes_288 compares with 128-token tiles and two widths as well, which this call does not have: few rows, where they lead)
   const double us192 = cost16(kTiles16[1], M, C, taps * C), us256 = cost16(kTiles16[2], M, C, taps * C);
   if (takes_288(M, C, taps * C, std::min(us192, us256)) && ldw < kMaxStride288)
     return gemm288_launch(x, w, e, o, M, C, taps * C, ldx, ldw, ldo, SANA_EPI_GATE_RES, false, &tp, s);

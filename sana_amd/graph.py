@@ -1,10 +1,10 @@
 """Replaying blocks from a HIP graph.
 
-At small shapes (one 1024 px image, the Sana-600M width) a block's launches (14, or up to ~25 where
-its modules are composed) take longer to issue from Python than to run; the library allocates, clears and synchronises nothing, so a block -- or a whole chain of
-blocks, one denoising step -- can be captured once and replayed with one launch.  The captured kernels hold raw
-addresses: inputs are copied into static buffers before each replay, the scratch buffers the library used stay
-alive for the life of the process, and the output tensor is overwritten by the next replay.
+At small shapes (one 1024 px image, the Sana-600M width) a block's launches (11 to 14, or up to ~25 where its modules are
+composed) take longer to issue from Python than to run; the library allocates, clears and synchronises nothing, so a
+block -- or a whole chain of blocks, one denoising step -- can be captured once and replayed with one launch.  The captured
+kernels hold raw addresses: inputs are copied into static buffers before each replay, the scratch buffers the library used
+stay alive for the life of the process (or are the graph's own), and the output tensor is overwritten by the next replay.
 """
 from __future__ import annotations
 
