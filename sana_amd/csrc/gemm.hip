@@ -836,78 +836,100 @@ GemmPlan plan_gemm(int M, int N, int K, bool w8) {
 size_t split_bytes(const GemmPlan& pl, int M, int N) { return pl.S > 1 ? (size_t)pl.S * M * N * sizeof(float) : 0; }
 
 // Time of an unsplit 16-bit GEMM in a given tile, us: ceil(K / 64) k-tiles per round of workgroups, at a rate per k-tile that
-// grows from `lone` (an eighth of the chip or less at work) to `full` (all of it: a compute unit takes 107 bytes/ns from
-// its L2 and about 50 while most of the chip misses it), plus launch, first loads and epilogue.  Fitted to 128 shapes
-// (64 .. 5000 tokens, the eight projections of the two image widths, weights cold): 8 - 13 % off, choice 2.5 % from the best.
+// grows from `lone` (lone_to workgroups or fewer in the round) to `full` (full_from or more: the weights come from HBM, the
+// matrix pipes share a power budget), plus launch, first loads and epilogue.
 struct Tile16 {
-  int bm, bn;    // tokens, channels; 256 tokens: gemm8_kernel, 288 channels: gemm288_kernel; else gemm_ring_kernel
+  int bm, bn;    // tokens, channels; 256 x 192 and 256 x 256: gemm8_kernel, 288 channels: gemm288_kernel; else gemm_ring_kernel
   int resident;  // workgroups on the chip at a time
+  int lone_to, full_from;
   double fixed, lone, full;
+  bool one_round = false;  // beyond one round of workgroups, every round is charged in full
 };
+// Fitted to 250 shapes (64 .. 32760 tokens, the eight projections of the two image widths and the text's, one block's and a
+// step's, weights cold, launches replayed from a graph: issued one by one, a launch of less than 20 us is timed by its issue):
+// 7 - 14 % off each, the choice 0.3 % from the best tile on the mean, more than 6 % in two shapes (9 and 7 %).  In a second round
+// the small tiles were never more than 2 % ahead, and 300 x 17920 x 2240 is 48.7 us in 128 x 128 and 40.4 in 256 x 192: hence
+// one_round.  us, the tile chosen before / now, both timed so: 256 x 1152 x 2880 14.9 / 13.8, 1024 x 2240 x 2240 24.3 / 19.0,
+// 1560 x 2304 x 1152 16.1 / 12.6, 2048 x 1152 x 2880 28.7 / 22.1, 4096 x 1152 x 1152 20.4 / 17.0, 4096 x 1152 x 2880
+// 38.6 / 30.5, 2916 x 2240 x 2240 33.0 / 32.1.
 constexpr Tile16 kTiles16[] = {
-    {256, 128, 256, 3.8, 0.73, 0.85}, {256, 192, 256, 5.7, 0.86, 1.17}, {256, 256, 256, 6.1, 1.12, 1.37},
-    {64, 64, 512, 2.1, 0.255, 0.466}, {64, 128, 256, 2.0, 0.42, 0.42},  {128, 128, 256, 2.4, 0.50, 0.59},
-    {128, 160, 256, 4.2, 0.58, 0.68},
+    {64, 64, 512, 256, 257, 3.0, 0.288, 0.503, true},  {64, 128, 256, 32, 256, 3.9, 0.350, 0.414, true},
+    {96, 128, 256, 32, 256, 3.7, 0.439, 0.466, true},  {128, 128, 256, 32, 256, 3.9, 0.454, 0.541, true},
+    {128, 160, 256, 32, 256, 4.3, 0.517, 0.643, true}, {192, 128, 256, 32, 256, 4.7, 0.497, 0.687, true},
+    {256, 128, 256, 32, 256, 5.1, 0.624, 0.825, true}, {256, 192, 256, 32, 256, 7.9, 0.628, 1.150},
+    {256, 256, 256, 32, 256, 5.3, 0.999, 1.404},       {256, 288, 256, 32, 256, 9.5, 0.955, 1.603},
+};
+constexpr int kTile192 = 7, kTile256 = 8, kTile288 = 9;
+// K below 1024: the rings fill and drain for much of the loop, and the constants above do not hold.  These are a fit of their own
+// (128 shapes), 8 - 13 % off.
+constexpr Tile16 kTilesShort[] = {
+    {256, 128, 256, 32, 256, 3.8, 0.73, 0.85}, {256, 192, 256, 32, 256, 5.7, 0.86, 1.17}, {256, 256, 256, 32, 256, 6.1, 1.12, 1.37},
+    {64, 64, 512, 64, 512, 2.1, 0.255, 0.466}, {64, 128, 256, 32, 256, 2.0, 0.42, 0.42},  {128, 128, 256, 32, 256, 2.4, 0.50, 0.59},
+    {128, 160, 256, 32, 256, 4.2, 0.58, 0.68},
 };
 double cost16(const Tile16& t, int64_t M, int64_t N, int K) {
   const int64_t n = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn), rounds = n / t.resident, rest = n % t.resident;
-  const double kt = (K + BK - 1) / BK, eighth = t.resident / 8;
+  const double kt = (K + BK - 1) / BK;
+  if (t.one_round && n > t.resident) return (rounds + (rest ? 1 : 0)) * (kt * t.full + t.fixed);
   double us = t.fixed + rounds * (kt * t.full + 0.5 * t.fixed);
-  if (rest) us += kt * (t.lone + (t.full - t.lone) * std::min(1.0, std::max(0.0, (rest - eighth) / (t.resident - eighth))));
+  if (rest)
+    us += kt * (t.lone + (t.full - t.lone) * std::min(1.0, std::max(0.0, double(rest - t.lone_to) / (t.full_from - t.lone_to))));
   return us;
 }
-// The 288-wide tile.  Its k-tile costs 1.18 times the 256-wide one's for 1.125 times the work, so it pays where it saves
-// rounds (2240 and 1152 channels are 8 and 4 tiles).  Fitted to 120 shapes (700 .. 32760 tokens, the same projections, weights
-// cold), and the tiles it is compared with to the same shapes, which reach further up than the ones above (two fits: the constants
-// of one tile differ by up to 30 % between them, and a plan's estimate is by one or the other): 7 % off each.  Taken
-// at 0.99 of the others' estimate or less: of 128 shapes 21, at 0.90 of the time on the mean, none slower, and two of the other
-// 107 would have been faster in it (3 and 6 %; profiles/gemm288_against_other_tiles.txt).  Of 330 random shapes that take it
-// (K 256 .. 5600, odd sizes) it is at 0.90 on the mean; three are 6 - 12 % slower, at K 600 - 830 with several rounds and no
-// epilogue, where the constants make too much of the 256- and 128-wide tiles.  us, best other / this:
-// 8192 x 2240 x 5600 225 / 152, 16384 x 2240 x 5600 352 / 308, 32760 x 2240 x 5600 751 / 642, 16384 x 1152 x 2880 103 / 84,
-// 9720 x 5760 x 1152 122 / 120; not taken: 4096 x 2240 x 2240 42 / 55, 16384 x 11200 x 2240 577 / 621, 12288 x 2240 x 2240 109 / 121.
-constexpr Tile16 kTile288 = {256, 288, 256, 11.3, 1.17, 1.61};
-constexpr Tile16 kBeside288[] = {
-    {256, 128, 256, 4.8, 0.75, 0.89}, {256, 192, 256, 7.4, 0.85, 1.18}, {256, 256, 256, 7.0, 1.20, 1.40},
-    {128, 128, 256, 2.3, 0.51, 0.61}, {128, 160, 256, 4.1, 0.62, 0.68},
+// The 288-wide tile at such K: its k-tile costs 1.18 times the 256-wide one's for 1.125 times the work, so it pays where it saves
+// rounds.  Fitted, and the tiles it is compared with too, to 120 shapes of 700 .. 32760 tokens; taken at 0.99 of the others'
+// estimate or less.  Of 330 random shapes that took it (K 256 .. 5600, odd sizes) it was at 0.90 of the time on the mean; three
+// were 6 - 12 % slower, at K 600 - 830 with several rounds and no epilogue.
+constexpr Tile16 kShort288 = {256, 288, 256, 32, 256, 11.3, 1.17, 1.61};
+constexpr Tile16 kBesideShort288[] = {
+    {256, 128, 256, 32, 256, 4.8, 0.75, 0.89}, {256, 192, 256, 32, 256, 7.4, 0.85, 1.18}, {256, 256, 256, 32, 256, 7.0, 1.20, 1.40},
+    {128, 128, 256, 32, 256, 2.3, 0.51, 0.61}, {128, 160, 256, 32, 256, 4.1, 0.62, 0.68},
 };
 constexpr int64_t kMaxStride288 = 1 << 21;  // rows of W from which the 32-bit offsets inside a tile could overflow
-bool takes_288(int M, int N, int K, double others_us) {  // others_us: by the constants above, which are lower
-  const double us = cost16(kTile288, M, N, K) / 0.99;
+bool short_takes_288(int M, int N, int K, double others_us) {  // others_us: by the constants above, which are lower
+  const double us = cost16(kShort288, M, N, K) / 0.99;
   if (us > 1.1 * others_us) return false;
-  for (const Tile16& t : kBeside288)
+  for (const Tile16& t : kBesideShort288)
     if (us > cost16(t, M, N, K)) return false;
   for (int a = 256; a < N; a += 256)
-    if (us > cost16(kBeside288[2], M, a, K) + cost16(kBeside288[1], M, N - a, K)) return false;
+    if (us > cost16(kBesideShort288[2], M, a, K) + cost16(kBesideShort288[1], M, N - a, K)) return false;
   return true;
 }
+constexpr int kShortK = 1024;
 struct Plan16 {
   const Tile16* tile;
   int n_wide;  // > 0: the first n_wide channels in 256 x 256 tiles, the rest in 256 x 192 ones, two launches
   double us;
 };
-Plan16 plan16(int M, int N, int K) {
-  Plan16 p = {&kTiles16[0], 0, 1e30};
-  for (const Tile16& t : kTiles16) {
+// the cheapest tile, or two widths where their last rounds fill better (4096 x 6720 tokens x channels, K = 2240: 432 tiles of 256
+// are 1.7 rounds, 15 x 16 and 15 x 16 tiles of the mix two that are 94 % full) by more than what the fit tells apart
+template <size_t TILES>
+Plan16 cheapest16(const Tile16 (&tiles)[TILES], const Tile16& t256, const Tile16& t192, double mix_below, int M, int N, int K) {
+  Plan16 p = {&tiles[0], 0, 1e30};
+  for (const Tile16& t : tiles) {
     const double us = cost16(t, M, N, K);
     if (us < p.us) p.tile = &t, p.us = us;
   }
-  // two widths, where their last rounds fill better (4096 x 6720 tokens x channels, K = 2240:
-  // 432 tiles of 256 are 1.7 rounds, 15 x 16 and 15 x 16 tiles of the mix two that are 94 % full)
   const double single = p.us;
   for (int a = 256; a < N; a += 256) {
-    const double us = cost16(kTiles16[2], M, a, K) + cost16(kTiles16[1], M, N - a, K);
-    if (us < 0.98 * single && us < p.us) p.n_wide = a, p.us = us;
+    const double us = cost16(t256, M, a, K) + cost16(t192, M, N - a, K);
+    if (us < mix_below * single && us < p.us) p.n_wide = a, p.us = us;
   }
-  if (takes_288(M, N, K, p.us)) p = {&kTile288, 0, cost16(kTile288, M, N, K)};
   return p;
 }
+Plan16 plan16(int M, int N, int K) {
+  if (K >= kShortK) return cheapest16(kTiles16, kTiles16[kTile256], kTiles16[kTile192], 0.992, M, N, K);
+  const Plan16 p = cheapest16(kTilesShort, kTilesShort[2], kTilesShort[1], 0.98, M, N, K);
+  return short_takes_288(M, N, K, p.us) ? Plan16{&kShort288, 0, cost16(kShort288, M, N, K)} : p;
+}
 // Split over k, or not: the split GEMM against the best unsplit one (16-bit and int8 weights decide alike, so that they
-// keep giving the same bits).  Time of the split one: fitted to 49 shapes, 4 % off.
+// keep giving the same bits).  Time of the split one: fitted to 49 shapes, 4 % off.  The unsplit tiles' fit is 3 - 13 % low at
+// the K of 5600 where it is taken (their weights come from HBM for longer than the prefetch reaches): 1024 x 2240 x 5600 is 46 us
+// either way, 256 x 2240 x 5600 27 split and 34 not.
 bool split_pays(const GemmPlan& pl, int M, int N, int K) {
   if (pl.S <= 1) return false;
   const int kt = (K + BK - 1) / BK;
-  return 9.4 + 1.12 * ((kt + pl.S - 1) / pl.S) + 0.139e-6 * pl.S * M * N * 8 < 0.97 * plan16(M, N, K).us;
+  return 9.4 + 1.12 * ((kt + pl.S - 1) / pl.S) + 0.139e-6 * pl.S * M * N * 8 < 1.04 * plan16(M, N, K).us;
 }
 
 // The pipelined kernel: split over k into pl.S ranges (ws holds the partial planes), or, int8 weights, unsplit (ws null).
@@ -1003,7 +1025,7 @@ int launch(const void* A, const void* W, const float* scale, const EpiArgs& ep, 
     if (p.tile->bn == 288 && ldw < kMaxStride288 && aligned16(ep.bias))  // (its bias row is loaded straight to LDS, 16 bytes a lane)
       return gemm288_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, nullptr, s);
     if (p.tile->bn == 288) return gemm8_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, 4, nullptr, s);
-    if (p.tile->bm == 256)
+    if (p.tile->bm == 256 && p.tile->bn >= 192)
       return gemm8_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, p.tile->bn / 64, nullptr, s);
     return gemm_ring_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, p.tile->bm, p.tile->bn, s);
   } else {
@@ -1225,11 +1247,13 @@ SANA_API int sana_hip_tconv_residual(const void* X, const void* W, void* out, in
   const uint16_t* w = static_cast<const uint16_t*>(W);
   uint16_t* o = static_cast<uint16_t*>(out);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // (takes_288 compares with 128-token tiles and two widths as well, which this call does not have: few rows, where they lead)
-  const double us192 = cost16(kTiles16[1], M, C, taps * C), us256 = cost16(kTiles16[2], M, C, taps * C);
-  if (takes_288(M, C, taps * C, std::min(us192, us256)) && ldw < kMaxStride288)
+  // one of the three widest tiles: the others have no taps
+  int best = kTile192;
+  for (int t : {kTile256, kTile288})
+    if ((t != kTile288 || ldw < kMaxStride288) && cost16(kTiles16[t], M, C, taps * C) < cost16(kTiles16[best], M, C, taps * C)) best = t;
+  if (best == kTile288)
     return gemm288_launch(x, w, e, o, M, C, taps * C, ldx, ldw, ldo, SANA_EPI_GATE_RES, false, &tp, s);
-  return gemm8_launch(x, w, e, o, M, C, taps * C, ldx, ldw, ldo, SANA_EPI_GATE_RES, false, us192 < us256 ? 3 : 4, &tp, s);
+  return gemm8_launch(x, w, e, o, M, C, taps * C, ldx, ldw, ldo, SANA_EPI_GATE_RES, false, best == kTile192 ? 3 : 4, &tp, s);
 }
 
 SANA_API int sana_hip_dequant_w8(const int8_t* Wq, const float* scale, void* W, int N, int K, int64_t ldw,

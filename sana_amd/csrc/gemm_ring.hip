@@ -5,7 +5,7 @@
 namespace sana {
 namespace {
 
-template <int WM, int WN, int TM, int TN, int ST, typename T>
+template <int WM, int WN, int TM, int TN, int ST, bool WHOLE, typename T>
 int launch_ring(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
                 int64_t ldw, int64_t ldc, int epilogue, hipStream_t s) {
   constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
@@ -20,7 +20,7 @@ int launch_ring(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_
     if (cost < best) best = cost, group = g;
   }
 #define SANA_LAUNCH_R(EPI)                                                                                              \
-  hipLaunchKernelGGL((gemm_ring_kernel<WM, WN, TM, TN, ST, EPI, T>), grid, block, 0, s, a, w, ep, c, M, N, K, lda, ldw, ldc, \
+  hipLaunchKernelGGL((gemm_ring_kernel<WM, WN, TM, TN, ST, WHOLE, EPI, T>), grid, block, 0, s, a, w, ep, c, M, N, K, lda, ldw, ldc, \
                      tiles_t, tiles_c, group)
   switch (epilogue) {
     case SANA_EPI_NONE: SANA_LAUNCH_R(SANA_EPI_NONE); break;
@@ -37,14 +37,20 @@ int launch_ring(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_
 
 int gemm_ring_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
                      int64_t ldw, int64_t ldc, int epilogue, bool f16, int bm, int bn, hipStream_t s) {
-#define SANA_RING(WM, WN, TM, TN, ST)                                                                          \
-  if (bm == 16 * TM * WM && bn == 16 * TN * WN)                                                                 \
-  return f16 ? launch_ring<WM, WN, TM, TN, ST, F16>(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, s)            \
-             : launch_ring<WM, WN, TM, TN, ST, BF16>(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, s)
-  SANA_RING(2, 2, 2, 2, 5);   // 64 x 64, 80 KB: two workgroups per compute unit
-  SANA_RING(2, 4, 2, 2, 6);   // 64 x 128
-  SANA_RING(4, 2, 2, 4, 4);   // 128 x 128 (five stages: the same time)
-  SANA_RING(4, 1, 2, 10, 4);  // 128 x 160
+#define SANA_RING(WM, WN, TM, TN, ST, WHOLE)                                                                           \
+  if (bm == 16 * TM * WM && bn == 16 * TN * WN)                                                                        \
+  return f16 ? launch_ring<WM, WN, TM, TN, ST, WHOLE, F16>(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, s)            \
+             : launch_ring<WM, WN, TM, TN, ST, WHOLE, BF16>(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, s)
+  SANA_RING(2, 2, 2, 2, 5, true);  // 64 x 64, 80 KB: two workgroups per compute unit
+  SANA_RING(2, 4, 2, 2, 6, true);  // 64 x 128
+  SANA_RING(2, 4, 3, 2, 5, true);  // 96 x 128
+  SANA_RING(2, 4, 4, 2, 4, true);  // 128 x 128
+  // 128 x 160.  The other loop (with 4 x 2 or 2 x 2 waves) needs 800 cycles a k-tile where this needs 977, but at 224 workgroups
+  // the chip then lowers its clock for what runs beside it as well: a step with int8 weights at 2048 rows takes 1721 us
+  // with that loop and 1642 with this one, at 1160 and 1245 W.
+  SANA_RING(4, 1, 2, 10, 4, false);
+  SANA_RING(4, 2, 3, 4, 4, true);  // 192 x 128
+  SANA_RING(4, 2, 4, 4, 3, true);  // 256 x 128
 #undef SANA_RING
   return SANA_ERR_ARG;
 }

@@ -1,0 +1,39 @@
+"""The ring tiles of the 16-bit GEMM at long k: rounds of the ring with and without a rest, k-tiles in odd and even number, k tails,
+ragged rows and channels, gate rows that change inside a tile.  Integer operands: every product and sum is exact in fp32, so the
+result is bit for bit the rounded integer one."""
+import ctypes
+
+import pytest
+import torch
+
+from sana_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+# 17 .. 27 k-tiles (every remainder of the rings' rounds of 4, 6 and 10), the last one of 8, 56, 0, .. values
+KS = [1032, 1080, 1152, 1216, 1288, 1344, 1408, 1472, 1536, 1600, 1664, 1720]
+TILES = {(64, 64): (195, 1048), (64, 128): (414, 2336), (96, 128): (1281, 2280), (128, 128): (1332, 2496),
+         (128, 160): (2349, 1800), (192, 128): (1872, 2992), (256, 128): (1935, 2968)}
+
+
+def _ints(*shape, hi=3, seed=0, dtype=torch.bfloat16):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randint(-hi, hi + 1, shape, generator=g).to(dtype)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_ring_tiles_are_exact_at_every_length_of_k(cuda, tile, dtype):
+    M, N = TILES[tile]
+    a_all, w_all = _ints(M, max(KS), seed=1, dtype=dtype).to(cuda), _ints(N, max(KS) + 8, seed=2, dtype=dtype).to(cuda)
+    bias, gate = _ints(N, hi=9, seed=3, dtype=dtype).to(cuda), _ints(3, 1, N, hi=4, seed=4, dtype=dtype).to(cuda)
+    res = _ints(3, M // 3, N, hi=99, seed=5, dtype=dtype).to(cuda)
+    for K in KS:
+        plan = (ctypes.c_int * 4)()
+        _lib.check(_lib.load().sana_hip_gemm_plan(M, N, K, plan), "sana_hip_gemm_plan")
+        assert tuple(plan) == (*tile, 0, 1), (tuple(plan), tile, K)
+        a, dense, apart = a_all[:, :K].contiguous(), w_all[:, :K].contiguous(), w_all[:, :K]   # rows of W one after the other, and not
+        y = (a.float() @ dense.float().T + bias.float()).to(dtype)      # |sum| <= 9 k < 2^24: exact in any order
+        assert torch.equal(ops.gemm_bf16(a, dense, bias, "bias"), y), K
+        assert torch.equal(ops.gemm_bf16(a, apart, bias, "bias"), y), K
+        assert torch.equal(ops.gemm_gate_residual(a.view(3, M // 3, K), dense, bias, gate, res), res + gate * y.view(3, M // 3, N)), K
