@@ -224,15 +224,24 @@ __global__ __launch_bounds__(256) void linattn_state16_kernel(
 // Bound by load latency: 64 tokens in flight without a branch around a load (it was 16 behind branches); the key sum is
 // adds, not a second MFMA chain.  Tokens x heads, us with the reduction: 1024 x 36 12.1 -> 7.6, 16384 x 70 136 -> 82.
 // ----------------------------------------------------------------------------
+// LINEAR: one chunk, the grid in one dimension of nsplit * B * ceil(h/4), an eighth of it in a row on each XCD: the phase 2 that
+// reads the partial states (linattn_apply32_partials_kernel) runs its heads there too.
+__device__ __forceinline__ int xcd_eighths(int id, int total) {  // workgroup -> its place in the order whose eighths are an XCD's
+  const int xcd = id & 7, base = total >> 3, rem = total & 7;
+  return xcd * base + min(xcd, rem) + (id >> 3);
+}
+template <bool LINEAR>
 __global__ __launch_bounds__(256) void linattn_state32_kernel(
     const float* __restrict__ K, const float* __restrict__ V, float* __restrict__ dst,
     const int32_t* __restrict__ chunk_starts, int N, int h, int n_chunks, int nsplit, int split_tokens,
     int64_t stride_b, int64_t stride_n) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int groups = (h + 3) >> 2;
-  const int b = blockIdx.z / groups, head = (blockIdx.z % groups) * 4 + wave;
+  const int at = LINEAR ? xcd_eighths(blockIdx.x, gridDim.x) : 0;
+  const int z = LINEAR ? at / nsplit : blockIdx.z, split = LINEAR ? at % nsplit : blockIdx.x;
+  const int b = z / groups, head = (z % groups) * 4 + wave;
   if (head >= h) return;  // no barriers below
-  const int c = blockIdx.y, split = blockIdx.x;
+  const int c = LINEAR ? 0 : blockIdx.y;
   const ChunkRange cr = chunk_range(chunk_starts, c, N);
   const int t0 = cr.begin + split * split_tokens;
   const int t1 = min(cr.end, t0 + split_tokens);
@@ -595,6 +604,70 @@ __global__ __launch_bounds__(256) void linattn_apply32_kernel(
       for (int r = 0; r < 16; r += 4)
         *reinterpret_cast<f32x4_t*>(op + 2 * r + 4 * g) = f32x4_t{num[r] / dd, num[r + 1] / dd, num[r + 2] / dd, num[r + 3] / dd};
     }
+  }
+}
+
+// ----------------------------------------------------------------------------
+// phase 2, fp32 io, on the partial states of one head (one chunk): the sum over the splits is formed here, in the order of
+// linattn_reduce_scan_kernel, so that a short sequence needs two launches.  grid: B * h * 128-token ranges; block 320: waves 0 .. 3
+// 32 tokens each, the fifth takes the state's 33rd row, so that the sums are one round of loads.  The queries are requested first;
+// a workgroup then reads nsplit x 4.2 KB of partial states, four times what its queries are at 16 splits, and that takes less than
+// the third launch: bound by the latency of the two loads.  us, issued eagerly on three sets of inputs in turn, three launches / two:
+// 1024 x 36 17.4 / 14.5, 2 x 1024 x 36 20.8 / 17.7, 400 x 70 17.2 / 14.2, 4 x 1000 x 36 27.2 / 26.3 (tokens x heads).  Both launches keep
+// a head on one XCD: with its partial states read by all eight, phase 1 of the next call takes 9.1 us instead of 5.9 to write
+// them again.  Beyond 1024 tokens the partial states that are read again outweigh the launch.
+// ----------------------------------------------------------------------------
+__global__ __launch_bounds__(320) void linattn_apply32_partials_kernel(
+    const float* __restrict__ Q, const float* __restrict__ partial, float* __restrict__ out, int N, int h, int nsplit,
+    int64_t q_stride_b, int64_t q_stride_n, int64_t o_stride_b, int64_t o_stride_n, float eps) {
+  constexpr int ROW = D + 4;  // floats of a state row in LDS (conflict-free 16-byte reads down a column)
+  __shared__ __attribute__((aligned(16))) float st[(D + 1) * ROW];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int ranges = (N + 127) >> 7, at = xcd_eighths(blockIdx.x, gridDim.x), bh = at / ranges;
+  const int b = bh / h, head = bh - b * h;
+  const int n = lane & 31, g = lane >> 5, tok = (at - bh * ranges) * 128 + wave * 32 + n;
+  const bool ok = tok < N && wave < 4;
+  f32x4_t q[4];
+  const float* qp = Q + (int64_t)b * q_stride_b + (int64_t)min(tok, N - 1) * q_stride_n + head * D + 16 * g;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) q[i] = *reinterpret_cast<const f32x4_t*>(qp + 4 * i);
+  const float* p0 = partial + (int64_t)bh * nsplit * STATE_ELEMS;
+  if (const int e = threadIdx.x; e < STATE_ELEMS / 4) {
+    f32x4_t v[16], s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = *reinterpret_cast<const f32x4_t*>(p0 + (int64_t)min(u, nsplit - 1) * STATE_ELEMS + 4 * e);
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      if (u < nsplit) s += v[u];
+    *reinterpret_cast<f32x4_t*>(st + (e >> 3) * ROW + 4 * (e & 7)) = s;
+  }
+  __syncthreads();
+  if (wave == 4) return;
+  float qv[16], den = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) qv[i] = ok ? fmaxf(q[i >> 2][i & 3], 0.f) : 0.f;
+  f32x16_t num;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) num[i] = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x4_t a = *reinterpret_cast<const f32x4_t*>(st + n * ROW + 16 * g + 4 * i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) num = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], qv[4 * i + e], num, 0, 0, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x4_t a = *reinterpret_cast<const f32x4_t*>(st + D * ROW + 16 * g + 4 * i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) den = fmaf(a[e], qv[4 * i + e], den);
+  }
+  den += __shfl_xor(den, 32, 64);
+  if (ok) {  // (layouts: linattn_apply32_kernel)
+    const float dd = den + eps;
+    float* op = out + (int64_t)b * o_stride_b + (int64_t)tok * o_stride_n + head * D;
+#pragma unroll
+    for (int r = 0; r < 16; r += 4)
+      *reinterpret_cast<f32x4_t*>(op + 2 * r + 4 * g) = f32x4_t{num[r] / dd, num[r + 1] / dd, num[r + 2] / dd, num[r + 3] / dd};
   }
 }
 
@@ -997,7 +1070,7 @@ static int state_impl(const void* k, const void* v, float* state, void* workspac
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (io_dtype == SANA_DT_F32) {
     dim3 grid(pl.nsplit, n_chunks, B * ((h + 3) / 4));
-    hipLaunchKernelGGL(linattn_state32_kernel, grid, dim3(256), 0, s, static_cast<const float*>(k),
+    hipLaunchKernelGGL(linattn_state32_kernel<false>, grid, dim3(256), 0, s, static_cast<const float*>(k),
                        static_cast<const float*>(v), dst, chunk_starts, N, h, n_chunks, pl.nsplit,
                        pl.split_tokens, stride_b, stride_n);
   } else {
@@ -1260,9 +1333,9 @@ extern "C" __attribute__((visibility("default"))) int sana_hip_linattn(
   if (!q || !k || !v || !out || B <= 0 || N <= 0 || h <= 0) return SANA_ERR_ARG;
   if (d != D) return SANA_ERR_SHAPE;
   if (io_dtype != SANA_DT_F32 && io_dtype != SANA_DT_BF16 && io_dtype != SANA_DT_F16) return SANA_ERR_DTYPE;
-  const int64_t C = (int64_t)h * d, vec = io_dtype == SANA_DT_F32 ? 4 : 8;  // values in 16 bytes
+  const int64_t C = (int64_t)h * d, heads = (int64_t)B * h, vec = io_dtype == SANA_DT_F32 ? 4 : 8;  // values in 16 bytes
   if (q_stride_n < C || stride_n < C || o_stride_n < C || q_stride_b < 0 || stride_b < 0 || o_stride_b < 0) return SANA_ERR_ARG;
-  if ((int64_t)B * h > (1 << 22)) return SANA_ERR_SHAPE;
+  if (heads > (1 << 22)) return SANA_ERR_SHAPE;
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out)) return SANA_ERR_ALIGN;
   for (int64_t x : {q_stride_b, q_stride_n, stride_b, stride_n, o_stride_b, o_stride_n})
     if (x % vec) return SANA_ERR_ALIGN;
@@ -1270,6 +1343,18 @@ extern "C" __attribute__((visibility("default"))) int sana_hip_linattn(
     const size_t at = state_bytes(B, h);
     if (!scratch || scratch_bytes < sana_hip_linattn_scratch_bytes(B, N, h, d, io_dtype)) return SANA_ERR_WORKSPACE;
     float* state = static_cast<float*>(scratch);
+    const StatePlan pl = plan_state(B, h, 1, N, io_dtype);
+    if (io_dtype == SANA_DT_F32 && N <= WHOLE_TOKENS && pl.nsplit > 1 && pl.nsplit <= 16 && heads <= (1 << 20)) {
+      float* partial = reinterpret_cast<float*>(static_cast<char*>(scratch) + at);
+      hipStream_t st = static_cast<hipStream_t>(stream);
+      hipLaunchKernelGGL(linattn_state32_kernel<true>, dim3(pl.nsplit * B * ((h + 3) / 4)), dim3(256), 0, st, static_cast<const float*>(k),
+                         static_cast<const float*>(v), partial, nullptr, N, h, 1, pl.nsplit, pl.split_tokens, stride_b, stride_n);
+      if (hipGetLastError() != hipSuccess) return SANA_ERR_LAUNCH;
+      hipLaunchKernelGGL(linattn_apply32_partials_kernel, dim3((N + 127) / 128 * (unsigned)heads), dim3(320), 0, st,
+                         static_cast<const float*>(q), partial, static_cast<float*>(out), N, h, pl.nsplit, q_stride_b, q_stride_n,
+                         o_stride_b, o_stride_n, eps);
+      return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
+    }
     const int rc = sana_hip_linattn_state(k, v, state, static_cast<char*>(scratch) + at, scratch_bytes - at, B, N, h, d, stride_b,
                                           stride_n, nullptr, 1, N, 0, io_dtype, stream);
     return rc != SANA_OK ? rc

@@ -109,3 +109,16 @@ def test_a_large_state_is_not_kept(cuda, monkeypatch):
         stream.synchronize()
         assert torch.equal(got, want)
         assert ((q.device.index, stream.cuda_stream) in ops._workspaces) == (kept == need)
+
+
+@pytest.mark.parametrize("B,N,h", [(1, 257, 5), (1, 300, 1), (2, 383, 7), (1, 384, 6), (1, 385, 9), (3, 1000, 13), (1, 1024, 3),
+                                   (1, 1008, 150), (53, 511, 3)])
+def test_two_launches_on_partial_states(cuda, B, N, h):
+    """fp32 between 257 and 1024 tokens: the sum over the splits inside phase 2, at the edges of its 128-token ranges, 32-token waves
+    and head groups, with rows and batch entries apart, is that of the reduction kernel bit for bit."""
+    C = 32 * h
+    gen = torch.Generator().manual_seed(N + h)
+    wide = torch.randn(B, N + 3, 3 * C + 4, generator=gen).to(cuda)[:, 1:N + 1]
+    q, k, v = (wide[:, :, i * C:(i + 1) * C] for i in range(3))
+    assert _lib.load().sana_hip_linattn_scratch_bytes(B, N, h, 32, ops._dt(q)) > 0
+    assert torch.equal(ops.relu_linear_attention(q, k, v, 1e-15), ops.linattn_apply(q, ops.linattn_state(k, v), 1e-15))
