@@ -13,8 +13,9 @@
 // feeds the probabilities straight back as the column operand of out^T = V^T . P^T -- the k index of that
 // product is permuted so that the 8 values a lane needs are the ones its own accumulators hold (keys
 // 32s + 4g + {0..3} and 32s + 16 + 4g + {0..3} for lane group g), and V^T is stored in that key order.
-// Few queries (one 512 px image: 32 workgroups of one item) are bound by the staging, a chain of load latencies: all of K
-// and V is requested before the first LDS write, and V is transposed four keys at a time (8-byte writes).
+// Few queries (one 512 px image: 32 workgroups of one item) are bound by the staging, a chain of load latencies: the queries and all
+// of K and V are requested before the first LDS write (the queries behind the staging: 0.3 us more a launch), and V is
+// transposed four keys at a time (8-byte writes).
 // Workgroups are persistent over consecutive (batch, head, query block) items and restage K / V only when the
 // (batch, head) changes.  Every K / V fragment read from LDS feeds QT MFMAs.
 #include "common.h"
@@ -69,6 +70,20 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
   for (int item = item0; item < item1; ++item) {
     const int bh = item / qblocks, qb = item - bh * qblocks;
     const int b = bh / H, h = bh - b * H;
+    const int q0 = qb * (NW * 16 * QT) + wave * (16 * QT);
+    // ---- Q fragments: column operand, lane -> query fr, k = 32*ks + 8*fg .. +7; requested in front of the staging
+    const uint16_t* qbase = q + ((int64_t)b * N) * ldq + (int64_t)h * d;
+    u32x4_t qf[QT][DK];
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+      const int qi = q0 + 16 * t + fr;
+#pragma unroll
+      for (int ks = 0; ks < DK; ++ks) {
+        const int k0 = 32 * ks + 8 * fg;
+        qf[t][ks] = (qi < N && k0 < d) ? *reinterpret_cast<const u32x4_t*>(qbase + (int64_t)qi * ldq + k0)
+                                       : u32x4_t{0u, 0u, 0u, 0u};
+      }
+    }
     if (bh != staged) {  // uniform
       __syncthreads();   // everyone is done with the previous head's K / V
       const uint16_t* kbase = kv + (int64_t)b * Nk * ldkv + (int64_t)h * d;
@@ -121,22 +136,7 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
       __syncthreads();
       staged = bh;
     }
-    const int q0 = qb * (NW * 16 * QT) + wave * (16 * QT);
     if (q0 >= N) continue;  // (no barrier inside the per-item work below)
-    const uint16_t* qbase = q + ((int64_t)b * N) * ldq + (int64_t)h * d;
-
-    // ---- Q fragments: column operand, lane -> query fr, k = 32*ks + 8*fg .. +7
-    u32x4_t qf[QT][DK];
-#pragma unroll
-    for (int t = 0; t < QT; ++t) {
-      const int qi = q0 + 16 * t + fr;
-#pragma unroll
-      for (int ks = 0; ks < DK; ++ks) {
-        const int k0 = 32 * ks + 8 * fg;
-        qf[t][ks] = (qi < N && k0 < d) ? *reinterpret_cast<const u32x4_t*>(qbase + (int64_t)qi * ldq + k0)
-                                       : u32x4_t{0u, 0u, 0u, 0u};
-      }
-    }
     // ---- scores^T = K . Q^T: acc[t][kt][r] = query 16t + fr, key 16*kt + 4*fg + r
     f32x4_t sc[QT][NKT];
 #pragma unroll
