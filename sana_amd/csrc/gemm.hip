@@ -844,6 +844,8 @@ struct Tile16 {
   int lone_to, full_from;
   double fixed, lone, full;
   bool one_round = false;  // beyond one round of workgroups, every round is charged in full
+  double halved = 0;       // > 0: k-tile where there are at most kHalvedTiles of them, in two workgroups each; a fit of its own:
+  double halved_row = 0;   // 4 % off.  One row of tiles: every weight comes from HBM to one workgroup (64 x 2240 x 5600 27 us, split 24)
 };
 // Fitted to 250 shapes (64 .. 32760 tokens, the eight projections of the two image widths and the text's, one block's and a
 // step's, weights cold, launches replayed from a graph: issued one by one, a launch of less than 20 us is timed by its issue):
@@ -853,7 +855,7 @@ struct Tile16 {
 // 1560 x 2304 x 1152 16.1 / 12.6, 2048 x 1152 x 2880 28.7 / 22.1, 4096 x 1152 x 1152 20.4 / 17.0, 4096 x 1152 x 2880
 // 38.6 / 30.5, 2916 x 2240 x 2240 33.0 / 32.1.
 constexpr Tile16 kTiles16[] = {
-    {64, 64, 512, 256, 257, 3.0, 0.288, 0.503, true},  {64, 128, 256, 32, 256, 3.9, 0.350, 0.414, true},
+    {64, 64, 512, 256, 257, 3.0, 0.288, 0.503, true, 0.165, 0.26}, {64, 128, 256, 32, 256, 3.9, 0.350, 0.414, true},
     {96, 128, 256, 32, 256, 3.7, 0.439, 0.466, true},  {128, 128, 256, 32, 256, 3.9, 0.454, 0.541, true},
     {128, 160, 256, 32, 256, 4.3, 0.517, 0.643, true}, {192, 128, 256, 32, 256, 4.7, 0.497, 0.687, true},
     {256, 128, 256, 32, 256, 5.1, 0.624, 0.825, true}, {256, 192, 256, 32, 256, 7.9, 0.628, 1.150},
@@ -870,6 +872,7 @@ constexpr Tile16 kTilesShort[] = {
 double cost16(const Tile16& t, int64_t M, int64_t N, int K) {
   const int64_t n = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn), rounds = n / t.resident, rest = n % t.resident;
   const double kt = (K + BK - 1) / BK;
+  if (t.halved > 0 && n <= kHalvedTiles) return t.fixed + kt * (M > t.bm ? t.halved : t.halved_row);
   if (t.one_round && n > t.resident) return (rounds + (rest ? 1 : 0)) * (kt * t.full + t.fixed);
   double us = t.fixed + rounds * (kt * t.full + 0.5 * t.fixed);
   if (rest)
@@ -925,7 +928,7 @@ Plan16 plan16(int M, int N, int K) {
 // Split over k, or not: the split GEMM against the best unsplit one (16-bit and int8 weights decide alike, so that they
 // keep giving the same bits).  Time of the split one: fitted to 49 shapes, 4 % off.  The unsplit tiles' fit is 3 - 13 % low at
 // the K of 5600 where it is taken (their weights come from HBM for longer than the prefetch reaches): 1024 x 2240 x 5600 is 46 us
-// either way, 256 x 2240 x 5600 27 split and 34 not.
+// either way, 256 x 2240 x 5600 27 split and 34 not, 144 x 2240 x 5600 27 and 20 (halved tiles).
 bool split_pays(const GemmPlan& pl, int M, int N, int K) {
   if (pl.S <= 1) return false;
   const int kt = (K + BK - 1) / BK;

@@ -12,8 +12,10 @@ pytestmark = pytest.mark.gpu
 
 # 17 .. 27 k-tiles (every remainder of the rings' rounds of 4, 6 and 10), the last one of 8, 56, 0, .. values
 KS = [1032, 1080, 1152, 1216, 1288, 1344, 1408, 1472, 1536, 1600, 1664, 1720]
-TILES = {(64, 64): (195, 1048), (64, 128): (414, 2336), (96, 128): (1281, 2280), (128, 128): (1332, 2496),
-         (128, 160): (2349, 1800), (192, 128): (1872, 2992), (256, 128): (1935, 2968)}
+# (64 x 64: up to 128 tiles as two workgroups of 32 channels each: 4 x 17 tiles, 3 x 42; whole: 4 x 33)
+TILES = [((64, 64), (195, 1048)), ((64, 64), (195, 2072)), ((64, 64), (192, 2688)), ((64, 64), (129, 1048)), ((64, 128), (414, 2336)),
+         ((96, 128), (1281, 2280)), ((128, 128), (1332, 2496)), ((128, 160), (2349, 1800)), ((192, 128), (1872, 2992)),
+         ((256, 128), (1935, 2968))]
 
 
 def _ints(*shape, hi=3, seed=0, dtype=torch.bfloat16):
@@ -21,10 +23,10 @@ def _ints(*shape, hi=3, seed=0, dtype=torch.bfloat16):
     return torch.randint(-hi, hi + 1, shape, generator=g).to(dtype)
 
 
-@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("tile,shape", TILES)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_ring_tiles_are_exact_at_every_length_of_k(cuda, tile, dtype):
-    M, N = TILES[tile]
+def test_ring_tiles_are_exact_at_every_length_of_k(cuda, tile, shape, dtype):
+    M, N = shape
     a_all, w_all = _ints(M, max(KS), seed=1, dtype=dtype).to(cuda), _ints(N, max(KS) + 8, seed=2, dtype=dtype).to(cuda)
     bias, gate = _ints(N, hi=9, seed=3, dtype=dtype).to(cuda), _ints(3, 1, N, hi=4, seed=4, dtype=dtype).to(cuda)
     res = _ints(3, M // 3, N, hi=99, seed=5, dtype=dtype).to(cuda)
