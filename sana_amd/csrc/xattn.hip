@@ -18,15 +18,14 @@
 // transposed four keys at a time (8-byte writes).
 // Workgroups are persistent over consecutive (batch, head, query block) items and restage K / V only when the
 // (batch, head) changes.  Every K / V fragment read from LDS feeds QT MFMAs.
+#include <type_traits>
+
 #include "common.h"
 
-// Tuning knobs: query tiles of 16 per wave and pass (every K / V fragment read feeds that many MFMAs), waves per
-// workgroup.  One tile and eight waves (two per SIMD, 196 registers) measured best: two tiles need either one wave
-// per SIMD (nothing hides the LDS latency: 112 us against 75 us at 16384 x 300 x 20 heads of 112) or spill.
-#ifndef SANA_XA_QT
-#define SANA_XA_QT 1
-#define SANA_XA_NW 8
-#endif
+// Query tiles of 16 per wave and pass (every K / V fragment read feeds that many MFMAs).  One measured best: two need either one wave
+// per SIMD (nothing hides the LDS latency: 112 us against 75 us at 16384 x 300 x 20 heads of 112) or, the keys in two groups, all
+// registers and a few more (92 us against 80).
+constexpr int XA_QT = 1;
 
 namespace sana {
 namespace {
@@ -137,125 +136,119 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
       staged = bh;
     }
     if (q0 >= N) continue;  // (no barrier inside the per-item work below)
-    // ---- scores^T = K . Q^T: acc[t][kt][r] = query 16t + fr, key 16*kt + 4*fg + r
-    f32x4_t sc[QT][NKT];
-#pragma unroll
-    for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-      for (int t = 0; t < QT; ++t) sc[t][kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    // key tiles in pairs (two independent accumulator chains), the next pair's fragments requested before
-    // this pair's MFMAs
-    u32x4_t kf[2][2][DK];
-    auto load_k = [&](int buf, int kp) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int row = 16 * (2 * kp + j) + fr;
-        const unsigned char* rp = sk + row * KPITCH;
-        const int key = xa_kkey<DK>(row);
-#pragma unroll
-        for (int ks = 0; ks < DK; ++ks) kf[buf][j][ks] = *reinterpret_cast<const u32x4_t*>(rp + (((4 * ks + fg) ^ key) << 4));
-      }
-    };
-    load_k(0, 0);
-#pragma unroll
-    for (int kp = 0; kp < NKT / 2; ++kp) {
-      if (kp + 1 < NKT / 2) load_k((kp + 1) & 1, kp + 1);
-#pragma unroll
-      for (int ks = 0; ks < DK; ++ks)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int t = 0; t < QT; ++t)
-            sc[t][2 * kp + j] = mfma_16x16x32<T>(kf[kp & 1][j][ks], qf[t][ks], sc[t][2 * kp + j]);
-    }
-    // ---- softmax over the keys of each query (log2 domain), probabilities back as packed 16-bit values.
-    // f16: the keys are two groups with a maximum each, combined in fp32 behind the product, and the sum is over the rounded
-    // probabilities.  A group's largest probability is 1 and has no rounding error; the stock fused kernels, which keep a
-    // running maximum over blocks of keys, have that in every block.  Error against 64 bits, one maximum / two / stock, e-4: 300 keys x 72
-    // 2.75 / 2.69 / 2.68, x 112 2.76 / 2.69 / 2.69, 10 keys 2.43 / 2.39 / 2.43.  us: 2048 queries x 16 heads 12.2 -> 12.9, 4096 22.6 ->
-    // 23.8, 77 keys 8.9 -> 8.4.
+    // Keys in NG groups, one after the other (scores, softmax, product; the first group's scores are gone before the second's come:
+    // 0.1 - 0.7 us less than all scores first).  f16: two, each with a maximum of its own, combined in fp32 at the end, and the sum
+    // is over the rounded probabilities.  A group's largest probability is 1 and has no rounding error; the stock fused kernels,
+    // which keep a running maximum over blocks of keys, have that in every block.  Error against 64 bits, one maximum / two /
+    // stock, e-4: 300 keys x 72 2.75 / 2.69 / 2.68, x 112 2.76 / 2.69 / 2.69, 10 keys 2.43 / 2.39 / 2.43.
     constexpr int NG = is_f16<T> ? 2 : 1, G0 = NG == 2 ? 2 * ((NKT + 3) / 4) : NKT;  // key tiles of the first group
-    float factor[QT][NG];
+    float mx[QT][NG], sum[QT][NG];
+    f32x4_t oc[NG][QT][DT];
+    auto group = [&](auto g_c) {
+      constexpr int g = decltype(g_c)::value, k0 = g * G0, k1 = g + 1 < NG ? G0 : NKT;
+      // ---- scores^T = K . Q^T: sc[t][kt][r] = query 16t + fr, key 16*(k0 + kt) + 4*fg + r
+      f32x4_t sc[QT][G0];
 #pragma unroll
-    for (int t = 0; t < QT; ++t) {
-      float mx[NG], sum[NG];
+      for (int kt = 0; kt < G0; ++kt)
 #pragma unroll
-      for (int g = 0; g < NG; ++g) {
-        mx[g] = -INFINITY;
+        for (int t = 0; t < QT; ++t) sc[t][kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      // key tiles in pairs (two independent accumulator chains), the next pair's fragments requested before this pair's MFMAs
+      u32x4_t kf[2][2][DK];
+      auto load_k = [&](int buf, int kt) {
 #pragma unroll
-        for (int kt = g * G0; kt < (g + 1 < NG ? G0 : NKT); ++kt) {
+        for (int j = 0; j < 2; ++j) {
+          const int row = 16 * (kt + j) + fr;
+          const unsigned char* rp = sk + row * KPITCH;
+          const int key = xa_kkey<DK>(row);
+#pragma unroll
+          for (int ks = 0; ks < DK; ++ks) kf[buf][j][ks] = *reinterpret_cast<const u32x4_t*>(rp + (((4 * ks + fg) ^ key) << 4));
+        }
+      };
+      load_k(0, k0);
+#pragma unroll
+      for (int kt = k0; kt < k1; kt += 2) {
+        const int buf = (kt - k0) / 2 & 1;
+        if (kt + 2 < k1) load_k(buf ^ 1, kt + 2);
+#pragma unroll
+        for (int ks = 0; ks < DK; ++ks)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int t = 0; t < QT; ++t)
+              sc[t][kt - k0 + j] = mfma_16x16x32<T>(kf[buf][j][ks], qf[t][ks], sc[t][kt - k0 + j]);
+      }
+      // ---- softmax over the group's keys (log2 domain), probabilities packed to 16 bits
+      u32x2_t pk[QT][G0];
+#pragma unroll
+      for (int t = 0; t < QT; ++t) {
+        float m = -INFINITY, l = 0.f;
+#pragma unroll
+        for (int kt = k0; kt < k1; ++kt) {
           const f32x4_t kb = *reinterpret_cast<const f32x4_t*>(sb + 16 * kt + 4 * fg);
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            sc[t][kt][r] = fmaf(sc[t][kt][r], scale_log2e, kb[r]);
-            mx[g] = fmaxf(mx[g], sc[t][kt][r]);
+            sc[t][kt - k0][r] = fmaf(sc[t][kt - k0][r], scale_log2e, kb[r]);
+            m = fmaxf(m, sc[t][kt - k0][r]);
           }
         }
-        mx[g] = fmaxf(mx[g], __shfl_xor(mx[g], 16));
-        mx[g] = fmaxf(mx[g], __shfl_xor(mx[g], 32));
-        if (NG == 2) mx[g] = fmaxf(mx[g], -3.0e38f);  // a group without keys: -inf - -inf
-        sum[g] = 0.f;
+        m = fmaxf(m, __shfl_xor(m, 16));
+        m = fmaxf(m, __shfl_xor(m, 32));
+        if (NG == 2) m = fmaxf(m, -3.0e38f);  // a group without keys: -inf - -inf
 #pragma unroll
-        for (int kt = g * G0; kt < (g + 1 < NG ? G0 : NKT); ++kt) {
+        for (int kt = 0; kt < k1 - k0; ++kt) {
+          float p[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            float p = __builtin_amdgcn_exp2f(sc[t][kt][r] - mx[g]);  // rounded to 16 bits where it is packed below
-            if constexpr (is_f16<T>) p = (float)(_Float16)p;
-            sc[t][kt][r] = p;
-            sum[g] += p;
+            p[r] = __builtin_amdgcn_exp2f(sc[t][kt][r] - m);
+            if constexpr (is_f16<T>) p[r] = (float)(_Float16)p[r];
+            l += p[r];
           }
+          pk[t][kt] = u32x2_t{pk16<T>(p[0], p[1]), pk16<T>(p[2], p[3])};
         }
-        sum[g] += __shfl_xor(sum[g], 16);
-        sum[g] += __shfl_xor(sum[g], 32);
+        l += __shfl_xor(l, 16);
+        l += __shfl_xor(l, 32);
+        mx[t][g] = m, sum[t][g] = l;
       }
-      if constexpr (NG == 2) {
-        const float m = fmaxf(mx[0], mx[1]), f0 = __builtin_amdgcn_exp2f(mx[0] - m), f1 = __builtin_amdgcn_exp2f(mx[1] - m);
-        const float inv = 1.0f / fmaf(sum[0], f0, sum[1] * f1);
-        factor[t][0] = f0 * inv, factor[t][1] = f1 * inv;
-      } else {
-        factor[t][0] = 1.0f / sum[0];
-      }
-    }
-    // ---- out^T = V^T . P^T: acc[t][dt][r] = query 16t + fr, channel 16*dt + 4*fg + r
-    f32x4_t oc[QT][DT], first[NG == 2 ? QT : 1][DT];  // first: the first group's part of the result
+      // ---- out^T = V^T . P^T: oc[t][dt][r] = query 16t + fr, channel 16*dt + 4*fg + r
 #pragma unroll
-    for (int t = 0; t < QT; ++t)
+      for (int t = 0; t < QT; ++t)
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) oc[t][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    u32x4_t vf[2][DT];
-    auto load_v = [&](int buf, int s) {
+        for (int dt = 0; dt < DT; ++dt) oc[g][t][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      u32x4_t vf[2][DT];
+      auto load_v = [&](int buf, int s) {
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        const int row = 16 * dt + fr;
-        vf[buf][dt] = *reinterpret_cast<const u32x4_t*>(sv + row * XA_VPITCH + (((4 * s + fg) ^ xa_vkey(row)) << 4));
-      }
-    };
-    load_v(0, 0);
+        for (int dt = 0; dt < DT; ++dt) {
+          const int row = 16 * dt + fr;
+          vf[buf][dt] = *reinterpret_cast<const u32x4_t*>(sv + row * XA_VPITCH + (((4 * s + fg) ^ xa_vkey(row)) << 4));
+        }
+      };
+      load_v(0, k0 / 2);
 #pragma unroll
-    for (int s = 0; s < NKT / 2; ++s) {
-      if (s + 1 < NKT / 2) load_v((s + 1) & 1, s + 1);
-      if (NG == 2 && 2 * s == G0) {
+      for (int s = 0; s < (k1 - k0) / 2; ++s) {
+        if (s + 1 < (k1 - k0) / 2) load_v((s + 1) & 1, k0 / 2 + s + 1);
+        u32x4_t pf[QT];
 #pragma unroll
         for (int t = 0; t < QT; ++t)
+          pf[t] = u32x4_t{pk[t][2 * s].x, pk[t][2 * s].y, pk[t][2 * s + 1].x, pk[t][2 * s + 1].y};
 #pragma unroll
-          for (int dt = 0; dt < DT; ++dt) {
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) first[t][dt][r] = oc[t][dt][r] * factor[t][0];
-            oc[t][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-          }
+          for (int t = 0; t < QT; ++t) oc[g][t][dt] = mfma_16x16x32<T>(vf[s & 1][dt], pf[t], oc[g][t][dt]);
       }
-      u32x4_t pf[QT];
+    };
+    group(std::integral_constant<int, 0>{});
+    if constexpr (NG == 2) group(std::integral_constant<int, 1>{});
+    float factor[QT][NG];
 #pragma unroll
-      for (int t = 0; t < QT; ++t) {
-        pf[t].x = pk16<T>(sc[t][2 * s][0], sc[t][2 * s][1]);
-        pf[t].y = pk16<T>(sc[t][2 * s][2], sc[t][2 * s][3]);
-        pf[t].z = pk16<T>(sc[t][2 * s + 1][0], sc[t][2 * s + 1][1]);
-        pf[t].w = pk16<T>(sc[t][2 * s + 1][2], sc[t][2 * s + 1][3]);
+    for (int t = 0; t < QT; ++t) {
+      if constexpr (NG == 2) {
+        const float m = fmaxf(mx[t][0], mx[t][1]);
+        const float f0 = __builtin_amdgcn_exp2f(mx[t][0] - m), f1 = __builtin_amdgcn_exp2f(mx[t][1] - m);
+        const float inv = 1.0f / fmaf(sum[t][0], f0, sum[t][1] * f1);
+        factor[t][0] = f0 * inv, factor[t][1] = f1 * inv;
+      } else {
+        factor[t][0] = 1.0f / sum[t][0];
       }
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int t = 0; t < QT; ++t) oc[t][dt] = mfma_16x16x32<T>(vf[s & 1][dt], pf[t], oc[t][dt]);
     }
     // ---- normalise and store: a lane holds 4 consecutive channels of its query per channel tile
     uint16_t* obase = out + ((int64_t)b * N) * ldo + (int64_t)h * d;
@@ -269,7 +262,7 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
           float v[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            v[r] = NG == 2 ? fmaf(oc[t][dt][r], factor[t][NG - 1], first[t][dt][r]) : oc[t][dt][r] * factor[t][0];
+            v[r] = NG == 2 ? fmaf(oc[NG - 1][t][dt][r], factor[t][NG - 1], oc[0][t][dt][r] * factor[t][0]) : oc[0][t][dt][r] * factor[t][0];
           const u32x2_t o = {pk16<T>(v[0], v[1]), pk16<T>(v[2], v[3])};
           *reinterpret_cast<u32x2_t*>(obase + (int64_t)qi * ldo + c0) = o;
         }
@@ -305,11 +298,17 @@ int cross_attention(const void* q, const void* kv, const float* key_bias, void* 
   const uint16_t* kp = static_cast<const uint16_t*>(kv);
   uint16_t* op = static_cast<uint16_t*>(out);
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define SANA_XA_GO(DK, DT, NKT) \
-  launch_xa<T, DK, DT, SANA_XA_QT, SANA_XA_NW, NKT>(qp, kp, key_bias, op, B, N, Nk, H, d, ldq, ldkv, ldo, bias_stride, scale, s)
+#define SANA_XA_GO(DK, DT, NW, NKT) \
+  launch_xa<T, DK, DT, XA_QT, NW, NKT>(qp, kp, key_bias, op, B, N, Nk, H, d, ldq, ldkv, ldo, bias_stride, scale, s)
+  // Waves per workgroup: eight, two per SIMD (up to 220 registers).  Four, half the queries, at up to 96 channels a head where these
+  // workgroups have a compute unit each: a unit then reads K and V from LDS for four waves.  us, 8 / 4 waves: 300 keys, 150 queries x
+  // 16 heads of 72 10.6 / 9.8, 512 11.5 / 10.1, 1024 11.7 / 10.5, f16 12.6 / 10.6, 77 keys 6.9 / 6.3; in two rounds 2 x 1024 13.8 / 16.2.
+  // 112 channels a head: 600 x 20 heads 13.1 / 12.7, 2 x 300 13.6 / 14.0 (the staging is more of it).
+  const bool few = d <= 96 && (int64_t)B * H * ((N + 64 * XA_QT - 1) / (64 * XA_QT)) <= 256;
   // key tiles of 16 that are multiplied: all 20, or 10 for up to 160 keys (tiles past Nk hold zeros and -inf)
-  if (d > 96) return Nk > 160 ? SANA_XA_GO(4, 7, 20) : SANA_XA_GO(4, 7, 10);
-  return Nk > 160 ? SANA_XA_GO(3, 6, 20) : SANA_XA_GO(3, 6, 10);
+  if (d > 96) return Nk > 160 ? SANA_XA_GO(4, 7, 8, 20) : SANA_XA_GO(4, 7, 8, 10);
+  if (few) return Nk > 160 ? SANA_XA_GO(3, 6, 4, 20) : SANA_XA_GO(3, 6, 4, 10);
+  return Nk > 160 ? SANA_XA_GO(3, 6, 8, 20) : SANA_XA_GO(3, 6, 8, 10);
 #undef SANA_XA_GO
 }
 

@@ -336,3 +336,18 @@ def test_tensor_subclass_weights_of_the_cross_attention_are_dispatched(cuda, dty
             lin.weight = own
             assert rel_l2(out, x + b.cross_attn(x, y)) <= (1e-2 if dtype == torch.bfloat16 else 2e-3), name
         assert torch.equal(b(x, y, t, None, (8, 8)), ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Nk", [1, 160, 161, 320])
+def test_few_queries_in_workgroups_of_four_waves_give_the_bits_of_eight(cuda, Nk, dtype):
+    """16 heads of 72: up to 1024 queries are at most 256 blocks of 64, four waves each; a query's result is its own, so it is that
+    of the call with more queries around it (eight waves)."""
+    H, d = 16, 72
+    g = torch.Generator().manual_seed(Nk)
+    q = (torch.randn(1, 1025, H * d, generator=g) * 1.5).to(dtype)
+    kv = torch.randn(1, Nk, 2 * H * d, generator=g).to(dtype)
+    many = ops.cross_attention16(q.to(cuda), kv.to(cuda), H)
+    assert rel_l2(many.cpu(), formula(q, kv, H)) <= 1e-2
+    for N in (1, 63, 64, 65, 130, 1024):
+        assert torch.equal(ops.cross_attention16(q[0, :N].clone()[None].to(cuda), kv.to(cuda), H), many[:, :N]), N
