@@ -65,6 +65,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
   const int fr = lane & 15, fg = lane >> 4, lr = lane >> 3;
 
   int m0, n0;
+  if (!WHOLE) asm volatile("" ::"s"(A), "s"(W), "s"(lda), "s"(ldw), "s"(M), "s"(N), "s"(K));  // (the arguments in one wait)
   gemm_tile_of(blockIdx.x, tiles_t, tiles_c, group, BM, BN, m0, n0);
 
   // ---- direct loads: rows past M / N, k pieces past K and k-tiles past the last one lie outside the resource: zeros
@@ -107,6 +108,12 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
     past_end(s);
 #pragma unroll
     for (int j = 0; j < (WHOLE || s + 1 < ST ? LOADS : L1); ++j) load1(j, s, s);
+    if (!WHOLE) {  // the next stages' offsets are computed behind these loads (all of them in front: 1 us a launch)
+#pragma unroll
+      for (int j = 0; j < NA; ++j) asm volatile("" : "+v"(va[j])::"memory");
+#pragma unroll
+      for (int j = 0; j < NWP; ++j) asm volatile("" : "+v"(vw[j])::"memory");
+    }
   }
   if (WHOLE) past_end(ST);
   // W towards the caches, an equal run of 128-byte lines per workgroup: k-tile by k-tile it comes from HBM in pieces of one line
