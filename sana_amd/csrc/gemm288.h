@@ -295,8 +295,9 @@ __global__ __launch_bounds__(512) void gemm288_kernel(const uint16_t* __restrict
     for (int i = 0; i < NT; ++i)
 #pragma unroll
       for (int j = 0; j < TM; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    // what the first phase reads: A and the first part of W of k-tile 0
-    wait_loads(C0{}, !fresh);
+    // what the first phase reads (everything requested so far, if no stores lie in between)
+    if (fresh) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else wait_loads(C0{}, true);
     half_end();
     // the MFMAs are asm statements: whatever wrote the accumulators last is done before the first of them
 #pragma unroll

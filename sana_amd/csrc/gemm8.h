@@ -389,9 +389,8 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
     for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    // what the first phase reads: W and the first half of A of k-tile 0
-    // (a workgroup's first tile waited for both of its first k-tiles here, 0.4 us; a bias in flight makes the wait stricter)
-    if (fresh) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+    // what the first phase reads (everything requested so far, if no stores lie in between)
+    if (fresh) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS + STORES) : "memory");
     half_end();
     // the MFMAs are asm statements: whatever wrote the accumulators last is done before the first of them
