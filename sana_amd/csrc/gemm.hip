@@ -845,7 +845,8 @@ struct Tile16 {
   double fixed, lone, full;
   bool one_round = false;  // beyond one round of workgroups, every round is charged in full
   double halved = 0;       // > 0: k-tile where there are at most kHalvedTiles of them, in two workgroups each; a fit of its own:
-  double halved_row = 0;   // 4 % off.  One row of tiles: every weight comes from HBM to one workgroup (64 x 2240 x 5600 27 us, split 24)
+  double halved_few = 0;   // 4 % off.  One row of tiles or a few: every weight comes from HBM to one workgroup (64 x 2240 x 5600 27 us,
+                           // split 24), or to few of them
 };
 // Fitted to 250 shapes (64 .. 32760 tokens, the eight projections of the two image widths and the text's, one block's and a
 // step's, weights cold, launches replayed from a graph: issued one by one, a launch of less than 20 us is timed by its issue):
@@ -872,7 +873,7 @@ constexpr Tile16 kTilesShort[] = {
 double cost16(const Tile16& t, int64_t M, int64_t N, int K) {
   const int64_t n = (M + t.bm - 1) / t.bm * ((N + t.bn - 1) / t.bn), rounds = n / t.resident, rest = n % t.resident;
   const double kt = (K + BK - 1) / BK;
-  if (t.halved > 0 && n <= kHalvedTiles) return t.fixed + kt * (M > t.bm ? t.halved : t.halved_row);
+  if (t.halved > 0 && n <= kHalvedTiles) return t.fixed + kt * (M > t.bm && n > kHalvedTiles / 4 ? t.halved : t.halved_few);
   if (t.one_round && n > t.resident) return (rounds + (rest ? 1 : 0)) * (kt * t.full + t.fixed);
   double us = t.fixed + rounds * (kt * t.full + 0.5 * t.fixed);
   if (rest)
