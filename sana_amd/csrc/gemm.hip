@@ -852,7 +852,7 @@ struct Tile16 {
 // step's, weights cold, launches replayed from a graph: issued one by one, a launch of less than 20 us is timed by its issue):
 // 7 - 14 % off each, the choice 0.3 % from the best tile on the mean, more than 6 % in two shapes (9 and 7 %).  In a second round
 // the small tiles were never more than 2 % ahead, and 300 x 17920 x 2240 is 48.7 us in 128 x 128 and 40.4 in 256 x 192: hence
-// one_round.  us, the tile chosen before / now, both timed so: 256 x 1152 x 2880 14.9 / 13.8, 1024 x 2240 x 2240 24.3 / 19.0,
+// one_round.  us, the tile chosen before / now, both timed so: 256 x 1152 x 2880 14.9 / 10.3 (halved), 1024 x 2240 x 2240 24.3 / 19.0,
 // 1560 x 2304 x 1152 16.1 / 12.6, 2048 x 1152 x 2880 28.7 / 22.1, 4096 x 1152 x 1152 20.4 / 17.0, 4096 x 1152 x 2880
 // 38.6 / 30.5, 2916 x 2240 x 2240 33.0 / 32.1.
 constexpr Tile16 kTiles16[] = {

@@ -43,8 +43,8 @@ __device__ __forceinline__ void gr_each(F&& f, std::integer_sequence<int, I...>)
 // halves.  Weights that come from HBM double the time of a k-tile without the prefetch (2048 x 1152 x 2880 in 128 x 128: 27.4 us,
 // with it 21.9, from the caches 19.9); on weights that the caches hold it costs 0.5 us.  From about 200 workgroups on the clock gives
 // way (2.4 GHz -> 1.8 - 2.1) and a denser loop gains little.  us, in a gated GEMM, the kernels before / now: 256 x 1152 x 2880
-// 14.9 / 13.8, 1024 x 2240 x 2240 24.3 / 19.0, 2048 x 1152 x 1152 15.0 / 12.3, 2048 x 1152 x 2880 28.7 / 22.1, 4096 x 1152 x 2880
-// 38.6 / 30.5.
+// 14.9 / 10.3 (halved tiles, gemm_ring.hip), 1024 x 2240 x 2240 24.3 / 19.0, 2048 x 1152 x 1152 15.0 / 11.9, 2048 x 1152 x 2880
+// 28.7 / 22.1, 4096 x 1152 x 2880 38.6 / 30.5.  Slower: 150 .. 200 x 3456 x 1152 7.5 / 8.2 (the prefetch is 0.4 of it).
 template <int WM, int WN, int TM, int TN, int ST, bool WHOLE, int EPI, typename T>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
                                                                  const EpiArgs ep, uint16_t* __restrict__ C, int M, int N,
