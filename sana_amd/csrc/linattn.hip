@@ -1342,6 +1342,7 @@ extern "C" __attribute__((visibility("default"))) int sana_hip_linattn(
   if (!one_launch(B, N, h, io_dtype)) {
     const size_t at = state_bytes(B, h);
     if (!scratch || scratch_bytes < sana_hip_linattn_scratch_bytes(B, N, h, d, io_dtype)) return SANA_ERR_WORKSPACE;
+    if (!aligned16(scratch)) return SANA_ERR_ALIGN;
     float* state = static_cast<float*>(scratch);
     const StatePlan pl = plan_state(B, h, 1, N, io_dtype);
     if (io_dtype == SANA_DT_F32 && N <= WHOLE_TOKENS && pl.nsplit > 1 && pl.nsplit <= 16 && heads <= (1 << 20)) {

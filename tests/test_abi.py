@@ -66,6 +66,19 @@ def test_argument_validation_needs_no_gpu():
     assert lib.sana_hip_tconv_residual(16, 16, 32, 64, 64, 3, 16, 80, None, 64, 192, 1 << 23, None) == -2   # 32-bit offsets
 
 
+@pytest.mark.parametrize("dtype,N", [(0, 257), (0, 1024), (0, 1025), (1, 1025), (2, 4096)])
+def test_one_call_attention_refuses_misaligned_scratch(dtype, N):
+    """Nothing is launched on scratch that the kernels' 16-byte accesses do not fit, whichever launches the sizes select."""
+    lib, h, C = _lib.load(), 5, 160
+    need = lib.sana_hip_linattn_scratch_bytes(1, N, h, 32, dtype)
+    assert need > 0
+    call = lambda scratch, size: lib.sana_hip_linattn(16, 16, 16, 16, scratch, size, 1, N, h, 32, N * C, C, N * C, C, N * C, C,
+                                                      1e-15, dtype, None)
+    for off in (2, 4, 8, 12):
+        assert call(4096 + off, need) == -3
+    assert call(4096, need - 1) == -4 and call(None, need) == -4
+
+
 def test_workspace_query():
     lib = _lib.load()
     # 1.6B @ 16384 tokens: 70 heads -> splits of the token axis need partial states
