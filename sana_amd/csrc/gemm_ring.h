@@ -121,6 +121,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
   // and of more k-tiles than the ring requests by itself.)
   uint32_t pf[WHOLE ? PF : 1];
   if (WHOLE) {
+    // (the waits count these loads as younger than the ring's: none of them moves in front of one)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
     const bool dense = ldw == K && (int64_t)N * K < ((int64_t)1 << 30) && KT > 2 * ST;
     const uint32_t bytes = dense ? (uint32_t)N * (uint32_t)K * 2u : 0u, run = (((bytes + 127) >> 7) + gridDim.x - 1) / gridDim.x;
     const __amdgpu_buffer_rsrc_t rsrc_all = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(W), 0, (int)bytes, 0x00020000);
