@@ -30,7 +30,7 @@ __device__ __forceinline__ void gr_each(F&& f, std::integer_sequence<int, I...>)
 // LDS: ST stages of a k-tile of 64 ([A rows | W rows], 128 bytes a row, the 16-byte piece index XORed with (row / 2) % 8),
 // filled by direct loads (1 KB = 8 rows per wave and instruction; swizzle and weight row order are applied to the global
 // address).  Between ST - 2 and ST - 1 k-tiles are in flight all the time.  Outputs sum their products in k order, as in all
-// GEMMs of this library.  Two loops:
+// GEMMs of this library.  Two loops (which of them runs: gemm_ring.hip):
 //  * WHOLE: a wave holds the fragments of two whole k-tiles: a pass multiplies one, reads the next and requests k-tile kt + ST
 //    into the stage that the pass before has emptied; the one barrier at its end says both that every wave has read stage
 //    kt + 1 and that k-tile kt + 2 has landed.
@@ -39,17 +39,19 @@ __device__ __forceinline__ void gr_each(F&& f, std::integer_sequence<int, I...>)
 //
 // What bounds it.  Few workgroups: latency -- 1.0 - 1.5 us to the first k-tile, then the loop's waits: a k-tile of 128 x 128 takes
 // 512 cycles of MFMAs, 512 of direct loads (64 bytes a cycle into LDS; LDS reads run at 254) and 660 in rounds of the ring,
-// where the half-k-tile loop needs 753; 256 x 128 1024 and 1137, in 4 x 2 waves, against 1455 of the many-token kernel's alternating
-// halves.  Weights that come from HBM double the time of a k-tile without the prefetch (2048 x 1152 x 2880 in 128 x 128: 27.4 us,
-// with it 21.9, from the caches 19.9); on weights that the caches hold it costs 0.5 us.  From about 200 workgroups on the clock gives
-// way (2.4 GHz -> 1.8 - 2.1) and a denser loop gains little.  us, in a gated GEMM, the kernels before / now: 256 x 1152 x 2880
-// 14.9 / 10.3 (halved tiles, gemm_ring.hip), 1024 x 2240 x 2240 24.3 / 19.0, 2048 x 1152 x 1152 15.0 / 11.9, 2048 x 1152 x 2880
-// 28.7 / 22.1, 4096 x 1152 x 2880 38.6 / 30.5.  Slower: 150 .. 200 x 3456 x 1152 7.5 / 8.2 (the prefetch is 0.4 of it).
+// where the half-k-tile loop needs 753.  Weights that come from HBM double the time of a k-tile without the prefetch where several
+// token tiles read them (2048 x 1152 x 2880 in 128 x 128: 27.4 us, with it 21.9, from the caches 19.9); on weights that the caches
+// hold it costs 0.5 us.  From about 200 workgroups on the clock gives way (2.4 GHz -> 1.8 - 2.1) and a denser loop gains little.
+// A branch in front of the first load costs a launch 0.3 us: a row is compared with BN only where rows are padded.  us, weights
+// cold, the kernels before the whole k-tiles / now: 256 x 1152 x 2880 15.3 / 10.4 (halved tiles, gemm_ring.hip), 1024 x 2240 x 2240
+// 23.7 / 18.5, 2048 x 1152 x 2880 28.7 / 21.8, 200 x 3456 x 1152 6.8 / 6.9; slower: 288 x 6720 x 2240 19.5 / 20.6, 150 x 11200 x 2240
+// 21.0 / 22.2 (96 x 128 instead of 128 x 128: a last token tile of few rows, which the plan's tile times do not know), 1260 x 5760 x
+// 1152 21.1 / 21.9 (256 x 128).
 template <int WM, int WN, int TM, int TN, int ST, bool WHOLE, int EPI, typename T>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
                                                                  const EpiArgs ep, uint16_t* __restrict__ C, int M, int N,
                                                                  int K, int64_t lda, int64_t ldw, int64_t ldc, int tiles_t,
-                                                                 int tiles_c, int group) {
+                                                                 int tiles_c, int group, uint32_t prefetch) {
   constexpr int NW = WM * WN, BM = 16 * TM * WM, BN = 16 * TN * WN;
   // load instructions per wave and k-tile (rows past the tile's, where its rows are no whole number of them, read as zeros)
   constexpr int NA = (BM / 8 + NW - 1) / NW, NWP = (BN / 8 + NW - 1) / NW, LOADS = NA + NWP;
@@ -65,7 +67,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
   const int fr = lane & 15, fg = lane >> 4, lr = lane >> 3;
 
   int m0, n0;
-  if (!WHOLE) asm volatile("" ::"s"(A), "s"(W), "s"(lda), "s"(ldw), "s"(M), "s"(N), "s"(K));  // (the arguments in one wait)
+  if (!WHOLE) asm volatile("" ::"s"(A), "s"(W), "s"(lda), "s"(ldw), "s"(M), "s"(N), "s"(K), "s"(tiles_t), "s"(tiles_c), "s"(group));  // (the arguments in one wait)
   gemm_tile_of(blockIdx.x, tiles_t, tiles_c, group, BM, BN, m0, n0);
 
   // ---- direct loads: rows past M / N, k pieces past K and k-tiles past the last one lie outside the resource: zeros
@@ -87,9 +89,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
   for (int j = 0; j < NWP; ++j) {
     const int row = 8 * (wave + NW * j) + lr, l = row % (16 * TN), i = l >> 4, g = (l >> 2) & 3;
     const int chan = 32 * (i >> 1) + 8 * g + 4 * (i & 1) + (l & 3);
-    vw[j] = row < BN ? ((uint32_t)(row - l + chan) * (uint32_t)ldw + 8 * piece) * 2 : kOut;
+    vw[j] = BN % (8 * NW) == 0 || row < BN ? ((uint32_t)(row - l + chan) * (uint32_t)ldw + 8 * piece) * 2 : kOut;
   }
   auto past_end = [&](int kl) {  // in front of the loads of k-tile kl (idempotent)
+    if (!WHOLE && __builtin_expect(kl < KT - 1, 1)) return;
     const uint32_t x = kl >= KT ? kOut : kl == KT - 1 ? tail_mask : 0u;
 #pragma unroll
     for (int j = 0; j < NA; ++j) va[j] |= x;
@@ -116,17 +119,16 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
     }
   }
   if (WHOLE) past_end(ST);
-  // W towards the caches, an equal run of 128-byte lines per workgroup: k-tile by k-tile it comes from HBM in pieces of one line
-  // a row, each with a row access of its own and a latency that ST - 1 k-tiles do not cover.  (Dense weights of less than 2 GB
-  // and of more k-tiles than the ring requests by itself.)
+  // W's first `prefetch` bytes (dense: all of it; or none) towards the caches, an equal run of 128-byte lines per workgroup: k-tile by
+  // k-tile it comes from HBM in pieces of one line a row, each with a row access of its own and a latency that ST - 1 k-tiles do
+  // not cover.
   uint32_t pf[WHOLE ? PF : 1];
   if (WHOLE) {
     // (the waits count these loads as younger than the ring's: none of them moves in front of one)
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    const bool dense = ldw == K && (int64_t)N * K < ((int64_t)1 << 30) && KT > 2 * ST;
-    const uint32_t bytes = dense ? (uint32_t)N * (uint32_t)K * 2u : 0u, run = (((bytes + 127) >> 7) + gridDim.x - 1) / gridDim.x;
-    const __amdgpu_buffer_rsrc_t rsrc_all = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(W), 0, (int)bytes, 0x00020000);
+    const uint32_t run = (((prefetch + 127) >> 7) + gridDim.x - 1) / gridDim.x;
+    const __amdgpu_buffer_rsrc_t rsrc_all = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(W), 0, (int)prefetch, 0x00020000);
 #pragma unroll
     for (int p = 0; p < PF; ++p) {
       const uint32_t i = p * 64 * NW + threadIdx.x;
@@ -155,7 +157,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
       const int col = ((4 * ks + fg) ^ key) << 4;
       ra[s][ks] = lds0 + s * STAGE + (16 * TM * wm + fr) * 128 + col;
       rw[s][ks] = lds0 + s * STAGE + W_OFF + (16 * TN * wn + fr) * 128 + col;
-      gr_here(ra[s][ks]), gr_here(rw[s][ks]);
+      if (WHOLE) gr_here(ra[s][ks]), gr_here(rw[s][ks]);
     }
   constexpr int KS = WHOLE ? 2 : 1;    // k-steps of a fragment set
   u32x4_t fa[2][KS][TM], fb[2][KS][TN];
