@@ -929,11 +929,23 @@ Plan16 plan16(int M, int N, int K) {
 // Split over k, or not: the split GEMM against the best unsplit one (16-bit and int8 weights decide alike, so that they
 // keep giving the same bits).  Time of the split one: fitted to 49 shapes, 4 % off.  The unsplit tiles' fit is 3 - 13 % low at
 // the K of 5600 where it is taken (their weights come from HBM for longer than the prefetch reaches): 1024 x 2240 x 5600 is 46 us
-// either way, 256 x 2240 x 5600 27 split and 34 not, 144 x 2240 x 5600 27 and 20 (halved tiles).
+// either way, 256 x 2240 x 5600 27 split and 34 not.
+// A split GEMM adds up short chains, so that its fp32 sums are closer to the 64-bit ones than those of one chain: 2240 x 5600, rms error
+// 1.0e-7 of the result in eight ranges, 2.4e-7 in one.  Precision is not given up for time: where the split was the faster one
+// against the tiles as they once were (kSplitRivals, their times then), it stays, though some tiles have become faster since
+// (144 x 2240 x 5600: 27 us split, 18 not; 400 x 2240 x 5600 31 and 25).
+constexpr Tile16 kSplitRivals[] = {
+    {256, 128, 256, 32, 256, 3.8, 0.73, 0.85}, {256, 192, 256, 32, 256, 5.7, 0.86, 1.17}, {256, 256, 256, 32, 256, 6.1, 1.12, 1.37},
+    {64, 64, 512, 64, 512, 2.1, 0.255, 0.466}, {64, 128, 256, 32, 256, 2.0, 0.42, 0.42},  {128, 128, 256, 32, 256, 2.4, 0.50, 0.59},
+    {128, 160, 256, 32, 256, 4.2, 0.58, 0.68},
+};
 bool split_pays(const GemmPlan& pl, int M, int N, int K) {
   if (pl.S <= 1) return false;
   const int kt = (K + BK - 1) / BK;
-  return 9.4 + 1.12 * ((kt + pl.S - 1) / pl.S) + 0.139e-6 * pl.S * M * N * 8 < 1.04 * plan16(M, N, K).us;
+  const double us = 9.4 + 1.12 * ((kt + pl.S - 1) / pl.S) + 0.139e-6 * pl.S * M * N * 8;
+  double rival = 1e30;
+  for (const Tile16& t : kSplitRivals) rival = std::min(rival, cost16(t, M, N, K));
+  return us < 0.97 * rival || us < 1.04 * plan16(M, N, K).us;
 }
 
 // The pipelined kernel: split over k into pl.S ranges (ws holds the partial planes), or, int8 weights, unsplit (ws null).

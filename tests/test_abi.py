@@ -127,6 +127,17 @@ def test_gemm_plan_query():
     assert lib.sana_hip_gemm_plan(8, 12, 8, plan) == -2 and lib.sana_hip_gemm_plan(8, 8, 12, plan) == -2
 
 
+@pytest.mark.parametrize("M,ranges", [(65, 8), (116, 8), (129, 8), (144, 8), (187, 8), (390, 8), (400, 8), (448, 8), (570, 7), (896, 5),
+                                      (1226, 4), (1280, 4), (2305, 2), (2560, 2)])
+def test_long_k_stays_split_where_a_small_tile_is_faster(M, ranges):
+    """The point conv of the 2240-wide model, both kinds of weights: sums over ranges of k are closer to the 64-bit ones than one
+    chain of 5600 products, and a faster tile is no reason to give that up."""
+    lib, plan = _lib.load(), (ctypes.c_int * 4)()
+    assert lib.sana_hip_gemm_plan(M, 2240, 5600, plan) == 0
+    assert plan[3] == ranges and lib.sana_hip_gemm_workspace_bytes(M, 2240, 5600) == ranges * M * 2240 * 4
+    assert lib.sana_hip_gemm_w8_expand(M, 2240, 5600) == 0
+
+
 @pytest.mark.parametrize("B,N,C,hidden", [(16, 4096, 1152, 2880), (2, 16384, 2240, 5600), (1, 256, 288, 720)])
 def test_block_scratch_is_no_more_than_the_calls_one_by_one_hold(B, N, C, hidden):
     """fp16 takes the block call at every size: its scratch stays within what the composition holds at its peak beside
