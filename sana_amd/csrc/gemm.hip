@@ -838,6 +838,7 @@ size_t split_bytes(const GemmPlan& pl, int M, int N) { return pl.S > 1 ? (size_t
 // Time of an unsplit 16-bit GEMM in a given tile, us: ceil(K / 64) k-tiles per round of workgroups, at a rate per k-tile that
 // grows from `lone` (lone_to workgroups or fewer in the round) to `full` (full_from or more: the weights come from HBM, the
 // matrix pipes share a power budget), plus launch, first loads and epilogue.
+constexpr int kHalvedTiles = 128;  // up to so many tiles of 64 x 64 run as two workgroups of 32 channels each
 struct Tile16 {
   int bm, bn;    // tokens, channels; 256 x 192 and 256 x 256: gemm8_kernel, 288 channels: gemm288_kernel; else gemm_ring_kernel
   int resident;  // workgroups on the chip at a time
@@ -902,6 +903,7 @@ bool short_takes_288(int M, int N, int K, double others_us) {  // others_us: by 
 constexpr int kShortK = 1024;
 struct Plan16 {
   const Tile16* tile;
+  int bn;      // channels of a workgroup: the tile's, or 32 (halved 64 x 64)
   int n_wide;  // > 0: the first n_wide channels in 256 x 256 tiles, the rest in 256 x 192 ones, two launches
   double us;
 };
@@ -909,7 +911,7 @@ struct Plan16 {
 // are 1.7 rounds, 15 x 16 and 15 x 16 tiles of the mix two that are 94 % full) by more than what the fit tells apart
 template <size_t TILES>
 Plan16 cheapest16(const Tile16 (&tiles)[TILES], const Tile16& t256, const Tile16& t192, double mix_below, int M, int N, int K) {
-  Plan16 p = {&tiles[0], 0, 1e30};
+  Plan16 p = {&tiles[0], 0, 0, 1e30};
   for (const Tile16& t : tiles) {
     const double us = cost16(t, M, N, K);
     if (us < p.us) p.tile = &t, p.us = us;
@@ -919,12 +921,14 @@ Plan16 cheapest16(const Tile16 (&tiles)[TILES], const Tile16& t256, const Tile16
     const double us = cost16(t256, M, a, K) + cost16(t192, M, N - a, K);
     if (us < mix_below * single && us < p.us) p.n_wide = a, p.us = us;
   }
+  const bool halved = p.tile->bm == 64 && p.tile->bn == 64 && (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= kHalvedTiles;
+  p.bn = p.n_wide ? 256 : halved ? 32 : p.tile->bn;
   return p;
 }
 Plan16 plan16(int M, int N, int K) {
   if (K >= kShortK) return cheapest16(kTiles16, kTiles16[kTile256], kTiles16[kTile192], 0.992, M, N, K);
   const Plan16 p = cheapest16(kTilesShort, kTilesShort[2], kTilesShort[1], 0.98, M, N, K);
-  return short_takes_288(M, N, K, p.us) ? Plan16{&kShort288, 0, cost16(kShort288, M, N, K)} : p;
+  return short_takes_288(M, N, K, p.us) ? Plan16{&kShort288, 288, 0, cost16(kShort288, M, N, K)} : p;
 }
 // Split over k, or not: the split GEMM against the best unsplit one (16-bit and int8 weights decide alike, so that they
 // keep giving the same bits).  Time of the split one: fitted to 49 shapes, 4 % off.  The unsplit tiles' fit is 3 - 13 % low at
@@ -1043,7 +1047,7 @@ int launch(const void* A, const void* W, const float* scale, const EpiArgs& ep, 
     if (p.tile->bn == 288) return gemm8_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, 4, nullptr, s);
     if (p.tile->bm == 256 && p.tile->bn >= 192)
       return gemm8_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, p.tile->bn / 64, nullptr, s);
-    return gemm_ring_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, p.tile->bm, p.tile->bn, s);
+    return gemm_ring_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, p.tile->bm, p.bn, s);
   } else {
     const bool pipelined = K % 32 == 0 && K >= 64;
     const int KT = (K + BK - 1) / BK;
@@ -1169,7 +1173,7 @@ SANA_API int sana_hip_gemm_plan(int M, int N, int K, int plan[4]) {
   const GemmPlan split = plan_gemm(M, N, K, false);
   const Plan16 p = plan16(M, N, K);
   const bool cut = split_pays(split, M, N, K);
-  plan[0] = cut ? BT : p.tile->bm, plan[1] = cut ? 64 * pick_ni(M, N) : p.n_wide ? 256 : p.tile->bn;
+  plan[0] = cut ? BT : p.tile->bm, plan[1] = cut ? 64 * pick_ni(M, N) : p.bn;
   plan[2] = cut ? 0 : p.n_wide, plan[3] = cut ? split.S : 1;
   return SANA_OK;
 }

@@ -55,9 +55,8 @@ int gemm288_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint
                    int64_t ldw, int64_t ldc, int epilogue, bool f16, const Taps* taps, hipStream_t s);
 
 // The GEMM for few tokens (gemm_ring.hip): the same operands and epilogues up to SANA_EPI_GATE_RES (gate not null), in tiles
-// of bm tokens x bn channels: 64 x 64 (up to kHalvedTiles of them as two workgroups of 32 channels each), 64 x 128, 96 x 128,
+// of bm tokens x bn channels: 64 x 32, 64 x 64, 64 x 128, 96 x 128,
 // 128 x 128, 128 x 160, 192 x 128 or 256 x 128.
-constexpr int kHalvedTiles = 128;
 int gemm_ring_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
                      int64_t ldw, int64_t ldc, int epilogue, bool f16, int bm, int bn, hipStream_t s);
 

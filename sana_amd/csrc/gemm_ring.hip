@@ -76,12 +76,11 @@ int gemm_ring_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, ui
   if (bm == 16 * TM * WM && bn == 16 * TN * WN)                                                                        \
   return f16 ? launch_ring<WM, WN, TM, TN, ST, AHEAD, HALF, F16>(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, s)      \
              : launch_ring<WM, WN, TM, TN, ST, AHEAD, HALF, BF16>(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, s)
-  // 64 x 64 where at most half the compute units would have a tile: each in two workgroups of 32 channels.  A compute unit takes 70 - 75
+  // 64 x 32: the plan's choice where 64 x 64 gives at most half the compute units a tile.  A compute unit takes 70 - 75
   // bytes/ns of such operands, whatever the ring's depth (8 and 10 stages: the same per k-tile, 1.1 and 1.9 us more in front of the
   // first), so a k-tile takes as long as its bytes: 12 KB 0.16 us, 16 KB 0.22.  us: 256 x 1152 x 1152 7.4 -> 6.0, x 2880
   // 13.4 -> 10.3, 144 x 2240 x 2240 11.7 -> 9.1; 32 tokens x 64 channels 6.2, 10.5, 9.6.  From 129 tiles on two workgroups would
   // share a compute unit: 512 x 1152 x 1152 7.4 in 64 x 64, 8.7 in halves.
-  if (bm == 64 && bn == 64 && ((M + 63) / 64) * (int64_t)((N + 63) / 64) <= kHalvedTiles) bn = 32;
   SANA_RING(4, 1, 1, 2, 6, true, false);  // 64 x 32, 72 KB
   SANA_RING(2, 2, 2, 2, 5, true, true);   // 64 x 64, 80 KB: two workgroups per compute unit
   SANA_RING(2, 4, 2, 2, 6, true, true);   // 64 x 128

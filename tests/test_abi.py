@@ -117,7 +117,8 @@ def test_gemm_plan_query():
     def of(*shape):
         assert lib.sana_hip_gemm_plan(*shape, plan) == 0
         return tuple(plan)
-    assert of(256, 1152, 1152) == (64, 64, 0, 1)
+    assert of(256, 1152, 1152) == (64, 32, 0, 1)                   # 4 x 18 tiles of 64 x 64, two workgroups each
+    assert of(512, 1152, 1152) == (64, 64, 0, 1)                   # 8 x 18
     assert of(16384, 11200, 2240) == (256, 256, 0, 1)
     assert of(4096, 6720, 2240) == (256, 256, 3840, 1)              # two widths, two launches
     assert of(1024, 2240, 5600) == (256, 192, 0, 5)                 # five ranges of k

@@ -15,7 +15,7 @@ KS = [1032, 1080, 1152, 1216, 1288, 1344, 1408, 1472, 1536, 1600, 1664, 1720]
 # (64 x 64: up to 128 tiles as two workgroups of 32 channels each: 4 x 17 tiles, 3 x 42; whole: 4 x 33)
 # Dense weights: with the weights requested ahead, in the loop over whole k-tiles, where that pays (the second shape of a tile, and
 # the only one of 64 x 128), else in the other loop, as rows of W apart always are.
-TILES = [((64, 64), (195, 1048)), ((64, 64), (195, 2072)), ((64, 64), (465, 1048)), ((64, 64), (192, 2688)), ((64, 64), (129, 1048)),
+TILES = [((64, 32), (195, 1048)), ((64, 64), (195, 2072)), ((64, 64), (465, 1048)), ((64, 32), (192, 2688)), ((64, 32), (129, 1048)),
          ((64, 128), (414, 2336)), ((96, 128), (1281, 2280)), ((96, 128), (1026, 2280)), ((128, 128), (1332, 2496)),
          ((128, 128), (2721, 1048)), ((128, 160), (2349, 1800)), ((192, 128), (1872, 2992)), ((192, 128), (3969, 1176)),
          ((256, 128), (1935, 2968))]

@@ -21,7 +21,8 @@ def _ints(*shape, lo=-3, hi=3, seed=0, dtype=torch.bfloat16):
 # of an odd and an even number, with tails of 8, 32 and 56; ragged rows and channels; one row; more tiles than workgroups
 # that are resident (persistent workgroups then take several).  128 x 160 is not chosen for short k or for many tiles.
 TILES = {
-    (64, 64): [(1, 8, 8), (65, 72, 40), (200, 264, 184), (33, 16, 320), (12300, 264, 72)],
+    (64, 32): [(1, 8, 8), (65, 72, 40), (200, 264, 184), (33, 16, 320)],
+    (64, 64): [(12300, 264, 72)],
     (64, 128): [(206, 3456, 8), (700, 2240, 328), (1500, 1160, 1152), (65, 6728, 40), (515, 6728, 64), (515, 6728, 136)],
     (128, 128): [(1030, 8200, 8), (1030, 8200, 64), (3679, 536, 8), (999, 2248, 392), (2049, 1160, 120), (1030, 6728, 40),
                  (1030, 6728, 184), (4100, 2240, 64)],
@@ -35,7 +36,7 @@ TILES = {
 }
 # the same for the gated residual, (batch entries, tokens of each, channels, k): boundaries between them inside a tile
 GATED = {
-    (64, 64): [(7, 9, 72, 40), (3, 67, 264, 184)],
+    (64, 32): [(7, 9, 72, 40), (3, 67, 264, 184)],
     (64, 128): [(5, 140, 2240, 328), (3, 172, 6728, 8)],
     (128, 128): [(9, 111, 2248, 392), (41, 100, 2240, 64), (5, 206, 6728, 40)],
     (128, 160): [(3, 667, 2232, 1032), (3, 1707, 776, 136)],
