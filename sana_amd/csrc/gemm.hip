@@ -840,7 +840,8 @@ size_t split_bytes(const GemmPlan& pl, int M, int N) { return pl.S > 1 ? (size_t
 // matrix pipes share a power budget), plus launch, first loads and epilogue.
 constexpr int kHalvedTiles = 128;  // up to so many tiles of 64 x 64 run as two workgroups of 32 channels each
 struct Tile16 {
-  int bm, bn;    // tokens, channels; 256 x 192 and 256 x 256: gemm8_kernel, 288 channels: gemm288_kernel; else gemm_ring_kernel
+  int bm, bn;    // tokens, channels; 256 x 192 and 256 x 256 (256 x 128 below kShortK): gemm8_kernel, 288 channels: gemm288_kernel; else
+                 // gemm_ring_kernel
   int resident;  // workgroups on the chip at a time
   int lone_to, full_from;
   double fixed, lone, full;
@@ -864,8 +865,11 @@ constexpr Tile16 kTiles16[] = {
     {256, 256, 256, 32, 256, 5.3, 0.999, 1.404},       {256, 288, 256, 32, 256, 9.5, 0.955, 1.603},
 };
 constexpr int kTile192 = 7, kTile256 = 8, kTile288 = 9;
-// K below 1024: the rings fill and drain for much of the loop, and the constants above do not hold.  These are a fit of their own
-// (128 shapes), 8 - 13 % off.
+// K below 1024.  These are the times that the tiles had in GEMMs of K = 1152 .. 5600 before the loop over whole k-tiles; at such K
+// no other loop runs, and 256 x 128 is gemm8_kernel's there.  As times they are up to 30 % off (epilogues and the fill of the rings are most of
+// a launch), as a choice they serve: of 560 shapes (64 .. 24576 tokens, 320 .. 6144 channels, K 64 .. 960, the ten tiles forced in turn)
+// 2.7 % from the best tile on the mean, more than 6 % in 91 (sizes just past a round of 256 x 192 or 256 x 128, mostly).  Constants fitted to
+// those shapes come to 2.0 %.
 constexpr Tile16 kTilesShort[] = {
     {256, 128, 256, 32, 256, 3.8, 0.73, 0.85}, {256, 192, 256, 32, 256, 5.7, 0.86, 1.17}, {256, 256, 256, 32, 256, 6.1, 1.12, 1.37},
     {64, 64, 512, 64, 512, 2.1, 0.255, 0.466}, {64, 128, 256, 32, 256, 2.0, 0.42, 0.42},  {128, 128, 256, 32, 256, 2.4, 0.50, 0.59},
@@ -1045,7 +1049,9 @@ int launch(const void* A, const void* W, const float* scale, const EpiArgs& ep, 
     if (p.tile->bn == 288 && ldw < kMaxStride288 && aligned16(ep.bias))  // (its bias row is loaded straight to LDS, 16 bytes a lane)
       return gemm288_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, nullptr, s);
     if (p.tile->bn == 288) return gemm8_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, 4, nullptr, s);
-    if (p.tile->bm == 256 && p.tile->bn >= 192)
+    // 256 x 128 at short k: the persistent kernel, whose next tile loads behind this one's epilogue.  us, ring / here: 16384 x 768 x 64
+    // 17.3 / 13.5, 2048 x 3072 x 512 13.2 / 12.5, 16384 x 1536 x 512 36.6 / 33.5, 8192 x 768 x 768 17.4 / 16.4; from K = 1024 on ties or worse
+    if (p.tile->bm == 256 && (p.tile->bn >= 192 || K < kShortK))
       return gemm8_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, p.tile->bn / 64, nullptr, s);
     return gemm_ring_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, p.tile->bm, p.bn, s);
   } else {

@@ -455,7 +455,7 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
     // (asm LDS accesses: see the fragment reads.)
     constexpr int PPR = 2 * NB;                       // 16-byte pieces of a row
     auto out_at = [&](int row, int pc) -> uint32_t {  // swizzled: conflict-free both ways (NB = 3: two-way)
-      const int k = NB == 4 ? (row >> 1) & 7 : 0;
+      const int k = NB == 4 ? (row >> 1) & 7 : NB == 2 ? (row >> 2) & 3 : 0;
       return row * OUT_ROW + ((pc ^ k) << 4);
     };
     const uint32_t out0 = lds0 + W_BASE + 2 * W_STAGE + wave * OUT_BYTES;

@@ -16,7 +16,7 @@ int launch_nb(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t*
   hipLaunchKernelGGL((gemm8_kernel<EPI, NB, TAPS, T>), grid, block, 0, s, a, w, ep, c, M, N, K, lda, ldw, ldc, (int)tiles_t, \
                      (int)tiles_c, TP)
   if (taps) {
-    if constexpr (!is_f16<T>) {
+    if constexpr (NB != 2 && !is_f16<T>) {
       if (epilogue != SANA_EPI_GATE_RES) return SANA_ERR_ARG;
       if (taps->zero_last) SANA_LAUNCH8(SANA_EPI_GATE_RES, 2, *taps);
       else SANA_LAUNCH8(SANA_EPI_GATE_RES, 1, *taps);
@@ -50,6 +50,7 @@ int gemm8_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16
   return f16 ? launch_nb<NB, F16>(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, taps, s)                             \
              : launch_nb<NB, BF16>(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, taps, s)
   switch (nb) {
+    case 2: SANA_NB8(2);
     case 3: SANA_NB8(3);
     case 4: SANA_NB8(4);
     default: return SANA_ERR_ARG;

@@ -43,7 +43,7 @@ struct Taps {
   const unsigned char* zero_last;
 };
 
-// The many-token GEMM (gemm8.hip): C = epilogue(A . W^T) in 256-token x 64*nb-channel tiles, nb = 3 or 4; operands
+// The many-token GEMM (gemm8.hip): C = epilogue(A . W^T) in 256-token x 64*nb-channel tiles, nb = 2, 3 or 4; operands
 // 16-bit (f16 or bf16), K % 8 == 0; epilogue SANA_EPI_NONE .. SANA_EPI_GATE_RES, or SANA_EPI_QKV_STATE with nb = 4
 // (bf16); taps (bf16, SANA_EPI_GATE_RES, nb = 3 or 4) or null.  Arguments are checked by the caller.
 int gemm8_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
