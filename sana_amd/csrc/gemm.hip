@@ -940,19 +940,14 @@ Plan16 plan16(int M, int N, int K) {
 // either way, 256 x 2240 x 5600 27 split and 34 not.
 // A split GEMM adds up short chains, so that its fp32 sums are closer to the 64-bit ones than those of one chain: 2240 x 5600, rms error
 // 1.0e-7 of the result in eight ranges, 2.4e-7 in one.  Precision is not given up for time: where the split was the faster one
-// against the tiles as they once were (kSplitRivals, their times then), it stays, though some tiles have become faster since
+// against the tiles as they once were (kTilesShort, their times then), it stays, though some tiles have become faster since
 // (144 x 2240 x 5600: 27 us split, 18 not; 400 x 2240 x 5600 31 and 25).
-constexpr Tile16 kSplitRivals[] = {
-    {256, 128, 256, 32, 256, 3.8, 0.73, 0.85}, {256, 192, 256, 32, 256, 5.7, 0.86, 1.17}, {256, 256, 256, 32, 256, 6.1, 1.12, 1.37},
-    {64, 64, 512, 64, 512, 2.1, 0.255, 0.466}, {64, 128, 256, 32, 256, 2.0, 0.42, 0.42},  {128, 128, 256, 32, 256, 2.4, 0.50, 0.59},
-    {128, 160, 256, 32, 256, 4.2, 0.58, 0.68},
-};
 bool split_pays(const GemmPlan& pl, int M, int N, int K) {
   if (pl.S <= 1) return false;
   const int kt = (K + BK - 1) / BK;
   const double us = 9.4 + 1.12 * ((kt + pl.S - 1) / pl.S) + 0.139e-6 * pl.S * M * N * 8;
   double rival = 1e30;
-  for (const Tile16& t : kSplitRivals) rival = std::min(rival, cost16(t, M, N, K));
+  for (const Tile16& t : kTilesShort) rival = std::min(rival, cost16(t, M, N, K));
   return us < 0.97 * rival || us < 1.04 * plan16(M, N, K).us;
 }
 
@@ -1274,12 +1269,13 @@ SANA_API int sana_hip_tconv_residual(const void* X, const void* W, void* out, in
   uint16_t* o = static_cast<uint16_t*>(out);
   hipStream_t s = static_cast<hipStream_t>(stream);
   // one of the three widest tiles: the others have no taps
-  int best = kTile192;
-  for (int t : {kTile256, kTile288})
-    if ((t != kTile288 || ldw < kMaxStride288) && cost16(kTiles16[t], M, C, taps * C) < cost16(kTiles16[best], M, C, taps * C)) best = t;
-  if (best == kTile288)
-    return gemm288_launch(x, w, e, o, M, C, taps * C, ldx, ldw, ldo, SANA_EPI_GATE_RES, false, &tp, s);
-  return gemm8_launch(x, w, e, o, M, C, taps * C, ldx, ldw, ldo, SANA_EPI_GATE_RES, false, best == kTile192 ? 3 : 4, &tp, s);
+  const int k = taps * C;
+  const bool brief = k < kShortK, may288 = ldw < kMaxStride288;
+  const double us192 = cost16(brief ? kTilesShort[1] : kTiles16[kTile192], M, C, k);
+  const double us256 = cost16(brief ? kTilesShort[2] : kTiles16[kTile256], M, C, k), us = std::min(us192, us256);
+  if (may288 && (brief ? short_takes_288(M, C, k, us) : cost16(kTiles16[kTile288], M, C, k) < us))
+    return gemm288_launch(x, w, e, o, M, C, k, ldx, ldw, ldo, SANA_EPI_GATE_RES, false, &tp, s);
+  return gemm8_launch(x, w, e, o, M, C, k, ldx, ldw, ldo, SANA_EPI_GATE_RES, false, us192 < us256 ? 3 : 4, &tp, s);
 }
 
 SANA_API int sana_hip_dequant_w8(const int8_t* Wq, const float* scale, void* W, int N, int K, int64_t ldw,
