@@ -124,8 +124,8 @@ int sana_hip_linattn_apply(const void* q, const float* state, void* out,
 
 /* ---------------------------------------------------------------------------
  * Both phases in one call: one chunk, d = 32, out in the io dtype, no state returned.  Short sequences are one kernel
- * that keeps the state on the compute unit and adds it up in the order of the two calls (the same bits),
- * others the launches of the two.  k and v share strides, as in sana_hip_linattn_state; q and out as in
+ * that keeps the state on the compute unit and adds it up in the order of the two calls (the same bits), others the launches
+ * of the two, or, fp32 of up to 1024 tokens and few heads, two: the second adds up the partial states itself (the same bits).  k and v share strides, as in sana_hip_linattn_state; q and out as in
  * sana_hip_linattn_apply; out must not overlap the inputs.
  *   scratch  at least sana_hip_linattn_scratch_bytes(...) bytes, 16-byte aligned (may be NULL when that is 0)
  */

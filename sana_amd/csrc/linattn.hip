@@ -613,9 +613,9 @@ __global__ __launch_bounds__(256) void linattn_apply32_kernel(
 // 32 tokens each, the fifth takes the state's 33rd row, so that the sums are one round of loads.  The queries are requested first;
 // a workgroup then reads nsplit x 4.2 KB of partial states, four times what its queries are at 16 splits, and that takes less than
 // the third launch: bound by the latency of the two loads.  us, issued eagerly on three sets of inputs in turn, three launches / two:
-// 1024 x 36 17.4 / 14.5, 2 x 1024 x 36 20.8 / 17.7, 400 x 70 17.2 / 14.2, 4 x 1000 x 36 27.2 / 26.3 (tokens x heads).  Both launches keep
-// a head on one XCD: with its partial states read by all eight, phase 1 of the next call takes 9.1 us instead of 5.9 to write
-// them again.  Beyond 1024 tokens the partial states that are read again outweigh the launch.
+// 1024 tokens x 36 heads 15.5 / 14.2, 400 x 70 14.2 / 13.8, 2 x 1024 x 36 20.6 / 17.7.  Both launches keep a head on one XCD: with its
+// partial states read by all eight, phase 1 of the next call takes 9.1 us instead of 5.9 to write them again.  Beyond 1024 tokens, and
+// beyond the heads that sana_hip_linattn takes it for, the partial states that are read again outweigh the launch.
 // ----------------------------------------------------------------------------
 __global__ __launch_bounds__(320) void linattn_apply32_partials_kernel(
     const float* __restrict__ Q, const float* __restrict__ partial, float* __restrict__ out, int N, int h, int nsplit,
@@ -1345,7 +1345,11 @@ extern "C" __attribute__((visibility("default"))) int sana_hip_linattn(
     if (!aligned16(scratch)) return SANA_ERR_ALIGN;
     float* state = static_cast<float*>(scratch);
     const StatePlan pl = plan_state(B, h, 1, N, io_dtype);
-    if (io_dtype == SANA_DT_F32 && N <= WHOLE_TOKENS && pl.nsplit > 1 && pl.nsplit <= 16 && heads <= (1 << 20)) {
+    // Short sequences of few heads: what phase 2 reads again, N / 128 times the partial states, grows with both.  us, three launches
+    // / two, three sets of inputs in turn, and in brackets sets that come from HBM: 2 x 1024 x 36 20.6 / 17.7 (23.5 / 21.5), 4 x 640 x 36 21.5 /
+    // 18.2 (24.8 / 22.3), 4 x 512 x 36 21.1 / 17.5, 2 x 1024 x 70 26.9 / 26.2 (30.3 / 31.6), 4 x 1024 x 36 27.0 / 26.4 (30.8 / 32.0), beyond the line
+    // 4 x 900 x 70 48.3 / 52.1, 8 x 1024 x 36 52.8 / 55.1, 8 x 400 x 70 43.9 / 47.5.  Below it 4 x 400 x 70 loses too, 22.9 / 23.5.
+    if (io_dtype == SANA_DT_F32 && N <= WHOLE_TOKENS && pl.nsplit > 1 && pl.nsplit <= 16 && heads * N <= (144 << 10)) {
       float* partial = reinterpret_cast<float*>(static_cast<char*>(scratch) + at);
       hipStream_t st = static_cast<hipStream_t>(stream);
       hipLaunchKernelGGL(linattn_state32_kernel<true>, dim3(pl.nsplit * B * ((h + 3) / 4)), dim3(256), 0, st, static_cast<const float*>(k),

@@ -122,3 +122,23 @@ def test_two_launches_on_partial_states(cuda, B, N, h):
     q, k, v = (wide[:, :, i * C:(i + 1) * C] for i in range(3))
     assert _lib.load().sana_hip_linattn_scratch_bytes(B, N, h, 32, ops._dt(q)) > 0
     assert torch.equal(ops.relu_linear_attention(q, k, v, 1e-15), ops.linattn_apply(q, ops.linattn_state(k, v), 1e-15))
+
+
+@pytest.mark.parametrize("B,N,h,two", [(1, 257, 5, True), (1, 1024, 3, True), (4, 1024, 36, True), (1, 980, 150, True), (2, 300, 140, True),
+                                       (1, 1025, 3, False), (1, 1008, 150, False), (5, 1024, 54, False)])
+def test_which_launches_read_the_partial_states(cuda, B, N, h, two):
+    """The two launches leave the front of the scratch, where the reduced state would be, as it was; the launches of the two calls
+    write it.  Up to 1024 tokens and 147456 head-tokens it is two."""
+    lib, C = _lib.load(), 32 * h
+    gen = torch.Generator().manual_seed(N + h)
+    q, k, v = (torch.randn(B, N, C, generator=gen).to(cuda) for _ in range(3))
+    need = lib.sana_hip_linattn_scratch_bytes(B, N, h, 32, _lib.DT_F32)
+    state = B * h * 33 * 32
+    assert need > 4 * state                                    # a state and partial states
+    scratch, out = torch.full((need // 4,), 7.25, device=cuda), torch.empty(B, N, C, device=cuda)
+    _lib.check(lib.sana_hip_linattn(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), scratch.data_ptr(), need, B, N, h, 32,
+                                    N * C, C, N * C, C, N * C, C, 1e-15, _lib.DT_F32, torch.cuda.current_stream().cuda_stream),
+               "sana_hip_linattn")
+    assert bool((scratch[:state] == 7.25).all()) == two
+    assert not bool((scratch[-(need // 4 - state) // 2:] == 7.25).any())
+    assert torch.equal(out, ops.linattn_apply(q, ops.linattn_state(k, v), 1e-15))
