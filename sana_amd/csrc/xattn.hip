@@ -13,7 +13,7 @@
 // feeds the probabilities straight back as the column operand of out^T = V^T . P^T -- the k index of that
 // product is permuted so that the 8 values a lane needs are the ones its own accumulators hold (keys
 // 32s + 4g + {0..3} and 32s + 16 + 4g + {0..3} for lane group g), and V^T is stored in that key order.
-// Few queries (one 512 px image: 32 workgroups of one item) are bound by the staging, a chain of load latencies: the queries and all
+// Few queries (one 512 px image: 64 workgroups of one item) are bound by the staging, a chain of load latencies: the queries and all
 // of K and V are requested before the first LDS write (the queries behind the staging: 0.3 us more a launch), and V is
 // transposed four keys at a time (8-byte writes).
 // Workgroups are persistent over consecutive (batch, head, query block) items and restage K / V only when the
@@ -304,7 +304,10 @@ int cross_attention(const void* q, const void* kv, const float* key_bias, void* 
   // workgroups have a compute unit each: a unit then reads K and V from LDS for four waves.  us, 8 / 4 waves: 300 keys, 150 queries x
   // 16 heads of 72 10.6 / 9.8, 512 11.5 / 10.1, 1024 11.7 / 10.5, f16 12.6 / 10.6, 77 keys 6.9 / 6.3; in two rounds 2 x 1024 13.8 / 16.2.
   // 112 channels a head: 600 x 20 heads 13.1 / 12.7, 2 x 300 13.6 / 14.0 (the staging is more of it).
-  const bool few = d <= 96 && (int64_t)B * H * ((N + 64 * XA_QT - 1) / (64 * XA_QT)) <= 256;
+  // Nor with the keys and values of 64 heads and more, each of which two workgroups then stage instead of one: 4 x 256 x 16 heads
+  // 12.7 / 13.8, 160 keys 8.9 / 9.2, f16 13.5 / 14.0; but 77 keys 8.1 / 7.8.
+  const bool restaged = (int64_t)B * H >= 64 && N > 64 * XA_QT && Nk > (is_f16<T> ? 256 : 128);
+  const bool few = d <= 96 && !restaged && (int64_t)B * H * ((N + 64 * XA_QT - 1) / (64 * XA_QT)) <= 256;
   // key tiles of 16 that are multiplied: all 20, or 10 for up to 160 keys (tiles past Nk hold zeros and -inf)
   if (d > 96) return Nk > 160 ? SANA_XA_GO(4, 7, 8, 20) : SANA_XA_GO(4, 7, 8, 10);
   if (few) return Nk > 160 ? SANA_XA_GO(3, 6, 4, 20) : SANA_XA_GO(3, 6, 4, 10);

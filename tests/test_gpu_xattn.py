@@ -351,3 +351,17 @@ def test_few_queries_in_workgroups_of_four_waves_give_the_bits_of_eight(cuda, Nk
     assert rel_l2(many.cpu(), formula(q, kv, H)) <= 1e-2
     for N in (1, 63, 64, 65, 130, 1024):
         assert torch.equal(ops.cross_attention16(q[0, :N].clone()[None].to(cuda), kv.to(cuda), H), many[:, :N]), N
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N,Nk", [(64, 300), (65, 128), (256, 129), (200, 257)])
+def test_few_queries_of_several_batch_entries(cuda, N, Nk, dtype):
+    """Four entries of 16 heads: four waves a workgroup, or eight where each head's keys would be staged twice; either way the bits
+    of the entries one by one."""
+    H, d = 16, 72
+    g = torch.Generator().manual_seed(N + Nk)
+    q, kv = (torch.randn(4, n, c * H * d, generator=g).to(dtype).to(cuda) for n, c in ((N, 1), (Nk, 2)))
+    out = ops.cross_attention16(q, kv, H)
+    assert rel_l2(out.cpu(), formula(q.cpu(), kv.cpu(), H)) <= 1e-2
+    for b in range(4):
+        assert torch.equal(out[b:b + 1], ops.cross_attention16(q[b:b + 1].clone(), kv[b:b + 1].clone(), H)), b
