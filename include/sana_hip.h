@@ -280,13 +280,15 @@ int sana_hip_dwconv3x3_silu_gate(const void* u, const void* w, const void* bias,
  * needs (0: this shape is never split); given it, the GEMM splits where that is expected to be faster than its best
  * unsplit tiling.  With workspace NULL, misaligned or smaller than that, the GEMM
  * runs unsplit -- same result up to the fp32 summation order.  The plan depends on (M, N, K) only, so the
- * int8-weight GEMM and the gated-residual GEMM split the same way and stay bit-identical to this one.
+ * int8-weight GEMM and the gated-residual GEMM split the same way and stay bit-identical to this one.  (16-bit weights of some
+ * of these shapes run as one kernel that adds the ranges' sums up itself: the same bits, the workspace untouched.)
  */
 size_t sana_hip_gemm_workspace_bytes(int M, int N, int K);
 
 /* What a 16-bit GEMM of this shape runs as, given that workspace: plan[0], plan[1] = tokens and channels of a workgroup's
  * tile; plan[2] > 0: its first plan[2] channels run in tiles of 256 x 256, the rest in tiles of 256 x 192 (two launches);
- * plan[3] > 1: split into that many ranges of K.  A host-side query for tests and measurements. */
+ * plan[3] > 1: K in that many ranges, by the split kernel (tiles of 256 channels or 192) or within a smaller tile.  A host-side
+ * query for tests and measurements. */
 int sana_hip_gemm_plan(int M, int N, int K, int plan[4]);
 
 int sana_hip_gemm_bf16(const void* A, const void* W, const void* bias, void* C,

@@ -937,19 +937,26 @@ Plan16 plan16(int M, int N, int K) {
 // Split over k, or not: the split GEMM against the best unsplit one (16-bit and int8 weights decide alike, so that they
 // keep giving the same bits).  Time of the split one: fitted to 49 shapes, 4 % off.  The unsplit tiles' fit is 3 - 13 % low at
 // the K of 5600 where it is taken (their weights come from HBM for longer than the prefetch reaches): 1024 x 2240 x 5600 is 46 us
-// either way, 256 x 2240 x 5600 27 split and 34 not.
+// either way, 256 x 2240 x 5600 30 split and 34 not.
 // A split GEMM adds up short chains, so that its fp32 sums are closer to the 64-bit ones than those of one chain: 2240 x 5600, rms error
 // 1.0e-7 of the result in eight ranges, 2.4e-7 in one.  Precision is not given up for time: where the split was the faster one
-// against the tiles as they once were (kTilesShort, their times then), it stays, though some tiles have become faster since
-// (144 x 2240 x 5600: 27 us split, 18 not; 400 x 2240 x 5600 31 and 25).
-bool split_pays(const GemmPlan& pl, int M, int N, int K) {
-  if (pl.S <= 1) return false;
+// against the tiles as they once were (kTilesShort, their times then), k stays in ranges though some tiles have become faster since.
+// 16-bit weights then take the faster tile all the same, which adds the ranges' sums up itself, in their order, with the same bits:
+// us, split / so: 72 x 2240 x 5600 24.9 / 17.4, 144 27.6 / 18.4, 400 30.9 / 25.7, 1260 49.9 / 48.1, 2400 74.8 / 68.4.
+enum class SplitWay { no, split, ranges };  // ranges: of a ring tile (16-bit weights; int8 ones are split)
+SplitWay split_way(const GemmPlan& pl, int M, int N, int K) {
+  if (pl.S <= 1) return SplitWay::no;
   const int kt = (K + BK - 1) / BK;
   const double us = 9.4 + 1.12 * ((kt + pl.S - 1) / pl.S) + 0.139e-6 * pl.S * M * N * 8;
+  const Plan16 p = plan16(M, N, K);
+  if (us < 1.04 * p.us) return SplitWay::split;
   double rival = 1e30;
   for (const Tile16& t : kTilesShort) rival = std::min(rival, cost16(t, M, N, K));
-  return us < 0.97 * rival || us < 1.04 * plan16(M, N, K).us;
+  if (us >= 0.97 * rival) return SplitWay::no;
+  const bool ring = !p.n_wide && (p.bn == 32 || (p.tile->bm == 64 && p.bn == 64) || (p.bn == 128 && (p.tile->bm == 96 || p.tile->bm == 192)));
+  return ring ? SplitWay::ranges : SplitWay::split;
 }
+bool split_pays(const GemmPlan& pl, int M, int N, int K) { return split_way(pl, M, N, K) != SplitWay::no; }
 
 // The pipelined kernel: split over k into pl.S ranges (ws holds the partial planes), or, int8 weights, unsplit (ws null).
 template <bool W8, int NI, typename T = BF16>
@@ -1025,7 +1032,8 @@ int launch(const void* A, const void* W, const float* scale, const EpiArgs& ep, 
   uint16_t* c = static_cast<uint16_t*>(C);
   const GemmPlan pl = plan_gemm(M, N, K, W8);
   float* ws = aligned16(workspace) ? static_cast<float*>(workspace) : nullptr;
-  if (ws && workspace_bytes >= split_bytes(pl, M, N) && split_pays(pl, M, N, K))
+  const SplitWay way = ws && workspace_bytes >= split_bytes(pl, M, N) ? split_way(pl, M, N, K) : SplitWay::no;
+  if (way == SplitWay::split || (W8 && way == SplitWay::ranges))
     return pick_ni(M, N) == 3 ? launch4<W8, 3, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, pl, ws)
                               : launch4<W8, 4, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, pl, ws);
   if constexpr (!W8) {
@@ -1048,7 +1056,8 @@ int launch(const void* A, const void* W, const float* scale, const EpiArgs& ep, 
     // 17.3 / 13.5, 2048 x 3072 x 512 13.2 / 12.5, 16384 x 1536 x 512 36.6 / 33.5, 8192 x 768 x 768 17.4 / 16.4; from K = 1024 on ties or worse
     if (p.tile->bm == 256 && (p.tile->bn >= 192 || K < kShortK))
       return gemm8_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, p.tile->bn / 64, nullptr, s);
-    return gemm_ring_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, p.tile->bm, p.bn, s);
+    return gemm_ring_launch(a, w, ep, c, M, N, K, lda, ldw, ldc, epilogue, is_f16<T>, p.tile->bm, p.bn,
+                            way == SplitWay::ranges ? KRanges{pl.tiles, pl.rem, pl.S} : KRanges{0, 0, 1}, s);
   } else {
     const bool pipelined = K % 32 == 0 && K >= 64;
     const int KT = (K + BK - 1) / BK;
@@ -1173,9 +1182,10 @@ SANA_API int sana_hip_gemm_plan(int M, int N, int K, int plan[4]) {
   if (N % 8 || K % 8) return SANA_ERR_SHAPE;
   const GemmPlan split = plan_gemm(M, N, K, false);
   const Plan16 p = plan16(M, N, K);
-  const bool cut = split_pays(split, M, N, K);
+  const SplitWay way = split_way(split, M, N, K);
+  const bool cut = way == SplitWay::split;
   plan[0] = cut ? BT : p.tile->bm, plan[1] = cut ? 64 * pick_ni(M, N) : p.bn;
-  plan[2] = cut ? 0 : p.n_wide, plan[3] = cut ? split.S : 1;
+  plan[2] = cut ? 0 : p.n_wide, plan[3] = way == SplitWay::no ? 1 : split.S;
   return SANA_OK;
 }
 

@@ -57,8 +57,13 @@ int gemm288_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint
 // The GEMM for few tokens (gemm_ring.hip): the same operands and epilogues up to SANA_EPI_GATE_RES (gate not null), in tiles
 // of bm tokens x bn channels: 64 x 32, 64 x 64, 64 x 128, 96 x 128,
 // 128 x 128, 128 x 160, 192 x 128 or 256 x 128.
+// ranges > 1: each output is the sum, in order, of the sums over that many ranges of k-tiles, the bits of the GEMM split over k; `tiles`
+// k-tiles each (8 or more), one more in the first `rem`.  64 x 32, 64 x 64, 96 x 128 and 192 x 128 only.
+struct KRanges {
+  int tiles, rem, ranges;
+};
 int gemm_ring_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
-                     int64_t ldw, int64_t ldc, int epilogue, bool f16, int bm, int bn, hipStream_t s);
+                     int64_t ldw, int64_t ldc, int epilogue, bool f16, int bm, int bn, const KRanges& kr, hipStream_t s);
 
 namespace {
 

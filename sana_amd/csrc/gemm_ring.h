@@ -25,6 +25,7 @@ template <typename F, int... I>
 __device__ __forceinline__ void gr_each(F&& f, std::integer_sequence<int, I...>) {
   (f(std::integral_constant<int, I>{}), ...);
 }
+// RANGES: sums over ranges of k (KRanges in gemm_common.h), added up here.
 // Workgroup tile BM = 16 TM WM tokens x BN = 16 TN WN channels, WM x WN waves of TM x TN MFMA tiles of 16x16x32.
 //
 // LDS: ST stages of a k-tile of 64 ([A rows | W rows], 128 bytes a row, the 16-byte piece index XORed with (row / 2) % 8),
@@ -47,11 +48,11 @@ __device__ __forceinline__ void gr_each(F&& f, std::integer_sequence<int, I...>)
 // 23.7 / 18.5, 2048 x 1152 x 2880 28.7 / 21.8, 200 x 3456 x 1152 6.8 / 6.9; slower: 288 x 6720 x 2240 19.5 / 20.6, 150 x 11200 x 2240
 // 21.0 / 22.2 (96 x 128 instead of 128 x 128: a last token tile of few rows, which the plan's tile times do not know), 1260 x 5760 x
 // 1152 21.1 / 21.9 (256 x 128).
-template <int WM, int WN, int TM, int TN, int ST, bool WHOLE, int EPI, typename T>
+template <int WM, int WN, int TM, int TN, int ST, bool WHOLE, bool RANGES, int EPI, typename T>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
                                                                  const EpiArgs ep, uint16_t* __restrict__ C, int M, int N,
                                                                  int K, int64_t lda, int64_t ldw, int64_t ldc, int tiles_t,
-                                                                 int tiles_c, int group, uint32_t prefetch) {
+                                                                 int tiles_c, int group, uint32_t prefetch, const KRanges kr) {
   constexpr int NW = WM * WN, BM = 16 * TM * WM, BN = 16 * TN * WN;
   // load instructions per wave and k-tile (rows past the tile's, where its rows are no whole number of them, read as zeros)
   constexpr int NA = (BM / 8 + NW - 1) / NW, NWP = (BN / 8 + NW - 1) / NW, LOADS = NA + NWP;
@@ -220,7 +221,39 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
       if (one_gate && n < N) gate[s] = *reinterpret_cast<const u32x4_t*>(ep.gate + (int64_t)g_first * ep.gate_stride + n);
     }
   };
-  constexpr bool EARLY = WHOLE && TN <= 4;  // (registers)
+  constexpr bool EARLY = WHOLE && TN <= 4 && !(RANGES && TM * TN > 8);  // (registers)
+
+  // RANGES: behind the last k-tile of a range of k (but the last one) its sum is added to those before it.
+  f32x4_t sum[RANGES ? TN : 1][RANGES ? TM : 1];
+  int range = 1, range_end = kr.tiles + (kr.rem > 0);
+  if constexpr (RANGES) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) sum[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  auto end_range = [&](int done) {  // done: k-tiles multiplied so far
+    if constexpr (RANGES) {
+      if (done != range_end || range >= kr.ranges) return;
+      asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");  // results of the last asm MFMAs
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) {
+          asm volatile("" : "+v"(acc[i][j]));
+          sum[i][j] += acc[i][j];
+          acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) asm volatile("" : "+v"(acc[i][j]));
+      asm volatile("s_nop 7" ::: "memory");
+      range_end += kr.tiles + (range < kr.rem);
+      ++range;
+    }
+  };
 
   int kt = 0;
   if constexpr (WHOLE) {
@@ -282,7 +315,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
 #pragma clang loop unroll(disable)
     for (; kt + UN + ST <= whole; kt += UN)
       gr_each([&](auto i_c) { constexpr int I = decltype(i_c)::value;
-                              pass(std::integral_constant<int, I & 1>{}, C1{}, C0{}, (HEAD + I) % ST, kt + I); },
+                              pass(std::integral_constant<int, I & 1>{}, C1{}, C0{}, (HEAD + I) % ST, kt + I);
+                              end_range(kt + I + 1); },
               std::make_integer_sequence<int, UN>{});
     if (GATED && EARLY) request();
     int st = HEAD;  // (rounds of the ring end where they began)
@@ -290,8 +324,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
 #pragma clang loop unroll(disable)
     for (; kt < KT; kt += 2) {  // (an odd number of them: one pass of zeros)
       pass(C0{}, C0{}, C0{}, st, kt);
+      end_range(kt + 1);
       st = st + 1 == ST ? 0 : st + 1;
       pass(C1{}, C0{}, C0{}, st, kt + 1);
+      end_range(kt + 2);
       st = st + 1 == ST ? 0 : st + 1;
     }
 #pragma unroll
@@ -334,6 +370,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
       past_end(kt + ST);
       kstep(C1{}, nxt, C0{}, J1{}, st, kt + ST);
       landed(C0{});
+      end_range(kt + 1);
       last = st;
       st = nxt;
     }
@@ -342,6 +379,12 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_ring_kernel(const uint16_t*
   asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_waitcnt vmcnt(0)" ::: "memory");
   GR_BARRIER();
 #undef GR_BARRIER
+  if constexpr (RANGES) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] += sum[i][j];
+  }
 
   // ---- epilogue: 16 tokens at a time through the wave's own corner of LDS (rows padded by 16 bytes: conflict-free both
   // ways), so that a store instruction writes whole row segments.
