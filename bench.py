@@ -491,11 +491,9 @@ def small_configs(dev):
     g = torch.Generator().manual_seed(0)
     qkv = torch.randn(B, N, 3, h * d, generator=g)
     qd = qkv.to(dev)
-    out = torch.empty(B, N, h * d, device=dev)
 
     def gpu_op():
-        st = ops.linattn_state(qd[:, :, 1], qd[:, :, 2])
-        ops.linattn_apply(qd[:, :, 0], st, 1e-15, out=out)
+        ops.relu_linear_attention(qd[:, :, 0], qd[:, :, 1], qd[:, :, 2], 1e-15)
 
     t_gpu = event_time_us(gpu_op, 200, 20)
     q4, k4, v4 = (qkv[:, :, i].reshape(B, N, h, d).permute(0, 2, 3, 1) for i in range(3))   # (B, h, d, N) views
@@ -507,11 +505,11 @@ def small_configs(dev):
         t_cpu = (time.perf_counter() - t0) / 50 * 1e6
     bytes1 = 4 * N * h * d * 4 + 2 * h * (d + 1) * d * 4
     res["cfg1"] = {"workload": "LiteLA ReLU linear attention op alone, fp32, B=1, 36 heads x 32, N=1024, eps 1e-15",
-                   "gpu_us": round(t_gpu, 2), "gpu_launches": 3, "algorithmic_bytes": bytes1,
+                   "gpu_us": round(t_gpu, 2), "gpu_launches": 2, "algorithmic_bytes": bytes1,
                    "achieved_GBps": round(bytes1 / t_gpu / 1e3, 1),
                    "cpu_baseline": {"value": round(t_cpu, 1), "unit": "us per op", "cores": threads, "kind": "port",
                                     "sample": "the whole workload, 50 timed iterations after 1 warm-up"},
-                   "note": "three launches of a few microseconds each: bound by launch latency, not by HBM"}
+                   "note": "two launches of a few microseconds each: bound by launch latency, not by HBM"}
     # ---- cfg2
     Cc, heads, Bb, HW = 1152, 16, 4, (32, 32)
     ob = O.init_block_(O.SanaMSBlock(Cc, heads, mlp_ratio=2.5, attn_type="linear", ffn_type="glumbconv"), 0)
