@@ -852,11 +852,11 @@ struct Tile16 {
 };
 // Fitted to 250 shapes (64 .. 32760 tokens, the eight projections of the two image widths and the text's, one block's and a
 // step's, weights cold, launches replayed from a graph: issued one by one, a launch of less than 20 us is timed by its issue):
-// 7 - 14 % off each, the choice 0.3 % from the best tile on the mean, more than 6 % in two shapes (9 and 7 %).  In a second round
+// 7 - 14 % off each.  Of 304 shapes timed since with every tile (profiles/gemm_tiles_by_shape.txt) the choice is 1.1 % from the
+// best on the mean, more than 6 % in ten.  In a second round
 // the small tiles were never more than 2 % ahead, and 300 x 17920 x 2240 is 48.7 us in 128 x 128 and 40.4 in 256 x 192: hence
-// one_round.  us, the tile chosen before / now, both timed so: 256 x 1152 x 2880 14.9 / 10.3 (halved), 1024 x 2240 x 2240 24.3 / 19.0,
-// 1560 x 2304 x 1152 16.1 / 12.6, 2048 x 1152 x 2880 28.7 / 22.1, 4096 x 1152 x 1152 20.4 / 17.0, 4096 x 1152 x 2880
-// 38.6 / 30.5, 2916 x 2240 x 2240 33.0 / 32.1.
+// one_round.  us, the tiles and kernels before this table / now, both timed so: 256 x 1152 x 2880 15.3 / 10.3 (halved), 1024 x 2240 x
+// 2240 23.6 / 18.7, 2048 x 1152 x 2880 28.6 / 21.6, 4096 x 1152 x 1152 20.7 / 17.7, 4096 x 1152 x 2880 35.0 / 31.4.
 constexpr Tile16 kTiles16[] = {
     {64, 64, 512, 256, 257, 3.0, 0.288, 0.503, true, 0.165, 0.26}, {64, 128, 256, 32, 256, 3.9, 0.350, 0.414, true},
     {96, 128, 256, 32, 256, 3.7, 0.439, 0.466, true},  {128, 128, 256, 32, 256, 3.9, 0.454, 0.541, true},
