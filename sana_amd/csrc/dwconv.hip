@@ -279,8 +279,11 @@ __device__ __forceinline__ float dot2_16_from<F16>(uint32_t a, uint32_t b, float
 // (x[j], x[j+1]) pairs as the kernel above.  Pixels and rows outside the image never need a branch or a
 // select: their lanes load through an offset outside the buffer resource, which writes zeros to LDS.
 // A row in LDS is [18 pixels][first half: 256 B | gate half: 256 B]; one load instruction fills 1 KB = two
-// pixels.  The 18 instructions of a group are dealt to the four waves five each (two pieces are written
-// twice, with the same data), so every wave can wait on its own counter with a constant.
+// pixels.  The 18 instructions of a group are dealt to the four waves, 5, 5, 4 and 4; each waits on its own count.
+// What bounds it: from about 4096 tokens the memory system; below, what a workgroup does before its first row counts: the taps value
+// by value, the border tests piece by piece and the arguments in five waits took longer than a band of 4 rows.  us, so / now
+// (bands included), cold inputs: 16 x 16 x 2880 6.3 / 4.8, 32 x 32 x 2880 11.5 / 8.3, 32 x 32 x 5600 15.5 / 13.1, 16 x 9 x 17 x 5600 38.2 /
+// 29.6, 4 x 32 x 32 x 2880 22.3 / 20.8, 64 x 64 x 5600 37.9 / 35.6, 128 x 128 x 5600 117 / 114 (behind the GEMM that wrote them 110 / 104).
 // ----------------------------------------------------------------------------
 constexpr int DWL_PIXB = 512, DWL_RING = 4;
 
@@ -290,6 +293,7 @@ __global__ __launch_bounds__(64 * NW, 16 / NW) void dwconv_gate16_lds_kernel(con
                                                                    int H, int W, int Ch, int R, int xgroups) {
   typedef Pair<T> P;
   constexpr int ESZ = 2, TW = 4, SW = TW * NW, FP = SW + 2, DWL_ROWB = FP * DWL_PIXB, NPIECE = FP / 2;
+  asm volatile("" ::"s"(u), "s"(w), "s"(bias), "s"(H), "s"(W), "s"(Ch), "s"(R), "s"(xgroups));  // (the arguments in one wait)
   __shared__ __attribute__((aligned(1024))) unsigned char ring[DWL_RING * DWL_ROWB];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -316,18 +320,21 @@ __global__ __launch_bounds__(64 * NW, 16 / NW) void dwconv_gate16_lds_kernel(con
   const int64_t img = (int64_t)bt * H * W;
   const uint32_t lane_b = (uint32_t)(2 * lane) * ESZ;
 
-  uint32_t w01[4][3], wz2[4][3];
-  float bs[4];
-  const uint16_t* wp = static_cast<const uint16_t*>(w);
+  // Filter taps: a channel pair's 18 values are 36 contiguous bytes, read as 16 + 16 + 4 per half, in front of the rows and unpacked
+  // behind the request of the first ones.  (Value by value they are 36 loads whose lanes stand 36 bytes apart, each over 18 lines of the
+  // vector cache.)
+  uint32_t raw_w[2][9], raw_b[2];
+  typedef uint32_t u32_a2 __attribute__((aligned(2)));  // (a channel's taps may stand on any 2-byte boundary)
+  typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int64_t ch = (lane_ok ? c : 0) + (q & 1) + (q >> 1) * Ch;
+  for (int q = 0; q < 2; ++q) {
+    const int64_t ch = (lane_ok ? c : 0) + q * (int64_t)Ch;
+    const u32x4_a2* p = reinterpret_cast<const u32x4_a2*>(static_cast<const uint16_t*>(w) + ch * 9);
+    const u32x4_a2 x = p[0], z = p[1];
 #pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      w01[q][r] = (uint32_t)wp[ch * 9 + 3 * r] | ((uint32_t)wp[ch * 9 + 3 * r + 1] << 16);
-      wz2[q][r] = (uint32_t)wp[ch * 9 + 3 * r + 2] << 16;
-    }
-    bs[q] = bias ? P::one(bias, ch) : 0.f;
+    for (int i = 0; i < 4; ++i) raw_w[q][i] = x[i], raw_w[q][4 + i] = z[i];
+    raw_w[q][8] = *reinterpret_cast<const u32_a2*>(p + 2);
+    raw_b[q] = bias ? *reinterpret_cast<const u32_a2*>(static_cast<const uint16_t*>(bias) + ch) : 0u;
   }
 
   // ---- global -> LDS.  Lane l of a load instruction: pixel parity l / 32, half (l / 16) % 2, 16-byte chunk l % 16.
@@ -339,21 +346,47 @@ __global__ __launch_bounds__(64 * NW, 16 / NW) void dwconv_gate16_lds_kernel(con
   const int d_chb = ((((lane >> 4) & 1) ? Ch : 0) + d_chan) * ESZ;
   const int d_col0 = x0wg - 1 + (lane >> 5);                             // footprint column of piece 0
   const bool d_ok = d_chan < Ch;                                         // Ch % 8 == 0: a chunk is in or out
+  // Piece j of a group's 2 * NPIECE goes to wave j % NW: its row of the two, its place in a row and its offset inside an image row are
+  // the same for every group.
+  constexpr int PMAX = (2 * NPIECE + NW - 1) / NW, NFULL = 2 * NPIECE - (PMAX - 1) * NW;  // waves < NFULL have PMAX pieces
+  int voff[PMAX];
+#pragma unroll
+  for (int k = 0; k < PMAX; ++k) {
+    const int j = wave + NW * k, col = d_col0 + 2 * (j < NPIECE ? j : j - NPIECE);
+    voff[k] = (d_ok & (col >= 0) & (col < W)) ? col * pix_b + d_chb : oob;
+  }
+  const int row_b = W * pix_b;
   auto issue_group = [&](int g) {   // rows 2g, 2g+1 of the band's row stream: image rows y0 - 1 + 2g (+1)
 #pragma unroll
-    for (int k = 0; k < (2 * NPIECE + NW - 1) / NW; ++k) {
+    for (int k = 0; k < PMAX; ++k) {
       const int j = wave + NW * k;
-      if (j >= 2 * NPIECE) break;                                         // wave-uniform
+      if (k == PMAX - 1 && wave >= NFULL) break;                          // wave-uniform
       const int r = j >= NPIECE ? 1 : 0, i = j - NPIECE * r;
       const int t = 2 * g + r, yy = y0 - 1 + t;
-      const bool row_ok = yy >= 0 && yy < H;
-      const int col = d_col0 + 2 * i;
-      const int voff = (d_ok && row_ok && col >= 0 && col < W) ? col * pix_b + d_chb : oob;
+      const bool row_ok = (unsigned)yy < (unsigned)H;
       unsigned char* dst = ring + (t & (DWL_RING - 1)) * DWL_ROWB + i * 1024;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_u, (__attribute__((address_space(3))) void*)dst, 16, voff,
-                                               row_ok ? yy * W * pix_b : 0, 0, 0);
+      const int off = voff[k] | (row_ok ? 0 : oob);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_u, (__attribute__((address_space(3))) void*)dst, 16, off,
+                                               row_ok ? yy * row_b : 0, 0, 0);
     }
   };
+
+  const int NT = y1 - y0 + 2, NGRP = (NT + 1) >> 1;
+  issue_group(0);
+  if (NGRP > 1) issue_group(1);
+  uint32_t w01[4][3], wz2[4][3];
+  float bs[4];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const uint32_t(&e)[9] = raw_w[q];  // channel c: values 0 .. 8, channel c + 1: 9 .. 17
+    w01[2 * q][0] = e[0], wz2[2 * q][0] = e[1] << 16;
+    w01[2 * q][1] = __builtin_amdgcn_alignbit(e[2], e[1], 16), wz2[2 * q][1] = e[2] & 0xffff0000u;
+    w01[2 * q][2] = e[3], wz2[2 * q][2] = e[4] << 16;
+    w01[2 * q + 1][0] = __builtin_amdgcn_alignbit(e[5], e[4], 16), wz2[2 * q + 1][0] = e[5] & 0xffff0000u;
+    w01[2 * q + 1][1] = e[6], wz2[2 * q + 1][1] = e[7] << 16;
+    w01[2 * q + 1][2] = __builtin_amdgcn_alignbit(e[8], e[7], 16), wz2[2 * q + 1][2] = e[8] & 0xffff0000u;
+    bs[2 * q] = P::lo(raw_b[q]), bs[2 * q + 1] = P::hi(raw_b[q]);
+  }
 
   uint32_t win[3][TW + 1][4];
   // the output image from this slab's first channel on: offsets past its end (and the 2^31 of a masked lane) are dropped
@@ -421,16 +454,12 @@ __global__ __launch_bounds__(64 * NW, 16 / NW) void dwconv_gate16_lds_kernel(con
     }
   };
 
-  const int NT = y1 - y0 + 2, NGRP = (NT + 1) >> 1;
-  issue_group(0);
-  if (NGRP > 1) issue_group(1);
   for (int g0 = 0; g0 < NGRP; g0 += 3) {
 #pragma unroll
     for (int gg = 0; gg < 3; ++gg) {
       const int g = g0 + gg;
       if (g >= NGRP) break;  // uniform over the workgroup
       // this wave's pieces of group g have landed: all but the pieces of group g + 1 it issued since
-      constexpr int PMAX = (2 * NPIECE + NW - 1) / NW, NFULL = 2 * NPIECE - (PMAX - 1) * NW;  // waves < NFULL issue PMAX
       if (g + 1 >= NGRP) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       else if (wave < NFULL) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PMAX) : "memory");
       else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PMAX - 1) : "memory");
@@ -459,15 +488,15 @@ int launch(const void* u, const void* w, const void* bias, void* y, int BT, int 
   // 16-bit io: the LDS kernel (32-bit byte offsets inside one image, 16-byte channel chunks)
   if constexpr (!std::is_same<T, float>::value) {
     if ((int64_t)H * W * 2 * Ch * 2 < ((int64_t)1 << 31) && Ch % 8 == 0) {
-      // Bands of rows so that the launch has at least SANA_DW_LDS_MINWG workgroups (four fit a compute unit).
-      // Two halo rows are re-read per band: no band shorter than 8 rows, or than 4 where even that leaves
-      // the chip short of work (single small images), or than 2 while those are at most one workgroup per compute unit:
-      // both groups of such a band's rows are requested at once, so it is one memory round trip instead of two.  us, bands of
-      // 4 / of 2: 16 x 16 x 2880 7.8 / 6.4 (184 workgroups of 2), 12 x 12 x 2880 7.7 / 6.3; 12 x 12 x 5600 7.8 / 8.5 (264).
+      // Bands of rows so that the launch has at least SANA_DW_LDS_MINWG workgroups (four fit a compute unit).  Two halo rows are re-read
+      // per band: none shorter than 4 rows, or than 2 where that many workgroups are not reached even so: both groups of such a
+      // band's rows are requested at once, one memory round trip instead of two.  us, bands of 8 / 4 / 2 rows: 16 x 16 x 2880 8.5 /
+      // 6.0 / 4.8, 32 x 32 x 2880 9.7 / 9.1 / 8.1, 24 x 24 x 5600 12.6 / 11.1 / 10.2, 32 x 32 x 5600 14.2 / 13.1 / 13.0; more workgroups
+      // 2 x 32 x 32 x 5600 20.8 / 20.8 / 20.6, 3 x 27 x 36 x 5600 30.8 / 28.8 / 32.0, 45 x 60 x 5600 26.8 / 25.0 / 26.1.
       constexpr int NW = 4;
       const int xg = (W + 4 * NW - 1) / (4 * NW);
       const int64_t base = (int64_t)slabs * xg * BT;
-      const int min_rows = base * ((H + 7) / 8) >= 512 ? 8 : base * ((H + 1) / 2) <= 256 ? 2 : 4;
+      const int min_rows = base * ((H + 1) / 2) <= SANA_DW_LDS_MINWG ? 2 : 4;
       int nb = (int)((SANA_DW_LDS_MINWG + base - 1) / base);
       nb = std::max(1, std::min(nb, (H + min_rows - 1) / min_rows));
       const int R = (H + nb - 1) / nb, bands = (H + R - 1) / R;
