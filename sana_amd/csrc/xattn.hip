@@ -6,16 +6,18 @@
 // q and out are token-major [B, N, H*d] (what the linear layers on either side read and write: no head
 // transposes), k and v are the two halves of the kv projection [B, Nk, 2, H*d].
 //
-// The key set of one (batch, head) fits LDS whole (Nk <= 320: K as [key][d padded to 32*DK] and V transposed as
-// [d][key]: 150 KB at d = 112), so there is no online softmax: a wave takes 16*QT queries, multiplies them with
+// The key set of one (batch, head) fits LDS whole (Nk <= 320: K as [key][d padded to 32*DK] and V as [key][112]: 151 KB at d = 112), so
+// there is no online softmax: a wave takes 16*QT queries, multiplies them with
 // all keys (v_mfma_f32_16x16x32_bf16, scores^T = K . Q^T: a lane owns one query and 4 keys of every 16-key tile),
 // takes max / exp2 / sum in registers (two cross-lane steps over the four lane groups that share a query), and
 // feeds the probabilities straight back as the column operand of out^T = V^T . P^T -- the k index of that
 // product is permuted so that the 8 values a lane needs are the ones its own accumulators hold (keys
-// 32s + 4g + {0..3} and 32s + 16 + 4g + {0..3} for lane group g), and V^T is stored in that key order.
-// Few queries (one 512 px image: 64 workgroups of one item) are bound by the staging, a chain of load latencies: the queries and all
-// of K and V are requested before the first LDS write (the queries behind the staging: 0.3 us more a launch), and V is
-// transposed four keys at a time (8-byte writes).
+// 32s + 4g + {0..3} and 32s + 16 + 4g + {0..3} for lane group g), and V is read transposed in that key order (ds_read_b64_tr_b16).
+// Few queries (one 512 px image: 64 workgroups of one item) are bound by the staging.  K and V go global -> LDS by direct loads: no
+// staging registers, no branch per piece (rows past Nk and pieces past d lie outside the resource: zeros), no transposing writes.
+// Through registers, each piece behind a branch of its own and V written transposed, the instructions in front of the last load alone
+// took over a microsecond.  us, before / now: 256 queries x 300 keys x 16 heads of 72 9.6 / 8.3 (launch 1.7, staging 3.0, the rest the
+// attention), 1024 9.9 / 8.5, 2 x 1024 12.6 / 11.8, 256 x 20 heads of 112 11.8 / 11.1, 1024 13.1 / 12.4, 4680 31.2 / 30.2, 16384 78 / 78; same bits.
 // Workgroups are persistent over consecutive (batch, head, query block) items and restage K / V only when the
 // (batch, head) changes.  Every K / V fragment read from LDS feeds QT MFMAs.
 #include <type_traits>
@@ -31,22 +33,17 @@ namespace sana {
 namespace {
 
 constexpr int XA_NKP = 320;       // keys an LDS image holds (padded)
-constexpr int XA_VPITCH = XA_NKP * 2;  // bytes per row of V^T
+constexpr int XA_VCH = 14, XA_VPITCH = 16 * XA_VCH;  // 16-byte pieces / bytes of a V row: 112 channels, and 8 rows cover all banks
 
 // 16-byte-slot swizzles that make 16 consecutive rows of one chunk hit 16 different bank groups
 template <int DK>
 __device__ __forceinline__ int xa_kkey(int row) {  // K rows of DK*64 bytes
   return DK == 4 ? (row & 15) : DK == 3 ? ((row >> 2) & 3) : DK == 2 ? ((row >> 1) & 7) : ((row >> 2) & 3);
 }
-// V^T rows of 640 bytes: rows alternate between the two halves of the bank space, (row / 2) % 8 spreads a 16-row
-// fragment read over the 8 slots of a half; the (row / 16) % 4 term does the same for the transposing writes of
-// the staging pass, whose lanes hold one key at rows 8 apart
-__device__ __forceinline__ int xa_vkey(int row) { return ((row >> 1) ^ ((row >> 4) & 3)) & 7; }
-
-// position of key m inside its group of 32 in V^T (and in the probability operand)
-__device__ __forceinline__ int xa_vpos(int m) {
-  const int s = m >> 5, w = m & 31, hi = w >> 4, g = (w >> 2) & 3, e = w & 3;
-  return 32 * s + 8 * g + 4 * hi + e;
+// 4 keys x 16 channels of row-major V -> this lane's channel, 4 keys: row i of a group of 16 lanes is addressed by its lanes 4 i .. 4 i + 3
+__device__ __forceinline__ u32x2_t xa_read_tr(uint32_t lds) {
+  typedef short s16x4_t __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(size_t)lds));
 }
 
 template <typename T, int DK, int DT, int QT, int NW, int NKT>
@@ -56,12 +53,12 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
                                                          int64_t bias_stride, float scale_log2e, int qblocks, int items,
                                                          int items_per_wg) {
   constexpr int KPITCH = DK * 64, KCH = DK * 4;  // bytes / 16-byte chunks per K row
-  constexpr int K_BYTES = XA_NKP * KPITCH, V_BYTES = DT * 16 * XA_VPITCH;
+  constexpr int K_BYTES = XA_NKP * KPITCH, V_BYTES = XA_NKP * XA_VPITCH;
   __shared__ __attribute__((aligned(16))) unsigned char smem[K_BYTES + V_BYTES + XA_NKP * 4];
   unsigned char* sk = smem;
   unsigned char* sv = smem + K_BYTES;
   float* sb = reinterpret_cast<float*>(smem + K_BYTES + V_BYTES);  // per key: bias * log2(e), -inf past Nk
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int fr = lane & 15, fg = lane >> 4;
 
   int staged = -1;
@@ -75,59 +72,76 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
     u32x4_t qf[QT][DK];
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
-      const int qi = q0 + 16 * t + fr;
+      const uint16_t* qrow = qbase + (int64_t)min(q0 + 16 * t + fr, N - 1) * ldq;  // (no branch around a load)
 #pragma unroll
       for (int ks = 0; ks < DK; ++ks) {
         const int k0 = 32 * ks + 8 * fg;
-        qf[t][ks] = (qi < N && k0 < d) ? *reinterpret_cast<const u32x4_t*>(qbase + (int64_t)qi * ldq + k0)
-                                       : u32x4_t{0u, 0u, 0u, 0u};
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(qrow + (k0 < d ? k0 : 0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) qf[t][ks][e] = k0 < d ? v[e] : 0u;
       }
     }
     if (bh != staged) {  // uniform
       __syncthreads();   // everyone is done with the previous head's K / V
       const uint16_t* kbase = kv + (int64_t)b * Nk * ldkv + (int64_t)h * d;
       const uint16_t* vbase = kbase + (int64_t)H * d;
-      // all of a thread's loads go out before its first LDS write.  K: pieces of 8 channels; V: 8 channels of 4 keys
-      // (key tiles past NKT are not read)
-      constexpr int NT = 64 * NW, KEYS = 16 * NKT, VCH = 2 * DT;
-      constexpr int KN = (KEYS * KCH + NT - 1) / NT, VN = (KEYS / 4 * VCH + NT - 1) / NT;
-      u32x4_t kval[KN], vval[VN][4];
-      int ht = tid;  // hidden from the optimiser: the addresses are not worth registers across the items
-      asm volatile("" : "+v"(ht));
+      // Rows past Nk and pieces past d lie outside the resources: zeros.  (key tiles past NKT are not read)
+      constexpr int NT = 64 * NW, KEYS = 16 * NKT;
+      constexpr uint32_t kOut = 0x80000000u;
+      if (ldkv < (1 << 21)) {
+        const uint32_t ld2 = 2 * (uint32_t)ldkv;
+        const int span = (int)((uint32_t)(Nk - 1) * ld2 + 2 * d);
+        const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kbase), 0, span, 0x00020000);
+        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(vbase), 0, span, 0x00020000);
+        auto load = [&](const __amdgpu_buffer_rsrc_t& r, unsigned char* dst, uint32_t off) {
+          const int o = (int)off;
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, o, 0, 0, 0);
+        };
+        // K: KI load instructions of 1 KB are 16 (12 pieces a row) or 4 rows (16 pieces); 16 rows and 4 waves repeat the swizzle
+        constexpr int KI = KCH == 16 ? 1 : KCH / 4, KR = 64 * KI / KCH;
+        static_assert(NW % 4 == 0 && (KR * NW) % 16 == 0 && KEYS % KR == 0, "");
+        uint32_t ko[KI];
 #pragma unroll
-      for (int i = 0; i < KN; ++i) {
-        const int idx = ht + i * NT, row = idx / KCH, c = idx - row * KCH;
-        kval[i] = u32x4_t{0u, 0u, 0u, 0u};
-        if (row < Nk && 8 * c < d) kval[i] = *reinterpret_cast<const u32x4_t*>(kbase + (int64_t)row * ldkv + 8 * c);
-      }
-#pragma unroll
-      for (int i = 0; i < VN; ++i) {
-        const int idx = ht + i * NT, quad = idx / VCH, c = idx - quad * VCH;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          vval[i][k] = u32x4_t{0u, 0u, 0u, 0u};
-          if (4 * quad + k < Nk && 8 * c < d)
-            vval[i][k] = *reinterpret_cast<const u32x4_t*>(vbase + (int64_t)(4 * quad + k) * ldkv + 8 * c);
+        for (int j = 0; j < KI; ++j) {
+          const int l = 64 * j + lane, row = l / KCH, c = (l - row * KCH) ^ xa_kkey<DK>(KR * wave + row);
+          ko[j] = 8 * c < d ? (uint32_t)(KR * wave + row) * ld2 + 16 * c : kOut;
         }
-      }
 #pragma unroll
-      for (int i = 0; i < KN; ++i) {
-        const int idx = ht + i * NT, row = idx / KCH, c = idx - row * KCH;
-        if (row < KEYS) *reinterpret_cast<u32x4_t*>(sk + row * KPITCH + ((c ^ xa_kkey<DK>(row)) << 4)) = kval[i];
-      }
+        for (int i = 0; i < (KEYS / KR + NW - 1) / NW; ++i) {
+          const int g = i * NW + wave;
+          if ((KEYS / KR) % NW && g >= KEYS / KR) break;  // uniform
 #pragma unroll
-      for (int i = 0; i < VN; ++i) {
-        const int idx = ht + i * NT, quad = idx / VCH, c = idx - quad * VCH;
-        if (quad < KEYS / 4) {
-          const int p = xa_vpos(4 * quad);  // four keys stand side by side
+          for (int j = 0; j < KI; ++j) load(rk, sk + (g * KI + j) * 1024, ko[j] + (uint32_t)(KR * NW * i) * ld2);
+        }
+        // V: 7 instructions are 32 rows
+        uint32_t vo[7];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const int dr = 8 * c + e;
-            const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;
-            const u32x2_t x = {__builtin_amdgcn_perm(vval[i][1][e >> 1], vval[i][0][e >> 1], sel),
-                               __builtin_amdgcn_perm(vval[i][3][e >> 1], vval[i][2][e >> 1], sel)};
-            *reinterpret_cast<u32x2_t*>(sv + dr * XA_VPITCH + (((p >> 3) ^ xa_vkey(dr)) << 4) + (p & 7) * 2) = x;
-          }
+        for (int j = 0; j < 7; ++j) {
+          const int l = 64 * j + lane, row = l / XA_VCH, c = l - row * XA_VCH;
+          vo[j] = 8 * c < d ? (uint32_t)(32 * wave + row) * ld2 + 16 * c : kOut;
+        }
+#pragma unroll
+        for (int i = 0; i < (KEYS / 32 + NW - 1) / NW; ++i) {
+          const int g = i * NW + wave;
+          if ((KEYS / 32) % NW && g >= KEYS / 32) break;  // uniform
+#pragma unroll
+          for (int j = 0; j < 7; ++j) load(rv, sv + (g * 7 + j) * 1024, vo[j] + (uint32_t)(32 * NW * i) * ld2);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      } else {  // rows too far apart for 32-bit offsets
+#pragma unroll 1
+        for (int i = tid; i < KEYS * KCH; i += NT) {
+          const int row = i / KCH, c = i - row * KCH;
+          u32x4_t x = {0u, 0u, 0u, 0u};
+          if (row < Nk && 8 * c < d) x = *reinterpret_cast<const u32x4_t*>(kbase + (int64_t)row * ldkv + 8 * c);
+          *reinterpret_cast<u32x4_t*>(sk + row * KPITCH + ((c ^ xa_kkey<DK>(row)) << 4)) = x;
+        }
+#pragma unroll 1
+        for (int i = tid; i < KEYS * XA_VCH; i += NT) {
+          const int row = i / XA_VCH, c = i - row * XA_VCH;
+          u32x4_t x = {0u, 0u, 0u, 0u};
+          if (row < Nk && 8 * c < d) x = *reinterpret_cast<const u32x4_t*>(vbase + (int64_t)row * ldkv + 8 * c);
+          *reinterpret_cast<u32x4_t*>(sv + 16 * i) = x;
         }
       }
       for (int m = tid; m < KEYS; m += NT)
@@ -215,11 +229,12 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) oc[g][t][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       u32x4_t vf[2][DT];
+      const uint32_t vrow = (uint32_t)(size_t)(__attribute__((address_space(3))) const unsigned char*)sv + (4 * fg + (fr >> 2)) * XA_VPITCH + 8 * (fr & 3);
       auto load_v = [&](int buf, int s) {
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
-          const int row = 16 * dt + fr;
-          vf[buf][dt] = *reinterpret_cast<const u32x4_t*>(sv + row * XA_VPITCH + (((4 * s + fg) ^ xa_vkey(row)) << 4));
+          const u32x2_t lo = xa_read_tr(vrow + 32 * s * XA_VPITCH + 32 * dt), hi = xa_read_tr(vrow + (32 * s + 16) * XA_VPITCH + 32 * dt);
+          vf[buf][dt] = u32x4_t{lo.x, lo.y, hi.x, hi.y};
         }
       };
       load_v(0, k0 / 2);
@@ -310,7 +325,10 @@ int cross_attention(const void* q, const void* kv, const float* key_bias, void* 
   const bool few = d <= 96 && !restaged && (int64_t)B * H * ((N + 64 * XA_QT - 1) / (64 * XA_QT)) <= 256;
   // key tiles of 16 that are multiplied: all 20, or 10 for up to 160 keys (tiles past Nk hold zeros and -inf)
   if (d > 96) return Nk > 160 ? SANA_XA_GO(4, 7, 8, 20) : SANA_XA_GO(4, 7, 8, 10);
+  // (the product with V in tiles of 16 channels: five up to 80)
+  if (few && d <= 80) return Nk > 160 ? SANA_XA_GO(3, 5, 4, 20) : SANA_XA_GO(3, 5, 4, 10);
   if (few) return Nk > 160 ? SANA_XA_GO(3, 6, 4, 20) : SANA_XA_GO(3, 6, 4, 10);
+  if (d <= 80) return Nk > 160 ? SANA_XA_GO(3, 5, 8, 20) : SANA_XA_GO(3, 5, 8, 10);
   return Nk > 160 ? SANA_XA_GO(3, 6, 8, 20) : SANA_XA_GO(3, 6, 8, 10);
 #undef SANA_XA_GO
 }

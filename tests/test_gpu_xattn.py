@@ -365,3 +365,21 @@ def test_few_queries_of_several_batch_entries(cuda, N, Nk, dtype):
     assert rel_l2(out.cpu(), formula(q.cpu(), kv.cpu(), H)) <= 1e-2
     for b in range(4):
         assert torch.equal(out[b:b + 1], ops.cross_attention16(q[b:b + 1].clone(), kv[b:b + 1].clone(), H)), b
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,d", [(2, 72), (3, 80), (2, 88), (1, 104), (2, 112)])
+@pytest.mark.parametrize("Nk", [1, 31, 160, 161, 319])
+def test_keys_of_any_distance_give_the_bits_of_dense_ones(cuda, dtype, H, d, Nk):
+    """Rows of K and V that are 32-bit offsets apart go to LDS by direct loads, others through registers; neither reads what stands
+    between the rows (NaN here)."""
+    gen = torch.Generator(device=cuda).manual_seed(Nk)
+    C = H * d
+    q = torch.randn(1, 70, C, generator=gen, device=cuda).to(dtype)
+    kv = torch.randn(1, Nk, 2 * C, generator=gen, device=cuda).to(dtype)
+    dense = ops.cross_attention16(q, kv, H)
+    assert (dense.double() - formula(q, kv, H)).norm() <= 1e-2 * dense.double().norm()
+    for ld in [2 * C + 8] + ([1 << 21] if Nk <= 31 else []):
+        rows = torch.full((Nk * ld,), float("nan"), dtype=dtype, device=cuda).view(1, Nk, ld)
+        rows[:, :, :2 * C] = kv
+        assert torch.equal(ops.cross_attention16(q, rows[:, :, :2 * C], H), dense)
