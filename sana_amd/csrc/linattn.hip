@@ -679,6 +679,8 @@ __global__ __launch_bounds__(320) void linattn_apply32_partials_kernel(
 // graph on one set of inputs (on 16 in turn): bf16, 36 heads x 256 tokens 9.8 / 5.2 (10.5 / 6.0), 36 x 1024 12.1 / 8.8 (13.3 /
 // 11.5), 140 x 1024 18.9 / 15.4 (22.2 / 17.0); fp16 36 x 256 10.5 / 5.8 (11.2 / 6.6); fp32 256 x 1024 35.9 / 26.7 (45.6 / 38.4).
 // (Adding the state up in the two calls' order costs 0.4 us at 1024 tokens: sixteen partial states in LDS, not eight.)
+// Two 16-bit heads share the 128-byte lines of their tokens: neighbours run on one XCD and meet in its L2 (workgroup ids alternate over
+// the XCDs: 210 heads x 972 tokens 19.0 -> 16.8 us behind the GEMM that wrote them, 70 x 1024 12.0 -> 11.8).
 // ----------------------------------------------------------------------------
 constexpr int WHOLE_TOKENS = 1024;  // the most that one round of loads covers
 template <int OFF>
@@ -705,7 +707,7 @@ __global__ __launch_bounds__(512) void linattn_whole16_kernel(
   __shared__ __attribute__((aligned(16))) unsigned char smem[STATE_AT + STATE_ELEMS * 4];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int b = blockIdx.x / h, head = blockIdx.x - b * h;
+  const int bh = xcd_eighths(blockIdx.x, gridDim.x), b = bh / h, head = bh - b * h;
   const int ld_tok = lane >> 2, ld_chunk = lane & 3;  // a load instruction: 16 tokens x 64 bytes
   const u32x4_t zero4 = {0u, 0u, 0u, 0u};
   const uint16_t* kbase = K + (int64_t)b * stride_b + head * D + 8 * ld_chunk;
