@@ -709,10 +709,10 @@ __global__ __launch_bounds__(512) void linattn_whole16_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int bh = xcd_eighths(blockIdx.x, gridDim.x), b = bh / h, head = bh - b * h;
   const int ld_tok = lane >> 2, ld_chunk = lane & 3;  // a load instruction: 16 tokens x 64 bytes
-  const u32x4_t zero4 = {0u, 0u, 0u, 0u};
-  const uint16_t* kbase = K + (int64_t)b * stride_b + head * D + 8 * ld_chunk;
-  const uint16_t* vbase = V + (int64_t)b * stride_b + head * D + 8 * ld_chunk;
-  const uint16_t* qbase = Q + (int64_t)b * q_stride_b + head * D + 8 * ld_chunk;
+  const uint16_t* kbase = K + (int64_t)b * stride_b + head * D;
+  const uint16_t* vbase = V + (int64_t)b * stride_b + head * D;
+  const uint16_t* qbase = Q + (int64_t)b * q_stride_b + head * D;
+  uint16_t* obase = out + (int64_t)b * o_stride_b + head * D;
 
   // ---- phase 1
   auto tile_of = [&](int u, int t) {
@@ -720,20 +720,46 @@ __global__ __launch_bounds__(512) void linattn_whole16_kernel(
     return SPLIT * (c >> 2) + TILE * (c & 3) + 128 * t;
   };
   u32x4_t kreg[U1][2][2], vreg[U1][2][2], raw[U2];
+  // Every load goes out without a branch: rows past N lie outside the resource (zeros).
+  const bool near = max(max(q_stride_n, stride_n), o_stride_n) < (1 << 20);  // 32-bit offsets over 1024 rows
+  auto resource = [&](const uint16_t* base, int64_t stride) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, (N - 1) * (int)stride * 2 + 2 * D, 0x00020000);
+  };
+  auto offset = [&](int tok0, int64_t stride) { return (tok0 + ld_tok) * (int)stride * 2 + 16 * ld_chunk; };
+  if (near) {
+    const __amdgpu_buffer_rsrc_t rk = resource(kbase, stride_n), rv = resource(vbase, stride_n), rq = resource(qbase, q_stride_n);
 #pragma unroll
-  for (int u = 0; u < U1; ++u)
+    for (int u = 0; u < U1; ++u)
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < 2; ++t) {
+        if (tile_of(u, t) >= N) break;  // uniform (and not read below)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int tok = tile_of(u, t) + 16 * i + ld_tok;
-        kreg[u][t][i] = tok < N ? *reinterpret_cast<const u32x4_t*>(kbase + (int64_t)tok * stride_n) : zero4;
-        vreg[u][t][i] = tok < N ? *reinterpret_cast<const u32x4_t*>(vbase + (int64_t)tok * stride_n) : zero4;
+        for (int i = 0; i < 2; ++i) {
+          const int o = offset(tile_of(u, t) + 16 * i, stride_n);
+          kreg[u][t][i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rk, o, 0, 0));
+          vreg[u][t][i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rv, o, 0, 0));
+        }
       }
 #pragma unroll
-  for (int u = 0; u < U2; ++u) {
-    const int tok = (wave + u * WAVES) * 16 + ld_tok;
-    raw[u] = tok < N ? *reinterpret_cast<const u32x4_t*>(qbase + (int64_t)tok * q_stride_n) : zero4;
+    for (int u = 0; u < U2; ++u) {
+      if ((wave + u * WAVES) * 16 >= N) break;  // uniform
+      raw[u] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rq, offset((wave + u * WAVES) * 16, q_stride_n), 0, 0));
+    }
+  } else {
+    auto row = [&](const uint16_t* base, int tok, int64_t stride) {
+      return tok < N ? *reinterpret_cast<const u32x4_t*>(base + (int64_t)tok * stride + 8 * ld_chunk) : u32x4_t{0u, 0u, 0u, 0u};
+    };
+#pragma unroll
+    for (int u = 0; u < U1; ++u)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int tok = tile_of(u, t) + 16 * i + ld_tok;
+          kreg[u][t][i] = row(kbase, tok, stride_n), vreg[u][t][i] = row(vbase, tok, stride_n);
+        }
+#pragma unroll
+    for (int u = 0; u < U2; ++u) raw[u] = row(qbase, (wave + u * WAVES) * 16 + ld_tok, q_stride_n);
   }
   // MFMA 32x32x16: lane -> channel lane % 32, element r of k-step s is token 16 s + 2 r + lane / 32 of the tile.  A transposing
   // read hands the 16 lanes of a group four rows, row i addressed by lanes 4 i .. 4 i + 3: two tokens apart here.
@@ -814,9 +840,11 @@ __global__ __launch_bounds__(512) void linattn_whole16_kernel(
   unsigned char* qstage = smem + wave * (U2 * 1024);
   const int slot_w = 16 * (4 * ld_tok + (ld_chunk ^ ((ld_tok >> 1) & 3)));
   const int slot_r = 16 * (4 * n + (g ^ ((n >> 1) & 3)));
-  uint16_t* obase = out + (int64_t)b * o_stride_b + head * D + 8 * ld_chunk;
 #pragma unroll
-  for (int u = 0; u < U2; ++u) *reinterpret_cast<u32x4_t*>(qstage + u * 1024 + slot_w) = relu_pk16(raw[u]);
+  for (int u = 0; u < U2; ++u) {
+    if ((wave + u * WAVES) * 16 >= N) break;  // uniform
+    *reinterpret_cast<u32x4_t*>(qstage + u * 1024 + slot_w) = relu_pk16(raw[u]);
+  }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
   for (int u = 0; u < U2; ++u) {
@@ -854,11 +882,21 @@ __global__ __launch_bounds__(512) void linattn_whole16_kernel(
     *reinterpret_cast<u32x4_t*>(slot) = o;  // in the place of this lane's queries
   }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  if (near) {
+    const __amdgpu_buffer_rsrc_t ro = resource(obase, o_stride_n);
 #pragma unroll
-  for (int u = 0; u < U2; ++u) {
-    const int tok = (wave + u * WAVES) * 16 + ld_tok;
-    const u32x4_t o = *reinterpret_cast<const u32x4_t*>(qstage + u * 1024 + slot_w);
-    if (tok < N) *reinterpret_cast<u32x4_t*>(obase + (int64_t)tok * o_stride_n) = o;
+    for (int u = 0; u < U2; ++u) {
+      if ((wave + u * WAVES) * 16 >= N) break;  // uniform
+      __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4_t*>(qstage + u * 1024 + slot_w), ro,
+                                             offset((wave + u * WAVES) * 16, o_stride_n), 0, 0);
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < U2; ++u) {
+      const int tok = (wave + u * WAVES) * 16 + ld_tok;
+      const u32x4_t o = *reinterpret_cast<const u32x4_t*>(qstage + u * 1024 + slot_w);
+      if (tok < N) *reinterpret_cast<u32x4_t*>(obase + (int64_t)tok * o_stride_n + 8 * ld_chunk) = o;
+    }
   }
 }
 

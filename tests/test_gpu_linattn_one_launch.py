@@ -142,3 +142,21 @@ def test_which_launches_read_the_partial_states(cuda, B, N, h, two):
     assert bool((scratch[:state] == 7.25).all()) == two
     assert not bool((scratch[-(need // 4 - state) // 2:] == 7.25).any())
     assert torch.equal(out, ops.linattn_apply(q, ops.linattn_state(k, v), 1e-15))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("far", ["q", "k and v", "out", "all"])
+def test_rows_of_any_distance(cuda, dtype, far):
+    """16-bit rows 2^20 values apart and more are addressed in 64 bits: the bits of dense rows, nothing written between the rows."""
+    lib, N, h, ld = _lib.load(), 37, 3, 1 << 20
+    C, gen = 32 * h, torch.Generator().manual_seed(7)
+    dense = torch.randn(N, 3 * C, generator=gen).to(dtype).to(cuda)
+    want = ops.relu_linear_attention(*(dense[None, :, i * C:(i + 1) * C] for i in range(3)), 1e-15)[0]
+    wide = torch.full((N, ld), float("nan"), dtype=dtype, device=cuda)
+    wide[:, :3 * C] = dense
+    src = [wide if far == "all" or name in far else dense for name in "qkv"]
+    out = torch.full((N, ld if far in ("out", "all") else C), 3.0, dtype=dtype, device=cuda)
+    ptr = [s.data_ptr() + 2 * C * i for i, s in enumerate(src)]
+    _lib.check(lib.sana_hip_linattn(*ptr, out.data_ptr(), None, 0, 1, N, h, 32, 0, src[0].stride(0), 0, src[1].stride(0), 0,
+                                    out.stride(0), 1e-15, ops._dt(out), torch.cuda.current_stream().cuda_stream), "sana_hip_linattn")
+    assert torch.equal(out[:, :C], want) and bool((out[:, C:] == 3.0).all())
