@@ -230,12 +230,16 @@ __device__ __forceinline__ int xcd_eighths(int id, int total) {  // workgroup ->
   const int xcd = id & 7, base = total >> 3, rem = total & 7;
   return xcd * base + min(xcd, rem) + (id >> 3);
 }
+// Short splits are one round trip behind what comes in front of their loads: with a 64-bit product and a clamp each, 64 loads went
+// out over more than a microsecond.  us, whole calls, before (the phase 2 on partial states with its divisions first) / now, inputs from
+// HBM: 1024 x 36 17.8 / 15.3 (from the caches 14.9 / 13.4), 400 x 70 14.3 / 12.9, 2 x 1024 x 36 22.5 / 19.8, 3 x 3000 x 36 67 / 56,
+// 16384 x 36 99 / 90, 4 x 5000 x 70 224 / 199.
 template <bool LINEAR>
 __global__ __launch_bounds__(256) void linattn_state32_kernel(
     const float* __restrict__ K, const float* __restrict__ V, float* __restrict__ dst,
     const int32_t* __restrict__ chunk_starts, int N, int h, int n_chunks, int nsplit, int split_tokens,
     int64_t stride_b, int64_t stride_n) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int groups = (h + 3) >> 2;
   const int at = LINEAR ? xcd_eighths(blockIdx.x, gridDim.x) : 0;
   const int z = LINEAR ? at / nsplit : blockIdx.z, split = LINEAR ? at % nsplit : blockIdx.x;
@@ -246,31 +250,59 @@ __global__ __launch_bounds__(256) void linattn_state32_kernel(
   const int t0 = cr.begin + split * split_tokens;
   const int t1 = min(cr.end, t0 + split_tokens);
   const int j = lane & 31, g = lane >> 5;
-  const float* kp = K + (int64_t)b * stride_b + head * D + j;
-  const float* vp = V + (int64_t)b * stride_b + head * D + j;
+  const float* kp = K + (int64_t)b * stride_b + (int64_t)t0 * stride_n + head * D;
+  const float* vp = V + (int64_t)b * stride_b + (int64_t)t0 * stride_n + head * D;
   f32x16_t accS;
   float accK = 0.f;  // the "1" row of [V|1]: this lane's half of the tokens
 #pragma unroll
   for (int i = 0; i < 16; ++i) accS[i] = 0.f;
-  constexpr int U = 32;  // 64 tokens in flight per wave: a small input is one round trip
-  for (int t = t0; t < t1; t += 2 * U) {
-    float kk[U], vv[U];
+  const int n = t1 - t0;
+  auto add = [&](auto& kk, auto& vv, auto u_c) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int tok = t + 2 * u + g;
-      const int64_t at = (int64_t)min(tok, t1 - 1) * stride_n;  // (no branch around a load)
-      kk[u] = kp[at], vv[u] = vp[at];
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const bool ok = t + 2 * u + g < t1;
-      kk[u] = ok ? fmaxf(kk[u], 0.f) : 0.f;
-      vv[u] = ok ? vv[u] : 0.f;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (int u = 0; u < decltype(u_c)::value; ++u) {
+      kk[u] = fmaxf(kk[u], 0.f);
       accS = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[u], kk[u], accS, 0, 0, 0);
       accK += kk[u];
+    }
+  };
+  using U32 = std::integral_constant<int, 32>;  // 64 tokens in flight per wave: a small input is one round trip
+  if ((int64_t)(split_tokens + 64) * stride_n < (1 << 29)) {  // 32-bit offsets; rows past t1 lie outside the resources: zeros
+    const int ld = (int)stride_n * 4, span = n > 0 ? (n - 1) * ld + 4 * D : 0;
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kp), 0, span, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vp), 0, span, 0x00020000);
+    auto pass = [&](int t, auto u_c) {
+      constexpr int U = decltype(u_c)::value;
+      float kk[U], vv[U];
+      int at = (t + g) * ld + 4 * j;
+#pragma unroll
+      for (int u = 0; u < U; ++u, at += 2 * ld) {
+        kk[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rk, at, 0, 0));
+        vv[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rv, at, 0, 0));
+      }
+      add(kk, vv, u_c);
+    };
+    int t = 0;
+#pragma unroll 1
+    for (; t + 64 <= n; t += 64) pass(t, U32{});
+    // (a load outside the resource takes its time all the same)
+    if (n - t > 32) pass(t, U32{});
+    else if (n - t > 16) pass(t, std::integral_constant<int, 16>{});
+    else if (n - t > 0) pass(t, std::integral_constant<int, 8>{});
+  } else {
+    constexpr int U = U32::value;
+    for (int t = 0; t < n; t += 2 * U) {
+      float kk[U], vv[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t at = (int64_t)min(t + 2 * u + g, n - 1) * stride_n + j;  // (no branch around a load)
+        kk[u] = kp[at], vv[u] = vp[at];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const bool ok = t + 2 * u + g < n;
+        kk[u] = ok ? kk[u] : 0.f, vv[u] = ok ? vv[u] : 0.f;
+      }
+      add(kk, vv, U32{});
     }
   }
   const int64_t slot = ((int64_t)(b * h + head) * n_chunks + c) * nsplit + split;
@@ -609,8 +641,9 @@ __global__ __launch_bounds__(256) void linattn_apply32_kernel(
 
 // ----------------------------------------------------------------------------
 // phase 2, fp32 io, on the partial states of one head (one chunk): the sum over the splits is formed here, in the order of
-// linattn_reduce_scan_kernel, so that a short sequence needs two launches.  grid: B * h * 128-token ranges; block 320: waves 0 .. 3
-// 32 tokens each, the fifth takes the state's 33rd row, so that the sums are one round of loads.  The queries are requested first;
+// linattn_reduce_scan_kernel, so that a short sequence needs two launches.  grid: B * h * 128-token ranges (per_range: 2^16 / ranges,
+// rounded up: exact for fewer than 2^13 workgroups); block 320: waves 0 .. 3
+// 32 tokens each, the fifth takes the state's 33rd row, so that the sums are one round of loads.  The partial states are requested first;
 // a workgroup then reads nsplit x 4.2 KB of partial states, four times what its queries are at 16 splits, and that takes less than
 // the third launch: bound by the latency of the two loads.  us, issued eagerly on three sets of inputs in turn, three launches / two:
 // 1024 tokens x 36 heads 15.5 / 14.2, 400 x 70 14.2 / 13.8, 2 x 1024 x 36 20.6 / 17.7.  Both launches keep a head on one XCD: with its
@@ -619,28 +652,30 @@ __global__ __launch_bounds__(256) void linattn_apply32_kernel(
 // ----------------------------------------------------------------------------
 __global__ __launch_bounds__(320) void linattn_apply32_partials_kernel(
     const float* __restrict__ Q, const float* __restrict__ partial, float* __restrict__ out, int N, int h, int nsplit,
-    int64_t q_stride_b, int64_t q_stride_n, int64_t o_stride_b, int64_t o_stride_n, float eps) {
+    uint32_t per_range, int64_t q_stride_b, int64_t q_stride_n, int64_t o_stride_b, int64_t o_stride_n, float eps) {
   constexpr int ROW = D + 4;  // floats of a state row in LDS (conflict-free 16-byte reads down a column)
   __shared__ __attribute__((aligned(16))) float st[(D + 1) * ROW];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int ranges = (N + 127) >> 7, at = xcd_eighths(blockIdx.x, gridDim.x), bh = at / ranges;
-  const int b = bh / h, head = bh - b * h;
+  asm volatile("" ::"s"(Q), "s"(partial), "s"(N), "s"(h), "s"(nsplit), "s"(per_range), "s"(q_stride_b), "s"(q_stride_n));  // (in one wait)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int ranges = (N + 127) >> 7, at = xcd_eighths(blockIdx.x, gridDim.x), bh = (int)((uint32_t)at * per_range >> 16);
+  // the partial states first: their sum is the longer way
+  const int e = min((int)threadIdx.x, STATE_ELEMS / 4 - 1);
+  const float* p0 = partial + (int64_t)bh * nsplit * STATE_ELEMS;
+  f32x4_t v[16];
+#pragma unroll
+  for (int u = 0; u < 16; ++u) v[u] = *reinterpret_cast<const f32x4_t*>(p0 + min(u, nsplit - 1) * STATE_ELEMS + 4 * e);
+  const int b = (int)((uint32_t)bh / (uint32_t)h), head = bh - b * h;
   const int n = lane & 31, g = lane >> 5, tok = (at - bh * ranges) * 128 + wave * 32 + n;
   const bool ok = tok < N && wave < 4;
   f32x4_t q[4];
   const float* qp = Q + (int64_t)b * q_stride_b + (int64_t)min(tok, N - 1) * q_stride_n + head * D + 16 * g;
 #pragma unroll
   for (int i = 0; i < 4; ++i) q[i] = *reinterpret_cast<const f32x4_t*>(qp + 4 * i);
-  const float* p0 = partial + (int64_t)bh * nsplit * STATE_ELEMS;
-  if (const int e = threadIdx.x; e < STATE_ELEMS / 4) {
-    f32x4_t v[16], s = {0.f, 0.f, 0.f, 0.f};
+  f32x4_t s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < 16; ++u) v[u] = *reinterpret_cast<const f32x4_t*>(p0 + (int64_t)min(u, nsplit - 1) * STATE_ELEMS + 4 * e);
-#pragma unroll
-    for (int u = 0; u < 16; ++u)
-      if (u < nsplit) s += v[u];
-    *reinterpret_cast<f32x4_t*>(st + (e >> 3) * ROW + 4 * (e & 7)) = s;
-  }
+  for (int u = 0; u < 16; ++u)
+    if (u < nsplit) s += v[u];
+  if (threadIdx.x < STATE_ELEMS / 4) *reinterpret_cast<f32x4_t*>(st + (e >> 3) * ROW + 4 * (e & 7)) = s;
   __syncthreads();
   if (wave == 4) return;
   float qv[16], den = 0.f;
@@ -1396,8 +1431,8 @@ extern "C" __attribute__((visibility("default"))) int sana_hip_linattn(
                          static_cast<const float*>(v), partial, nullptr, N, h, 1, pl.nsplit, pl.split_tokens, stride_b, stride_n);
       if (hipGetLastError() != hipSuccess) return SANA_ERR_LAUNCH;
       hipLaunchKernelGGL(linattn_apply32_partials_kernel, dim3((N + 127) / 128 * (unsigned)heads), dim3(320), 0, st,
-                         static_cast<const float*>(q), partial, static_cast<float*>(out), N, h, pl.nsplit, q_stride_b, q_stride_n,
-                         o_stride_b, o_stride_n, eps);
+                         static_cast<const float*>(q), partial, static_cast<float*>(out), N, h, pl.nsplit,
+                         (65536u + (N + 127) / 128 - 1) / ((N + 127) / 128), q_stride_b, q_stride_n, o_stride_b, o_stride_n, eps);
       return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
     }
     const int rc = sana_hip_linattn_state(k, v, state, static_cast<char*>(scratch) + at, scratch_bytes - at, B, N, h, d, stride_b,

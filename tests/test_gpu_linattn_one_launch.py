@@ -160,3 +160,19 @@ def test_rows_of_any_distance(cuda, dtype, far):
     _lib.check(lib.sana_hip_linattn(*ptr, out.data_ptr(), None, 0, 1, N, h, 32, 0, src[0].stride(0), 0, src[1].stride(0), 0,
                                     out.stride(0), 1e-15, ops._dt(out), torch.cuda.current_stream().cuda_stream), "sana_hip_linattn")
     assert torch.equal(out[:, :C], want) and bool((out[:, C:] == 3.0).all())
+
+
+@pytest.mark.parametrize("N", [1, 16, 17, 33, 64, 65, 81, 97, 130])
+def test_fp32_splits_of_any_length_and_row_distance(cuda, N):
+    """Phase 1 in passes of 64, 32 and 16 tokens with 32-bit offsets, and on rows too far apart for those, against 64 bits and each other;
+    nothing between the rows or behind them (NaN) is read."""
+    h, C, gen = 3, 96, torch.Generator().manual_seed(N)
+    k, v = (torch.randn(1, N, C, generator=gen).to(cuda) for _ in range(2))
+    want = torch.einsum("nhi,nhj->hij", v[0].double().view(N, h, 32), k[0].double().clamp(min=0).view(N, h, 32))
+    near = ops.linattn_state(k, v)
+    assert _rel(near.view(h, 33, 32)[:, :32], want) < 1e-6
+    assert _rel(near.view(h, 33, 32)[:, 32], k[0].double().clamp(min=0).sum(0).view(h, 32)) < 1e-6
+    for ld in [4 * C] + ([1 << 23] if N <= 17 else []):
+        wide = torch.full(((N + 1) * ld,), float("nan"), device=cuda)[:N * ld].view(1, N, ld)
+        wide[:, :, :C], wide[:, :, C:2 * C] = k, v
+        assert torch.equal(ops.linattn_state(wide[:, :, :C], wide[:, :, C:2 * C]), near)
