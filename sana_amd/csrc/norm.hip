@@ -15,7 +15,8 @@
 // with the row, and the wave sums stay in the vector unit (through LDS a step of the butterfly takes over 100 cycles, twelve of
 // them a row); the row is unpacked once.  us, rows x channels, before and now: 256 x 1152 3.8 -> 3.2, 1024 x 1152 4.3 -> 3.8,
 // 2048 x 1152 5.6 -> 5.0, 1024 x 2240 5.9 -> 5.2, 2048 x 2240 7.6 -> 6.9; 16384 x 2240 33.5 -> 32.5 (vector unit 0.99 busy, at the copy rate).
-// Same bits.
+// Same bits.  The row of a wave is uniform, its offsets 32-bit and its division too, the arguments one wait: from a graph, so / before
+// 256 x 1152 2.6 / 2.7, 1024 x 1152 3.4 / 3.7, 1024 x 2240 5.0 / 5.5, 2916 x 2240 9.1 / 9.7, 4680 x 2240 13.1 / 13.7, 16384 x 2240 33.1 / 33.3.
 #include "common.h"
 
 // No implicit fused multiply-adds in this file: the epilogues reproduce the stock op chain's roundings (product
@@ -62,15 +63,17 @@ __global__ __launch_bounds__(256) void ln_modulate_kernel(const uint16_t* __rest
                                                           uint16_t* __restrict__ out, int64_t M, int C,
                                                           int64_t ldx, int64_t ldy, int64_t lds, int64_t ldo,
                                                           int rows_per_mod, int64_t mod_stride, float eps) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  asm volatile("" ::"s"(x), "s"(scale), "s"(shift), "s"(M), "s"(C), "s"(ldx), "s"(rows_per_mod), "s"(mod_stride));  // (the arguments in one wait)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + wave;
   if (row >= M) return;  // no barriers in this kernel
   const int nchunks = C >> 3;
   const uint16_t* xr = x + row * ldx;
-  const int64_t mod = (row / rows_per_mod) * mod_stride;
+  // (one row of the modulation, or rows that 32 bits count: a 64-bit division is longer than the wait for the row)
+  const int64_t mod = M <= rows_per_mod ? 0 : (M >> 32 ? row / rows_per_mod : (int64_t)((uint32_t)row / (uint32_t)rows_per_mod)) * mod_stride;
   // A lane's chunks, past the row's end its last one once more: no branch around a load, all of them in flight at once.
   auto chunk = [&](const uint16_t* p, int i) {
-    return reinterpret_cast<const u32x4_t*>(p + 8 * min(lane + 64 * i, nchunks - 1));
+    return reinterpret_cast<const u32x4_t*>(reinterpret_cast<const char*>(p) + 16u * (uint32_t)min(lane + 64 * i, nchunks - 1));
   };
   constexpr bool AHEAD = NCH <= 5;  // the modulation rows with the row itself, while registers allow
   u32x4_t raw[NCH], b[ADD ? NCH : 1], sc[AHEAD ? NCH : 1], sh[AHEAD ? NCH : 1];
