@@ -132,7 +132,11 @@ __device__ __forceinline__ void g8_state_tile(f32x4_t (&acc)[4][8], const float 
 //
 // Workgroups are persistent (one per compute unit, every 256th tile): the first two k-tiles of the next tile are
 // requested in front of a tile's epilogue, whose rows go through 8 KB (NB = 4) per wave beside the stages and leave those to
-// the loads.
+// the loads.  At NB = 3 the four waves of a wm share the rows: a wave's 48 channels are 96 bytes, and 64-byte sectors written half by one
+// wave and half by another made the epilogue 8 - 9 us a tile, whatever it computes, where the wider tile of NB = 4 takes 6.  us, so /
+// now, weights cold: 2048 x 5760 x 1152 SiLU 31.3 / 28.2, 4096 x 5760 x 1152 SiLU 59.4 / 50.8, 1024 x 11200 x 2240 SiLU 51.0 / 48.5, 2916 x 6720 x
+// 2240 84.6 / 78.0, 4680 x 2240 x 2240 bias 46.1 / 43.1, gated 48.3 / 47.6.  (The residual touched from within the loop, six k-tiles in front of
+// the epilogue: 1 us more a launch.)
 template <int EPI, int NB, int TAPS = 0, typename T = BF16>
 __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
                                                     const EpiArgs ep, uint16_t* __restrict__ C, int M, int N, int K,
@@ -142,9 +146,12 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
   constexpr int A_STAGE = BM * 128, W_STAGE = BN * 128, W_BASE = 2 * A_STAGE;
   constexpr int NP = (NB + 1) / 2;  // pieces of 8 (the last one of 4 if NB is odd) channels per lane and token
   constexpr int STORES = 4 * NB;    // store instructions of an epilogue, per wave
-  constexpr int OUT_ROW = 32 * NB, OUT_BYTES = 32 * OUT_ROW;  // per wave: 32 finished rows of its 16*NB channels
+  // The epilogue's rows, 32 at a time: per wave its 16*NB channels; NB = 3, whose 96 bytes a wave are no whole 64-byte sectors: the
+  // tile's 192 channels by the four waves of a wm, in two buffers.
+  constexpr bool SHARED = NB == 3;
+  constexpr int OUT_ROW = SHARED ? 2 * BN : 32 * NB, OUT_BYTES = 32 * OUT_ROW, OUT_BUF = SHARED ? 2 * OUT_BYTES : 0;
   static_assert(EPI != SANA_EPI_QKV_STATE || (NB == 4 && !is_f16<T> && !TAPS), "the fused qkv projection: 256-wide bf16 tiles");
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[W_BASE + 2 * W_STAGE + 8 * OUT_BYTES];
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[W_BASE + 2 * W_STAGE + (SHARED ? 4 : 8) * OUT_BYTES];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave >> 2, wn = wave & 3;
   // The lane index, hidden from the optimiser: what is derived from it per tile (load offsets, epilogue addresses) would
@@ -453,24 +460,25 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
     // 64 separate 16-byte pieces (measured ~100 cycles each, against ~12 for whole row segments), so the rows go
     // through the wave's own corner of LDS, 32 tokens at a time: written as the lane holds them, read back row by row.
     // (asm LDS accesses: see the fragment reads.)
-    constexpr int PPR = 2 * NB;                       // 16-byte pieces of a row
-    auto out_at = [&](int row, int pc) -> uint32_t {  // swizzled: conflict-free both ways (NB = 3: two-way)
-      const int k = NB == 4 ? (row >> 1) & 7 : NB == 2 ? (row >> 2) & 3 : 0;
+    constexpr int PPR = OUT_ROW / 16;                 // 16-byte pieces of a row
+    auto out_at = [&](int row, int pc) -> uint32_t {  // swizzled (NB = 3: within eight pieces): conflict-free both ways
+      const int k = NB == 2 ? (row >> 2) & 3 : (row >> 1) & 7;
       return row * OUT_ROW + ((pc ^ k) << 4);
     };
-    const uint32_t out0 = lds0 + W_BASE + 2 * W_STAGE + wave * OUT_BYTES;
+    const uint32_t out0 = lds0 + W_BASE + 2 * W_STAGE + (SHARED ? wm : wave) * OUT_BYTES;
+    const int pc0 = SHARED ? 2 * NB * wn : 0;         // the wave's first piece of a row
     uint32_t wr[NP], rd[NB];   // LDS addresses: written pieces of row fr; pieces read for store s of a round
     int coff[NB], roff[NB];    // byte offsets of store s of the first round in C and in the residual
     int row_s[NB], n_s[NB];
 #pragma unroll
     for (int c = 0; c < NP; ++c)
-      wr[c] = out0 + ((NB & 1) && c == NP - 1 ? out_at(fr, 4 * c + (fg >> 1)) + 8 * (fg & 1) : out_at(fr, 4 * c + fg));
+      wr[c] = out0 + ((NB & 1) && c == NP - 1 ? out_at(fr, pc0 + 4 * c + (fg >> 1)) + 8 * (fg & 1) : out_at(fr, pc0 + 4 * c + fg));
 #pragma unroll
     for (int s = 0; s < NB; ++s) {
-      const int idx = lane + 64 * s, row = idx / PPR, pc = idx % PPR;
+      const int idx = lane + 64 * s, row = (SHARED ? 8 * wn : 0) + idx / PPR, pc = idx % PPR;
       rd[s] = out0 + out_at(row, pc);
       row_s[s] = 128 * wm + row;
-      n_s[s] = n0t + wn * 16 * NB + 8 * pc;
+      n_s[s] = n0t + (SHARED ? 0 : wn * 16 * NB) + 8 * pc;
       coff[s] = n_s[s] < n_end ? (row * (int)ldc + n_s[s]) * 2 : (int)kOut;
       roff[s] = n_s[s] < n_end ? (row_s[s] * (int)ep.ldr + n_s[s]) * 2 : (int)kOut;
     }
@@ -502,7 +510,7 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
     auto convert = [&](auto g_c) {  // round g: token tiles 2g, 2g + 1
       constexpr int g = decltype(g_c)::value;
       auto tile = [&](auto jj_c) {
-        constexpr int jj = decltype(jj_c)::value, j = 2 * g + jj, O = jj * 16 * OUT_ROW;  // (the swizzle repeats every 16 rows)
+        constexpr int jj = decltype(jj_c)::value, j = 2 * g + jj, O = jj * 16 * OUT_ROW + (g & 1) * OUT_BUF;  // (the swizzle repeats every 16 rows)
 #pragma unroll
         for (int c = 0; c < NP; ++c) {
           if ((NB & 1) && c == NP - 1) {
@@ -518,15 +526,20 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
       tile(C0{});
       tile(C1{});
     };
-    auto store = [&](int g) {
+    auto store = [&](auto g_c) {
+      constexpr int g = decltype(g_c)::value;
+      if (SHARED) {  // (a wave that is here has read the round before the last, whose buffer the next round is written to)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        half_end();
+      }
       u32x4_t o[NB];
 #pragma unroll
-      for (int s = 0; s < NB; ++s) o[s] = gemm_lds_read<0>(rd[s]);  // (a wave's LDS accesses are in order)
+      for (int s = 0; s < NB; ++s) o[s] = gemm_lds_read<(g & 1) * OUT_BUF>(rd[s]);  // (a wave's LDS accesses are in order)
 #pragma unroll
       for (int s = 0; s < NB; ++s) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(o[s])::"memory");
 #pragma unroll
       for (int s = 0; s < NB; ++s) {
-        if (GATED) {
+        if constexpr (GATED) {
           u32x4_t gt8 = gate[s];
           if (ep.gate && !one_gate) {
             const int m = min(m0t + row_s[s] + 32 * g, M - 1);
@@ -540,14 +553,16 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
         __builtin_amdgcn_raw_buffer_store_b128(o[s], rsrc_c, coff[s] + 64 * g * (int)ldc, 0, kBufferNt);
       }
     };
+    using C2 = std::integral_constant<int, 2>;
+    using C3 = std::integral_constant<int, 3>;
     convert(C0{});
-    store(0);
+    store(C0{});
     convert(C1{});
-    store(1);
-    convert(std::integral_constant<int, 2>{});
-    store(2);
-    convert(std::integral_constant<int, 3>{});
-    store(3);
+    store(C1{});
+    convert(C2{});
+    store(C2{});
+    convert(C3{});
+    store(C3{});
     if (id >= total) return;
   }
 #undef G8_PIN
