@@ -857,11 +857,15 @@ struct Tile16 {
 // the small tiles were never more than 2 % ahead, and 300 x 17920 x 2240 is 48.7 us in 128 x 128 and 40.4 in 256 x 192: hence
 // one_round.  us, the tiles and kernels before this table / now, both timed so: 256 x 1152 x 2880 15.3 / 10.3 (halved), 1024 x 2240 x
 // 2240 23.6 / 18.7, 2048 x 1152 x 2880 28.6 / 21.6, 4096 x 1152 x 1152 20.7 / 17.7, 4096 x 1152 x 2880 35.0 / 31.4.
+// The 192-wide tile's fixed part was 7.9 before the waves shared its rows (gemm8.h).  With 4.9, of the shapes that this changes (200 ..
+// 20000 tokens, widths as above), kernel as it is, 7.9 / 4.9: 14208 x 3456 x 1152 109 / 98, 16576 x 2240 x 2240 167 / 157, 7246 x 9216 x 1152 140 /
+// 133, 6017 x 11200 x 2240 251 / 241, 2079 x 18432 x 1152 88 / 84, 12423 x 2240 x 2240 115 / 111; 18219 x 9216 x 1152 307 / 311, 6400 x 6720 x 2240
+// 145 / 151; 0.979 on the mean of 48.  (3.9: 993 x 18432 x 1152 42.7 / 48.1.)
 constexpr Tile16 kTiles16[] = {
     {64, 64, 512, 256, 257, 3.0, 0.288, 0.503, true, 0.165, 0.26}, {64, 128, 256, 32, 256, 3.9, 0.350, 0.414, true},
     {96, 128, 256, 32, 256, 3.7, 0.439, 0.466, true},  {128, 128, 256, 32, 256, 3.9, 0.454, 0.541, true},
     {128, 160, 256, 32, 256, 4.3, 0.517, 0.643, true}, {192, 128, 256, 32, 256, 4.7, 0.497, 0.687, true},
-    {256, 128, 256, 32, 256, 5.1, 0.624, 0.825, true}, {256, 192, 256, 32, 256, 7.9, 0.628, 1.150},
+    {256, 128, 256, 32, 256, 5.1, 0.624, 0.825, true}, {256, 192, 256, 32, 256, 4.9, 0.628, 1.150},
     {256, 256, 256, 32, 256, 5.3, 0.999, 1.404},       {256, 288, 256, 32, 256, 9.5, 0.955, 1.603},
 };
 constexpr int kTile192 = 7, kTile256 = 8, kTile288 = 9;
@@ -1281,7 +1285,9 @@ SANA_API int sana_hip_tconv_residual(const void* X, const void* W, void* out, in
   // one of the three widest tiles: the others have no taps
   const int k = taps * C;
   const bool brief = k < kShortK, may288 = ldw < kMaxStride288;
-  const double us192 = cost16(brief ? kTilesShort[1] : kTiles16[kTile192], M, C, k);
+  // (192 channels: with the residual the epilogue is still what it was before its rows were shared)
+  constexpr Tile16 gated192 = {256, 192, 256, 32, 256, 7.9, 0.628, 1.150};
+  const double us192 = cost16(brief ? kTilesShort[1] : gated192, M, C, k);
   const double us256 = cost16(brief ? kTilesShort[2] : kTiles16[kTile256], M, C, k), us = std::min(us192, us256);
   if (may288 && (brief ? short_takes_288(M, C, k, us) : cost16(kTiles16[kTile288], M, C, k) < us))
     return gemm288_launch(x, w, e, o, M, C, k, ldx, ldw, ldo, SANA_EPI_GATE_RES, false, &tp, s);
