@@ -414,7 +414,9 @@ __global__ __launch_bounds__(512) void gemm288_kernel(const uint16_t* __restrict
           }
           o[s] = gate_res8v<T>(o[s], g8, res[j][s]);
         }
-        __builtin_amdgcn_raw_buffer_store_b128(o[s], rsrc_c, off[s], 0, kBufferNt);  // (the hint: as in gemm8_kernel)
+        // (cacheable: a wave column's 288 bytes end within a 64-byte sector, which the L2 puts together; with the non-temporal hint of gemm8_kernel /
+        // without: a step of 16 x 1024 px 8276 / 8217 us, 4096 px 7993 / 7906, a streamed chunk 856 / 847)
+        __builtin_amdgcn_raw_buffer_store_b128(o[s], rsrc_c, off[s], 0, 0);
       }
       if constexpr (GATED && j + 2 < TM) fetch(j + 2);
     };
