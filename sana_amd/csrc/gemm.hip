@@ -449,7 +449,7 @@ __device__ __forceinline__ void finish_tile16(f32x4_t (&acc)[2 * NI][8], const u
 }
 
 // ============================================================================
-// Pipelined kernel (K % 32 == 0, K >= 64; bf16 and int8 weights): 256 threads, one
+// Pipelined kernel (K % 32 == 0, K >= 64; int8 weights): 256 threads, one
 // wave per SIMD with the whole register file (256 accumulators + 256 VGPRs), each
 // wave a sub-tile of 128 tokens x 32*NI channels = 2*NI x 8 MFMA tiles of 16x16
 // (NI = 4: 128x128; NI = 3 narrows the workgroup's channel tile to 192 where that fills
@@ -458,16 +458,13 @@ __device__ __forceinline__ void finish_tile16(f32x4_t (&acc)[2 * NI][8], const u
 // else hides a stalled memory instruction, so the main loop is one hand-ordered
 // stream (pinned with sched_barrier): a k-tile is two k-steps of 32 = 2 * 16*NI MFMA
 // slots of 16 cycles, and a lone wave issues about one other instruction per 5 cycles,
-// so a slot carries at most a fragment read, a store or a load (bf16):
-//   * k-step 0: the fragments of k-step 1, and all staging -- quad q (k-tile kt+1) is
-//     stored into the other LDS stage and the same registers are re-loaded with
-//     k-tile kt+2 one slot later, so every global load has a whole k-tile (about
-//     1 us) to land and one 64-register set is enough;
-//   * the only barrier sits right behind it, and the next tile's k-step-0 fragments
-//     are read over the rest of k-step 1, which runs from the other fragment buffer
-//     (int8 weights: 16 values per quad, converted two at a time in the MFMA slots
-//     before they are stored, the quad reloaded after its last piece; their barrier
-//     stays at the end of the k-tile).
+// so a slot carries at most a fragment read, a store or a load:
+//   * k-step 0: the fragments of k-step 1; A quad q (k-tile kt+1) is stored into the
+//     other LDS stage and the same registers are re-loaded with k-tile kt+2 one slot
+//     later, so every global load has a whole k-tile (about 1 us) to land;
+//   * weights, 16 values per quad, are converted two at a time in the MFMA slots before
+//     they are stored, the quad reloaded after its last piece; the only barrier stands
+//     at the end of the k-tile.
 // The MFMAs are asm statements with the accumulator tied in and out (see mfma_acc).
 // Rows past M / N read as zero (buffer range check) and only feed outputs that are
 // never stored; the last k-tile runs just the k-steps that exist.
@@ -475,23 +472,24 @@ __device__ __forceinline__ void finish_tile16(f32x4_t (&acc)[2 * NI][8], const u
 // SPLIT (split-k, for shapes with too few tiles to fill the chip): grid row z multiplies its own range of
 // k-tiles and stores the raw fp32 accumulators to C taken as float [gridDim.y][M][N]; splitk_epilogue_kernel
 // adds the ranges up in order and applies the epilogue.
-template <bool W8, int EPI, int NI, bool SPLIT = false, typename T = BF16>
-__global__ __launch_bounds__(256) void gemm4_kernel(const uint16_t* __restrict__ A_, const void* __restrict__ Wv_,
+template <int EPI, int NI, bool SPLIT = false>
+__global__ __launch_bounds__(256) void gemm4_kernel(const uint16_t* __restrict__ A_, const int8_t* __restrict__ W_,
                                                     const float* __restrict__ scale, const EpiArgs ep,
                                                     uint16_t* __restrict__ C, int M, int N, int K_, int64_t lda,
                                                     int64_t ldw, int64_t ldc, int tiles_t, int tiles_c,
                                                     const Taps tp) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * TILE_BYTES];  // [stage][A | W]
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  typedef BF16 T;
   const uint16_t* A = A_;
-  const void* Wv = Wv_;
+  const int8_t* W = W_;
   int K = K_;
   if (SPLIT) {  // this grid row's k range becomes "the" K of everything below
     const int z = blockIdx.y;
     const int kb = (z * tp.split_tiles + min(z, tp.split_rem)) * BK;
     const int kn = (tp.split_tiles + (z < tp.split_rem ? 1 : 0)) * BK;
     A += kb;
-    Wv = static_cast<const char*>(Wv_) + (int64_t)kb * (W8 ? 1 : 2);
+    W += kb;
     K = min(K_ - kb, kn);
   }
   const int total = tiles_t * tiles_c;
@@ -513,35 +511,29 @@ __global__ __launch_bounds__(256) void gemm4_kernel(const uint16_t* __restrict__
   constexpr int BCN = 64 * NI;  // channels per workgroup: two waves x NI MFMA tiles of 32
   const int m0 = tile_t * BT, n0 = tile_c * BCN;
 
-  // global -> VGPR -> LDS: thread -> k chunk tid%8, rows tid/8 + 32*q, q < 8 for A and q < 2*NI for bf16 W.
-  // int8 W: thread -> 16-value chunk tid%4, rows tid/4 + 64*q (q < NI); dequantised on the way to LDS.
+  // global -> VGPR -> LDS: thread -> k chunk tid%8, rows tid/8 + 32*q, q < 8 for A.
+  // W: thread -> 16-value chunk tid%4, rows tid/4 + 64*q (q < NI); dequantised on the way to LDS.
   const int g_chunk = tid & 7, g_row = tid >> 3;
   const int a_last = min(BT, M - m0) - 1, w_last = min(BCN, N - n0) - 1;  // last valid row of each tile
-  const uint32_t ulda = (uint32_t)lda, uldw = (uint32_t)ldw;
+  const uint32_t ulda = (uint32_t)lda;
   const int a_dst0 = swz(g_row, g_chunk);               // rows +32*q keep the key: +4096 bytes each
-  const int w_dst0 = TILE_BYTES + swz(g_row, g_chunk);  // LDS rows g_row + 32*q; the weight-row permutation is on the global side
   // LDS row L of a wave's block of 32*NI weight rows belongs to MFMA tile L / 16 as its row L % 16 = 4*g + r, and
   // holds channel 8*NI*g + 4*(L / 16) + r of the block: a lane's accumulators (tile i, registers r) are then the
-  // 8*NI contiguous channels 8*NI*g + 4*i + r.  The thread's quad q (LDS rows g_row + 32*q) is channel
-  // w_chan0 + 8*(q % NI) + 32*NI*(q / NI) of the tile.
-  const int w_chan0 = 8 * NI * ((g_row >> 2) & 3) + 4 * (g_row >> 4) + (g_row & 3);
-  constexpr int NWQ = W8 ? NI : 2 * NI;  // W quads per thread
-  constexpr int NQ = 8 + NWQ;
+  // 8*NI contiguous channels 8*NI*g + 4*i + r.
+  constexpr int NQ = 8 + NI;
   u32x4_t rs[NQ];  // the k-tile in flight: A quads 0..7, then the W quads
   const int q_chunk = tid & 3, q_row = tid >> 2;
   const int q_dst_lo = TILE_BYTES + swz(q_row, 2 * q_chunk);  // LDS rows q_row + 64*q: +8192 bytes, same key
   const int q_dst_hi = TILE_BYTES + swz(q_row, 2 * q_chunk + 1);
   float wscale[NI], woff[NI];
   int q_voff[NI];  // int8 quads: byte offset of the channel that LDS row q_row + 64*q holds
-  if (W8) {
 #pragma unroll
-    for (int q = 0; q < NI; ++q) {
-      const int L = q_row + 64 * q, blk = L / (32 * NI), l = L % (32 * NI);
-      const int chan = blk * 32 * NI + 8 * NI * ((l >> 2) & 3) + 4 * (l >> 4) + (l & 3);
-      q_voff[q] = chan * (int)ldw + 16 * q_chunk;
-      wscale[q] = scale[n0 + min(chan, w_last)];
-      woff[q] = -128.f * wscale[q];
-    }
+  for (int q = 0; q < NI; ++q) {
+    const int L = q_row + 64 * q, blk = L / (32 * NI), l = L % (32 * NI);
+    const int chan = blk * 32 * NI + 8 * NI * ((l >> 2) & 3) + 4 * (l >> 4) + (l & 3);
+    q_voff[q] = chan * (int)ldw + 16 * q_chunk;
+    wscale[q] = scale[n0 + min(chan, w_last)];
+    woff[q] = -128.f * wscale[q];
   }
   u32x4_t dq[2];  // dequantised halves of the int8 quad being converted
 
@@ -569,27 +561,21 @@ __global__ __launch_bounds__(256) void gemm4_kernel(const uint16_t* __restrict__
   const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(A + (int64_t)m0 * lda), 0, (int)a_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<char*>(static_cast<const char*>(Wv) + (int64_t)n0 * ldw * (W8 ? 1 : 2)), 0,
-      (int)(((int64_t)w_last * ldw + K) * (W8 ? 1 : 2)), 0x00020000);
+      const_cast<int8_t*>(W + (int64_t)n0 * ldw), 0, (int)((int64_t)w_last * ldw + K), 0x00020000);
   const int voff_a = (g_row * (int)ulda + 8 * g_chunk) * 2;
-  const int voff_w = (w_chan0 * (int)uldw + 8 * g_chunk) * 2;  // bf16 weights
-  const int step_a = 32 * (int)ulda * 2, step_w1 = (int)uldw * 2;
+  const int step_a = 32 * (int)ulda * 2;
   auto gload = [&](int q, int k0) {
     if (q < 8) {
       const int off = voff_a + (q * step_a + k0 * 2);
       const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, off, 0, 0);
       rs[q] = __builtin_bit_cast(u32x4_t, v);
     } else {
-      const int wq = q - 8;
-      const int off = W8 ? q_voff[wq] + k0 : voff_w + ((8 * (wq % NI) + 32 * NI * (wq / NI)) * step_w1 + k0 * 2);
-      const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, off, 0, 0);
+      const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, q_voff[q - 8] + k0, 0, 0);
       rs[q] = __builtin_bit_cast(u32x4_t, v);
     }
   };
-  auto lstore = [&](int q, int stage) {  // A quads, bf16 W quads
-    unsigned char* base = smem + stage * 2 * TILE_BYTES;
-    if (q < 8) *reinterpret_cast<u32x4_t*>(base + a_dst0 + 4096 * q) = rs[q];
-    else *reinterpret_cast<u32x4_t*>(base + w_dst0 + 4096 * (q - 8)) = rs[q];
+  auto lstore = [&](int q, int stage) {  // A quads
+    *reinterpret_cast<u32x4_t*>(smem + stage * 2 * TILE_BYTES + a_dst0 + 4096 * q) = rs[q];
   };
   // int8 quad wq (16 values), piece 0..7 = two values each: convert, and store a 16-byte half when complete
   auto dequant_piece = [&](int wq, int piece, int stage) {
@@ -624,11 +610,9 @@ __global__ __launch_bounds__(256) void gemm4_kernel(const uint16_t* __restrict__
 #pragma unroll
   for (int q = 0; q < NQ; ++q) gload(q, 0);
 #pragma unroll
-  for (int q = 0; q < (W8 ? 8 : NQ); ++q) lstore(q, 0);
-  if (W8) {
+  for (int q = 0; q < 8; ++q) lstore(q, 0);
 #pragma unroll
-    for (int n = 0; n < 8 * NI; ++n) dequant_piece(n >> 3, n & 7, 0);
-  }
+  for (int n = 0; n < 8 * NI; ++n) dequant_piece(n >> 3, n & 7, 0);
 #pragma unroll
   for (int q = 0; q < NQ; ++q) gload(q, BK);
   __syncthreads();
@@ -637,19 +621,12 @@ __global__ __launch_bounds__(256) void gemm4_kernel(const uint16_t* __restrict__
 
   // Slots: a k-tile is two k-steps of 32 = 2 * SL MFMAs of 16 cycles each, and a lone wave issues about one
   // other instruction per 5 cycles, so no slot carries more than a fragment read or a store or a load.
-  //  * k-step 0: the fragments of k-step 1 (read r at slot r*SL/NFR), and all staging -- quad q stored to the other
-  //    LDS stage at slot 1 + q*QSTRIDE and re-loaded (k-tile kt+2) one slot later;
-  //  * the barrier right behind it (slot SL + 2), and the next tile's k-step-0 fragments spread over the rest
-  //    of k-step 1, which runs from the other fragment buffer.
-  // int8 weights convert 8*NI pieces in the MFMA slots as well, so their barrier stays at the end of the k-tile.
+  // The fragments of k-step 1 are read in k-step 0 (read r at slot r*SL/NFR), the weights converted in 8*NI pieces over the whole
+  // k-tile; the barrier and the next tile's k-step-0 fragments stand at its end.
   constexpr int SL = 8 * NWT, TS = 2 * SL;
-  constexpr int BAR = W8 ? TS - NFR - 1 : SL + 2;
-  constexpr int RSTR = W8 ? 1 : (TS - BAR - 1 - 8) / NFR;  // spacing of the reads behind the barrier
-  constexpr int QSTRIDE = SL / NQ;                           // bf16: spacing of the staging quads
-  constexpr int PSTR = (BAR - 4) / (8 * NI);                 // int8: piece n (two values) at slot 2 + n*PSTR
-  static_assert(W8 || (QSTRIDE >= 2 && 1 + (NQ - 1) * QSTRIDE < BAR - 2 && RSTR >= 1 && BAR + 1 + (NFR - 1) * RSTR < TS),
-                "staging does not fit in front of the barrier");
-  static_assert(!W8 || (4 * 7 + 1 < BAR && PSTR >= 1), "staging does not fit in front of the barrier");
+  constexpr int BAR = TS - NFR - 1;
+  constexpr int PSTR = (BAR - 4) / (8 * NI);                 // piece n (two values) at slot 2 + n*PSTR
+  static_assert(4 * 7 + 1 < BAR && PSTR >= 1, "staging does not fit in front of the barrier");
   // The MFMAs below are asm statements: the compiler neither knows that they read the accumulators through the
   // matrix pipe nor places the wait states such a read needs behind the VALU writes that zeroed them.  Pin the
   // order by hand: every accumulator passes through an empty asm statement (its zeroing is complete, in program
@@ -679,23 +656,17 @@ __global__ __launch_bounds__(256) void gemm4_kernel(const uint16_t* __restrict__
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // own LDS stores done; no fence: loads stay in flight
           __builtin_amdgcn_s_barrier();
           asm volatile("" ::: "memory");
-        } else if (slot > BAR && (slot - BAR - 1) % RSTR == 0 && (slot - BAR - 1) / RSTR < NFR) {
-          fread(stn, 0, 0, (slot - BAR - 1) / RSTR);
+        } else if (slot > BAR && slot - BAR - 1 < NFR) {
+          fread(stn, 0, 0, slot - BAR - 1);
         }
-        if (!W8) {
-          if (slot >= 1 && (slot - 1) % QSTRIDE == 0 && (slot - 1) / QSTRIDE < NQ) lstore((slot - 1) / QSTRIDE, cur ^ 1);
-          if (slot >= 2 && (slot - 2) % QSTRIDE == 0 && (slot - 2) / QSTRIDE < NQ)
-            gload((slot - 2) / QSTRIDE, (kt + 2) * BK);
-        } else {
-          // A quad q: store at slot 4q, reload at 4q+1.  int8 piece n at slot 2 + n*PSTR (its half is stored
-          // with pieces 3 and 7), the quad is reloaded one slot after its last piece.
-          if (slot % 4 == 0 && slot / 4 < 8) lstore(slot / 4, cur ^ 1);
-          if (slot % 4 == 1 && slot / 4 < 8) gload(slot / 4, (kt + 2) * BK);
-          if (slot >= 2 && (slot - 2) % PSTR == 0 && (slot - 2) / PSTR < 8 * NI)
-            dequant_piece(((slot - 2) / PSTR) >> 3, ((slot - 2) / PSTR) & 7, cur ^ 1);
-          if (slot >= 3 && (slot - 3) % PSTR == 0 && (slot - 3) / PSTR < 8 * NI && (((slot - 3) / PSTR) & 7) == 7)
-            gload(8 + (((slot - 3) / PSTR) >> 3), (kt + 2) * BK);
-        }
+        // A quad q: store at slot 4q, reload at 4q+1.  Piece n at slot 2 + n*PSTR (its half is stored with pieces 3 and 7), the quad
+        // is reloaded one slot after its last piece.
+        if (slot % 4 == 0 && slot / 4 < 8) lstore(slot / 4, cur ^ 1);
+        if (slot % 4 == 1 && slot / 4 < 8) gload(slot / 4, (kt + 2) * BK);
+        if (slot >= 2 && (slot - 2) % PSTR == 0 && (slot - 2) / PSTR < 8 * NI)
+          dequant_piece(((slot - 2) / PSTR) >> 3, ((slot - 2) / PSTR) & 7, cur ^ 1);
+        if (slot >= 3 && (slot - 3) % PSTR == 0 && (slot - 3) / PSTR < 8 * NI && (((slot - 3) / PSTR) & 7) == 7)
+          gload(8 + (((slot - 3) / PSTR) >> 3), (kt + 2) * BK);
         SANA_G4_PIN();
       }
     }
@@ -738,35 +709,52 @@ __global__ __launch_bounds__(256) void gemm4_kernel(const uint16_t* __restrict__
   finish_tile16<EPI, NI, SPLIT, T>(acc, bpk, smem, ep, C, M, N, ldc, m0, n0);
 }
 
-// Second half of a split-k GEMM: partial[S][M][N] (fp32) -> C = epilogue(sum over the S k-ranges, added in
-// order).  One thread per row and 8 channels; the same epilogue functions as the fused path.
+// Second half of a split-k GEMM: partial[S][M][N] (fp32) -> C = epilogue(sum over the S <= 8 k-ranges, added in
+// order).  One thread per row and 8 channels; the same epilogue functions as the fused path.  All planes, the residual and the gate are
+// requested at once (plane by plane 0.3 us more a launch); the rest is the planes, 46 MB written and read at 1024 x 2240 in five ranges.
 template <int EPI, typename T = BF16>
 __global__ __launch_bounds__(256) void splitk_epilogue_kernel(const float* __restrict__ partial, int S,
                                                                const EpiArgs ep, uint16_t* __restrict__ C, int M, int N,
                                                                int64_t ldc) {
-  const int chunks = N >> 3;
-  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (id >= (int64_t)M * chunks) return;
-  const int m = (int)(id / chunks), n = (int)(id - (int64_t)m * chunks) * 8;
+  const uint32_t chunks = N >> 3, id = blockIdx.x * 256u + threadIdx.x;  // (M * N * 4 < 2^31)
+  if (id >= M * chunks) return;
+  const int m = (int)(id / chunks), n = (int)(id - m * chunks) * 8;
   const f32x4_t* p = reinterpret_cast<const f32x4_t*>(partial + (int64_t)m * N + n);
   const int64_t plane = (int64_t)M * N / 4;
-  f32x4_t lo = p[0], hi = p[1];
-  for (int z = 1; z < S; ++z) {
-    lo += p[z * plane];
-    hi += p[z * plane + 1];
+  constexpr bool GATED = EPI == SANA_EPI_GATE_RES;
+  u32x4_t b = {0u, 0u, 0u, 0u}, g, r;
+  if (EPI != SANA_EPI_NONE && ep.bias) b = *reinterpret_cast<const u32x4_t*>(ep.bias + n);
+  if constexpr (GATED) {
+    g = *reinterpret_cast<const u32x4_t*>(ep.gate + (int64_t)((uint32_t)m / (uint32_t)ep.rows_per_gate) * ep.gate_stride + n);
+    r = *reinterpret_cast<const u32x4_t*>(ep.res + (int64_t)m * ep.ldr + n);
   }
-  const float a[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-  float bv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if (EPI != SANA_EPI_NONE && ep.bias) {
-    const u32x4_t b = *reinterpret_cast<const u32x4_t*>(ep.bias + n);
+  f32x4_t lo, hi;
+  auto sum = [&](auto s_c) {
+    constexpr int Z = decltype(s_c)::value;
+    f32x4_t l[Z], h[Z];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      bv[2 * e] = lo16<T>(b[e]);
-      bv[2 * e + 1] = hi16<T>(b[e]);
-    }
+    for (int z = 0; z < Z; ++z) l[z] = p[z * plane], h[z] = p[z * plane + 1];
+    lo = l[0], hi = h[0];
+#pragma unroll
+    for (int z = 1; z < Z; ++z) lo += l[z], hi += h[z];
+  };
+  switch (S) {
+    case 2: sum(std::integral_constant<int, 2>{}); break;
+    case 3: sum(std::integral_constant<int, 3>{}); break;
+    case 4: sum(std::integral_constant<int, 4>{}); break;
+    case 5: sum(std::integral_constant<int, 5>{}); break;
+    case 6: sum(std::integral_constant<int, 6>{}); break;
+    case 7: sum(std::integral_constant<int, 7>{}); break;
+    default: sum(std::integral_constant<int, 8>{}); break;  // (plan_gemm: 2 .. 8)
   }
-  u32x4_t o = epi_pack8<EPI == SANA_EPI_GATE_RES ? SANA_EPI_BIAS : EPI, T>(a, bv);
-  if (EPI == SANA_EPI_GATE_RES) o = gate_res8<T>(o, ep, m, n);
+  float a[8], bv[8];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    a[e] = lo[e], a[4 + e] = hi[e];
+    bv[2 * e] = lo16<T>(b[e]), bv[2 * e + 1] = hi16<T>(b[e]);
+  }
+  u32x4_t o = epi_pack8<GATED ? SANA_EPI_BIAS : EPI, T>(a, bv);
+  if constexpr (GATED) o = gate_res8v<T>(o, g, r);
   *reinterpret_cast<u32x4_t*>(C + (int64_t)m * ldc + n) = o;
 }
 
@@ -962,48 +950,53 @@ SplitWay split_way(const GemmPlan& pl, int M, int N, int K) {
 }
 bool split_pays(const GemmPlan& pl, int M, int N, int K) { return split_way(pl, M, N, K) != SplitWay::no; }
 
-// The pipelined kernel: split over k into pl.S ranges (ws holds the partial planes), or, int8 weights, unsplit (ws null).
-template <bool W8, int NI, typename T = BF16>
+// K split into pl.S ranges (ws holds the partial planes): tiles of 256 x 192, which is pick_ni's choice wherever plan_gemm splits (one round).
+template <bool W8, typename T>
+int launch_split(const uint16_t* a, const void* W, const float* scale, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
+                 int64_t ldw, int64_t ldc, int epilogue, hipStream_t s, const GemmPlan& pl, float* ws) {
+  const int tiles_t = (M + BT - 1) / BT, tiles_c = (N + 191) / 192;
+  if constexpr (W8) {
+    const Taps split = {0, 0, 0, pl.tiles, pl.rem, nullptr};
+    hipLaunchKernelGGL((gemm4_kernel<SANA_EPI_NONE, 3, true>), dim3((unsigned)(tiles_t * tiles_c), (unsigned)pl.S), dim3(256), 0, s, a,
+                       static_cast<const int8_t*>(W), scale, ep, reinterpret_cast<uint16_t*>(ws), M, N, K, lda, ldw, ldc, tiles_t, tiles_c,
+                       split);
+    if (hipGetLastError() != hipSuccess) return SANA_ERR_LAUNCH;
+  } else {
+    const int rc = gemm8_planes_launch(a, static_cast<const uint16_t*>(W), ws, M, N, K, lda, ldw, is_f16<T>, pl.tiles, pl.rem, pl.S, s);
+    if (rc != SANA_OK) return rc;
+  }
+  const dim3 egrid((unsigned)(((int64_t)M * (N / 8) + 255) / 256));
+#define SANA_SPLIT_EPI(EPI) hipLaunchKernelGGL((splitk_epilogue_kernel<EPI, T>), egrid, dim3(256), 0, s, ws, pl.S, ep, c, M, N, ldc)
+  switch (epilogue) {
+    case SANA_EPI_NONE: SANA_SPLIT_EPI(SANA_EPI_NONE); break;
+    case SANA_EPI_BIAS: SANA_SPLIT_EPI(SANA_EPI_BIAS); break;
+    case SANA_EPI_BIAS_SILU: SANA_SPLIT_EPI(SANA_EPI_BIAS_SILU); break;
+    case SANA_EPI_GATE_RES: SANA_SPLIT_EPI(SANA_EPI_GATE_RES); break;
+    default: return SANA_ERR_ARG;
+  }
+#undef SANA_SPLIT_EPI
+  return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
+}
+
+// The pipelined kernel (int8 weights).
+template <int NI>
 int launch4(const uint16_t* a, const void* W, const float* scale, const EpiArgs& ep, uint16_t* c, int M, int N, int K,
-            int64_t lda, int64_t ldw, int64_t ldc, int epilogue, hipStream_t s, const GemmPlan& pl, float* ws) {
+            int64_t lda, int64_t ldw, int64_t ldc, int epilogue, hipStream_t s) {
   const int tiles_t = (M + BT - 1) / BT, tiles_c = (N + 64 * NI - 1) / (64 * NI);
   dim3 grid((unsigned)(tiles_t * tiles_c)), block(256);
-  if constexpr (NI != 2) {  // the 128-wide tile exists unsplit only
-    if (ws) {
-      const Taps split = {0, 0, 0, pl.tiles, pl.rem, nullptr};
-      hipLaunchKernelGGL((gemm4_kernel<W8, SANA_EPI_NONE, NI, true, T>), dim3(grid.x, (unsigned)pl.S), block, 0, s, a, W,
-                         scale, ep, reinterpret_cast<uint16_t*>(ws), M, N, K, lda, ldw, ldc, tiles_t, tiles_c, split);
-      if (hipGetLastError() != hipSuccess) return SANA_ERR_LAUNCH;
-      const int64_t threads = (int64_t)M * (N / 8);
-      dim3 egrid((unsigned)((threads + 255) / 256));
-#define SANA_SPLIT_EPI(EPI) hipLaunchKernelGGL((splitk_epilogue_kernel<EPI, T>), egrid, block, 0, s, ws, pl.S, ep, c, M, N, ldc)
-      switch (epilogue) {
-        case SANA_EPI_NONE: SANA_SPLIT_EPI(SANA_EPI_NONE); break;
-        case SANA_EPI_BIAS: SANA_SPLIT_EPI(SANA_EPI_BIAS); break;
-        case SANA_EPI_BIAS_SILU: SANA_SPLIT_EPI(SANA_EPI_BIAS_SILU); break;
-        case SANA_EPI_GATE_RES: SANA_SPLIT_EPI(SANA_EPI_GATE_RES); break;
-        default: return SANA_ERR_ARG;
-      }
-#undef SANA_SPLIT_EPI
-      return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
-    }
-  }
-  if constexpr (W8) {
-    const Taps none = {0, 0, 0, 0, 0, nullptr};
-#define SANA_LAUNCH4(EPI)                                                                                              \
-  hipLaunchKernelGGL((gemm4_kernel<W8, EPI, NI, false, T>), grid, block, 0, s, a, W, scale, ep, c, M, N, K, lda, ldw, ldc, \
+  const Taps none = {0, 0, 0, 0, 0, nullptr};
+#define SANA_LAUNCH4(EPI)                                                                                                     \
+  hipLaunchKernelGGL((gemm4_kernel<EPI, NI>), grid, block, 0, s, a, static_cast<const int8_t*>(W), scale, ep, c, M, N, K, lda, ldw, ldc, \
                      tiles_t, tiles_c, none)
-    switch (epilogue) {
-      case SANA_EPI_NONE: SANA_LAUNCH4(SANA_EPI_NONE); break;
-      case SANA_EPI_BIAS: SANA_LAUNCH4(SANA_EPI_BIAS); break;
-      case SANA_EPI_BIAS_SILU: SANA_LAUNCH4(SANA_EPI_BIAS_SILU); break;
-      case SANA_EPI_GATE_RES: SANA_LAUNCH4(SANA_EPI_GATE_RES); break;
-      default: return SANA_ERR_ARG;
-    }
-#undef SANA_LAUNCH4
-    return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
+  switch (epilogue) {
+    case SANA_EPI_NONE: SANA_LAUNCH4(SANA_EPI_NONE); break;
+    case SANA_EPI_BIAS: SANA_LAUNCH4(SANA_EPI_BIAS); break;
+    case SANA_EPI_BIAS_SILU: SANA_LAUNCH4(SANA_EPI_BIAS_SILU); break;
+    case SANA_EPI_GATE_RES: SANA_LAUNCH4(SANA_EPI_GATE_RES); break;
+    default: return SANA_ERR_ARG;
   }
-  return SANA_ERR_ARG;
+#undef SANA_LAUNCH4
+  return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
 }
 
 // The compiler-scheduled kernel (int8 weights): 64*TT tokens x 64*TC channels.
@@ -1038,8 +1031,7 @@ int launch(const void* A, const void* W, const float* scale, const EpiArgs& ep, 
   float* ws = aligned16(workspace) ? static_cast<float*>(workspace) : nullptr;
   const SplitWay way = ws && workspace_bytes >= split_bytes(pl, M, N) ? split_way(pl, M, N, K) : SplitWay::no;
   if (way == SplitWay::split || (W8 && way == SplitWay::ranges))
-    return pick_ni(M, N) == 3 ? launch4<W8, 3, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, pl, ws)
-                              : launch4<W8, 4, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, pl, ws);
+    return launch_split<W8, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, pl, ws);
   if constexpr (!W8) {
     const uint16_t* w = static_cast<const uint16_t*>(W);
     const Plan16 p = plan16(M, N, K);
@@ -1074,9 +1066,9 @@ int launch(const void* A, const void* W, const float* scale, const EpiArgs& ep, 
     // Taken when the 192-wide grid leaves a fifth of the CUs idle and the 128-wide one still fits.
     const int64_t t128 = tiles_t * ((N + 127) / 128), t192 = tiles_t * ((N + 191) / 192);
     if (t128 <= compute_units() && t192 < compute_units() * 4 / 5)
-      return launch4<true, 2>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, pl, nullptr);
-    return pick_ni(M, N) == 3 ? launch4<true, 3>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, pl, nullptr)
-                              : launch4<true, 4>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, pl, nullptr);
+      return launch4<2>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s);
+    return pick_ni(M, N) == 3 ? launch4<3>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s)
+                              : launch4<4>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s);
   }
 }
 

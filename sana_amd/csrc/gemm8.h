@@ -142,6 +142,12 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
                                                     const EpiArgs ep, uint16_t* __restrict__ C, int M, int N, int K,
                                                     int64_t lda, int64_t ldw, int64_t ldc, int tiles_t, int tiles_c,
                                                     const Taps tp) {
+  constexpr bool PLANES = EPI == SANA_EPI_PLANES;
+  if constexpr (PLANES) {  // this grid row's range of k-tiles
+    const int z = blockIdx.y, kt0 = z * tp.split_tiles + min(z, tp.split_rem);
+    A += 64 * kt0, W += 64 * kt0;
+    K = min(K - 64 * kt0, 64 * (tp.split_tiles + (z < tp.split_rem)));
+  }
   constexpr int BM = 256, BN = 64 * NB;
   constexpr int A_STAGE = BM * 128, W_STAGE = BN * 128, W_BASE = 2 * A_STAGE;
   constexpr int NP = (NB + 1) / 2;  // pieces of 8 (the last one of 4 if NB is odd) channels per lane and token
@@ -150,6 +156,7 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
   // tile's 192 channels by the four waves of a wm, in two buffers.
   constexpr bool SHARED = NB == 3;
   constexpr int OUT_ROW = SHARED ? 2 * BN : 32 * NB, OUT_BYTES = 32 * OUT_ROW, OUT_BUF = SHARED ? 2 * OUT_BYTES : 0;
+  static_assert(!PLANES || NB == 3, "rows of 48 floats a wave");
   static_assert(EPI != SANA_EPI_QKV_STATE || (NB == 4 && !is_f16<T> && !TAPS), "the fused qkv projection: 256-wide bf16 tiles");
   __shared__ __attribute__((aligned(1024))) unsigned char smem[W_BASE + 2 * W_STAGE + (SHARED ? 4 : 8) * OUT_BYTES];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -284,7 +291,7 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
   }
   u32x4_t fa[2][4], fb[2][NB];
   f32x4_t acc[NB][8];
-  constexpr bool HAS_BIAS = EPI != SANA_EPI_NONE;
+  constexpr bool HAS_BIAS = EPI != SANA_EPI_NONE && !PLANES;
 
   constexpr int LOADS = 4 + NB;  // per wave and k-tile
 #define G8_PIN() __builtin_amdgcn_sched_barrier(0)
@@ -444,6 +451,37 @@ __global__ __launch_bounds__(512) void gemm8_kernel(const uint16_t* __restrict__
         fresh = true;
         continue;
       }
+    }
+    if constexpr (PLANES) {
+      // 32 rows of the wave's 48 floats at a time through its eighth of the epilogue's LDS (swizzled: conflict-free both ways): whole
+      // segments of 192 bytes leave, for the kernel that adds the planes up to find in the caches
+      const int prows = min(128, M - m0t - 128 * wm);
+      const __amdgpu_buffer_rsrc_t rsrc_p = __builtin_amdgcn_make_buffer_rsrc(
+          reinterpret_cast<float*>(C) + ((int64_t)blockIdx.y * M + m0t + 128 * wm) * N, 0, prows > 0 ? prows * N * 4 : 0, 0x00020000);
+      const uint32_t corner = lds0 + W_BASE + 2 * W_STAGE + wave * 6144;
+      auto place = [&](int row, int pc) -> uint32_t { return corner + row * 192 + ((pc ^ ((row >> 2) & 3)) << 4); };
+      const uint32_t wr[3] = {place(fr, 2 * fg), place(fr, 2 * fg + 1), place(fr, 8 + fg)};
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          gemm_lds_write<0>(wr[i], __builtin_bit_cast(u32x4_t, acc[i][2 * g]));
+          gemm_lds_write<16 * 192>(wr[i], __builtin_bit_cast(u32x4_t, acc[i][2 * g + 1]));  // (the swizzle repeats every 16 rows)
+        }
+        u32x4_t o[6];
+        int off[6];
+#pragma unroll
+        for (int s = 0; s < 6; ++s) {
+          const int idx = lane + 64 * s, row = idx / 12, pc = idx - 12 * row, n = n0t + 48 * wn + 4 * pc;
+          off[s] = n < N ? ((row + 32 * g) * N + n) * 4 : (int)kOut;
+          o[s] = gemm_lds_read<0>(place(row, pc));  // (a wave's LDS accesses are in order)
+        }
+#pragma unroll
+        for (int s = 0; s < 6; ++s) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(o[s])::"memory");
+#pragma unroll
+        for (int s = 0; s < 6; ++s) __builtin_amdgcn_raw_buffer_store_b128(o[s], rsrc_p, off[s], 0, 0);
+      }
+      return;  // (one tile a workgroup)
     }
     if (id < total) start_tile(id);
     fresh = false;

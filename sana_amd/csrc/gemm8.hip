@@ -44,6 +44,23 @@ int launch_nb(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t*
 
 }  // namespace
 
+// Against the one-wave-per-SIMD kernel that split 16-bit GEMMs before (gemm4_kernel, int8 weights only now), with the epilogue launch, us,
+// weights cold: 1024 x 2240 x 5600 in five ranges 47.9 / 45.6, 600 in seven 36.8 / 35.0, 500 x 1152 x 5600 in eight 31.5 / 29.7; same bits.
+int gemm8_planes_launch(const uint16_t* a, const uint16_t* w, float* planes, int M, int N, int K, int64_t lda, int64_t ldw, bool f16,
+                        int tiles, int rem, int ranges, hipStream_t s) {
+  const int tiles_t = (M + 255) / 256, tiles_c = (N + 191) / 192;
+  const dim3 grid((unsigned)(tiles_t * tiles_c), (unsigned)ranges), block(512);
+  const Taps split = {0, 0, 0, tiles, rem, nullptr};
+  uint16_t* c = reinterpret_cast<uint16_t*>(planes);
+  if (f16)
+    hipLaunchKernelGGL((gemm8_kernel<SANA_EPI_PLANES, 3, 0, F16>), grid, block, 0, s, a, w, EpiArgs{}, c, M, N, K, lda, ldw, (int64_t)N, tiles_t,
+                       tiles_c, split);
+  else
+    hipLaunchKernelGGL((gemm8_kernel<SANA_EPI_PLANES, 3, 0, BF16>), grid, block, 0, s, a, w, EpiArgs{}, c, M, N, K, lda, ldw, (int64_t)N, tiles_t,
+                       tiles_c, split);
+  return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
+}
+
 int gemm8_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
                  int64_t ldw, int64_t ldc, int epilogue, bool f16, int nb, const Taps* taps, hipStream_t s) {
 #define SANA_NB8(NB)                                                                                            \

@@ -26,6 +26,8 @@ struct EpiArgs {
 // (not part of the C ABI's epilogue codes) qkv projection of the linear attention with the k / v column tiles
 // contracted over their tokens in the epilogue instead of stored: see g8_state_tile
 #define SANA_EPI_QKV_STATE 4
+// (nor this) K split into ranges, one grid row each: the fp32 accumulators to plane blockIdx.y of C, [M][N] floats each
+#define SANA_EPI_PLANES 5
 
 // Virtual concatenation of the A operand along k: columns [t*kc, (t+1)*kc) of the GEMM's A are columns
 // [0, kc) of the matrix whose row m is row m + t*stride of the buffer (a convolution over rows as one GEMM,
@@ -48,6 +50,11 @@ struct Taps {
 // (bf16); taps (bf16, SANA_EPI_GATE_RES, nb = 3 or 4) or null.  Arguments are checked by the caller.
 int gemm8_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, uint16_t* c, int M, int N, int K, int64_t lda,
                  int64_t ldw, int64_t ldc, int epilogue, bool f16, int nb, const Taps* taps, hipStream_t s);
+
+// K split into `ranges` ranges of `tiles` k-tiles (one more in the first `rem`), tiles of 256 x 192: the fp32 sums of range z to plane z of
+// `planes`, [M][N] each.  One workgroup a tile and range; M * N * 4 < 2^31.
+int gemm8_planes_launch(const uint16_t* a, const uint16_t* w, float* planes, int M, int N, int K, int64_t lda, int64_t ldw, bool f16,
+                        int tiles, int rem, int ranges, hipStream_t s);
 
 // The same in tiles of 256 tokens x 288 channels (gemm288.hip); no SANA_EPI_QKV_STATE; rows of W less than 2^21 values apart,
 // bias 16-byte aligned (or null).
