@@ -66,25 +66,35 @@ __device__ __forceinline__ uint32_t dequant2(uint32_t q4, int which, float s, fl
 }
 
 // int8 weight [N][K] + per-row scale -> bf16 [N][K], with the rounding of dequant2: the expansion the GEMM's
-// int8 path performs on its way to LDS, as a streaming kernel of its own (16 values per thread).
+// int8 path performs on its way to LDS, as a streaming kernel of its own.  A wave takes a row, a lane 8 values (a store instruction is
+// 1 KB in a row), six of them requested at once: no division, whole sectors.  HBM bound.  us, 16 values a thread with a 64-bit division
+// for its row / so: 11200 x 2240 18.1 / 16.1, 6720 x 2240 11.9 / 9.7, 5760 x 1152 6.0 / 5.4, 2240 x 5600 8.9 / 8.8.
+// grid: ceil(N / 4); block 256.
 __global__ __launch_bounds__(256) void dequant_w8_kernel(const int8_t* __restrict__ wq, const float* __restrict__ scale,
                                                          uint16_t* __restrict__ out, int N, int K, int64_t ldw,
                                                          int64_t ldo) {
-  const int pieces = K >> 4;
-  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (id >= (int64_t)N * pieces) return;
-  const int n = (int)(id / pieces), p = (int)(id - (int64_t)n * pieces);
-  u32x4_t q = *reinterpret_cast<const u32x4_t*>(wq + n * ldw + 16 * p);
+  constexpr int U = 6;
+  const int n = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (n >= N) return;
+  const int pieces = K >> 3;
+  const char* row = reinterpret_cast<const char*>(wq + n * ldw);
+  char* orow = reinterpret_cast<char*>(out + n * ldo);
   const float s = scale[n], off = -128.f * s;
-  u32x4_t lo, hi;
-  q.x ^= 0x80808080u, q.y ^= 0x80808080u, q.z ^= 0x80808080u, q.w ^= 0x80808080u;
-  lo.x = dequant2(q.x, 0, s, off), lo.y = dequant2(q.x, 1, s, off);
-  lo.z = dequant2(q.y, 0, s, off), lo.w = dequant2(q.y, 1, s, off);
-  hi.x = dequant2(q.z, 0, s, off), hi.y = dequant2(q.z, 1, s, off);
-  hi.z = dequant2(q.w, 0, s, off), hi.w = dequant2(q.w, 1, s, off);
-  uint16_t* o = out + n * ldo + 16 * p;
-  *reinterpret_cast<u32x4_t*>(o) = lo;
-  *reinterpret_cast<u32x4_t*>(o + 8) = hi;
+  for (int p0 = 0; p0 < pieces; p0 += 64 * U) {
+    u32x2_t q[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (p0 + 64 * u < pieces) q[u] = *reinterpret_cast<const u32x2_t*>(row + 8u * (uint32_t)min(p0 + 64 * u + lane, pieces - 1));
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int p = p0 + 64 * u + lane;
+      if (p < pieces) {
+        const uint32_t x = q[u].x ^ 0x80808080u, y = q[u].y ^ 0x80808080u;
+        *reinterpret_cast<u32x4_t*>(orow + 16u * (uint32_t)p) =
+            u32x4_t{dequant2(x, 0, s, off), dequant2(x, 1, s, off), dequant2(y, 0, s, off), dequant2(y, 1, s, off)};
+      }
+    }
+  }
 }
 
 // Compiler-scheduled kernel for int8 weights, any K % 16 == 0.  Workgroup tile 64*TT tokens x 64*TC channels,
@@ -1185,15 +1195,18 @@ SANA_API int sana_hip_gemm_plan(int M, int N, int K, int plan[4]) {
   return SANA_OK;
 }
 
-// From 4096 rows on always (converting in the main loop costs it 14 % at every M, the expansion a fixed 10 - 20 us); below
-// that where N <= K and the GEMM is not split: there the bf16 GEMM has its small tiles and the int8 one a chain of long
-// k-tiles.  us, converting / expanding (the weights of 12 calls in turn): 256 x 1152 x 2880 37 / 20, 2048 x 2240 x 2240 36 / 32,
-// 2048 x 2240 x 5600 90 / 76; but 2048 x 5760 x 1152 32 / 41, 1024 x 11200 x 2240 56 / 65, and split 512 x 2240 x 5600 33 / 42.
-// Wide weights of 2240 at 2000 - 3000 rows are the tie between: 2048 x 11200 x 2240 107 - 112 / 109 - 110, 2048 x 6720 x 2240
-// 63 / 60, 2916 x 11200 x 2240 155 / 152, 2916 x 6720 x 2240 98 / 97.
+// From 4096 rows on always (converting in the main loop costs it 14 % at every M, the expansion a fixed 5 - 16 us); below that, of GEMMs that
+// are not split, where
+//  * N <= K: there the bf16 GEMM has its small tiles and the int8 one a chain of long k-tiles.  us, converting / expanding (the weights of
+//    12 calls in turn): 256 x 1152 x 2880 37 / 20, 2048 x 2240 x 2240 36 / 32, 2048 x 2240 x 5600 91 / 79; split 1024 x 2240 x 5600 45 / 54;
+//  * the int8 tiles need a second round: 1536 x 11200 x 2240 98 / 82, 2916 x 5760 x 1152 57 / 49, 3584 x 5760 x 1152 59.1 / 58.4;
+//  * long rows of weights meet more than six token tiles: 1600 x 6720 x 2240 55.2 / 54.4, 2048 x 6720 x 2240 64 / 59, 2300 x 4480 x 2240 53 / 49; but
+//    1024 x 11200 x 2240 58 / 60, 2048 x 5760 x 1152 33 / 38, 3072 x 3456 x 1152 30 / 33.
 SANA_API int sana_hip_gemm_w8_expand(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return M >= 4096 || (N <= K && !split_pays(plan_gemm(M, N, K, true), M, N, K));
+  if (M >= 4096) return 1;
+  const int64_t tiles = (int64_t)((M + BT - 1) / BT) * ((N + 64 * pick_ni(M, N) - 1) / (64 * pick_ni(M, N)));
+  return (N <= K || tiles > compute_units() || (K >= 2048 && M > 6 * BT)) && !split_pays(plan_gemm(M, N, K, true), M, N, K);
 }
 
 SANA_API int sana_hip_gemm_bf16(const void* A, const void* W, const void* bias, void* C, int M, int N, int K,
@@ -1292,9 +1305,8 @@ SANA_API int sana_hip_dequant_w8(const int8_t* Wq, const float* scale, void* W, 
   if (K % 16) return SANA_ERR_SHAPE;
   if (ldw < K || ldo < K) return SANA_ERR_ARG;
   if (ldw % 16 || ldo % 8 || !aligned16(Wq) || !aligned16(W)) return SANA_ERR_ALIGN;
-  const int64_t threads = (int64_t)N * (K / 16);
-  if ((threads + 255) / 256 > 0x7fffffff) return SANA_ERR_SHAPE;
-  hipLaunchKernelGGL(dequant_w8_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+  if ((int64_t)N * (K / 16) > (int64_t)0x7fffffff * 256) return SANA_ERR_SHAPE;
+  hipLaunchKernelGGL(dequant_w8_kernel, dim3((unsigned)(((int64_t)N + 3) / 4)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), Wq, scale, static_cast<uint16_t*>(W), N, K, ldw, ldo);
   return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
 }

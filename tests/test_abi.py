@@ -202,3 +202,11 @@ def test_gemm_qkv_state_refuses_bad_arguments_before_any_launch():
     assert call(*bad(11, 64)) == -1                                                                # lda < C
     assert call(*bad(0, P + 2)) == -3 and call(*bad(12, 100)) == -3                                # SANA_ERR_ALIGN
     assert call(*bad(6, 1024)) == -4 and call(*bad(5, None)) == -4                                 # SANA_ERR_WORKSPACE
+
+
+@pytest.mark.parametrize("M,N,K,expand", [(4096, 3456, 1152, 1), (256, 1152, 2880, 1), (1024, 2240, 5600, 0), (0, 8, 16, 0),
+                                          (1537, 6720, 2240, 1), (1536, 6720, 2240, 0), (3072, 3456, 1152, 0), (2048, 5760, 1152, 0),
+                                          (1280, 11200, 2240, 0), (1281, 11200, 2240, 1), (2816, 5760, 1152, 0), (2817, 5760, 1152, 1)])
+def test_which_int8_weights_are_expanded(M, N, K, expand):
+    """Narrow outputs that are not split, a second round of int8 tiles, more than six token tiles on long rows of weights."""
+    assert _lib.load().sana_hip_gemm_w8_expand(M, N, K) == expand

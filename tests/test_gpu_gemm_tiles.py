@@ -80,3 +80,27 @@ def test_many_token_gated_residual_across_batch_boundaries(cuda, tile, B, Ntok, 
     gate, res = ints(B, 1, C, hi=4, seed=4), ints(B, Ntok, C, hi=99, seed=5)
     y = (a.float() @ w.float().T + bias.float()).to(dtype)
     assert torch.equal(ops.gemm_gate_residual(a, w, bias, gate, res), res + gate * y)   # the stock pair's roundings
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 264, 5664), (257, 200, 4128), (700, 1160, 6432), (130, 3000, 8192), (1025, 2232, 5600)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_split_over_k_is_exact_on_integers(cuda, M, N, K, dtype):
+    """Partial planes of 256 x 192 tiles: ragged rows and channels, token halves without rows, ranges of unequal length, a k tail."""
+    plan = (ctypes.c_int * 4)()
+    _lib.check(_lib.load().sana_hip_gemm_plan(M, N, K, plan), "sana_hip_gemm_plan")
+    assert tuple(plan[:2]) == (256, 192) and plan[3] > 1
+    a, w, bias = (_ints(M, K, seed=1, dtype=dtype).to(cuda), _ints(N, K, seed=2, dtype=dtype).to(cuda),
+                  _ints(N, lo=-9, hi=9, seed=3, dtype=dtype).to(cuda))
+    ref = a.float() @ w.float().T        # |sum| <= 9 k < 2^24: exact in any order
+    assert torch.equal(ops.gemm_bf16(a, w), ref.to(dtype))
+    assert torch.equal(ops.gemm_bf16(a, w, bias, "bias"), (ref + bias.float()).to(dtype))
+
+
+@pytest.mark.parametrize("N", [1, 5, 64])
+@pytest.mark.parametrize("K", [16, 512, 3072, 3088, 5600])
+def test_expanded_weights_are_the_rounded_products(cuda, N, K):
+    """Pieces of 8 values, 64 lanes, six pieces a lane: one piece, whole passes, one more piece."""
+    gen = torch.Generator().manual_seed(K + N)
+    wq = torch.randint(-128, 128, (N, K + 16), generator=gen).to(torch.int8).to(cuda)[:, :K]
+    scale = (0.001 + torch.rand(N, generator=gen)).to(cuda)
+    assert torch.equal(ops.dequant_w8(wq, scale), (wq.float() * scale[:, None]).bfloat16())
