@@ -401,13 +401,17 @@ struct Quotient {
 
 // T = F16 replaces MFMAs in fp32 (32x32x2) and 2-byte loads and stores: tokens x heads, us: 2048 x 36
 // 16.5 -> 7.2, 16384 x 70 125 -> 36.
+// The state, then the first queries, are requested before anything is computed, later ones a pass ahead; the wave is uniform.  bf16, us,
+// before / so, inputs from HBM: 16384 x 70 40.3 / 35.5, 16 x 1024 x 70 38.5 / 34.5, 4096 x 70 14.6 / 13.9, 2048 x 36 6.3 / 5.8, 4 x 1024 x 36 9.2 / 9.2.
 template <typename T, bool OUT_F32, int PRE>
 __global__ __launch_bounds__(256) void linattn_apply16_kernel(
     const uint16_t* __restrict__ Q, const float* __restrict__ state, void* __restrict__ out,
     const int32_t* __restrict__ chunk_starts, int N, int h, int n_chunks, int wg_tokens,
     int64_t q_stride_b, int64_t q_stride_n, int64_t o_stride_b, int64_t o_stride_n, float eps,
     const QkPre pre, int xranges, int ngroups) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  asm volatile("" ::"s"(Q), "s"(state), "s"(chunk_starts), "s"(N), "s"(h), "s"(n_chunks), "s"(wg_tokens), "s"(q_stride_b), "s"(q_stride_n),
+               "s"(xranges), "s"(ngroups));  // (the arguments in one wait)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int pairs = (h + 1) >> 1;
   const int pgroups = (pairs + 3) >> 2;
   // 3-D grid (token range, chunk, batch x head group), or -- with many (chunk, batch, head group)
@@ -415,12 +419,11 @@ __global__ __launch_bounds__(256) void linattn_apply16_kernel(
   // (workgroup ids go round-robin to the 8 XCDs): their common state is then fetched into one L2 only.
   int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
   if (ngroups > 0) {
-    const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-    const int grp = xcd + 8 * (idx / xranges);
-    if (grp >= ngroups) return;  // no barriers below
-    bx = idx % xranges, by = grp % n_chunks, bz = grp / n_chunks;
+    const uint32_t xcd = blockIdx.x & 7, idx = blockIdx.x >> 3, grp = xcd + 8 * (idx / (uint32_t)xranges);
+    if (grp >= (uint32_t)ngroups) return;  // no barriers below
+    bx = (int)(idx % (uint32_t)xranges), by = (int)(grp % (uint32_t)n_chunks), bz = (int)(grp / (uint32_t)n_chunks);
   }
-  const int b = bz / pgroups, p = (bz % pgroups) * 4 + wave;
+  const int b = (int)((uint32_t)bz / (uint32_t)pgroups), p = (bz - b * pgroups) * 4 + wave;
   if (p >= pairs) return;  // no barriers below
   const int c = by;
   const ChunkRange cr = chunk_range(chunk_starts, c, N);
@@ -430,32 +433,6 @@ __global__ __launch_bounds__(256) void linattn_apply16_kernel(
   const int n = lane & 15, g = lane >> 4;
   const int nheads = (2 * p + 1 < h) ? 2 : 1;
 
-  // A operands.  MFMA 16x16x32: A lane -> row lane%16, k = 8*(lane/16)+e.  Output
-  // lane (token n, g') register s of row block rb is row 4*g'+s; we place channel
-  // 8*(r/4) + 4*rb + r%4 in row r so that a lane ends up with 8 contiguous channels.
-  SplitState st[2];
-#pragma unroll
-  for (int hh = 0; hh < 2; ++hh) {
-    const int head = min(2 * p + hh, h - 1);
-    const float* sp = state + ((int64_t)(b * h + head) * n_chunks + c) * STATE_ELEMS;
-#pragma unroll
-    for (int rb = 0; rb < 3; ++rb) {
-      const int row = (rb < 2) ? (8 * (n >> 2) + 4 * rb + (n & 3)) : D;
-      const f32x4_t x0 = *reinterpret_cast<const f32x4_t*>(sp + row * D + 8 * g);
-      const f32x4_t x1 = *reinterpret_cast<const f32x4_t*>(sp + row * D + 8 * g + 4);
-      const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-      split3(x, st[hh].a[rb]);
-    }
-  }
-
-  const u32x4_t zero4 = {0u, 0u, 0u, 0u};
-  constexpr bool has_norm = (PRE & 1) != 0, has_rope = (PRE & 2) != 0, rope_first = (PRE & 4) != 0;
-  u32x4_t qw[2] = {zero4, zero4};
-  if (has_norm) {
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh)
-      if (hh < nheads) qw[hh] = *reinterpret_cast<const u32x4_t*>(pre.weight + p * 64 + hh * D + 8 * g);
-  }
   // Global accesses are whole 128-byte lines: lane l fetches 16-byte chunk l%8 of token l/8 (both heads
   // of the pair), two instructions per 16-token step, and the step goes through wave-private LDS to
   // reach the MFMA layout (lane = token n, channel group g); results return the same way, so a store
@@ -466,8 +443,8 @@ __global__ __launch_bounds__(256) void linattn_apply16_kernel(
   __shared__ __attribute__((aligned(16))) unsigned char stage_all[4 * (SANA_LA_APPLY_U + 1) * 2048];
   unsigned char* stage = stage_all + wave * ((SANA_LA_APPLY_U + 1) * 2048);
   const int ld_tok = lane >> 3, ld_chunk = lane & 7;
-  const uint16_t* qrow = Q + (int64_t)b * q_stride_b + p * 64 + 8 * ld_chunk;
   const bool ld_ok = nheads == 2 || ld_chunk < 4;   // the second head of the last pair may not exist
+  const uint16_t* qrow = Q + (int64_t)b * q_stride_b + p * 64 + 8 * (ld_ok ? ld_chunk : ld_chunk - 4);
   int slot_w[2], slot_r[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -476,17 +453,58 @@ __global__ __launch_bounds__(256) void linattn_apply16_kernel(
   }
 #pragma unroll
   for (int hh = 0; hh < 2; ++hh) slot_r[hh] = 16 * (8 * n + ((4 * hh + g) ^ ((n >> 1) & 7)));
+  // The queries of a pass are requested a pass ahead, the first ones behind the state's loads and in front of its split: it was one memory
+  // latency after the other.  Past the range its last token once more (not stored), for the head that does not exist the one that does: no
+  // branch around a load.
+  u32x4_t raw[U][2];
+  auto fetch = [&](int t) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        raw[u][j] = *reinterpret_cast<const u32x4_t*>(qrow + (int64_t)min(t + 16 * u + 8 * j + ld_tok, t1 - 1) * q_stride_n);
+  };
+
+  // A operands.  MFMA 16x16x32: A lane -> row lane%16, k = 8*(lane/16)+e.  Output
+  // lane (token n, g') register s of row block rb is row 4*g'+s; we place channel
+  // 8*(r/4) + 4*rb + r%4 in row r so that a lane ends up with 8 contiguous channels.
+  SplitState st[2];
+  f32x4_t x[2][3][2];
+#pragma unroll
+  for (int hh = 0; hh < 2; ++hh) {
+    const int head = min(2 * p + hh, h - 1);
+    const float* sp = state + ((int64_t)(b * h + head) * n_chunks + c) * STATE_ELEMS;
+#pragma unroll
+    for (int rb = 0; rb < 3; ++rb) {
+      const int row = (rb < 2) ? (8 * (n >> 2) + 4 * rb + (n & 3)) : D;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) x[hh][rb][e] = *reinterpret_cast<const f32x4_t*>(sp + row * D + 8 * g + 4 * e);
+    }
+  }
+  fetch(t0);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+    for (int rb = 0; rb < 3; ++rb) {
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = x[hh][rb][e >> 2][e & 3];
+      split3(v, st[hh].a[rb]);
+    }
+
+  constexpr bool has_norm = (PRE & 1) != 0, has_rope = (PRE & 2) != 0, rope_first = (PRE & 4) != 0;
+  u32x4_t qw[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
+  if (has_norm) {
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh)
+      if (hh < nheads) qw[hh] = *reinterpret_cast<const u32x4_t*>(pre.weight + p * 64 + hh * D + 8 * g);
+  }
   for (int t = t0; t < t1; t += 16 * U) {
-    u32x4_t raw[U][2];
     float rin[has_norm ? U : 1];
     f32x4_t cs[has_rope ? U : 1][2];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int tok = t + 16 * u + 8 * j + ld_tok;
-        raw[u][j] = (tok < t1 && ld_ok) ? load_stream<SANA_LA_NT_LOAD != 0>(reinterpret_cast<const u32x4_t*>(qrow + (int64_t)tok * q_stride_n)) : zero4;
-      }
       const int tok = t + 16 * u + n;
       if (has_norm) rin[u] = tok < t1 ? pre.rinv[(int64_t)b * N + tok] : 0.f;
       if (has_rope) {
@@ -500,6 +518,7 @@ __global__ __launch_bounds__(256) void linattn_apply16_kernel(
 #pragma unroll
       for (int j = 0; j < 2; ++j) *reinterpret_cast<u32x4_t*>(stage + u * 2048 + slot_w[j]) = raw[u][j];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // wave-private LDS: in-order, no barrier needed
+    if (t + 16 * U < t1) fetch(t + 16 * U);  // uniform
     unsigned char* ostage = stage + SANA_LA_APPLY_U * 2048;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
