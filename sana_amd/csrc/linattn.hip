@@ -726,10 +726,11 @@ __global__ __launch_bounds__(320) void linattn_apply32_partials_kernel(
 }
 
 // ----------------------------------------------------------------------------
-// Both phases in one launch, for short sequences: one workgroup = one head of one batch entry, the state never leaves LDS.
+// Both phases in one launch, for short sequences: one workgroup = one head of one batch entry (16-bit io, few heads: its state and
+// a share of its queries), the state never leaves LDS.
 // Three launches (phase 1, reduction, phase 2) are 3 - 6 us of work each with a gap in front; here everything a head needs
 // for 1024 tokens is requested at once and the rest is one memory round trip, the transposes and the matrix products of one
-// compute unit.  That is also the bound: a head's tokens are one compute unit's work.  us, two calls / this, replayed from a
+// compute unit.  That is also the bound: a head's keys and values are one compute unit's work.  us, two calls / this, replayed from a
 // graph on one set of inputs (on 16 in turn): bf16, 36 heads x 256 tokens 9.8 / 5.2 (10.5 / 6.0), 36 x 1024 12.1 / 8.8 (13.3 /
 // 11.5), 140 x 1024 18.9 / 15.4 (22.2 / 17.0); fp16 36 x 256 10.5 / 5.8 (11.2 / 6.6); fp32 256 x 1024 35.9 / 26.7 (45.6 / 38.4).
 // (Adding the state up in the two calls' order costs 0.4 us at 1024 tokens: sixteen partial states in LDS, not eight.)
@@ -744,24 +745,24 @@ __device__ __forceinline__ u32x2_t lds_read_tr16(uint32_t addr) {  // 4 tokens x
   return v;
 }
 
-// 16-bit io.  grid: B * h; block 512.  The state is formed by the sums of linattn_state16_kernel and its reduction, in their
+// 16-bit io.  grid: B * h * R; block 512: R workgroups form the state of a head each for itself and share its queries.  The state is formed by the sums of linattn_state16_kernel and its reduction, in their
 // order (at most 256 heads: always splits of 256 tokens), so that the result is that of the two calls bit for bit: "chain" c is
 // what wave c % 4 of split c / 4 adds up there, the 32-token tiles 256 (c / 4) + 32 (c % 4) + {0, 128}.  Wave w takes chains w and
 // w + 8 through its own LDS (rows of 96 bytes: conflict-free transposing reads).  Phase 2 as linattn_apply16_kernel, on the
-// 16-token steps w, w + 8, ..
-template <typename T>
+// 16-token steps R w + part, R (w + 8) + part, ..
+template <typename T, int R>
 __global__ __launch_bounds__(512) void linattn_whole16_kernel(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V, uint16_t* __restrict__ out,
     int N, int h, int64_t q_stride_b, int64_t q_stride_n, int64_t stride_b, int64_t stride_n, int64_t o_stride_b,
     int64_t o_stride_n, float eps) {
   constexpr int WAVES = 8, ROW = 96, SPLIT = 256, CHAINS = 4 * WHOLE_TOKENS / SPLIT, U1 = CHAINS / WAVES,
-                U2 = WHOLE_TOKENS / (WAVES * 16);
+                U2 = (WHOLE_TOKENS / 16 + WAVES * R - 1) / (WAVES * R);
   constexpr int STATE_AT = CHAINS * STATE_ELEMS * 4;
   static_assert(STATE_AT >= WAVES * 2 * TILE * ROW && STATE_AT >= WAVES * U2 * 1024, "the state lies behind the stages");
   __shared__ __attribute__((aligned(16))) unsigned char smem[STATE_AT + STATE_ELEMS * 4];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int bh = xcd_eighths(blockIdx.x, gridDim.x), b = bh / h, head = bh - b * h;
+  const int at = xcd_eighths(blockIdx.x, gridDim.x), bh = at / R, part = at % R, b = bh / h, head = bh - b * h;
   const int ld_tok = lane >> 2, ld_chunk = lane & 3;  // a load instruction: 16 tokens x 64 bytes
   const uint16_t* kbase = K + (int64_t)b * stride_b + head * D;
   const uint16_t* vbase = V + (int64_t)b * stride_b + head * D;
@@ -773,6 +774,7 @@ __global__ __launch_bounds__(512) void linattn_whole16_kernel(
     const int c = wave + WAVES * u;
     return SPLIT * (c >> 2) + TILE * (c & 3) + 128 * t;
   };
+  auto query_of = [&](int u) { return ((wave + u * WAVES) * R + part) * 16; };  // phase 2, step u of this wave: its first token
   u32x4_t kreg[U1][2][2], vreg[U1][2][2], raw[U2];
   // Every load goes out without a branch: rows past N lie outside the resource (zeros).
   const bool near = max(max(q_stride_n, stride_n), o_stride_n) < (1 << 20);  // 32-bit offsets over 1024 rows
@@ -796,8 +798,8 @@ __global__ __launch_bounds__(512) void linattn_whole16_kernel(
       }
 #pragma unroll
     for (int u = 0; u < U2; ++u) {
-      if ((wave + u * WAVES) * 16 >= N) break;  // uniform
-      raw[u] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rq, offset((wave + u * WAVES) * 16, q_stride_n), 0, 0));
+      if (query_of(u) >= N) break;  // uniform
+      raw[u] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rq, offset(query_of(u), q_stride_n), 0, 0));
     }
   } else {
     auto row = [&](const uint16_t* base, int tok, int64_t stride) {
@@ -813,7 +815,7 @@ __global__ __launch_bounds__(512) void linattn_whole16_kernel(
           kreg[u][t][i] = row(kbase, tok, stride_n), vreg[u][t][i] = row(vbase, tok, stride_n);
         }
 #pragma unroll
-    for (int u = 0; u < U2; ++u) raw[u] = row(qbase, (wave + u * WAVES) * 16 + ld_tok, q_stride_n);
+    for (int u = 0; u < U2; ++u) raw[u] = row(qbase, query_of(u) + ld_tok, q_stride_n);
   }
   // MFMA 32x32x16: lane -> channel lane % 32, element r of k-step s is token 16 s + 2 r + lane / 32 of the tile.  A transposing
   // read hands the 16 lanes of a group four rows, row i addressed by lanes 4 i .. 4 i + 3: two tokens apart here.
@@ -896,13 +898,13 @@ __global__ __launch_bounds__(512) void linattn_whole16_kernel(
   const int slot_r = 16 * (4 * n + (g ^ ((n >> 1) & 3)));
 #pragma unroll
   for (int u = 0; u < U2; ++u) {
-    if ((wave + u * WAVES) * 16 >= N) break;  // uniform
+    if (query_of(u) >= N) break;  // uniform
     *reinterpret_cast<u32x4_t*>(qstage + u * 1024 + slot_w) = relu_pk16(raw[u]);
   }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
   for (int u = 0; u < U2; ++u) {
-    if ((wave + u * WAVES) * 16 >= N) break;  // uniform
+    if (query_of(u) >= N) break;  // uniform
     unsigned char* slot = qstage + u * 1024 + slot_r;
     const u32x4_t qd = *reinterpret_cast<const u32x4_t*>(slot);
     u32x4_t q_hi, q_lo;
@@ -940,14 +942,14 @@ __global__ __launch_bounds__(512) void linattn_whole16_kernel(
     const __amdgpu_buffer_rsrc_t ro = resource(obase, o_stride_n);
 #pragma unroll
     for (int u = 0; u < U2; ++u) {
-      if ((wave + u * WAVES) * 16 >= N) break;  // uniform
+      if (query_of(u) >= N) break;  // uniform
       __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4_t*>(qstage + u * 1024 + slot_w), ro,
-                                             offset((wave + u * WAVES) * 16, o_stride_n), 0, 0);
+                                             offset(query_of(u), o_stride_n), 0, 0);
     }
   } else {
 #pragma unroll
     for (int u = 0; u < U2; ++u) {
-      const int tok = (wave + u * WAVES) * 16 + ld_tok;
+      const int tok = query_of(u) + ld_tok;
       const u32x4_t o = *reinterpret_cast<const u32x4_t*>(qstage + u * 1024 + slot_w);
       if (tok < N) *reinterpret_cast<u32x4_t*>(obase + (int64_t)tok * o_stride_n + 8 * ld_chunk) = o;
     }
@@ -1460,16 +1462,29 @@ extern "C" __attribute__((visibility("default"))) int sana_hip_linattn(
                          : sana_hip_linattn_apply(q, state, out, B, N, h, d, q_stride_b, q_stride_n, o_stride_b, o_stride_n,
                                                   nullptr, 1, N, eps, io_dtype, io_dtype, stream);
   }
-  const dim3 grid((unsigned)(B * h));
+  // 16-bit io: up to four workgroups a head while the chip has room for all of them at once.  us, one / so (two, three or four), behind
+  // the launch that writes q, k and v: 36 heads x 256 tokens 5.6 / 4.8, 36 x 1024 11.3 / 8.7, 70 x 576 8.2 / 7.2, 70 x 1024 11.0 / 9.0,
+  // fp16 72 x 1024 13.8 / 10.1, 128 x 1000 13.5 / 11.4; with more of them than compute units 140 x 1024 12.2 / 14.6, 210 x 972 13.8 / 15.1.
+  // (Seven for 36 x 1024: 8.3.)
+  const int parts = io_dtype == SANA_DT_F32 ? 1 : heads <= 64 ? 4 : heads <= 85 ? 3 : heads <= 128 ? 2 : 1;
+  const dim3 grid((unsigned)(heads * parts));
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define SANA_WHOLE(kernel, threads, E, ...)                                                                            \
   hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, static_cast<const E*>(q), static_cast<const E*>(k),           \
                      static_cast<const E*>(v), static_cast<E*>(out), N, h, __VA_ARGS__, q_stride_n, stride_b, stride_n, \
                      o_stride_b, o_stride_n, eps)
+#define SANA_WHOLE16(R)                                                                                       \
+  do {                                                                                                        \
+    if (io_dtype == SANA_DT_F16) SANA_WHOLE((linattn_whole16_kernel<F16, R>), 512, uint16_t, q_stride_b);      \
+    else SANA_WHOLE((linattn_whole16_kernel<BF16, R>), 512, uint16_t, q_stride_b);                             \
+  } while (0)
   if (io_dtype == SANA_DT_F32)
     SANA_WHOLE(linattn_whole32_kernel, WHOLE_TOKENS, float, plan_state(B, h, 1, N, io_dtype).split_tokens, q_stride_b);
-  else if (io_dtype == SANA_DT_F16) SANA_WHOLE(linattn_whole16_kernel<F16>, 512, uint16_t, q_stride_b);
-  else SANA_WHOLE(linattn_whole16_kernel<BF16>, 512, uint16_t, q_stride_b);
+  else if (parts == 1) SANA_WHOLE16(1);
+  else if (parts == 2) SANA_WHOLE16(2);
+  else if (parts == 3) SANA_WHOLE16(3);
+  else SANA_WHOLE16(4);
+#undef SANA_WHOLE16
 #undef SANA_WHOLE
   return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
 }

@@ -162,6 +162,22 @@ def test_rows_of_any_distance(cuda, dtype, far):
     assert torch.equal(out[:, :C], want) and bool((out[:, C:] == 3.0).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,h", [(2, 32), (1, 65), (5, 17), (2, 43), (1, 128), (3, 43)])
+@pytest.mark.parametrize("N", [16, 47, 49, 385, 1009])
+def test_workgroups_that_share_a_head(cuda, B, h, N, dtype):
+    """16 bits: four, three, two and one workgroup a head (64, 65 .. 85, 86 .. 128 and more heads), with steps of 16 queries that run out
+    within one of them: every query is answered, with the bits of the two calls."""
+    C, gen = 32 * h, torch.Generator().manual_seed(N + h)
+    q, k, v = (torch.randn(B, N, C, generator=gen).to(dtype).to(cuda) for _ in range(3))
+    out = torch.full((B, N + 1, C), float("nan"), dtype=dtype, device=cuda)       # (a row behind each batch entry's that stays)
+    _lib.check(_lib.load().sana_hip_linattn(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), None, 0, B, N, h, 32, N * C, C,
+                                            N * C, C, (N + 1) * C, C, 1e-8, ops._dt(q), torch.cuda.current_stream().cuda_stream),
+               "sana_hip_linattn")
+    assert torch.equal(out[:, :N], ops.linattn_apply(q, ops.linattn_state(k, v), 1e-8))
+    assert bool(torch.isnan(out[:, N]).all())
+
+
 @pytest.mark.parametrize("N", [1, 16, 17, 33, 64, 65, 81, 97, 130])
 def test_fp32_splits_of_any_length_and_row_distance(cuda, N):
     """Phase 1 in passes of 64, 32 and 16 tokens with 32-bit offsets, and on rows too far apart for those, against 64 bits and each other;
