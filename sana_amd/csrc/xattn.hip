@@ -20,6 +20,11 @@
 // attention), 1024 9.9 / 8.5, 2 x 1024 12.6 / 11.8, 256 x 20 heads of 112 11.8 / 11.1, 1024 13.1 / 12.4, 4680 31.2 / 30.2, 16384 78 / 78; same bits.
 // Workgroups are persistent over consecutive (batch, head, query block) items and restage K / V only when the
 // (batch, head) changes.  Every K / V fragment read from LDS feeds QT MFMAs.
+// Many queries: of an item of 128 queries (8 us at 112 channels) the matrix pipes take 2 us, the vector units 2.6 and the LDS reads, eight
+// waves reading all of K and V, 2 - 4; the waves of a unit, in step, overlap little of it.  What a wave need not wait for is requested ahead:
+// an item's queries behind the scores of the one before it, and a new head's V, which the scores do not need, behind its K.  us, all in front of
+// the scores / so: 256 queries x 300 keys x 16 heads of 72 8.3 / 7.5, 2 x 1024 11.8 / 11.4, 16 x 1024 56 / 49, 1024 x 20 heads of 112 12.4 / 12.1, 4096
+// 30.6 / 27.0, 16 x 1024 87 / 76, 16384 79 / 69, 32760 152 / 132.
 #include <type_traits>
 
 #include "common.h"
@@ -46,12 +51,26 @@ __device__ __forceinline__ u32x2_t xa_read_tr(uint32_t lds) {
   return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(size_t)lds));
 }
 
-template <typename T, int DK, int DT, int QT, int NW, int NKT>
+// n / by of n < 2^31 with magic = (2^32 - 1) / by, which is at most one too small
+__device__ __forceinline__ int xa_div(int n, int by, uint32_t magic) {
+  const int z = (int)__umulhi((uint32_t)n, magic);
+  return n - z * by >= by ? z + 1 : z;
+}
+// What this wave wrote to LDS is there, and what it reads from there has come; loads from memory stay in flight.
+__device__ __forceinline__ void xa_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <typename T, int DK, int DT, int QT, int NW, int NKT, bool FAR>
 __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv,
                                                          const float* __restrict__ bias, uint16_t* __restrict__ out, int B,
                                                          int N, int Nk, int H, int d, int64_t ldq, int64_t ldkv, int64_t ldo,
                                                          int64_t bias_stride, float scale_log2e, int qblocks, int items,
-                                                         int items_per_wg) {
+                                                         int items_per_wg, uint32_t qblocks_magic, uint32_t h_magic) {
+  asm volatile("" ::"s"(q), "s"(kv), "s"(bias), "s"(B), "s"(N), "s"(Nk), "s"(H), "s"(d), "s"(ldq), "s"(ldkv), "s"(bias_stride), "s"(qblocks),
+               "s"(items), "s"(items_per_wg), "s"(qblocks_magic), "s"(h_magic));  // (the arguments in one wait)
   constexpr int KPITCH = DK * 64, KCH = DK * 4;  // bytes / 16-byte chunks per K row
   constexpr int K_BYTES = XA_NKP * KPITCH, V_BYTES = XA_NKP * XA_VPITCH;
   __shared__ __attribute__((aligned(16))) unsigned char smem[K_BYTES + V_BYTES + XA_NKP * 4];
@@ -61,95 +80,159 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int fr = lane & 15, fg = lane >> 4;
 
-  int staged = -1;
-  const int item0 = blockIdx.x * items_per_wg, item1 = min(items, item0 + items_per_wg);
-  for (int item = item0; item < item1; ++item) {
-    const int bh = item / qblocks, qb = item - bh * qblocks;
-    const int b = bh / H, h = bh - b * H;
-    const int q0 = qb * (NW * 16 * QT) + wave * (16 * QT);
-    // ---- Q fragments: column operand, lane -> query fr, k = 32*ks + 8*fg .. +7; requested in front of the staging
+  // ---- Q fragments: column operand, lane -> query fr, k = 32*ks + 8*fg .. +7; requested an item ahead
+  u32x4_t qn[QT][DK];
+  int bh, b, h, q0;  // of the item requested last
+  auto request = [&](int item) {
+    bh = xa_div(item, qblocks, qblocks_magic), b = xa_div(bh, H, h_magic), h = bh - b * H;
+    q0 = (item - bh * qblocks) * (NW * 16 * QT) + wave * (16 * QT);
     const uint16_t* qbase = q + ((int64_t)b * N) * ldq + (int64_t)h * d;
-    u32x4_t qf[QT][DK];
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
       const uint16_t* qrow = qbase + (int64_t)min(q0 + 16 * t + fr, N - 1) * ldq;  // (no branch around a load)
 #pragma unroll
+      for (int ks = 0; ks < DK; ++ks) qn[t][ks] = *reinterpret_cast<const u32x4_t*>(qrow + (32 * ks + 8 * fg < d ? 32 * ks + 8 * fg : 0));
+    }
+  };
+  u32x4_t qf[QT][DK];
+  auto take = [&]() {  // (here, not behind the stores or the branches that follow)
+#pragma unroll
+    for (int t = 0; t < QT; ++t)
+#pragma unroll
       for (int ks = 0; ks < DK; ++ks) {
-        const int k0 = 32 * ks + 8 * fg;
-        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(qrow + (k0 < d ? k0 : 0));
+        asm volatile("" : "+v"(qn[t][ks]));
 #pragma unroll
-        for (int e = 0; e < 4; ++e) qf[t][ks][e] = k0 < d ? v[e] : 0u;
+        for (int e = 0; e < 4; ++e) qf[t][ks][e] = 32 * ks + 8 * fg < d ? qn[t][ks][e] : 0u;
+        asm volatile("" : "+v"(qf[t][ks]));
+      }
+  };
+  const uint32_t sk0 = (uint32_t)(size_t)(__attribute__((address_space(3))) const unsigned char*)sk + fr * KPITCH;
+  uint32_t ka[DK];  // this lane's piece of K row fr, per k-step (rows 16 apart have the same swizzle)
+#pragma unroll
+  for (int ks = 0; ks < DK; ++ks) ka[ks] = sk0 + (((4 * ks + fg) ^ xa_kkey<DK>(fr)) << 4);
+
+  const int item0 = blockIdx.x * items_per_wg, item1 = min(items, item0 + items_per_wg);
+  auto stage = [&](bool first) {  // K and V of b, h
+    // the biases first, and K in front of V: the scores are multiplied while V is on its way
+    constexpr int NB = (16 * NKT + 64 * NW - 1) / (64 * NW);
+    float key_bias[NB];
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(bias + (bias ? (int64_t)b * bias_stride : 0)), 0, bias ? 4 * Nk : 0, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int m = tid + 64 * NW * i;
+      key_bias[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, 4 * m, 0, 0));  // (past Nk, and without biases: 0)
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    auto older = [&]() {  // the biases and the first item's queries, which are older than K, have landed (the compiler, too, knows it in here)
+#pragma unroll
+      for (int i = 0; i < NB; ++i) asm volatile("" : "+v"(key_bias[i]));
+      if (first) {
+#pragma unroll
+        for (int t = 0; t < QT; ++t)
+#pragma unroll
+          for (int ks = 0; ks < DK; ++ks) asm volatile("" : "+v"(qn[t][ks]));
+      }
+    };
+    const uint16_t* kbase = kv + (int64_t)b * Nk * ldkv + (int64_t)h * d;
+    const uint16_t* vbase = kbase + (int64_t)H * d;
+    // Rows past Nk and pieces past d lie outside the resources: zeros.  (key tiles past NKT are not read)
+    constexpr int NT = 64 * NW, KEYS = 16 * NKT;
+    constexpr uint32_t kOut = 0x80000000u;
+    if constexpr (!FAR) {
+      const uint32_t ld2 = 2 * (uint32_t)ldkv;
+      const int span = (int)((uint32_t)(Nk - 1) * ld2 + 2 * d);
+      const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kbase), 0, span, 0x00020000);
+      const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(vbase), 0, span, 0x00020000);
+      auto load = [&](const __amdgpu_buffer_rsrc_t& r, unsigned char* dst, uint32_t off) {
+        const int o = (int)off;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, o, 0, 0, 0);
+      };
+      // K: KI load instructions of 1 KB are 16 (12 pieces a row) or 4 rows (16 pieces); 16 rows and 4 waves repeat the swizzle
+      constexpr int KI = KCH == 16 ? 1 : KCH / 4, KR = 64 * KI / KCH;
+      static_assert(NW % 4 == 0 && (KR * NW) % 16 == 0 && KEYS % KR == 0, "");
+      uint32_t ko[KI];
+#pragma unroll
+      for (int j = 0; j < KI; ++j) {
+        const int l = 64 * j + lane, row = l / KCH, c = (l - row * KCH) ^ xa_kkey<DK>(KR * wave + row);
+        ko[j] = 8 * c < d ? (uint32_t)(KR * wave + row) * ld2 + 16 * c : kOut;
+      }
+#pragma unroll
+      for (int i = 0; i < (KEYS / KR + NW - 1) / NW; ++i) {
+        const int g = i * NW + wave;
+        if (i == KEYS / KR / NW && g >= KEYS / KR) break;  // uniform
+#pragma unroll
+        for (int j = 0; j < KI; ++j) load(rk, sk + (g * KI + j) * 1024, ko[j] + (uint32_t)(KR * NW * i) * ld2);
+      }
+      // V: 7 instructions are 32 rows
+      uint32_t vo[7];
+#pragma unroll
+      for (int j = 0; j < 7; ++j) {
+        const int l = 64 * j + lane, row = l / XA_VCH, c = l - row * XA_VCH;
+        vo[j] = 8 * c < d ? (uint32_t)(32 * wave + row) * ld2 + 16 * c : kOut;
+      }
+#pragma unroll
+      for (int i = 0; i < (KEYS / 32 + NW - 1) / NW; ++i) {
+        const int g = i * NW + wave;
+        if (i == KEYS / 32 / NW && g >= KEYS / 32) break;  // uniform
+#pragma unroll
+        for (int j = 0; j < 7; ++j) load(rv, sv + (g * 7 + j) * 1024, vo[j] + (uint32_t)(32 * NW * i) * ld2);
+      }
+      // K has landed (and what was requested before it); V is waited for behind the scores
+      constexpr int VI = KEYS / 32 / NW * 7;
+      if (wave < KEYS / 32 % NW) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(VI + 7) : "memory");
+      else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(VI) : "memory");
+      older();
+    } else {  // rows too far apart for 32-bit offsets
+      older();
+#pragma unroll 1
+      for (int i = tid; i < KEYS * KCH; i += NT) {
+        const int row = i / KCH, c = i - row * KCH;
+        u32x4_t x = {0u, 0u, 0u, 0u};
+        if (row < Nk && 8 * c < d) x = *reinterpret_cast<const u32x4_t*>(kbase + (int64_t)row * ldkv + 8 * c);
+        *reinterpret_cast<u32x4_t*>(sk + row * KPITCH + ((c ^ xa_kkey<DK>(row)) << 4)) = x;
+      }
+#pragma unroll 1
+      for (int i = tid; i < KEYS * XA_VCH; i += NT) {
+        const int row = i / XA_VCH, c = i - row * XA_VCH;
+        u32x4_t x = {0u, 0u, 0u, 0u};
+        if (row < Nk && 8 * c < d) x = *reinterpret_cast<const u32x4_t*>(vbase + (int64_t)row * ldkv + 8 * c);
+        *reinterpret_cast<u32x4_t*>(sv + 16 * i) = x;
       }
     }
-    if (bh != staged) {  // uniform
-      __syncthreads();   // everyone is done with the previous head's K / V
-      const uint16_t* kbase = kv + (int64_t)b * Nk * ldkv + (int64_t)h * d;
-      const uint16_t* vbase = kbase + (int64_t)H * d;
-      // Rows past Nk and pieces past d lie outside the resources: zeros.  (key tiles past NKT are not read)
-      constexpr int NT = 64 * NW, KEYS = 16 * NKT;
-      constexpr uint32_t kOut = 0x80000000u;
-      if (ldkv < (1 << 21)) {
-        const uint32_t ld2 = 2 * (uint32_t)ldkv;
-        const int span = (int)((uint32_t)(Nk - 1) * ld2 + 2 * d);
-        const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kbase), 0, span, 0x00020000);
-        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(vbase), 0, span, 0x00020000);
-        auto load = [&](const __amdgpu_buffer_rsrc_t& r, unsigned char* dst, uint32_t off) {
-          const int o = (int)off;
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, o, 0, 0, 0);
-        };
-        // K: KI load instructions of 1 KB are 16 (12 pieces a row) or 4 rows (16 pieces); 16 rows and 4 waves repeat the swizzle
-        constexpr int KI = KCH == 16 ? 1 : KCH / 4, KR = 64 * KI / KCH;
-        static_assert(NW % 4 == 0 && (KR * NW) % 16 == 0 && KEYS % KR == 0, "");
-        uint32_t ko[KI];
 #pragma unroll
-        for (int j = 0; j < KI; ++j) {
-          const int l = 64 * j + lane, row = l / KCH, c = (l - row * KCH) ^ xa_kkey<DK>(KR * wave + row);
-          ko[j] = 8 * c < d ? (uint32_t)(KR * wave + row) * ld2 + 16 * c : kOut;
-        }
-#pragma unroll
-        for (int i = 0; i < (KEYS / KR + NW - 1) / NW; ++i) {
-          const int g = i * NW + wave;
-          if ((KEYS / KR) % NW && g >= KEYS / KR) break;  // uniform
-#pragma unroll
-          for (int j = 0; j < KI; ++j) load(rk, sk + (g * KI + j) * 1024, ko[j] + (uint32_t)(KR * NW * i) * ld2);
-        }
-        // V: 7 instructions are 32 rows
-        uint32_t vo[7];
-#pragma unroll
-        for (int j = 0; j < 7; ++j) {
-          const int l = 64 * j + lane, row = l / XA_VCH, c = l - row * XA_VCH;
-          vo[j] = 8 * c < d ? (uint32_t)(32 * wave + row) * ld2 + 16 * c : kOut;
-        }
-#pragma unroll
-        for (int i = 0; i < (KEYS / 32 + NW - 1) / NW; ++i) {
-          const int g = i * NW + wave;
-          if ((KEYS / 32) % NW && g >= KEYS / 32) break;  // uniform
-#pragma unroll
-          for (int j = 0; j < 7; ++j) load(rv, sv + (g * 7 + j) * 1024, vo[j] + (uint32_t)(32 * NW * i) * ld2);
-        }
+    for (int i = 0; i < NB; ++i) {
+      const int m = tid + NT * i;
+      if (m < KEYS) sb[m] = m < Nk ? key_bias[i] * 1.44269504088896341f : -INFINITY;
+    }
+    if (first) take();
+    xa_barrier();
+  };
+  request(item0);
+  stage(true);
+  int staged = -1;
+  for (int item = item0; item < item1; ++item) {
+    const bool fresh = bh != staged;  // uniform
+    if (fresh && item > item0) {
+      xa_barrier();  // everyone is done with the previous head's K / V
+      stage(false);
+    }
+    staged = bh;
+    const int first_query = q0;
+    uint16_t* obase = out + ((int64_t)b * N) * ldo + (int64_t)h * d;
+    auto scores_done = [&]() {
+      if (fresh) {  // V has landed, everyone's
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      } else {  // rows too far apart for 32-bit offsets
-#pragma unroll 1
-        for (int i = tid; i < KEYS * KCH; i += NT) {
-          const int row = i / KCH, c = i - row * KCH;
-          u32x4_t x = {0u, 0u, 0u, 0u};
-          if (row < Nk && 8 * c < d) x = *reinterpret_cast<const u32x4_t*>(kbase + (int64_t)row * ldkv + 8 * c);
-          *reinterpret_cast<u32x4_t*>(sk + row * KPITCH + ((c ^ xa_kkey<DK>(row)) << 4)) = x;
-        }
-#pragma unroll 1
-        for (int i = tid; i < KEYS * XA_VCH; i += NT) {
-          const int row = i / XA_VCH, c = i - row * XA_VCH;
-          u32x4_t x = {0u, 0u, 0u, 0u};
-          if (row < Nk && 8 * c < d) x = *reinterpret_cast<const u32x4_t*>(vbase + (int64_t)row * ldkv + 8 * c);
-          *reinterpret_cast<u32x4_t*>(sv + 16 * i) = x;
-        }
+        xa_barrier();
       }
-      for (int m = tid; m < KEYS; m += NT)
-        sb[m] = m < Nk ? (bias ? bias[(int64_t)b * bias_stride + m] * 1.44269504088896341f : 0.f) : -INFINITY;
-      __syncthreads();
-      staged = bh;
+      request(min(item + 1, item1 - 1));
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if (first_query >= N) {
+      scores_done();
+      take();
+      continue;  // (no barrier below)
     }
-    if (q0 >= N) continue;  // (no barrier inside the per-item work below)
     // Keys in NG groups, one after the other (scores, softmax, product; the first group's scores are gone before the second's come:
     // 0.1 - 0.7 us less than all scores first).  f16: two, each with a maximum of its own, combined in fp32 at the end, and the sum
     // is over the rounded probabilities.  A group's largest probability is 1 and has no rounding error; the stock fused kernels,
@@ -168,21 +251,30 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
         for (int t = 0; t < QT; ++t) sc[t][kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       // key tiles in pairs (two independent accumulator chains), the next pair's fragments requested before this pair's MFMAs
       u32x4_t kf[2][2][DK];
+      // (asm reads: to the compiler an ordinary one may alias the loads of V in flight)
       auto load_k = [&](int buf, int kt) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int row = 16 * (kt + j) + fr;
-          const unsigned char* rp = sk + row * KPITCH;
-          const int key = xa_kkey<DK>(row);
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-          for (int ks = 0; ks < DK; ++ks) kf[buf][j][ks] = *reinterpret_cast<const u32x4_t*>(rp + (((4 * ks + fg) ^ key) << 4));
-        }
+          for (int ks = 0; ks < DK; ++ks) {
+            const uint32_t at = ka[ks] + (kt + j < 10 ? 0 : 160 * KPITCH);  // (an offset has 16 bits)
+            asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(kf[buf][j][ks]) : "v"(at), "n"((kt + j) % 10 * 16 * KPITCH));
+          }
+      };
+      auto landed = [&](int buf, bool more) {
+        if (more) asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(2 * DK) : "memory");
+        else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int ks = 0; ks < DK; ++ks) asm volatile("" : "+v"(kf[buf][j][ks])::"memory");
       };
       load_k(0, k0);
 #pragma unroll
       for (int kt = k0; kt < k1; kt += 2) {
         const int buf = (kt - k0) / 2 & 1;
         if (kt + 2 < k1) load_k(buf ^ 1, kt + 2);
+        landed(buf, kt + 2 < k1);
 #pragma unroll
         for (int ks = 0; ks < DK; ++ks)
 #pragma unroll
@@ -190,7 +282,9 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
 #pragma unroll
             for (int t = 0; t < QT; ++t)
               sc[t][kt - k0 + j] = mfma_16x16x32<T>(kf[buf][j][ks], qf[t][ks], sc[t][kt - k0 + j]);
+        __builtin_amdgcn_sched_barrier(0);
       }
+      if constexpr (g == 0) scores_done();
       // ---- softmax over the group's keys (log2 domain), probabilities packed to 16 bits
       u32x2_t pk[QT][G0];
 #pragma unroll
@@ -265,11 +359,11 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
         factor[t][0] = 1.0f / sum[t][0];
       }
     }
+    take();  // (in front of the stores, which it need not wait for)
     // ---- normalise and store: a lane holds 4 consecutive channels of its query per channel tile
-    uint16_t* obase = out + ((int64_t)b * N) * ldo + (int64_t)h * d;
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
-      const int qi = q0 + 16 * t + fr;
+      const int qi = first_query + 16 * t + fr;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         const int c0 = 16 * dt + 4 * fg;
@@ -286,7 +380,7 @@ __global__ __launch_bounds__(64 * NW) void cross_attn_kernel(const uint16_t* __r
   }
 }
 
-template <typename T, int DK, int DT, int QT, int NW, int NKT>
+template <typename T, int DK, int DT, int QT, int NW, int NKT, bool FAR = false>
 int launch_xa(const uint16_t* q, const uint16_t* kv, const float* bias, uint16_t* out, int B, int N, int Nk, int H, int d,
               int64_t ldq, int64_t ldkv, int64_t ldo, int64_t bias_stride, float scale, hipStream_t s) {
   const int qblocks = (N + NW * 16 * QT - 1) / (NW * 16 * QT);
@@ -295,8 +389,8 @@ int launch_xa(const uint16_t* q, const uint16_t* kv, const float* bias, uint16_t
   const int items = (int)items64, cus = 256;
   const int ipw = (items + cus - 1) / cus;
   const int grid = (items + ipw - 1) / ipw;
-  hipLaunchKernelGGL((cross_attn_kernel<T, DK, DT, QT, NW, NKT>), dim3((unsigned)grid), dim3(64 * NW), 0, s, q, kv, bias, out, B, N, Nk, H, d,
-                     ldq, ldkv, ldo, bias_stride, scale * 1.44269504088896341f, qblocks, items, ipw);
+  hipLaunchKernelGGL((cross_attn_kernel<T, DK, DT, QT, NW, NKT, FAR>), dim3((unsigned)grid), dim3(64 * NW), 0, s, q, kv, bias, out, B, N, Nk, H, d,
+                     ldq, ldkv, ldo, bias_stride, scale * 1.44269504088896341f, qblocks, items, ipw, 0xffffffffu / (uint32_t)qblocks, 0xffffffffu / (uint32_t)H);
   return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
 }
 
@@ -323,6 +417,9 @@ int cross_attention(const void* q, const void* kv, const float* key_bias, void* 
   // 12.7 / 13.8, 160 keys 8.9 / 9.2, f16 13.5 / 14.0; but 77 keys 8.1 / 7.8.
   const bool restaged = (int64_t)B * H >= 64 && N > 64 * XA_QT && Nk > (is_f16<T> ? 256 : 128);
   const bool few = d <= 96 && !restaged && (int64_t)B * H * ((N + 64 * XA_QT - 1) / (64 * XA_QT)) <= 256;
+  if (ldkv >= (1 << 21))  // rows of K and V too far apart for 32-bit offsets: staged through registers (the same bits)
+    return Nk > 160 ? launch_xa<T, 4, 7, XA_QT, 8, 20, true>(qp, kp, key_bias, op, B, N, Nk, H, d, ldq, ldkv, ldo, bias_stride, scale, s)
+                    : launch_xa<T, 4, 7, XA_QT, 8, 10, true>(qp, kp, key_bias, op, B, N, Nk, H, d, ldq, ldkv, ldo, bias_stride, scale, s);
   // key tiles of 16 that are multiplied: all 20, or 10 for up to 160 keys (tiles past Nk hold zeros and -inf)
   if (d > 96) return Nk > 160 ? SANA_XA_GO(4, 7, 8, 20) : SANA_XA_GO(4, 7, 8, 10);
   // (the product with V in tiles of 16 channels: five up to 80)

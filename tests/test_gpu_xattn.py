@@ -383,3 +383,19 @@ def test_keys_of_any_distance_give_the_bits_of_dense_ones(cuda, dtype, H, d, Nk)
         rows = torch.full((Nk * ld,), float("nan"), dtype=dtype, device=cuda).view(1, Nk, ld)
         rows[:, :, :2 * C] = kv
         assert torch.equal(ops.cross_attention16(q, rows[:, :, :2 * C], H), dense)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,N,H,d", [(9, 130, 20, 112), (5, 1000, 16, 72), (3, 1, 150, 96), (2, 2300, 17, 104)])
+@pytest.mark.parametrize("Nk", [33, 230])
+def test_workgroups_of_several_heads(cuda, B, N, H, d, Nk, dtype):
+    """Workgroups whose items run over query blocks, heads and batch entries, with waves that have no query in a head's last block and
+    biases of each batch entry's own: queries requested an item ahead and K and V of the next head give the bits of one entry at a time."""
+    g = torch.Generator().manual_seed(N + d + Nk)
+    q, kv = (torch.randn(B, n, c * H * d, generator=g).to(dtype).to(cuda) for n, c in ((N, 1), (Nk, 2)))
+    bias = torch.where(torch.rand(B, Nk, generator=g) < 0.3, -10000.0, 0.0).to(cuda)
+    got = ops.cross_attention16(q, kv, H, bias)
+    for b in range(B):
+        assert torch.equal(got[b], ops.cross_attention16(q[b:b + 1], kv[b:b + 1], H, bias[b:b + 1])[0])
+    ref = formula(q[-1:].cpu(), kv[-1:].cpu(), H, bias[-1:].cpu())
+    assert rel_l2(got[-1:].cpu(), ref) <= 1e-2
