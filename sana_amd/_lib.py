@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 from ctypes import c_float, c_int, c_int64, c_size_t, c_void_p
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -27,6 +28,10 @@ class BlockArgs(ctypes.Structure):
                              "split_k", "io_dtype")] + [
         (n, c_float) for n in ("eps_norm1", "eps_norm2", "eps_attn", "cross_scale")]
 
+
+# its fields in order ("0q": padded at the end as the structure is)
+BLOCK_ARGS = struct.Struct("@26PN3q11i4f0q")
+assert BLOCK_ARGS.size == ctypes.sizeof(BlockArgs)
 
 # name -> (restype, argtypes); must list every symbol include/sana_hip.h declares
 SIGNATURES = {

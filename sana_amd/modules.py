@@ -1085,16 +1085,26 @@ class SanaMSBlock(nn.Module):
                 return None
         ic, pc, dc = mlp._pointwise_params(mlp.inverted_conv), mlp._pointwise_params(mlp.point_conv), mlp.depth_conv.conv
         hid, dt, dev = mlp.hidden_features, x.dtype, x.get_device()
-        ps = []
-        for m, shape in zip((*linears, ic, dc, pc), ((3 * C, C), (C, C), (C, C), (C, C), (2 * hid, C), (2 * hid, 1), (C, hid))):
-            w, b = m._parameters.get("weight"), m._parameters.get("bias")
-            if type(w) not in _PLAIN or w.dtype != dt or w.shape[:2] != shape or w.get_device() != dev or not w.is_contiguous() or w.data_ptr() % 16:
+        ps = []     # (a small image waits for this walk, a block at a time: each attribute is read once)
+        qkv, proj, q_linear, o_linear = linears
+        for m, rows, cols in ((qkv, 3 * C, C), (proj, C, C), (q_linear, C, C), (o_linear, C, C), (ic, 2 * hid, C), (dc, 2 * hid, 1),
+                              (pc, C, hid)):
+            own = m._parameters
+            w, b = own.get("weight"), own.get("bias")
+            if type(w) not in _PLAIN or w.dtype is not dt or w.get_device() != dev or not w.is_contiguous():
                 return None
-            if b is not None and (type(b) not in _PLAIN or b.dtype != dt or b.numel() != shape[0] or b.get_device() != dev or not b.is_contiguous()
-                                  or b.data_ptr() % 16):
+            at = w.data_ptr()
+            if w.shape[:2] != (rows, cols) or at % 16:
                 return None
-            ps += (w.data_ptr(), None if b is None else b.data_ptr())
-        if None in (ps[3], ps[5], ps[7], ps[9]) or dc.weight.numel() != 18 * hid or hid % 8 or not x.is_contiguous() \
+            ps.append(at)
+            if b is None:
+                ps.append(0)
+                continue
+            at = b.data_ptr() if type(b) in _PLAIN else 1
+            if at % 16 or b.dtype is not dt or b.get_device() != dev or b.numel() != rows or not b.is_contiguous():
+                return None
+            ps.append(at)
+        if not (ps[3] and ps[5] and ps[7] and ps[9]) or dc.weight.numel() != 18 * hid or hid % 8 or not x.is_contiguous() \
                 or x.data_ptr() % 16 or modulation.shape != (B, 6, C) or not modulation.is_contiguous() \
                 or modulation.get_device() != dev or modulation.data_ptr() % 16 \
                 or (mask is not None and mask.get_device() != dev) or not ca._residual_in_gemm(x, y, mask, text_kv):
@@ -1116,11 +1126,11 @@ class SanaMSBlock(nn.Module):
         text_kv, modulation = kwargs.get("text_kv"), kwargs.get("modulation")
         if modulation is None:
             modulation = self.scale_shift_table[None] + t.reshape(B, 6, -1)
-        shift_msa, scale_msa, gate_msa, shift_mlp, scale_mlp, gate_mlp = modulation.chunk(6, dim=1)
         # (conditioning in another dtype than x -- an fp32 t with a bf16 x -- promotes in the stock op chain; the
         # fused kernels read the modulation rows as x's dtype, so that case takes the stock composition below)
-        if x.is_cuda and x.dtype in ops.IO16 and shift_msa.dtype == x.dtype and C % 8 == 0 and C <= 8192 \
-                and not torch.is_grad_enabled():
+        fused = (x.is_cuda and x.dtype in ops.IO16 and modulation.dtype == x.dtype and C % 8 == 0 and C <= 8192
+                 and not torch.is_grad_enabled())
+        if fused:
             attn = self.attn
             # the block as one call; with many bf16 tokens the qkv projection takes the attention's first phase along, and
             # the host is ahead anyway
@@ -1129,6 +1139,8 @@ class SanaMSBlock(nn.Module):
                 out = self._one_call(x, y, modulation, mask, HW, text_kv)
                 if out is not None:
                     return out
+        shift_msa, scale_msa, gate_msa, shift_mlp, scale_mlp, gate_mlp = modulation.chunk(6, dim=1)
+        if fused:
             # fused seams: LayerNorm + modulate in one kernel, gate * out + residual in the GEMM epilogue
             h = ops.layernorm_modulate(x, scale_msa, shift_msa, self.norm1.eps)
             if "forward" in attn.__dict__:
@@ -1213,7 +1225,7 @@ class StepConditioning:
                    for b in self.blocks):
             return [dict(modulation=mod[i]) for i in range(L)]
         kv = ops.gemm_bf16(y.reshape(B * Nk, C), w, b, "bias").view(B, Nk, L, 2 * C)
-        return [dict(text_kv=kv[:, :, i], modulation=mod[i]) for i in range(L)]
+        return [dict(text_kv=k, modulation=m) for k, m in zip(kv.unbind(2), mod.unbind(0))]
 
 
 class ChunkedLiteLAReLURope(LiteLAReLURope):

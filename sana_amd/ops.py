@@ -85,9 +85,10 @@ def chunk_table(chunk_tokens: Optional[Sequence[int]], N: int, device) -> Tuple[
 
 def _token_major_view(t: torch.Tensor, what: str) -> Tuple[int, int]:
     """t: [B, N, C] with unit channel stride -> (stride_b, stride_n) in elements."""
-    if t.dim() != 3 or t.stride(2) != 1:
-        raise SanaHipError(f"{what} must be a [B, N, C] view with unit channel stride, got strides {t.stride()}")
-    return (t.stride(0) if t.shape[0] > 1 else 0), t.stride(1)
+    strides = t.stride()
+    if len(strides) != 3 or strides[2] != 1:
+        raise SanaHipError(f"{what} must be a [B, N, C] view with unit channel stride, got strides {strides}")
+    return (strides[0] if t.shape[0] > 1 else 0), strides[1]
 
 
 class QkPre:
@@ -332,11 +333,14 @@ STATE_SCRATCH_KEPT = 64 << 20   # bytes of attention state and partial states th
 def _one_call(q, k, v, d: int) -> bool:
     """Whether ``sana_hip_linattn`` takes these.  What it does not (mixed dtypes or shapes, k and v of different
     strides, other head dims) goes to the two calls, which serve or refuse it."""
-    if d != HEAD_DIM or q.dim() != 3 or not q.is_cuda or q.shape != k.shape or k.shape != v.shape:
+    if d != HEAD_DIM or q.dim() != 3 or not q.is_cuda:
         return False
-    if q.dtype != k.dtype or k.dtype != v.dtype or q.dtype not in _DT or q.shape[2] % d or q.numel() == 0:
+    shape, dt, dev = q.shape, q.dtype, q.get_device()
+    if k.shape != shape or v.shape != shape or k.dtype is not dt or v.dtype is not dt or dt not in _DT or shape[2] % d or q.numel() == 0 \
+            or k.get_device() != dev or v.get_device() != dev:
         return False
-    return q.device == k.device == v.device and all(a == b or n == 1 for a, b, n in zip(k.stride(), v.stride(), k.shape))
+    ks, vs = k.stride(), v.stride()
+    return ks == vs or all(a == b or n == 1 for a, b, n in zip(ks, vs, shape))
 
 
 def relu_linear_attention(q, k, v, eps: float, chunk_tokens=None, out_dtype=None,
@@ -345,21 +349,22 @@ def relu_linear_attention(q, k, v, eps: float, chunk_tokens=None, out_dtype=None
     causal = chunk_tokens is not None and len(chunk_tokens) > 1
     if not causal and out_dtype in (None, q.dtype) and _one_call(q, k, v, head_dim):
         B, N, C = q.shape
-        h, dt, lib, stream = C // head_dim, _dt(q), _lib.load(), _stream()
-        qs, ks = _token_major_view(q, "q"), _token_major_view(k, "k")
-        out = torch.empty(B, N, C, dtype=q.dtype, device=q.device)
+        h, dt, lib, stream, device = C // head_dim, _DT[q.dtype], _lib.load(), _stream(), q.device
+        (qb, qn), (kb, kn) = _token_major_view(q, "q"), _token_major_view(k, "k")
+        out = torch.empty((B, N, C), dtype=q.dtype, device=device)
         nbytes = lib.sana_hip_linattn_scratch_bytes(B, N, h, head_dim, dt)
         # The state is in there as well: of this call's own under capture (graphs that a caller captures on one stream and
         # replays side by side must not share it) and where it is too large to be kept.  us, fp32 1024 tokens x 36 heads, own
         # always / the stream's where it may be: 17.8 / 17.2.
         if nbytes and (nbytes > STATE_SCRATCH_KEPT or torch._C._cuda_isCurrentStreamCapturing()):
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
         else:
-            ws = _workspace(q.device, nbytes, stream)
+            ws = _workspace(device, nbytes, stream)
         code = lib.sana_hip_linattn(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                                    ws.data_ptr() if ws is not None else None, nbytes, B, N, h, head_dim, *qs, *ks,
+                                    ws.data_ptr() if ws is not None else None, nbytes, B, N, h, head_dim, qb, qn, kb, kn,
                                     N * C if B > 1 else 0, C, float(eps), dt, stream)
-        _lib.check(code, "sana_hip_linattn")
+        if code:
+            _lib.check(code, "sana_hip_linattn")
         return out
     state = linattn_state(k, v, chunk_tokens, causal=causal, head_dim=head_dim)
     return linattn_apply(q, state, eps, chunk_tokens, out_dtype)
@@ -754,22 +759,24 @@ def block(x, text_kv, key_bias, modulation, weights, ones, hidden, cross_heads, 
           eps_norm2, eps_attn) -> torch.Tensor:
     """A whole image block in one call (``sana_hip_block``).  The caller has checked devices, dtypes, shapes and alignment:
     x [B, N, C] and modulation [B, 6, C] dense, text_kv [B, Nk, 2C] rows, key_bias fp32 [B, Nk] or None, ``weights`` the
-    weight and bias pointers of qkv, proj, q_linear, cross-attention proj, inverted, depthwise and point convolution."""
+    weight and bias pointers (0: no bias) of qkv, proj, q_linear, cross-attention proj, inverted, depthwise and point convolution."""
     B, N, C = x.shape
     lib = _lib.load()
     out = torch.empty_like(x)
     mod = modulation.data_ptr()
     if key_bias is not None:
         key_bias = key_bias.contiguous()
-    args = _lib.BlockArgs(
+    Nk = text_kv.shape[1]
+    args = _lib.BlockArgs.from_buffer_copy(_lib.BLOCK_ARGS.pack(     # (half the time of a constructor of as many fields)
         x.data_ptr(), text_kv.data_ptr(), mod, mod + 2 * C, mod + 4 * C, mod + 6 * C, mod + 8 * C, mod + 10 * C,
-        *weights[:8], ones.data_ptr(), *weights[8:], None if key_bias is None else key_bias.data_ptr(), out.data_ptr(), None, 0,
-        text_kv.stride(1), text_kv.shape[1], 6 * C if B > 1 else 0,
-        B, N, C, hidden, cross_heads, text_kv.shape[1], int(HW[0]), int(HW[1]), 1 if round_like_reference else 0, 1 if SPLIT_K else 0,
-        _dt(x), eps_norm1, eps_norm2, eps_attn, (C // cross_heads) ** -0.5)
+        *weights[:8], ones.data_ptr(), *weights[8:], 0 if key_bias is None else key_bias.data_ptr(), out.data_ptr(), 0, 0,
+        text_kv.stride(1), Nk, 6 * C if B > 1 else 0,
+        B, N, C, hidden, cross_heads, Nk, int(HW[0]), int(HW[1]), 1 if round_like_reference else 0, 1 if SPLIT_K else 0,
+        _dt(x), eps_norm1, eps_norm2, eps_attn, (C // cross_heads) ** -0.5))
     ref = _lib.ctypes.byref(args)
-    scratch = torch.empty(lib.sana_hip_block_scratch_bytes(ref), dtype=torch.uint8, device=x.device)
-    args.scratch, args.scratch_bytes = scratch.data_ptr(), scratch.numel()
+    need = lib.sana_hip_block_scratch_bytes(ref)
+    scratch = torch.empty(need, dtype=torch.uint8, device=x.device)
+    args.scratch, args.scratch_bytes = scratch.data_ptr(), need
     _lib.check(lib.sana_hip_block(ref, _stream()), "sana_hip_block")
     return out
 
