@@ -859,12 +859,16 @@ struct Tile16 {
 // 20000 tokens, widths as above), kernel as it is, 7.9 / 4.9: 14208 x 3456 x 1152 109 / 98, 16576 x 2240 x 2240 167 / 157, 7246 x 9216 x 1152 140 /
 // 133, 6017 x 11200 x 2240 251 / 241, 2079 x 18432 x 1152 88 / 84, 12423 x 2240 x 2240 115 / 111; 18219 x 9216 x 1152 307 / 311, 6400 x 6720 x 2240
 // 145 / 151; 0.979 on the mean of 48.  (3.9: 993 x 18432 x 1152 42.7 / 48.1.)
+// 160 x 192 is chosen between 257 and 320 tokens where both of its rows of tiles run in one round, the tiles of 256 rows padding two fifths and
+// the smaller ones taking two rounds; 256 x 192 / so, weights cold: 260 x 17920 x 2240 39.2 / 33.7, 288 x 18432 x 1152 25.1 / 20.7, 300 x 24000 x 1152 26.2 / 22.6,
+// 320 x 24000 x 3072 60.7 / 54.7, 300 x 20480 x 1536 with a gate 34.0 / 31.6.
 constexpr Tile16 kTiles16[] = {
     {64, 64, 512, 256, 257, 3.0, 0.288, 0.503, true, 0.165, 0.26}, {64, 128, 256, 32, 256, 3.9, 0.350, 0.414, true},
     {96, 128, 256, 32, 256, 3.7, 0.439, 0.466, true},  {128, 128, 256, 32, 256, 3.9, 0.454, 0.541, true},
     {128, 160, 256, 32, 256, 4.3, 0.517, 0.643, true}, {192, 128, 256, 32, 256, 4.7, 0.497, 0.687, true},
     {256, 128, 256, 32, 256, 5.1, 0.624, 0.825, true}, {256, 192, 256, 32, 256, 4.9, 0.628, 1.150},
     {256, 256, 256, 32, 256, 5.3, 0.999, 1.404},       {256, 288, 256, 32, 256, 9.5, 0.955, 1.603},
+    {160, 192, 256, 32, 256, 7.4, 0.487, 0.975, true},
 };
 constexpr int kTile192 = 7, kTile256 = 8, kTile288 = 9;
 // K below 1024.  These are the times that the tiles had in GEMMs of K = 1152 .. 5600 before the loop over whole k-tiles; at such K

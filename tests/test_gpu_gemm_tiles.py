@@ -82,6 +82,15 @@ def test_many_token_gated_residual_across_batch_boundaries(cuda, tile, B, Ntok, 
     assert torch.equal(ops.gemm_gate_residual(a, w, bias, gate, res), res + gate * y)   # the stock pair's roundings
 
 
+@pytest.mark.parametrize("M,N,K", [(257, 18440, 1152), (300, 17920, 2240), (320, 18376, 1208), (290, 20480, 1064)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_two_tiles_of_160_tokens_are_exact_on_integers(cuda, M, N, K, dtype):
+    """160 x 192: a prompt's tokens by many channels, with ragged tokens and channels, k tails and gate rows that change inside a tile."""
+    test_many_token_tiles_are_exact_on_integers(cuda, (160, 192), M, N, K, dtype)
+    if M % 2 == 0:
+        test_many_token_gated_residual_across_batch_boundaries(cuda, (160, 192), 2, M // 2, N, K, dtype)
+
+
 @pytest.mark.parametrize("M,N,K", [(300, 264, 5664), (257, 200, 4128), (700, 1160, 6432), (130, 3000, 8192), (1025, 2232, 5600)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_split_over_k_is_exact_on_integers(cuda, M, N, K, dtype):
