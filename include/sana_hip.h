@@ -287,7 +287,7 @@ size_t sana_hip_gemm_workspace_bytes(int M, int N, int K);
 
 /* What a 16-bit GEMM of this shape runs as, given that workspace: plan[0], plan[1] = tokens and channels of a workgroup's
  * tile; plan[2] > 0: its first plan[2] channels run in tiles of 256 x 256, the rest in tiles of 256 x 192 (two launches);
- * plan[3] > 1: K in that many ranges, by the split kernel (tiles of 256 channels or 192) or within a smaller tile.  A host-side
+ * plan[3] > 1: K in that many ranges, by the split kernel (tiles of 192 channels) or within a smaller tile.  A host-side
  * query for tests and measurements. */
 int sana_hip_gemm_plan(int M, int N, int K, int plan[4]);
 

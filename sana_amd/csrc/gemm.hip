@@ -1,7 +1,7 @@
 // bf16 MFMA GEMM for gfx950:  C[M][N] = epilogue(A[M][K] . W[N][K]^T), with an int8-weight (W8A16) variant
 // dequantised on the way into LDS: the C entry points, the choice of a kernel by shape, and the kernels for int8
-// weights and for k split into ranges, which the rest of this comment describes.  Unsplit 16-bit GEMMs run the kernels of
-// gemm8.h (many tokens) and gemm_ring.h (few).
+// weights, which the rest of this comment describes.  16-bit GEMMs run the kernels of gemm8.h and gemm288.h (many tokens, and k
+// split into ranges) and gemm_ring.h (few).
 //
 // Both operands are K-contiguous, which is exactly the MFMA operand layout (a
 // lane holds 8 consecutive k of one row), so nothing is transposed.  The MFMA

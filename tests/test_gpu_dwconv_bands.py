@@ -1,5 +1,5 @@
 """The depthwise kernel's bands of 2, 4 and 8 rows give the same bits: a small image alone (bands of 2 where those are at most
-256 workgroups) and as one of a batch whose launch is large enough for taller bands."""
+1536 workgroups) and as one of a batch whose launch is large enough for taller bands."""
 import pytest
 import torch
 
