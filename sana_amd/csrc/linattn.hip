@@ -48,10 +48,20 @@ constexpr int D = 32;
 constexpr int STATE_ELEMS = (D + 1) * D;  // 1056
 constexpr int TILE = 32;                  // tokens per phase-1 tile
 
+template <int OFF>
+__device__ __forceinline__ u32x2_t lds_read_tr16(uint32_t addr) {  // 4 tokens x 16 channels -> this lane's channel, 4 tokens
+  u32x2_t v;
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+  return v;
+}
+
 // ----------------------------------------------------------------------------
 // phase 1, 16-bit io
 // grid: x = nsplit, y = n_chunks, z = B * pairs;  block 256
 // dst: when nsplit == 1 the final state, else partial[(bh*n_chunks + c)*nsplit + split][1056]
+// At a few thousand tokens bound by latency: a split is one or two tiles a wave.  Loads without a branch and a 64-bit product each, and 16
+// transposing reads a tile where 64 two-byte ones were packed in pairs (same bits).  us with the reduction, before / now: 1600 tokens x 20 heads
+// 7.8 / 7.1, 2048 x 36 8.7 / 8.1, 4096 x 70 14.4 / 13.7, with the norm 16.2 / 15.5, with the rotation 15.8 / 15.3, 16384 x 70 35.7 / 34.9.
 // ----------------------------------------------------------------------------
 // PRE: on-load transforms as compile-time bits (1 = q/k RMSNorm, 2 = rotary embedding, 4 = the rotation comes before
 // the ReLU and ksum is taken from the rotated values: QkPre::rope_first)
@@ -60,12 +70,14 @@ __global__ __launch_bounds__(256) void linattn_state16_kernel(
     const uint16_t* __restrict__ K, const uint16_t* __restrict__ V, float* __restrict__ dst,
     const int32_t* __restrict__ chunk_starts, int N, int h, int n_chunks, int nsplit, int split_tokens,
     int64_t stride_b, int64_t stride_n, const QkPre pre) {
-  // staging: per wave K tile [32 tok][64 ch] + V tile, 16-bit -> 8 KB per wave.
+  // staging: per wave K tile [32 tok][64 ch] + V tile, 16-bit, rows of ROW bytes -> 10 KB per wave (four workgroups per CU).
   // reduction: per wave 2 heads x 1056 fp32 -> 8448 B per wave.  The two uses
   // never overlap in time, so they share one buffer.
-  __shared__ __attribute__((aligned(16))) unsigned char smem[4 * 2 * STATE_ELEMS * 4];
+  constexpr int ROW = 160;  // 40 banks: the eight rows of a transposing read meet every bank twice
+  static_assert(2 * TILE * ROW >= 2 * STATE_ELEMS * 4, "the reduction fits in the stages");
+  __shared__ __attribute__((aligned(16))) unsigned char smem[4 * 2 * TILE * ROW];
   const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int pairs = (h + 1) >> 1;
   const int b = blockIdx.z / pairs, p = blockIdx.z % pairs;
   const int c = blockIdx.y, split = blockIdx.x;
@@ -74,9 +86,8 @@ __global__ __launch_bounds__(256) void linattn_state16_kernel(
   const int t0 = cr.begin + split * split_tokens;
   const int t1 = min(cr.end, t0 + split_tokens);
 
-  uint16_t* stage = reinterpret_cast<uint16_t*>(smem) + wave * (2 * TILE * 64);
-  uint16_t* lds_k = stage;
-  uint16_t* lds_v = stage + TILE * 64;
+  unsigned char* lds_k = smem + wave * (2 * TILE * ROW);
+  unsigned char* lds_v = lds_k + TILE * ROW;
 
   // load mapping: lane -> token (lane/8 + 8*i), 16-byte channel chunk lane%8
   const int ld_tok = lane >> 3;
@@ -104,7 +115,33 @@ __global__ __launch_bounds__(256) void linattn_state16_kernel(
   u32x4_t kw = zero4;
   float ks8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (has_norm && ch_ok) kw = *reinterpret_cast<const u32x4_t*>(pre.weight + ld_ch);
+  // Loads without a branch each: tokens from t1 on and channels past C lie outside the resources, zeros.
+  const bool near = (int64_t)(t1 - t0 + TILE) * stride_n < (1 << 29);  // 32-bit offsets
+  constexpr uint32_t kOut = 0x80000000u;
   auto issue_loads = [&](int tile) {
+    if (near) {
+      const int span = ((t1 - t0 - 1) * (int)stride_n + min(64, C - p * 64)) * 2;
+      const int64_t at = (int64_t)b * stride_b + (int64_t)t0 * stride_n + p * 64;
+      const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(K + at), 0, span, 0x00020000);
+      const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(V + at), 0, span, 0x00020000);
+      const __amdgpu_buffer_rsrc_t rn = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<float*>(has_norm ? pre.rinv + (int64_t)b * N + t0 : nullptr), 0, has_norm ? (t1 - t0) * 4 : 0, 0x00020000);
+      const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<float*>(has_rope ? pre.rope + (int64_t)t0 * 32 : nullptr), 0, has_rope ? (t1 - t0) * 128 : 0, 0x00020000);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int tok = tile - t0 + ld_tok + 8 * i, o = ch_ok ? (tok * (int)stride_n + (lane & 7) * 8) * 2 : (int)kOut;
+        kreg[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rk, o, 0, 0));
+        vreg[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rv, o, 0, 0));
+        if (has_norm) rin[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rn, tok * 4, 0, 0));
+        if (has_rope) {
+          const int ro = tok * 128 + (lane & 3) * 32;
+          cs[i][0] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rr, ro, 0, 0));
+          cs[i][1] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rr, ro + 16, 0, 0));
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int tok = tile + ld_tok + 8 * i;
@@ -135,6 +172,9 @@ __global__ __launch_bounds__(256) void linattn_state16_kernel(
   // element r of k-step s is token 16*s + 2*r + g of the tile (any bijection works as
   // long as both operands use the same one: the MFMA contracts over tokens).
   const int j = lane & 31, g = lane >> 5;
+  // A transposing read hands the 16 lanes of a group four rows, row i addressed by lanes 4 i .. 4 i + 3: two tokens apart here.
+  const uint32_t k_at = (uint32_t)(size_t)(__attribute__((address_space(3))) const unsigned char*)lds_k +
+                        (2 * ((lane >> 2) & 3) + g) * ROW + ((lane >> 4) & 1) * 32 + (lane & 3) * 8, v_at = k_at + TILE * ROW;
   for (; tile < t1; tile += 4 * TILE) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -152,32 +192,47 @@ __global__ __launch_bounds__(256) void linattn_state16_kernel(
       } else {
         kk = relu_pk16(kk);
       }
-      *reinterpret_cast<u32x4_t*>(lds_k + (ld_tok + 8 * i) * 64 + (lane & 7) * 8) = kk;
-      *reinterpret_cast<u32x4_t*>(lds_v + (ld_tok + 8 * i) * 64 + (lane & 7) * 8) = vreg[i];
+      *reinterpret_cast<u32x4_t*>(lds_k + (ld_tok + 8 * i) * ROW + (lane & 7) * 16) = kk;
+      *reinterpret_cast<u32x4_t*>(lds_v + (ld_tok + 8 * i) * ROW + (lane & 7) * 16) = vreg[i];
     }
     if (tile + 4 * TILE < t1) issue_loads(tile + 4 * TILE);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // wave-private LDS: in-order, no barrier needed
+    u32x2_t kf[2][2][2], vf[2][2][2];  // [head][k-step][elements 4 i ..]
+    auto read = [&](auto hh_c) {
+      constexpr int hh = decltype(hh_c)::value;
+      kf[hh][0][0] = lds_read_tr16<64 * hh>(k_at), kf[hh][0][1] = lds_read_tr16<64 * hh + 8 * ROW>(k_at);
+      vf[hh][0][0] = lds_read_tr16<64 * hh>(v_at), vf[hh][0][1] = lds_read_tr16<64 * hh + 8 * ROW>(v_at);
+      kf[hh][1][0] = lds_read_tr16<64 * hh + 16 * ROW>(k_at), kf[hh][1][1] = lds_read_tr16<64 * hh + 24 * ROW>(k_at);
+      vf[hh][1][0] = lds_read_tr16<64 * hh + 16 * ROW>(v_at), vf[hh][1][1] = lds_read_tr16<64 * hh + 24 * ROW>(v_at);
+    };
+    read(std::integral_constant<int, 0>{});
+    if (!has_rope) read(std::integral_constant<int, 1>{});  // (with the rotation: later, for the registers of a third workgroup)
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
+      if (hh == 1 && has_rope) read(std::integral_constant<int, 1>{});
+      if (hh == 0 && has_rope)
+        asm volatile("s_waitcnt lgkmcnt(0)"
+                     : "+v"(kf[0][0][0]), "+v"(kf[0][0][1]), "+v"(kf[0][1][0]), "+v"(kf[0][1][1]), "+v"(vf[0][0][0]), "+v"(vf[0][0][1]),
+                       "+v"(vf[0][1][0]), "+v"(vf[0][1][1])::"memory");
+      else if (hh == 0)  // (the reads come in order: the second head's eight are behind)
+        asm volatile("s_waitcnt lgkmcnt(8)"
+                     : "+v"(kf[0][0][0]), "+v"(kf[0][0][1]), "+v"(kf[0][1][0]), "+v"(kf[0][1][1]), "+v"(vf[0][0][0]), "+v"(vf[0][0][1]),
+                       "+v"(vf[0][1][0]), "+v"(vf[0][1][1])::"memory");
+      else
+        asm volatile("s_waitcnt lgkmcnt(0)"  // (and before the next tile overwrites)
+                     : "+v"(kf[1][0][0]), "+v"(kf[1][0][1]), "+v"(kf[1][1][0]), "+v"(kf[1][1][1]), "+v"(vf[1][0][0]), "+v"(vf[1][0][1]),
+                       "+v"(vf[1][1][0]), "+v"(vf[1][1][1])::"memory");
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
-        u32x4_t fk, fv;
-#pragma unroll
-        for (int r2 = 0; r2 < 4; ++r2) {
-          const int ta = 16 * s + 2 * (2 * r2) + g, tb = 16 * s + 2 * (2 * r2 + 1) + g;
-          const uint32_t klo = lds_k[ta * 64 + hh * 32 + j], khi = lds_k[tb * 64 + hh * 32 + j];
-          const uint32_t vlo = lds_v[ta * 64 + hh * 32 + j], vhi = lds_v[tb * 64 + hh * 32 + j];
-          fk[r2] = klo | (khi << 16);
-          fv[r2] = vlo | (vhi << 16);
-        }
-        accS[hh] = mfma_32x32x16<T>(fv, fk, accS[hh]);  // S[i][j] += sum_tok V[tok][i] K[tok][j]
+        const u32x4_t fk = {kf[hh][s][0].x, kf[hh][s][0].y, kf[hh][s][1].x, kf[hh][s][1].y};
+        accS[hh] = mfma_32x32x16<T>(u32x4_t{vf[hh][s][0].x, vf[hh][s][0].y, vf[hh][s][1].x, vf[hh][s][1].y}, fk,
+                                    accS[hh]);  // S[i][j] += sum_tok V[tok][i] K[tok][j]
         if (!PRE) {
 #pragma unroll
           for (int r2 = 0; r2 < 4; ++r2) accK[hh] = add_pk16<T>(fk[r2], accK[hh]);  // the "1" row of [V|1]
         }
       }
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // reads done before the next tile overwrites
   }
 
   // cross-wave reduction in LDS.  D layout of 32x32 MFMA: lane -> column j = lane%32,
@@ -738,12 +793,6 @@ __global__ __launch_bounds__(320) void linattn_apply32_partials_kernel(
 // the XCDs: 210 heads x 972 tokens 19.0 -> 16.8 us behind the GEMM that wrote them, 70 x 1024 12.0 -> 11.8).
 // ----------------------------------------------------------------------------
 constexpr int WHOLE_TOKENS = 1024;  // the most that one round of loads covers
-template <int OFF>
-__device__ __forceinline__ u32x2_t lds_read_tr16(uint32_t addr) {  // 4 tokens x 16 channels -> this lane's channel, 4 tokens
-  u32x2_t v;
-  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
-  return v;
-}
 
 // 16-bit io.  grid: B * h * R; block 512: R workgroups form the state of a head each for itself and share its queries.  The state is formed by the sums of linattn_state16_kernel and its reduction, in their
 // order (at most 256 heads: always splits of 256 tokens), so that the result is that of the two calls bit for bit: "chain" c is

@@ -192,3 +192,20 @@ def test_fp32_splits_of_any_length_and_row_distance(cuda, N):
         wide = torch.full(((N + 1) * ld,), float("nan"), device=cuda)[:N * ld].view(1, N, ld)
         wide[:, :, :C], wide[:, :, C:2 * C] = k, v
         assert torch.equal(ops.linattn_state(wide[:, :, :C], wide[:, :, C:2 * C]), near)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N,h", [(1, 3), (31, 2), (33, 5), (159, 3), (290, 1)])
+def test_16_bit_splits_of_any_length_and_row_distance(cuda, N, h, dtype):
+    """Phase 1 in 16 bits with 32-bit offsets, and on rows too far apart for those, against 64 bits and each other; nothing between the
+    rows, behind the last channel of an odd head or behind the last token (NaN) is read."""
+    C, gen = 32 * h, torch.Generator().manual_seed(N + h)
+    k, v = (torch.randn(1, N, C, generator=gen).to(dtype).to(cuda) for _ in range(2))
+    want = torch.einsum("nhi,nhj->hij", v[0].double().view(N, h, 32), k[0].double().clamp(min=0).view(N, h, 32))
+    near = ops.linattn_state(k, v)
+    assert _rel(near.view(h, 33, 32)[:, :32], want) < 1e-6
+    assert _rel(near.view(h, 33, 32)[:, 32], k[0].double().clamp(min=0).sum(0).view(h, 32)) < 1e-6
+    for ld in [2 * C + 8] + ([1 << 24] if N <= 33 else []):
+        wide = torch.full(((N + 1) * ld,), float("nan"), dtype=dtype, device=cuda)[:N * ld].view(1, N, ld)
+        wide[:, :, :C], wide[:, :, C:2 * C] = k, v
+        assert torch.equal(ops.linattn_state(wide[:, :, :C], wide[:, :, C:2 * C]), near)
