@@ -287,9 +287,11 @@ __device__ __forceinline__ int xcd_eighths(int id, int total) {  // workgroup ->
 }
 // Short splits are one round trip behind what comes in front of their loads: with a 64-bit product and a clamp each, 64 loads went
 // out over more than a microsecond.  us, whole calls, before (the phase 2 on partial states with its divisions first) / now, inputs from
-// HBM: 1024 x 36 17.8 / 15.3 (from the caches 14.9 / 13.4), 400 x 70 14.3 / 12.9, 2 x 1024 x 36 22.5 / 19.8, 3 x 3000 x 36 67 / 56,
-// 16384 x 36 99 / 90, 4 x 5000 x 70 224 / 199.
-template <bool LINEAR>
+// HBM: 1024 x 36 17.7 / 15.1 (from the caches 14.9 / 13.4), 400 x 70 14.0 / 12.5, 2 x 1024 x 36 22.4 / 19.8, 4 x 1737 x 36 46.4 / 45.7, 3 x 3000 x 36 68 / 58,
+// 16384 x 36 99 / 89, 4 x 5000 x 70 224 / 207.
+// FAR: rows too far apart for 32-bit offsets, an instance of its own: both ways in one kernel take the registers of a fourth workgroup per compute
+// unit, of which plan_state's 1000 or so of a few thousand tokens need all (4 x 1500 x 36 45.5, so 42.5).
+template <bool LINEAR, bool FAR>
 __global__ __launch_bounds__(256) void linattn_state32_kernel(
     const float* __restrict__ K, const float* __restrict__ V, float* __restrict__ dst,
     const int32_t* __restrict__ chunk_starts, int N, int h, int n_chunks, int nsplit, int split_tokens,
@@ -321,7 +323,7 @@ __global__ __launch_bounds__(256) void linattn_state32_kernel(
     }
   };
   using U32 = std::integral_constant<int, 32>;  // 64 tokens in flight per wave: a small input is one round trip
-  if ((int64_t)(split_tokens + 64) * stride_n < (1 << 29)) {  // 32-bit offsets; rows past t1 lie outside the resources: zeros
+  if constexpr (!FAR) {  // 32-bit offsets; rows past t1 lie outside the resources: zeros
     const int ld = (int)stride_n * 4, span = n > 0 ? (n - 1) * ld + 4 * D : 0;
     const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kp), 0, span, 0x00020000);
     const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vp), 0, span, 0x00020000);
@@ -1215,7 +1217,8 @@ static int state_impl(const void* k, const void* v, float* state, void* workspac
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (io_dtype == SANA_DT_F32) {
     dim3 grid(pl.nsplit, n_chunks, B * ((h + 3) / 4));
-    hipLaunchKernelGGL(linattn_state32_kernel<false>, grid, dim3(256), 0, s, static_cast<const float*>(k),
+    const bool far = (int64_t)(pl.split_tokens + 64) * stride_n >= (1 << 29);  // beyond the 32-bit offsets
+    hipLaunchKernelGGL((far ? linattn_state32_kernel<false, true> : linattn_state32_kernel<false, false>), grid, dim3(256), 0, s, static_cast<const float*>(k),
                        static_cast<const float*>(v), dst, chunk_starts, N, h, n_chunks, pl.nsplit,
                        pl.split_tokens, stride_b, stride_n);
   } else {
@@ -1497,7 +1500,8 @@ extern "C" __attribute__((visibility("default"))) int sana_hip_linattn(
     if (io_dtype == SANA_DT_F32 && N <= WHOLE_TOKENS && pl.nsplit > 1 && pl.nsplit <= 16 && heads * N <= (144 << 10)) {
       float* partial = reinterpret_cast<float*>(static_cast<char*>(scratch) + at);
       hipStream_t st = static_cast<hipStream_t>(stream);
-      hipLaunchKernelGGL(linattn_state32_kernel<true>, dim3(pl.nsplit * B * ((h + 3) / 4)), dim3(256), 0, st, static_cast<const float*>(k),
+      const bool far = (int64_t)(pl.split_tokens + 64) * stride_n >= (1 << 29);  // beyond the 32-bit offsets
+      hipLaunchKernelGGL((far ? linattn_state32_kernel<true, true> : linattn_state32_kernel<true, false>), dim3(pl.nsplit * B * ((h + 3) / 4)), dim3(256), 0, st, static_cast<const float*>(k),
                          static_cast<const float*>(v), partial, nullptr, N, h, 1, pl.nsplit, pl.split_tokens, stride_b, stride_n);
       if (hipGetLastError() != hipSuccess) return SANA_ERR_LAUNCH;
       hipLaunchKernelGGL(linattn_apply32_partials_kernel, dim3((N + 127) / 128 * (unsigned)heads), dim3(320), 0, st,
