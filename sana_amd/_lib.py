@@ -29,8 +29,9 @@ class BlockArgs(ctypes.Structure):
         (n, c_float) for n in ("eps_norm1", "eps_norm2", "eps_attn", "cross_scale")]
 
 
-# its fields in order ("0q": padded at the end as the structure is)
-BLOCK_ARGS = struct.Struct("@26PN3q11i4f0q")
+# its fields in order, packed in one call ("0q": padded at the end as the structure is)
+BLOCK_ARGS = struct.Struct("@" + "".join({c_void_p: "P", c_size_t: "N", c_int64: "q", c_int: "i", c_float: "f"}[t]
+                                         for _, t in BlockArgs._fields_) + "0q")
 assert BLOCK_ARGS.size == ctypes.sizeof(BlockArgs)
 
 # name -> (restype, argtypes); must list every symbol include/sana_hip.h declares

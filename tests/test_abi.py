@@ -210,3 +210,49 @@ def test_gemm_qkv_state_refuses_bad_arguments_before_any_launch():
 def test_which_int8_weights_are_expanded(M, N, K, expand):
     """Narrow outputs that are not split, a second round of int8 tiles, more than six token tiles on long rows of weights."""
     assert _lib.load().sana_hip_gemm_w8_expand(M, N, K) == expand
+
+
+def test_packed_block_arguments_are_the_structure():
+    """A value of its own for each field, packed in the fields' order, is read back under each field's name."""
+    names = [n for n, _ in _lib.BlockArgs._fields_]
+    values = [float(1 + i) if t is ctypes.c_float else 1 + i for i, (_, t) in enumerate(_lib.BlockArgs._fields_)]
+    args = _lib.BlockArgs.from_buffer_copy(_lib.BLOCK_ARGS.pack(*values))
+    assert [getattr(args, n) for n in names] == values
+
+
+def test_the_block_call_fills_each_field(monkeypatch):
+    """ops.block against the structure by name (a stand-in library: nothing is launched)."""
+    import torch
+
+    from sana_amd import ops
+
+    seen = {}
+
+    class Lib:
+        def sana_hip_block_scratch_bytes(self, ref):
+            return 64
+
+        def sana_hip_block(self, ref, stream):
+            a = ref._obj
+            seen.update({n: getattr(a, n) for n, _ in _lib.BlockArgs._fields_})
+            return 0
+
+    monkeypatch.setattr(_lib, "load", lambda: Lib())
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    B, H, W, C, Nk, hid, heads = 2, 3, 5, 64, 7, 160, 4
+    x, kv, mod = torch.zeros(B, H * W, C, dtype=torch.float16), torch.zeros(B, Nk, 3, 2 * C, dtype=torch.float16)[:, :, 1], \
+        torch.zeros(B, 6, C, dtype=torch.float16)
+    bias, ones, weights = torch.zeros(B, Nk), torch.ones(C), list(range(101, 115))
+    weights[1] = 0                                # qkv without a bias
+    out = ops.block(x, kv, bias, mod, weights, ones, hid, heads, (H, W), True, 1e-6, 2e-6, 1e-8)
+    m = mod.data_ptr()
+    want = dict(x=x.data_ptr(), text_kv=kv.data_ptr(), shift_msa=m, scale_msa=m + 2 * C, gate_msa=m + 4 * C, shift_mlp=m + 6 * C,
+                scale_mlp=m + 8 * C, gate_mlp=m + 10 * C, ones=ones.data_ptr(), key_bias=bias.data_ptr(), out=out.data_ptr(),
+                scratch_bytes=64, text_ld=6 * C, key_bias_ld=Nk, mod_stride=6 * C, B=B, N=H * W, C=C, hidden=hid, cross_heads=heads,
+                text_len=Nk, H=H, W=W, round_like_reference=1, split_k=1 if ops.SPLIT_K else 0, io_dtype=_lib.DT_F16)
+    want.update(zip(("qkv_w", "qkv_b", "proj_w", "proj_b", "q_w", "q_b", "o_w", "o_b", "inv_w", "inv_b", "dw_w", "dw_b", "point_w",
+                     "point_b"), [w or None for w in weights]))
+    floats = dict(eps_norm1=1e-6, eps_norm2=2e-6, eps_attn=1e-8, cross_scale=0.25)
+    assert {n: seen[n] for n in want} == want and seen["scratch"]
+    assert all(seen[n] == pytest.approx(v, rel=1e-6) for n, v in floats.items())
+    assert set(want) | set(floats) | {"scratch"} == set(seen)
