@@ -31,9 +31,6 @@
 #ifndef SANA_LA_APPLY_TOKENS
 #define SANA_LA_APPLY_TOKENS 128
 #endif
-#ifndef SANA_LA_NT_LOAD
-#define SANA_LA_NT_LOAD 0
-#endif
 #ifndef SANA_LA_NT_STORE
 #define SANA_LA_NT_STORE 0
 #endif
@@ -146,8 +143,8 @@ __global__ __launch_bounds__(256) void linattn_state16_kernel(
     for (int i = 0; i < 4; ++i) {
       const int tok = tile + ld_tok + 8 * i;
       if (ch_ok && tok < t1) {
-        kreg[i] = load_stream<SANA_LA_NT_LOAD != 0>(reinterpret_cast<const u32x4_t*>(kbase + (int64_t)tok * stride_n));
-        vreg[i] = load_stream<SANA_LA_NT_LOAD != 0>(reinterpret_cast<const u32x4_t*>(vbase + (int64_t)tok * stride_n));
+        kreg[i] = *reinterpret_cast<const u32x4_t*>(kbase + (int64_t)tok * stride_n);
+        vreg[i] = *reinterpret_cast<const u32x4_t*>(vbase + (int64_t)tok * stride_n);
         if (has_norm) rin[i] = pre.rinv[(int64_t)b * N + tok];
         if (has_rope) {
           const float* rp = pre.rope + ((int64_t)tok * 16 + (lane & 3) * 4) * 2;
