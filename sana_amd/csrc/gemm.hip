@@ -1294,9 +1294,9 @@ SANA_API int sana_hip_tconv_residual(const void* X, const void* W, void* out, in
   // one of the three widest tiles: the others have no taps
   const int k = taps * C;
   const bool brief = k < kShortK, may288 = ldw < kMaxStride288;
-  // (192 channels: with the residual the epilogue is still what it was before its rows were shared)
-  constexpr Tile16 gated192 = {256, 192, 256, 32, 256, 7.9, 0.628, 1.150};
-  const double us192 = cost16(brief ? kTilesShort[1] : gated192, M, C, k);
+  // (192 channels at the price that they have in every GEMM; with 7.9, what its fixed part was, / so: 39680 x 1152 taken from 288 channels 265 / 252,
+  // 50160 x 1152 320 / 316, 55760 x 1536 from 256 channels 606 / 596; 27 shapes 0.96 .. 1.00; at 2240 channels the choice is the same)
+  const double us192 = cost16(brief ? kTilesShort[1] : kTiles16[kTile192], M, C, k);
   const double us256 = cost16(brief ? kTilesShort[2] : kTiles16[kTile256], M, C, k), us = std::min(us192, us256);
   if (may288 && (brief ? short_takes_288(M, C, k, us) : cost16(kTiles16[kTile288], M, C, k) < us))
     return gemm288_launch(x, w, e, o, M, C, k, ldx, ldw, ldo, SANA_EPI_GATE_RES, false, &tp, s);
