@@ -399,3 +399,22 @@ def test_workgroups_of_several_heads(cuda, B, N, H, d, Nk, dtype):
         assert torch.equal(got[b], ops.cross_attention16(q[b:b + 1], kv[b:b + 1], H, bias[b:b + 1])[0])
     ref = formula(q[-1:].cpu(), kv[-1:].cpu(), H, bias[-1:].cpu())
     assert rel_l2(got[-1:].cpu(), ref) <= 1e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,N,H,d,Nk,masked", [(1, 70, 2, 112, 161, False), (1, 70, 2, 72, 161, True), (3, 600, 20, 112, 31, True),
+                                               (3, 600, 20, 72, 31, False), (2, 1100, 15, 88, 165, True)])
+def test_far_keys_of_many_heads(cuda, dtype, B, N, H, d, Nk, masked):
+    """Rows of K and V too far apart for 32-bit offsets: both numbers of key tiles, biases, and workgroups of two items that stage the
+    keys of a second head or batch entry over the first ones (from 257 items on): the bits of dense rows."""
+    assert Nk > 160 or B * H * (-(-N // 128)) > 256
+    gen = torch.Generator(device=cuda).manual_seed(Nk + d)
+    C, ld = H * d, 1 << 21
+    q = torch.randn(B, N, C, generator=gen, device=cuda).to(dtype)
+    kv = torch.randn(B, Nk, 2 * C, generator=gen, device=cuda).to(dtype)
+    bias = torch.where(torch.rand(B, Nk, generator=gen, device=cuda) < 0.3, -10000.0, 0.0) if masked else None
+    rows = torch.full((B * Nk * ld,), float("nan"), dtype=dtype, device=cuda).view(B, Nk, ld)
+    rows[:, :, :2 * C] = kv
+    dense = ops.cross_attention16(q, kv, H, bias)
+    assert bool(torch.isfinite(dense).all())
+    assert torch.equal(ops.cross_attention16(q, rows[:, :, :2 * C], H, bias), dense)
