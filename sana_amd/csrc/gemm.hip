@@ -920,24 +920,27 @@ struct Plan16 {
 // the cheapest tile, or two widths where their last rounds fill better (4096 x 6720 tokens x channels, K = 2240: 432 tiles of 256
 // are 1.7 rounds, 15 x 16 and 15 x 16 tiles of the mix two that are 94 % full) by more than what the fit tells apart
 template <size_t TILES>
-Plan16 cheapest16(const Tile16 (&tiles)[TILES], const Tile16& t256, const Tile16& t192, double mix_below, int M, int N, int K) {
+Plan16 cheapest16(const Tile16 (&tiles)[TILES], const Tile16& t256, const Tile16& t192, double mix_below, double mix_below_288, int M, int N, int K) {
   Plan16 p = {&tiles[0], 0, 0, 1e30};
   for (const Tile16& t : tiles) {
     const double us = cost16(t, M, N, K);
     if (us < p.us) p.tile = &t, p.us = us;
   }
-  const double single = p.us;
+  const double below = (p.tile->bn == 288 ? mix_below_288 : mix_below) * p.us;
   for (int a = 256; a < N; a += 256) {
     const double us = cost16(t256, M, a, K) + cost16(t192, M, N - a, K);
-    if (us < mix_below * single && us < p.us) p.n_wide = a, p.us = us;
+    if (us < below && us < p.us) p.n_wide = a, p.us = us;
   }
   const bool halved = p.tile->bm == 64 && p.tile->bn == 64 && (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= kHalvedTiles;
   p.bn = p.n_wide ? 256 : halved ? 32 : p.tile->bn;
   return p;
 }
-Plan16 plan16(int M, int N, int K) {
-  if (K >= kShortK) return cheapest16(kTiles16, kTiles16[kTile256], kTiles16[kTile192], 0.992, M, N, K);
-  const Plan16 p = cheapest16(kTilesShort, kTilesShort[2], kTilesShort[1], 0.98, M, N, K);
+// gated: with a residual, two widths take the place of 288 channels by 2 % at least: both launches' epilogues wait for it.  us, two widths by 0.8 % /
+// so: 31676 x 2240 x 2240 286 / 274, 39680 x 2240 x 5600 946 / 830, 26420 x 3912 x 5504 928 / 890, 24455 x 2224 x 2368 225 / 223; 17757 x 4800 x 5248 689 / 702;
+// 0.978 on the mean of 40 shapes.  Without one they are the faster ones: 31250 x 2240 x 2240 238, 288 channels 247.
+Plan16 plan16(int M, int N, int K, bool gated = false) {
+  if (K >= kShortK) return cheapest16(kTiles16, kTiles16[kTile256], kTiles16[kTile192], 0.992, gated ? 0.98 : 0.992, M, N, K);
+  const Plan16 p = cheapest16(kTilesShort, kTilesShort[2], kTilesShort[1], 0.98, 0.98, M, N, K);
   return short_takes_288(M, N, K, p.us) ? Plan16{&kShort288, 288, 0, cost16(kShort288, M, N, K)} : p;
 }
 // Split over k, or not: the split GEMM against the best unsplit one (16-bit and int8 weights decide alike, so that they
@@ -1048,7 +1051,7 @@ int launch(const void* A, const void* W, const float* scale, const EpiArgs& ep, 
     return launch_split<W8, T>(a, W, scale, ep, c, M, N, K, lda, ldw, ldc, epilogue, s, pl, ws);
   if constexpr (!W8) {
     const uint16_t* w = static_cast<const uint16_t*>(W);
-    const Plan16 p = plan16(M, N, K);
+    const Plan16 p = plan16(M, N, K, epilogue == SANA_EPI_GATE_RES);
     if (p.n_wide) {
       const int rc = gemm8_launch(a, w, ep, c, M, p.n_wide, K, lda, ldw, ldc, epilogue, is_f16<T>, 4, nullptr, s);
       if (rc != SANA_OK) return rc;
