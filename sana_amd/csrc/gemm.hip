@@ -935,11 +935,13 @@ Plan16 cheapest16(const Tile16 (&tiles)[TILES], const Tile16& t256, const Tile16
   p.bn = p.n_wide ? 256 : halved ? 32 : p.tile->bn;
   return p;
 }
-// gated: with a residual, two widths take the place of 288 channels by 2 % at least: both launches' epilogues wait for it.  us, two widths by 0.8 % /
-// so: 31676 x 2240 x 2240 286 / 274, 39680 x 2240 x 5600 946 / 830, 26420 x 3912 x 5504 928 / 890, 24455 x 2224 x 2368 225 / 223; 17757 x 4800 x 5248 689 / 702;
-// 0.978 on the mean of 40 shapes.  Without one they are the faster ones: 31250 x 2240 x 2240 238, 288 channels 247.
+// gated: with a residual, two widths take the place of 288 channels by 4 % at least: both launches' epilogues wait for it.  us, two widths / 288
+// channels, weights cold, by how far the estimates are apart: 0.8 - 2 % 31676 x 2240 x 2240 286 / 274, 39680 x 2240 x 5600 946 / 830, 24455 x 2224 x 2368 225 /
+// 223, 17757 x 4800 x 5248 689 / 702, 1.02 on the mean of 40 shapes; 2 - 4 % 38042 x 2240 x 5600 905 / 801, 17604 x 4968 x 3584 512 / 505, 30494 x 3112 x 5440 872 /
+// 841, 1.03 of 22; beyond a tie with cold rows too (1.01 of 38) and 36897 x 2240 x 2240 323 / 335 without.  With no residual they are the faster ones:
+// 31250 x 2240 x 2240 238 / 247.
 Plan16 plan16(int M, int N, int K, bool gated = false) {
-  if (K >= kShortK) return cheapest16(kTiles16, kTiles16[kTile256], kTiles16[kTile192], 0.992, gated ? 0.98 : 0.992, M, N, K);
+  if (K >= kShortK) return cheapest16(kTiles16, kTiles16[kTile256], kTiles16[kTile192], 0.992, gated ? 0.96 : 0.992, M, N, K);
   const Plan16 p = cheapest16(kTilesShort, kTilesShort[2], kTilesShort[1], 0.98, 0.98, M, N, K);
   return short_takes_288(M, N, K, p.us) ? Plan16{&kShort288, 288, 0, cost16(kShort288, M, N, K)} : p;
 }
