@@ -871,6 +871,16 @@ constexpr Tile16 kTiles16[] = {
     {160, 192, 256, 32, 256, 7.4, 0.487, 0.975, true},
 };
 constexpr int kTile192 = 7, kTile256 = 8, kTile288 = 9;
+// The same for K % 32, where rows that follow one another straddle the 64-byte sectors, with no residual: the price that the 192-wide tile had
+// before (above), which keeps such GEMMs in 256 or 288 channels; two widths read the rows of A twice.  us, 4.9 / 7.9, weights cold: 6893 x 4016 x 2064
+// 119 / 107 (but x 2048 99 / 97), 12506 x 5144 x 4584 511 / 476, 17278 x 3928 x 1200 177 / 145, 4502 x 11456 x 1656 165 / 148, 28755 x 1128 x 1264 85 / 75;
+// one round of 192 the slower way: 2100 x 5280 x 1072 28 / 31; 0.963 on the mean of the 100 shapes timed.  With a residual 4.9 gains there too (0.98 of 37).
+constexpr auto kTilesStraddling = [] {
+  struct { Tile16 t[sizeof(kTiles16) / sizeof(Tile16)]; } r = {};
+  for (size_t i = 0; i < sizeof(kTiles16) / sizeof(Tile16); ++i) r.t[i] = kTiles16[i];
+  r.t[kTile192].fixed = 7.9;
+  return r;
+}();
 // K below 1024.  These are the times that the tiles had in GEMMs of K = 1152 .. 5600 before the loop over whole k-tiles; at such K
 // no other loop runs, and 256 x 128 is gemm8_kernel's there.  As times they are up to 30 % off (epilogues and the fill of the rings are most of
 // a launch), as a choice they serve: of 560 shapes (64 .. 24576 tokens, 320 .. 6144 channels, K 64 .. 960, the ten tiles forced in turn)
@@ -941,6 +951,8 @@ Plan16 cheapest16(const Tile16 (&tiles)[TILES], const Tile16& t256, const Tile16
 // 841, 1.03 of 22; beyond a tie with cold rows too (1.01 of 38) and 36897 x 2240 x 2240 323 / 335 without.  With no residual they are the faster ones:
 // 31250 x 2240 x 2240 238 / 247.
 Plan16 plan16(int M, int N, int K, bool gated = false) {
+  if (K >= kShortK && K % 32 && !gated)
+    return cheapest16(kTilesStraddling.t, kTilesStraddling.t[kTile256], kTilesStraddling.t[kTile192], 0.992, 0.992, M, N, K);
   if (K >= kShortK) return cheapest16(kTiles16, kTiles16[kTile256], kTiles16[kTile192], 0.992, gated ? 0.96 : 0.992, M, N, K);
   const Plan16 p = cheapest16(kTilesShort, kTilesShort[2], kTilesShort[1], 0.98, 0.98, M, N, K);
   return short_takes_288(M, N, K, p.us) ? Plan16{&kShort288, 288, 0, cost16(kShort288, M, N, K)} : p;

@@ -256,3 +256,12 @@ def test_the_block_call_fills_each_field(monkeypatch):
     assert {n: seen[n] for n in want} == want and seen["scratch"]
     assert all(seen[n] == pytest.approx(v, rel=1e-6) for n, v in floats.items())
     assert set(want) | set(floats) | {"scratch"} == set(seen)
+
+
+@pytest.mark.parametrize("M,N,K,straddling", [(6893, 4016, 2048, 2064), (12506, 5144, 4544, 4584), (13663, 1760, 1280, 1304),
+                                              (17278, 3928, 1184, 1200)])
+def test_rows_that_straddle_sectors_are_not_read_in_two_widths(M, N, K, straddling):
+    """K % 32: one launch of 256 or 288 channels where k of whole sectors takes two widths."""
+    plan = (ctypes.c_int * 4)()
+    assert _lib.load().sana_hip_gemm_plan(M, N, K, plan) == 0 and plan[2] > 0
+    assert _lib.load().sana_hip_gemm_plan(M, N, straddling, plan) == 0 and plan[1] in (256, 288) and plan[2:] == [0, 1]
