@@ -850,18 +850,22 @@ struct Tile16 {
 };
 // Fitted to 250 shapes (64 .. 32760 tokens, the eight projections of the two image widths and the text's, one block's and a
 // step's, weights cold, launches replayed from a graph: issued one by one, a launch of less than 20 us is timed by its issue):
-// 7 - 14 % off each.  Of 304 shapes timed since with every tile (profiles/gemm_tiles_by_shape.txt) the choice is 1.1 % from the
-// best on the mean, more than 6 % in ten.  In a second round
+// 7 - 14 % off each.  Of 304 shapes timed with every tile as it is now (profiles/gemm_tiles_by_shape.txt) the choice is 0.6 % from the
+// best on the mean, more than 6 % in seven; of 124 at random token counts 0.6 %, more than 6 % in one.  In a second round
 // the small tiles were never more than 2 % ahead, and 300 x 17920 x 2240 is 48.7 us in 128 x 128 and 40.4 in 256 x 192: hence
 // one_round.  us, the tiles and kernels before this table / now, both timed so: 256 x 1152 x 2880 15.3 / 10.3 (halved), 1024 x 2240 x
 // 2240 23.6 / 18.7, 2048 x 1152 x 2880 28.6 / 21.6, 4096 x 1152 x 1152 20.7 / 17.7, 4096 x 1152 x 2880 35.0 / 31.4.
 // The 192-wide tile's fixed part was 7.9 before the waves shared its rows (gemm8.h).  With 4.9, of the shapes that this changes (200 ..
 // 20000 tokens, widths as above), kernel as it is, 7.9 / 4.9: 14208 x 3456 x 1152 109 / 98, 16576 x 2240 x 2240 167 / 157, 7246 x 9216 x 1152 140 /
 // 133, 6017 x 11200 x 2240 251 / 241, 2079 x 18432 x 1152 88 / 84, 12423 x 2240 x 2240 115 / 111; 18219 x 9216 x 1152 307 / 311, 6400 x 6720 x 2240
-// 145 / 151; 0.979 on the mean of 48.  (3.9: 993 x 18432 x 1152 42.7 / 48.1.)
-// 160 x 192 is chosen between 257 and 320 tokens where both of its rows of tiles run in one round, the tiles of 256 rows padding two fifths and
-// the smaller ones taking two rounds; 256 x 192 / so, weights cold: 260 x 17920 x 2240 39.2 / 33.7, 288 x 18432 x 1152 25.1 / 20.7, 300 x 24000 x 1152 26.2 / 22.6,
-// 320 x 24000 x 3072 60.7 / 54.7, 300 x 20480 x 1536 with a gate 34.0 / 31.6.
+// 145 / 151; 0.979 on the mean of 48.  (Against the former kernel at its price those two are ties, 313 / 312 and 151 / 151.  3.9: 993 x 18432 x
+// 1152 42.7 / 48.1.)
+// 160 x 192 is chosen where one, two, four or five rows of its tiles are one round, and the rows of 256 would be padded by two fifths and
+// more, smaller tiles take two rounds: 71 .. 160 tokens from 32800 channels, 257 .. 320 from 16500, 519 .. 640 from 10900 (K > 4096), 771 .. 799 from
+// 8300 (K > 2800).  us, the best other tile / so, weights cold: 150 x 46080 x 2240 47.1 / 42.8, 260 x 17920 x 2240 39.2 / 33.7, 300 x 24000 x 1152 26.2 / 22.6,
+// 300 x 20480 x 1536 with a gate 34.0 / 31.6, 519 x 10960 x 4608 74.0 / 55.5, 784 x 9216 x 4096 58.5 / 52.4; 0.75 .. 1.00 of it at 247 such shapes; 57 of K =
+// 5600, whose rows are 87.5 lines of 128 bytes, 0.88 .. 1.10 (784 x 9216 x 5600 83.6 / 92.4).  A prompt's 300 tokens take it for the keys and values of 8 blocks
+// of 1152 channels or 4 of 2240; for those of 28 and 20 256 channels or two widths are faster (55.5 / 57.5, 134.6 / 137.1) and chosen.
 constexpr Tile16 kTiles16[] = {
     {64, 64, 512, 256, 257, 3.0, 0.288, 0.503, true, 0.165, 0.26}, {64, 128, 256, 32, 256, 3.9, 0.350, 0.414, true},
     {96, 128, 256, 32, 256, 3.7, 0.439, 0.466, true},  {128, 128, 256, 32, 256, 3.9, 0.454, 0.541, true},
@@ -958,9 +962,9 @@ Plan16 plan16(int M, int N, int K, bool gated = false) {
   return short_takes_288(M, N, K, p.us) ? Plan16{&kShort288, 288, 0, cost16(kShort288, M, N, K)} : p;
 }
 // Split over k, or not: the split GEMM against the best unsplit one (16-bit and int8 weights decide alike, so that they
-// keep giving the same bits).  Time of the split one: fitted to 49 shapes, 4 % off.  The unsplit tiles' fit is 3 - 13 % low at
-// the K of 5600 where it is taken (their weights come from HBM for longer than the prefetch reaches): 1024 x 2240 x 5600 is 46 us
-// either way, 256 x 2240 x 5600 30 split and 34 not.
+// keep giving the same bits).  Time of the split one: fitted to 49 shapes when gemm4_kernel ran the ranges; gemm8_kernel's are 3 - 8 % longer with
+// cold weights (42.3 estimated, 46.1 taken at 1024 x 2240 x 5600).  So is the unsplit tiles' fit, by 3 - 13 %, at the K of 5600 where it is taken (their
+// weights come from HBM for longer than the prefetch reaches): 1024 x 2240 x 5600 is 46 us either way, 256 x 2240 x 5600 30 split and 34 not, 1560 58 and 53.
 // A split GEMM adds up short chains, so that its fp32 sums are closer to the 64-bit ones than those of one chain: 2240 x 5600, rms error
 // 1.0e-7 of the result in eight ranges, 2.4e-7 in one.  Precision is not given up for time: where the split was the faster one
 // against the tiles as they once were (kTilesShort, their times then), k stays in ranges though some tiles have become faster since.

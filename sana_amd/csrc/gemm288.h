@@ -14,11 +14,11 @@ __device__ __forceinline__ u32x2_t g288_read2(uint32_t addr) {
   return v;
 }
 
-// What bounds it: the matrix pipes' power where the rounds are full (16384 x 2240 x 5600: 308 us = 1.34 PFLOP/s with the gated
-// residual at 1.76 GHz; 192-wide tiles, which it replaced there, 352), else the half phases: a k-tile takes 2525 cycles for 2304
-// of MFMAs (2750 with the gated residual).  What is not k-tiles -- first loads and epilogue -- is 23 k cycles a tile with a bias,
-// 29 k with the gated residual, of 270 k at K = 5600: the whole chip reads its residual and writes its rows at once, at memory
-// rate.  (Counters at K = 2240 and 5600: profiles/kernels_cfg3_mfma_util.txt.)
+// What bounds it: the matrix pipes' power where the rounds are full (16384 x 2240 x 5600: 306 us = 1.34 PFLOP/s with the gated
+// residual at 1.88 GHz; 192-wide tiles, which it replaced there, 352), else the half phases: a k-tile takes 2670 cycles for 2304
+// of MFMAs (3120 with the gated residual, at a higher clock).  What is not k-tiles -- first loads and epilogue -- is 11 k cycles a
+// tile with a bias, 15 k with the gated residual, of 245 k and 288 k at K = 5600: the whole chip reads its residual and writes its rows at
+// once, at memory rate.  (Counters at K = 2240 and 5600: profiles/kernels_cfg3_mfma_util.txt.)
 //
 // Waves (wm, wn) = (wave % 4, wave / 4): 64 tokens x 144 channels each = 4 x 9 tiles of v_mfma_f32_16x16x32 (the weight tile
 // is the row operand: a lane owns one token and, by the order in which weight rows are placed in LDS, 8 contiguous channels

@@ -90,7 +90,7 @@ int gemm_ring_launch(const uint16_t* a, const uint16_t* w, const EpiArgs& ep, ui
   // workgroups the chip then lowers its clock for what runs beside it as well: a step with int8 weights at 2048 rows takes 1721 us
   // with that loop and 1642 with this one, at 1160 and 1245 W.
   SANA_RING(4, 1, 2, 10, 4, false, false);
-  // 160 x 192: the 300 tokens of a prompt by the keys and values of all blocks, two tiles of 256 rows a fifth longer than these.  us, weights
+  // 160 x 192: the 300 tokens of a prompt by the keys and values of a few blocks, two tiles of 256 rows a fifth longer than these.  us, weights
   // cold (each call others, tokens the same): 300 x 18432 x 1152 25.4 / 22.4 (23.7 / 20.5), 300 x 17920 x 2240 41.5 / 36.6 (37.7 / 33.9).  In 320 x 96,
   // with more operand bytes, 23.3 and 39.4; in 2 x 6 waves 23.2 and 36.6.
   SANA_RING(2, 2, 5, 6, 3, false, false);
