@@ -66,35 +66,23 @@ __device__ __forceinline__ uint32_t dequant2(uint32_t q4, int which, float s, fl
 }
 
 // int8 weight [N][K] + per-row scale -> bf16 [N][K], with the rounding of dequant2: the expansion the GEMM's
-// int8 path performs on its way to LDS, as a streaming kernel of its own.  A wave takes a row, a lane 8 values (a store instruction is
-// 1 KB in a row), six of them requested at once: no division, whole sectors.  HBM bound.  us, 16 values a thread with a 64-bit division
-// for its row / so: 11200 x 2240 18.1 / 16.1, 6720 x 2240 11.9 / 9.7, 5760 x 1152 6.0 / 5.4, 2240 x 5600 8.9 / 8.8.
-// grid: ceil(N / 4); block 256.
+// int8 path performs on its way to LDS, as a streaming kernel of its own.  A wave takes 512 values of a row, a lane 8 (a store instruction is
+// 1 KB in a row): no division, whole sectors.  HBM bound; short rows by latency, for which a wave is to have one round trip: with a whole row a wave, six
+// pieces a lane requested at once, it was the longer way for narrow weights.  us, 16 values a thread with a 64-bit division for its row / a row a wave / so:
+// 504 x 2208 2.8 / 3.4 / 2.6, 1152 x 1152 2.9 / 3.2 / 2.7, 1152 x 2880 4.5 / 5.1 / 4.0, 2240 x 5600 11.2 / 11.9 / 10.0, 5760 x 1152 7.1 / 6.5 / 6.8, 6720 x 2240 12.9 /
+// 11.2 / 11.2, 11200 x 2240 19.6 / 17.9 / 16.3.
+// grid: ceil(K / 512), rows by four in y and, 2^15 of them each, z; block 256.
 __global__ __launch_bounds__(256) void dequant_w8_kernel(const int8_t* __restrict__ wq, const float* __restrict__ scale,
                                                          uint16_t* __restrict__ out, int N, int K, int64_t ldw,
                                                          int64_t ldo) {
-  constexpr int U = 6;
-  const int n = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (n >= N) return;
-  const int pieces = K >> 3;
-  const char* row = reinterpret_cast<const char*>(wq + n * ldw);
-  char* orow = reinterpret_cast<char*>(out + n * ldo);
+  const uint32_t n = (blockIdx.z << 15 | blockIdx.y) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t p = blockIdx.x * 64 + (threadIdx.x & 63);
+  if (n >= (uint32_t)N || p >= (uint32_t)K >> 3) return;
+  const u32x2_t q = *reinterpret_cast<const u32x2_t*>(wq + n * ldw + 8 * (int64_t)p);
   const float s = scale[n], off = -128.f * s;
-  for (int p0 = 0; p0 < pieces; p0 += 64 * U) {
-    u32x2_t q[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (p0 + 64 * u < pieces) q[u] = *reinterpret_cast<const u32x2_t*>(row + 8u * (uint32_t)min(p0 + 64 * u + lane, pieces - 1));
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int p = p0 + 64 * u + lane;
-      if (p < pieces) {
-        const uint32_t x = q[u].x ^ 0x80808080u, y = q[u].y ^ 0x80808080u;
-        *reinterpret_cast<u32x4_t*>(orow + 16u * (uint32_t)p) =
-            u32x4_t{dequant2(x, 0, s, off), dequant2(x, 1, s, off), dequant2(y, 0, s, off), dequant2(y, 1, s, off)};
-      }
-    }
-  }
+  const uint32_t x = q.x ^ 0x80808080u, y = q.y ^ 0x80808080u;
+  *reinterpret_cast<u32x4_t*>(out + n * ldo + 8 * (int64_t)p) =
+      u32x4_t{dequant2(x, 0, s, off), dequant2(x, 1, s, off), dequant2(y, 0, s, off), dequant2(y, 1, s, off)};
 }
 
 // Compiler-scheduled kernel for int8 weights, any K % 16 == 0.  Workgroup tile 64*TT tokens x 64*TC channels,
@@ -1331,7 +1319,8 @@ SANA_API int sana_hip_dequant_w8(const int8_t* Wq, const float* scale, void* W, 
   if (ldw < K || ldo < K) return SANA_ERR_ARG;
   if (ldw % 16 || ldo % 8 || !aligned16(Wq) || !aligned16(W)) return SANA_ERR_ALIGN;
   if ((int64_t)N * (K / 16) > (int64_t)0x7fffffff * 256) return SANA_ERR_SHAPE;
-  hipLaunchKernelGGL(dequant_w8_kernel, dim3((unsigned)(((int64_t)N + 3) / 4)), dim3(256), 0,
+  const unsigned rows = ((unsigned)N + 3) / 4, y = std::min(rows, 1u << 15);
+  hipLaunchKernelGGL(dequant_w8_kernel, dim3(((unsigned)K + 511) / 512, y, (rows + y - 1) / y), dim3(256), 0,
                      static_cast<hipStream_t>(stream), Wq, scale, static_cast<uint16_t*>(W), N, K, ldw, ldo);
   return hipGetLastError() == hipSuccess ? SANA_OK : SANA_ERR_LAUNCH;
 }

@@ -129,3 +129,12 @@ def test_expanded_weights_are_the_rounded_products(cuda, N, K):
     wq = torch.randint(-128, 128, (N, K + 16), generator=gen).to(torch.int8).to(cuda)[:, :K]
     scale = (0.001 + torch.rand(N, generator=gen)).to(cuda)
     assert torch.equal(ops.dequant_w8(wq, scale), (wq.float() * scale[:, None]).bfloat16())
+
+
+@pytest.mark.parametrize("N,K,ld", [(131069, 16, 16), (131073, 48, 64), (262150, 16, 32), (7, 520 * 16, 521 * 16), (3, 496, 496)])
+def test_int8_weights_of_many_rows_and_of_rows_apart_are_expanded(cuda, N, K, ld):
+    """More rows than one grid plane takes (2^17), fewer and more than 512 values a row, the last wave's lanes past it, rows apart."""
+    gen = torch.Generator().manual_seed(N)
+    wq = torch.randint(-127, 128, (N, ld), generator=gen, dtype=torch.int8).to(cuda)[:, :K]
+    scale = (0.001 + torch.rand(N, generator=gen)).to(cuda)
+    assert torch.equal(ops.dequant_w8(wq, scale), (wq.float() * scale[:, None]).bfloat16())
